@@ -249,11 +249,13 @@ int rumus_hip_f16_to_f32(const uint16_t* in, float* out, uint64_t numel,
  * row and eighth of K beyond), so single outlier channels of thousands of
  * sigma keep the tolerance.  The u4-zero-point decode entry point
  * (rumus_hip_qmatmul_int4_decode_zp4) does not make that exception and keeps
- * the plain bound.  Larger batches, and those the f16 tile kernel takes, keep
- * 22 bits of every element and add in f32.  That kernel is faster on tables
- * of integer zero-points (what AWQ and GPTQ checkpoints hold; it looks before
- * it multiplies): an eighth of its work at groups of 128, more at smaller
- * groups, exists only for their fractional part. */
+ * the plain bound.  Batches of more than 256 rows that the six-bit-float
+ * kernel takes (group_size % 64 == 0, k from 1024 to 16384, where it is the faster one)
+ * keep 24 bits below the largest of 32 consecutive k, and 39 where an
+ * eighth of those lies 2^8 or more below it.  The others, which the f16 tile
+ * kernel takes, keep 22 bits of every element and add in f32.  Both are
+ * faster on tables of integer zero-points (what AWQ and GPTQ checkpoints hold;
+ * they look first): part of the work exists only for their fractional part. */
 int rumus_hip_qmatmul_int4(const float* x, const uint32_t* packed,
                            const float* scales, const float* zero_points,
                            const float* bias, const int32_t* g_idx, float* y,

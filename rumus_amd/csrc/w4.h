@@ -80,9 +80,14 @@ uint32_t w4_decode_max_rows(uint32_t padded_k, uint32_t n);   // w4_gemv.hip
 int w4_launch_gemm(const W4Args& a, hipStream_t s);
 
 // int8 matrix cores for up to 128 rows (w4_gemm_i8.hip): group_size % 64 == 0, n % 4 == 0, 16-byte aligned
-// buffers, no g_idx.
-bool w4_gemm_i8_supported(const W4Args& a);
+// buffers, no g_idx.  Larger batches where an estimate says that it beats the f16 tiles; us: the faster one's estimate.
+bool w4_gemm_i8_supported(const W4Args& a, double* us = nullptr);
 int w4_launch_gemm_i8(const W4Args& a, hipStream_t s);
+
+// six-bit-float matrix cores for large batches (w4_gemm_f6.hip): whether they take the call (more than 256 rows, group_size % 64 == 0,
+// n % 4 == 0, 16-byte aligned buffers, no g_idx, and the faster kernel by estimate).
+bool w4_gemm_f6_chosen(const W4Args& a);
+int w4_launch_gemm_f6(const W4Args& a, hipStream_t s);
 
 // grad_x on the f16 matrix cores (w4_gemm_t.hip): group_size 32, 64 or a multiple of 128, n % 4 == 0, k % 4 == 0,
 // 16-byte aligned buffers.

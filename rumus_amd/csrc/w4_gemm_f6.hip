@@ -1,0 +1,884 @@
+// INT4 engine: dequant-fused GEMM on the six-bit-float matrix cores, for large batches.
+//
+//   y[m,n] = sum_g scale[g,n] * ( sum_{k in g} x[m,k] (q[k,n] - z[g,n])  -  rest[g,n] * sum_{k in g} x[m,k] )
+//
+// with z the zero-point's nearest integer (within 0..15) and rest = zp - z.  v_mfma_scale_f32_32x32x64_f8f6f4 runs
+// operands of six bits (e2m3: sign, 0 .. 7.5, integers up to 16 in units of 1/8 .. 1/2) at four times the f16 rate:
+//   - q - z is -15 .. 15: exact as (q - z) / 8;
+//   - x becomes five six-bit digits.  Per row and 32 consecutive k, x 2^-e (largest magnitude below 7.5) is rounded to
+//     the nearest e2m3, the exact remainder, at most 1/4, is rounded again in units of 2^-4, the remainder of that, at
+//     most 2^-7, in units of 2^-9, then 2^-14 and 2^-19: what is left is below 2^-22, i.e. 24 bits below the largest of
+//     the 32 values.  The exponent e is the MFMA's own block scale (one E8M0 byte per row and 32 k), and the
+//     digits' constant offsets ride on the block scale of the weight operand, so all five products add up in one f32
+//     accumulator.
+// Five products at four times the rate take 5/8 of the two f16 products of the hi/lo split (w4_gemm_tile.hip), and what a
+// launch can issue is limited by the board's power: from registers, on digits of N(0,1) activations against quantized
+// normal weights, 1275 useful TFLOP/s (at 1.63 GHz) against 961 (at 1.94 GHz).
+// What bounds the whole call: power.  2048 x 4096 -> 11008 takes 265 us with integer zero-points, 284 with fractional ones (f16
+// tiles: 344 and 365), of which the preparation is 14 and the tables of fractional zero-points 12; a step of 64 k takes 3938 clocks at
+// 1.71 GHz where its 80 MFMAs per wave pair alone take 2680.  The conversion of the weights draws about 12 % of the loop's
+// energy, the loads into LDS 7 %, the change of scale from group to group 5 %.  Other sizes, before -> after (fractional
+// zero-points): 4096 x 4096 -> 22016 1430 -> 1002 us, 4096 x 11008 -> 4096 751 -> 553, 4096 x 4096 -> 4096 285 -> 198;
+// groups of 64: 2048 x 4096 -> 11008 426 -> 328.
+//
+// Elements that tower over some of their 32 neighbours would cost those their low bits: where an octet of the 32 lies 2^8
+// or more below the largest, the run of 32 is marked, and a second pass over such steps, after the main loop, multiplies
+// three more digits (2^-24, 2^-29, 2^-34: 39 bits below the largest).
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
+#include "w4.h"
+
+namespace rumus {
+
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v32h __attribute__((ext_vector_type(32)));
+typedef short v8s __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v32f __attribute__((ext_vector_type(32)));
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef uint32_t v6u __attribute__((ext_vector_type(6)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef float v3fa4 __attribute__((ext_vector_type(3), aligned(4)));
+
+typedef const void __attribute__((address_space(1)))* gptr_t;
+typedef void __attribute__((address_space(3)))* lptr_t;
+
+constexpr int kF6BM = 128;                      // rows per workgroup
+constexpr int kF6Tiles = kF6BM / 32;            // row tiles of 32 per workgroup
+constexpr int kF6Digits = 5;
+constexpr int kF6Tile = kF6Digits * 1536;       // bytes of one row tile and one step of 64 k: 64 lanes x 24 bytes per digit
+constexpr int kF6Step = kF6Tiles * kF6Tile;     // 30 KB
+constexpr int kF6Lo = kF6Digits * 1024;         // inside a tile: the lanes' first 16 bytes of every digit, then their last 8
+constexpr int kF6BTile = 1024 + 512 + 32;       // the same for 32 columns of weights; 32 bytes of skew against bank conflicts
+constexpr uint32_t kF6Flags = 256;              // parts of the zero-point table, one flag word each
+constexpr int kF6Deep = 3;                      // further digits where a run of 32 k spans many binades
+constexpr uint32_t kF6DeepBit = 0x80;           // of an exponent byte: the run needs them (the exponents themselves stay below 128)
+// digit d counts in units of 2^-shift
+constexpr int kF6Shift[kF6Digits + kF6Deep] = {0, 4, 9, 14, 19, 24, 29, 34};
+
+struct F6Args {
+    const uint32_t* packed;
+    const float* scales;
+    const float* zp;
+    const uint32_t* zp4;
+    const float* bias;
+    const uint8_t* planes;     // [row block][step][kF6Step]
+    const uint16_t* exps;      // [row block][pair of steps][row tile][64 lanes]: two E8M0 bytes
+    const float* sums;         // [row block][step][kF6BM rows]: sum of x over the step's 64 k
+    const float* x;            // for the further digits of marked runs, with its gather and width
+    const int32_t* perm;
+    const float* rfac;         // [row]: back to the row's own scale (NaN: the row holds a NaN or an infinity)
+    const uint32_t* zflags;    // kF6Flags words, nonzero where a part of the zero-point table holds a value that is no integer in 0..15
+    float* y;
+    uint32_t m, k, n, steps, steps_per_group, num_groups;
+};
+
+__device__ __forceinline__ v8i f6_operand(const v6u& a) {
+    return v8i{(int)a[0], (int)a[1], (int)a[2], (int)a[3], (int)a[4], (int)a[5], 0, 0};
+}
+
+// Fragment order of the weights (nibble conversion): field 8 w + {0..7} of a lane holds k offsets 8 w + {0,4,1,5,2,6,3,7}:
+// even fields come from one register vector, odd ones from the other.
+__device__ __forceinline__ void f6_order(const float (&v)[32], v16f& ev, v16f& od) {
+#pragma unroll
+    for (int w = 0; w < 4; w++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            ev[4 * w + j] = v[8 * w + j];
+            od[4 * w + j] = v[8 * w + 4 + j];
+        }
+}
+// the next digit of 32 values, in units of `unit`, and what it leaves (exact)
+__device__ __forceinline__ v6u f6_digit(v16f& ev, v16f& od, float unit) {
+    const v6u code = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ev, od, unit);
+    const v32f back = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(code, unit);
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        ev[i] -= back[2 * i];
+        od[i] -= back[2 * i + 1];
+    }
+    return code;
+}
+
+// ---- activations -> digits ---------------------------------------------------------------------------
+// A workgroup takes `rows` rows (a power of two up to 8): copies them into LDS with contiguous reads, finding each row's
+// largest magnitude on the way, and then every thread turns one unit, 32 consecutive k of one row, into five digits
+// (rows * units <= 512 threads).  The gather of act-order weights happens on the way out of LDS: from global memory a wave
+// instruction would touch 64 cache lines for 256 bytes.  Memory bound: 2048 x 4096 reads 33.5 and writes 32 MB in 14 us.
+// LDS: row r at r * pitch floats, 4 floats of padding after every 32, so that the 16-byte reads of threads 32 floats
+// apart fall on different banks (likewise rows: pitch / 4 is odd).
+// Beyond the row groups, kF6Flags more workgroups look at the zero-points.
+__device__ __forceinline__ uint32_t f6_padded(uint32_t j) { return j + (j >> 5) * 4; }
+
+template <bool PERM>
+__global__ __launch_bounds__(512) void w4_f6_prepare_kernel(const float* __restrict__ x, const int32_t* __restrict__ perm,
+                                                            uint8_t* __restrict__ planes, uint8_t* __restrict__ exps,
+                                                            float* __restrict__ sums, float* __restrict__ rfac,
+                                                            uint32_t m, uint32_t k, uint32_t steps, uint32_t rows,
+                                                            uint32_t pitch, const float4* __restrict__ zp, uint32_t zp_count4,
+                                                            uint32_t* __restrict__ zflags, uint32_t row_groups) {
+    extern __shared__ __attribute__((aligned(16))) float lds_x[];
+    __shared__ uint32_t rowmax[8];
+    constexpr uint32_t T = 512;
+    const uint32_t tid = threadIdx.x;
+    if (blockIdx.x >= row_groups) {
+        const uint32_t part = blockIdx.x - row_groups;
+        bool mine = false;
+        for (uint32_t i = part * T + tid; i < zp_count4; i += kF6Flags * T) {
+            const float4 z = zp[i];
+            const float v[4] = {z.x, z.y, z.z, z.w};
+#pragma unroll
+            for (int j = 0; j < 4; j++) mine = mine || !(v[j] == rintf(v[j]) && v[j] >= 0.0f && v[j] <= 15.0f);   // a NaN counts
+        }
+        const int any = __syncthreads_or(mine);
+        if (tid == 0) zflags[part] = any ? 1u : 0u;
+        return;
+    }
+    const uint32_t row0 = xcd_contiguous(blockIdx.x, row_groups) * rows;   // neighbours fill the same cache lines of the planes
+    const uint32_t live = row0 < m ? min(rows, m - row0) : 0;
+    if (tid < 8) rowmax[tid] = 0;
+    const uint32_t units = 2 * steps, r = tid % rows, unit = tid / rows, row = row0 + r;
+    const bool mine = unit < units;
+    int4 from[PERM ? 8 : 1];                                     // act-order: where the unit's values come from
+    if constexpr (PERM) {                                                // (k is a multiple of the group size then, and so of 64)
+#pragma unroll
+        for (int q = 0; q < 8; q++) from[q] = reinterpret_cast<const int4*>(perm)[mine ? 8 * unit + q : q];
+    }
+    __syncthreads();
+    // rows into LDS, largest magnitudes on the bit patterns (a NaN or an infinity sorts highest)
+    const bool vec = k % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+    const uint32_t per_row = T / rows, r1 = tid / per_row, t1 = tid % per_row;   // (a wave's threads share a row)
+    {
+        uint32_t am = 0;
+        if (r1 < live) {
+            const float* src = x + (uint64_t)(row0 + r1) * k;
+            float* dst = lds_x + r1 * pitch;
+            if (vec) {
+                const uint32_t last = k / 4 - 1;
+                for (uint32_t i0 = t1; i0 <= last; i0 += 8 * per_row) {
+                    float4 v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) v[u] = reinterpret_cast<const float4*>(src)[min(i0 + u * per_row, last)];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        *reinterpret_cast<float4*>(dst + f6_padded(4 * min(i0 + u * per_row, last))) = v[u];
+                        am = max(max(am, __float_as_uint(v[u].x) & 0x7fffffffu), __float_as_uint(v[u].y) & 0x7fffffffu);
+                        am = max(max(am, __float_as_uint(v[u].z) & 0x7fffffffu), __float_as_uint(v[u].w) & 0x7fffffffu);
+                    }
+                }
+            } else {
+                for (uint32_t i = t1; i < k; i += per_row) {
+                    const float v = src[i];
+                    dst[f6_padded(i)] = v;
+                    am = max(am, __float_as_uint(v) & 0x7fffffffu);
+                }
+            }
+        }
+        am = wave_max(am);
+        if ((tid & 63) == 0) atomicMax(&rowmax[r1], am);
+    }
+    __syncthreads();
+    // 2^(113 - E) brings the row's largest magnitude into [2^-14, 2^-13) (rows beyond 2^112: below 4): the accumulators then
+    // stay inside f32's range whatever the row's own size; the factor and its reciprocal are normal numbers
+    const uint32_t e8 = rowmax[r] >> 23, fb = e8 == 0 || e8 == 255 ? 127u : 240u > e8 ? 240u - e8 : 1u;
+    const bool filled = mine && row < m && e8 != 255;
+    float v[32];
+    {
+        const float rv = __uint_as_float(fb << 23);
+        const float* lr = lds_x + r * pitch;
+        const uint32_t left = filled && k > 32 * unit ? k - 32 * unit : 0;   // columns past k are zeros
+        if constexpr (PERM) {
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                v[4 * q] = lr[f6_padded((uint32_t)from[q].x)]; v[4 * q + 1] = lr[f6_padded((uint32_t)from[q].y)];
+                v[4 * q + 2] = lr[f6_padded((uint32_t)from[q].z)]; v[4 * q + 3] = lr[f6_padded((uint32_t)from[q].w)];
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                const float4 f = *reinterpret_cast<const float4*>(lr + (mine ? unit * 36 : 0) + 4 * q);
+                v[4 * q] = f.x; v[4 * q + 1] = f.y; v[4 * q + 2] = f.z; v[4 * q + 3] = f.w;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 32; j++) v[j] = (uint32_t)j < left ? v[j] * rv : 0.0f;
+    }
+    float o4[4], top = 0.0f, low = 3.4e38f;                      // the octets' largest magnitudes, over all of them: largest and smallest
+#pragma unroll
+    for (int o = 0; o < 4; o++) {
+        o4[o] = fabsf(v[8 * o]);
+#pragma unroll
+        for (int j = 1; j < 8; j++) o4[o] = fmaxf(o4[o], fabsf(v[8 * o + j]));
+        top = fmaxf(top, o4[o]);
+        low = o4[o] > 0.0f ? fminf(low, o4[o]) : low;            // (octets of zeros have nothing to lose)
+    }
+    const bool is_deep = low < top * 0.00390625f;
+    if (!mine) return;                                           // whole waves or the tail of one: no barrier follows
+    float sum = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 32; j++) sum += v[j];
+    // the other half of the step: threads tid and tid ^ rows (rows divides 64, units is even)
+    sum += __shfl_xor(sum, (int)rows);
+    // 2^e with top 2^-e in [3.75, 7.5); units far below the row's size keep a floor
+    const uint32_t eb = max(__float_as_uint(top * (8.0f / 7.5f)) >> 23, 37u) - 2;
+    v16f ev, od;
+    f6_order(v, ev, od);
+    const uint32_t step = unit >> 1, half = unit & 1, blk = row / kF6BM, rt = row / 32 % kF6Tiles, ln = half * 32 + (row & 31);
+    uint8_t* const tile = planes + ((uint64_t)blk * steps + step) * kF6Step + rt * kF6Tile;
+#pragma unroll
+    for (int d = 0; d < kF6Digits; d++) {
+        const v6u code = f6_digit(ev, od, __uint_as_float((eb - kF6Shift[d]) << 23));
+        *reinterpret_cast<uint4*>(tile + d * 1024 + ln * 16) = make_uint4(code[0], code[1], code[2], code[3]);
+        *reinterpret_cast<uint2*>(tile + kF6Lo + d * 512 + ln * 8) = make_uint2(code[4], code[5]);
+    }
+    uint8_t* const e_at = exps + ((((uint64_t)blk * ((steps + 1) / 2) + step / 2) * kF6Tiles + rt) * 64 + ln) * 2;
+    e_at[step & 1] = (uint8_t)(eb | (is_deep ? kF6DeepBit : 0u));
+    if ((steps & 1) && step + 1 == steps) e_at[1] = 0;           // a step that does not exist is not marked either
+    if (half == 0) sums[((uint64_t)blk * steps + step) * kF6BM + row % kF6BM] = sum;
+    if (unit == 0 && row < m) {
+        rfac[row] = e8 == 255 ? __uint_as_float(0x7fc00000u) : __uint_as_float((254u - fb) << 23);
+    }
+}
+
+// ---- the matmul ----------------------------------------------------------------------------------------
+// one packed word -> eight f16, k order 0,4,1,5,2,6,3,7, the integer z taken off on the way (1024 + n - (1024 + z), and
+// (1024 + 16 n) / 16 - (64 + z)): exact
+__device__ __forceinline__ v8h f6_nibbles(uint32_t w, v2h big, v2h small) {
+    const v2h k16th = {(_Float16)0.0625f, (_Float16)0.0625f};
+    const uint32_t m_lo = 0x000F000Fu, m_hi = 0x00F000F0u, magic = 0x64006400u;
+    const uint32_t w8 = w >> 8;
+    uint32_t t0, t1, t2, t3;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(t0) : "v"(w), "v"(m_lo), "s"(magic));
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(t1) : "v"(w), "v"(m_hi), "s"(magic));
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(t2) : "v"(w8), "v"(m_lo), "s"(magic));
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(t3) : "v"(w8), "v"(m_hi), "s"(magic));
+    const v2h h0 = __builtin_bit_cast(v2h, t0) - big;
+    const v2h h1 = __builtin_elementwise_fma(__builtin_bit_cast(v2h, t1), k16th, small);
+    const v2h h2 = __builtin_bit_cast(v2h, t2) - big;
+    const v2h h3 = __builtin_elementwise_fma(__builtin_bit_cast(v2h, t3), k16th, small);
+    return v8h{h0[0], h0[1], h1[0], h1[1], h2[0], h2[1], h3[0], h3[1]};
+}
+
+// TN adjacent columns' floats (TN = 2, 3 or 4; 8-byte aligned)
+template <int TN> struct F6Floats { float v[TN]; };
+template <int TN>
+__device__ __forceinline__ void f6_cols_store(float* p, const F6Floats<TN>& o) {
+    if constexpr (TN == 4) *reinterpret_cast<float4*>(p) = make_float4(o.v[0], o.v[1], o.v[2], o.v[3]);
+    else if constexpr (TN == 3) *reinterpret_cast<v3fa4*>(p) = v3fa4{o.v[0], o.v[1], o.v[2]};
+    else *reinterpret_cast<float2*>(p) = make_float2(o.v[0], o.v[1]);
+}
+// An array as a buffer resource: addresses are an offset that is the same for the whole wave (scalar) plus one per lane,
+// and reads beyond its end give zeros.  (gfx9 descriptor: no swizzle, raw 32-bit data.)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t f6_array(const void* p, uint64_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)(uint32_t)min(bytes, (uint64_t)0xffffffffu), 0x00027000);
+}
+template <int TN>
+__device__ __forceinline__ F6Floats<TN> f6_cols_at(__amdgpu_buffer_rsrc_t p, uint32_t lane_bytes, uint32_t uniform) {
+    F6Floats<TN> o;
+    if constexpr (TN == 4) {
+        const v4u f = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(p, (int)lane_bytes, (int)uniform, 0));
+#pragma unroll
+        for (int j = 0; j < 4; j++) o.v[j] = __uint_as_float(f[j]);
+    } else if constexpr (TN == 3) {
+        const auto f = __builtin_amdgcn_raw_buffer_load_b96(p, (int)lane_bytes, (int)uniform, 0);
+#pragma unroll
+        for (int j = 0; j < 3; j++) o.v[j] = __uint_as_float(f[j]);
+    } else {
+        const v2u f = __builtin_bit_cast(v2u, __builtin_amdgcn_raw_buffer_load_b64(p, (int)lane_bytes, (int)uniform, 0));
+        o.v[0] = __uint_as_float(f[0]);
+        o.v[1] = __uint_as_float(f[1]);
+    }
+    return o;
+}
+__device__ __forceinline__ uint32_t lds_offset(const void* p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p; }
+
+// Loads into LDS (16 bytes per lane, to `to` + 16 * lane) and writes to it, spelled out: the compiler would make every
+// LDS access wait for all loads into LDS in flight (it cannot see that they go to another buffer).  The waits that it counts
+// for its own accesses only get longer for operations it does not know of; the barrier that publishes a buffer waits for
+// these explicitly.
+__device__ __forceinline__ void lds_load16(uint32_t to, const uint8_t* from, uint32_t lane_bytes) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(lane_bytes), "s"(from));
+}
+template <int OFF>
+__device__ __forceinline__ void lds_write24(uint32_t hi_at, uint32_t lo_at, const v6u& v) {
+    const v4u hi = {v[0], v[1], v[2], v[3]};
+    const v2u lo = {v[4], v[5]};
+    asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(hi_at), "v"(hi), "n"(OFF));
+    asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(lo_at), "v"(lo), "n"(OFF));
+}
+
+// s_waitcnt vmcnt(n) lgkmcnt(0)
+#define RUMUS_F6_WAIT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | 0x70)
+
+// Eight waves as 2 (rows) x 4 (columns); a wave owns 64 rows (two row tiles) and 32 TN columns, lane l's columns being
+// TN adjacent ones per tile set.  The accumulators (32 TN registers) set the tile: with 128 TN columns by 128 rows every
+// converted weight serves two row tiles and every activation digit TN column tiles, two steps of both fill the LDS
+// (156 KB at TN = 4), and one workgroup runs per compute unit; w4_launch_gemm_f6 picks TN.
+template <int TN, int FOLD, bool ZP4>
+__global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
+    constexpr int BN = 128 * TN, CPT = TN == 2 ? 1 : 2;          // columns per workgroup; columns each thread converts per step
+    constexpr int BBYTES = 4 * TN * kF6BTile;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // A[2][kF6Step], B[2][BBYTES]
+    uint8_t* const lds_b = lds + 2 * kF6Step;
+
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wm = wave >> 2, wn = wave & 3, l32 = lane & 31, kb = lane >> 5;
+    const uint32_t blk = blockIdx.y, m0 = blk * kF6BM, n0 = blockIdx.x * BN;
+    // whether some zero-point of the table is no integer in 0..15 (found by w4_f6_prepare_kernel)
+    uint4 zflag = make_uint4(0, 0, 0, 0);
+    if constexpr (!ZP4) zflag = reinterpret_cast<const uint4*>(a.zflags)[lane];
+    const uint32_t my_col = n0 + wn * (32 * TN) + TN * l32;       // first of the lane's TN output columns
+    const uint32_t my_col_c = my_col < a.n ? my_col : 0;          // n % 4 == 0
+
+    // ---- weights: thread converts CPT adjacent columns of one half (32 k) of a step --------------------
+    // (TN = 3: 192 pairs of columns, the last 64 threads of a half repeat the last pair)
+    const uint32_t c_half = wave >> 2, c_first = CPT * min(tid & 255, (uint32_t)(BN / CPT - 1)), c_col = n0 + c_first;
+    const uint32_t c_col_c = c_col < a.n ? c_col : 0;
+    uint32_t c_hi[CPT], c_lo[CPT];                                 // where the column's codes go
+#pragma unroll
+    for (int c = 0; c < CPT; c++) {
+        const uint32_t w = (c_first + c) / (32 * TN), r = (c_first + c) % (32 * TN);
+        const uint32_t tile = lds_offset(lds_b) + (w * TN + r % TN) * kF6BTile, ln = c_half * 32 + r / TN;
+        c_hi[c] = tile + ln * 16;
+        c_lo[c] = tile + 1024 + ln * 8;
+    }
+    const uint32_t row_bytes = a.n * 4;
+    const auto b_packed = f6_array(a.packed, (uint64_t)a.steps * 8 * row_bytes), b_scales = f6_array(a.scales, (uint64_t)a.num_groups * row_bytes);
+    const auto b_zp = ZP4 ? f6_array(a.zp4, (uint64_t)a.num_groups * (a.n / 2)) : f6_array(a.zp, (uint64_t)a.num_groups * row_bytes);
+    const uint32_t c_bytes = c_col_c * 4;
+    uint32_t raw[2][4][CPT];                                       // words of an even and an odd step
+    auto word_load = [&](uint32_t s, int set, int i) __attribute__((always_inline)) {
+        const uint32_t row = min(s, a.steps - 1) * 8 + c_half * 4 + i;
+        if constexpr (CPT == 2) {
+            const v2u w = __builtin_bit_cast(v2u, __builtin_amdgcn_raw_buffer_load_b64(b_packed, (int)c_bytes, (int)(row * row_bytes), 0));
+            raw[set][i][0] = w[0]; raw[set][i][1] = w[1];
+        } else {
+            raw[set][i][0] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(b_packed, (int)c_bytes, (int)(row * row_bytes), 0);
+        }
+    };
+    constexpr int ZSETS = FOLD == 1 ? 2 : 1;                       // zero-points in flight: of every step, or of every even one
+    float raw_zp[ZSETS][CPT];
+    uint32_t raw_zp4[ZSETS];
+    auto zp_load = [&](uint32_t s, int set) __attribute__((always_inline)) {
+        const uint32_t g = min(s, a.steps - 1) / a.steps_per_group;
+        if constexpr (ZP4) {
+            raw_zp4[set] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(b_zp, (int)(c_col_c / 8 * 4), (int)(g * (a.n / 2)), 0);
+        } else if constexpr (CPT == 2) {
+            const v2u z = __builtin_bit_cast(v2u, __builtin_amdgcn_raw_buffer_load_b64(b_zp, (int)c_bytes, (int)(g * row_bytes), 0));
+            raw_zp[set][0] = __uint_as_float(z[0]); raw_zp[set][1] = __uint_as_float(z[1]);
+        } else {
+            raw_zp[set][0] = __uint_as_float((uint32_t)__builtin_amdgcn_raw_buffer_load_b32(b_zp, (int)c_bytes, (int)(g * row_bytes), 0));
+        }
+    };
+    v2h z_big[CPT], z_small[CPT];
+    auto zero_points = [&](int set) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < CPT; c++) {
+            float z;
+            if constexpr (ZP4) {
+                z = (float)((raw_zp4[set] >> (4 * (c_col_c & 7u) + 4 * c)) & 15u);
+            } else {
+                z = fminf(fmaxf(rintf(raw_zp[set][c]), 0.0f), 15.0f);    // (a NaN becomes 0 and stays whole in the rest)
+            }
+            const _Float16 b = (_Float16)(1024.0f + z), sm = (_Float16)(-64.0f - z);
+            z_big[c] = v2h{b, b};
+            z_small[c] = v2h{sm, sm};
+        }
+    };
+    v32h halves;
+    auto convert_words = [&](int set, int c, int first) __attribute__((always_inline)) {   // two of the four words of column c
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const v8h f = f6_nibbles(raw[set][first + i][c], z_big[c], z_small[c]);
+#pragma unroll
+            for (int e = 0; e < 8; e++) halves[8 * (first + i) + e] = f[e];
+        }
+    };
+    auto column_store = [&](int c, auto buf_tag) __attribute__((always_inline)) {
+        constexpr int OFF = decltype(buf_tag)::value * BBYTES;
+        const v6u code = __builtin_amdgcn_cvt_scalef32_pk32_fp6_f16(halves, 8.0f);
+        lds_write24<OFF>(c_hi[c], c_lo[c], code);
+    };
+
+    // ---- activations: a step is 30 KB, straight into LDS; wave w takes KB w, w + 8, w + 16, w + 24 (the last two waves
+    // repeat one: same bytes to the same place, so that every wave counts the same loads) ------------------
+    const uint8_t* const a_blk = a.planes + (uint64_t)blk * a.steps * kF6Step;
+    const uint32_t a_lds = lds_offset(lds), a_lane = lane * 16;
+    auto digits_load = [&](uint32_t s, uint32_t buf) __attribute__((always_inline)) {
+        const uint8_t* src = a_blk + (uint64_t)min(s, a.steps - 1) * kF6Step;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const uint32_t c = min(wave + 8 * q, 29u) * 1024;
+            lds_load16(a_lds + buf * kF6Step + c, src + c, a_lane);
+        }
+    };
+    uint32_t exps[2], exps_next[2];                                // E8M0 bytes of two steps, per row tile of this wave
+    const uint32_t e_pairs = (a.steps + 1) / 2;
+    const auto b_exps = f6_array(a.exps + (uint64_t)blk * e_pairs * (kF6Tiles * 64), (uint64_t)e_pairs * (kF6Tiles * 128));
+    auto exps_load = [&](uint32_t s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+            exps_next[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(
+                b_exps, (int)(lane * 2), (int)(min(s, a.steps - 1) / 2 * (kF6Tiles * 128) + (wm * 2 + i) * 128), 0);
+    };
+
+    uint32_t deep = 0;                                             // kF6DeepBit of any run seen
+    auto take_exps = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            deep |= exps_next[i];
+            exps[i] = exps_next[i] & (0x0101u * (kF6DeepBit - 1));
+        }
+    };
+
+    v16f acc[2][TN];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+
+    auto scales_of = [&](uint32_t g) __attribute__((always_inline)) {
+        return f6_cols_at<TN>(b_scales, my_col_c * 4, min(g, a.num_groups - 1) * row_bytes);
+    };
+    auto nonzero = [](float s) { return s == 0.0f ? 1e-30f : s; };
+    F6Floats<TN> sc_cur, sc_next, ratio;
+#pragma unroll
+    for (int j = 0; j < TN; j++) ratio.v[j] = 1.0f;
+
+    constexpr int kB0 = 130 | (126 << 8) | (121 << 16) | (116 << 24), kB1 = 111;   // 2^3 / 2^shift of every digit
+
+    auto read6 = [&](const uint8_t* hi, const uint8_t* lo) __attribute__((always_inline)) {
+        const uint4 h = *reinterpret_cast<const uint4*>(hi + lane * 16);
+        const uint2 l = *reinterpret_cast<const uint2*>(lo + lane * 8);
+        return v6u{h.x, h.y, h.z, h.w, l.x, l.y};
+    };
+
+    // Step s from buffer P, in ten sections of TN MFMAs (row tile i, digit d): a section's A fragment is read one section
+    // ahead, and the vector work of a step is dealt out over its sections so that every MFMA has its share: the change of
+    // the accumulators from one group's scale to the next (a row tile undergoes it while the other one multiplies, in the
+    // second half of an odd step and the first half of an even one), and in the other halves the next step's weights.
+    auto step = [&](uint32_t s, auto p_tag) __attribute__((always_inline)) {
+        constexpr int P = decltype(p_tag)::value;
+        constexpr bool ENDS = P == 1 || FOLD == 1, STARTS = P == 0 || FOLD == 1;   // a group may end / start with this step
+        constexpr int C0 = P == 0 ? 5 : 0;                       // first section of the conversion
+        constexpr int SET = P ^ 1;                               // of step s + 1
+        typedef std::integral_constant<int, P ^ 1> other;
+        const uint8_t* const pa = lds + P * kF6Step + wm * 2 * kF6Tile;
+        const uint8_t* const pb = lds_b + P * BBYTES + wn * TN * kF6BTile;
+        v6u bf[TN], af[2];
+        af[0] = read6(pa, pa + kF6Lo);
+#pragma unroll
+        for (int j = 0; j < TN; j++) bf[j] = read6(pb + j * kF6BTile, pb + j * kF6BTile + 1024);
+#pragma unroll
+        for (int t = 0; t < 10; t++) {
+            const int i = t / 5, d = t % 5;
+            if (t + 1 < 10) {
+                const int i2 = (t + 1) / 5, d2 = (t + 1) % 5;
+                af[(t + 1) & 1] = read6(pa + i2 * kF6Tile + d2 * 1024, pa + i2 * kF6Tile + kF6Lo + d2 * 512);
+            }
+            if (t == 0) digits_load(s + 1, P ^ 1);
+            if (P == 1 && t == 1) exps_load(s + 1);
+            if (t == C0 && ENDS) zero_points(FOLD == 1 ? SET : 0);
+            if (t == C0 + 1 && ENDS) zp_load(s + 3, FOLD == 1 ? SET : 0);
+            if (t == C0 || t == C0 + 1) convert_words(SET, 0, 2 * (t - C0));
+            if (t == C0 + 2) column_store(0, other{});
+            if (CPT == 2 && (t == C0 + 2 || t == C0 + 3)) convert_words(SET, 1, 2 * (t - C0 - 2));
+            if (CPT == 2 && t == C0 + 4) column_store(1, other{});
+            if (t == C0 + 3) { word_load(s + 3, SET, 0); word_load(s + 3, SET, 1); }
+            if (t == C0 + 4) { word_load(s + 3, SET, 2); word_load(s + 3, SET, 3); }
+            if (STARTS && t >= 1 && t <= TN) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[1][t - 1][r] *= ratio.v[t - 1];
+            }
+            // the scales of this step's group and the next step's
+            if (ENDS && t == 1) {
+                sc_cur = scales_of(min(s, a.steps - 1) / a.steps_per_group);
+                sc_next = scales_of(min(s + 1, a.steps - 1) / a.steps_per_group);
+            }
+            if (ENDS && t == 5) {
+#pragma unroll
+                for (int j = 0; j < TN; j++) {
+                    const float sc = nonzero(sc_cur.v[j]), sn = nonzero(sc_next.v[j]);
+                    const float rc = __builtin_amdgcn_rcpf(sn);
+                    const float q = sc * rc;
+                    ratio.v[j] = fmaf(fmaf(-q, sn, sc), rc, q);   // one correction step: within an ulp of the quotient, and 1 for the same group
+                }
+            }
+            if (ENDS && t >= 6 && t < 6 + TN) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[0][t - 6][r] *= ratio.v[t - 6];
+            }
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                const v8i fa = f6_operand(af[t & 1]), fb = f6_operand(bf[j]);
+                // (the byte selectors are immediates)
+                if (d == 0) acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa, fb, acc[i][j], 2, 2, P, (int)exps[i], 0, kB0);
+                if (d == 1) acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa, fb, acc[i][j], 2, 2, P, (int)exps[i], 1, kB0);
+                if (d == 2) acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa, fb, acc[i][j], 2, 2, P, (int)exps[i], 2, kB0);
+                if (d == 3) acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa, fb, acc[i][j], 2, 2, P, (int)exps[i], 3, kB0);
+                if (d == 4) acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa, fb, acc[i][j], 2, 2, P, (int)exps[i], 0, kB1);
+            }
+            // the reads of the next section, then MFMAs with a share of the vector work behind each
+            if (t + 1 < 10) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, FOLD == 1 ? 10 : 6, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (P == 1) take_exps();
+        // this step's digits have landed once only the loads issued behind them are outstanding: words, exponents,
+        // zero-points, scales
+        RUMUS_F6_WAIT(4 + (ENDS ? 3 : 0) + (P == 1 ? 2 : 0));
+        __builtin_amdgcn_s_barrier();
+    };
+
+    digits_load(0, 0);
+    exps_load(0);
+    take_exps();
+    if constexpr (FOLD == 1) zp_load(1, 1);
+    zp_load(0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; i++) word_load(0, 0, i);
+#pragma unroll
+    for (int i = 0; i < 4; i++) word_load(1, 1, i);
+    zero_points(0);
+#pragma unroll
+    for (int c = 0; c < CPT; c++) {
+        convert_words(0, c, 0);
+        convert_words(0, c, 2);
+        column_store(c, std::integral_constant<int, 0>{});
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) word_load(2, 0, i);
+    zp_load(2, 0);
+    RUMUS_F6_WAIT(0);
+    __builtin_amdgcn_s_barrier();
+    uint32_t s = 0;
+    for (; s + 1 < a.steps; s += 2) {
+        step(s, std::integral_constant<int, 0>{});
+        step(s + 1, std::integral_constant<int, 1>{});
+    }
+    if (s < a.steps) step(s, std::integral_constant<int, 0>{});
+    RUMUS_F6_WAIT(0);                                              // the loads past the last step have landed: the LDS is free
+    __syncthreads();
+
+    sc_cur = scales_of(a.num_groups - 1);
+#pragma unroll
+    for (int j = 0; j < TN; j++) sc_cur.v[j] = nonzero(sc_cur.v[j]);
+
+    // ---- the further digits of marked runs; ordinary data has none --------------------------------------------------
+    if (__syncthreads_or((deep & (0x0101u * kF6DeepBit)) != 0)) {
+        for (uint32_t s = 0; s < a.steps; s++) {
+            if ((s & 1) == 0) exps_load(s);
+            const uint32_t e_shift = 8 * (s & 1);
+            if (!__syncthreads_or(((exps_next[0] | exps_next[1]) >> e_shift & kF6DeepBit) != 0)) continue;
+            // this step's weights once more
+#pragma unroll
+            for (int i = 0; i < 4; i++) word_load(s, 0, i);
+            zp_load(s, 0);
+            zero_points(0);
+#pragma unroll
+            for (int c = 0; c < CPT; c++) {
+                convert_words(0, c, 0);
+                convert_words(0, c, 2);
+                column_store(c, std::integral_constant<int, 0>{});
+            }
+            // and the runs: a thread each, from x itself, past the digits that the planes hold
+            constexpr int DTILE = kF6Deep * 1536;
+            if (tid < 2 * kF6BM) {
+                const uint32_t r = tid % kF6BM, half = tid / kF6BM, rt = r / 32, ln = half * 32 + (r & 31), row = m0 + r;
+                const uint32_t e = a.exps[(((uint64_t)blk * e_pairs + s / 2) * kF6Tiles + rt) * 64 + ln] >> e_shift & 0xffu;
+                const bool marked = (e & kF6DeepBit) != 0;        // (rows past m are not)
+                uint8_t* const to = lds + rt * DTILE;
+                v16f ev, od;
+                if (marked) {
+                    const float rv = __uint_as_float((254u - (__float_as_uint(a.rfac[row]) >> 23)) << 23);
+                    const float* const xr = a.x + (uint64_t)row * a.k;
+                    const uint32_t k0 = 64 * s + 32 * half;
+                    uint32_t from[32];
+                    float v[32];
+#pragma unroll
+                    for (int j = 0; j < 32; j++) from[j] = min(k0 + j, a.k - 1);
+                    if (a.perm) {
+#pragma unroll
+                        for (int j = 0; j < 32; j++) from[j] = (uint32_t)a.perm[from[j]];
+                    }
+#pragma unroll
+                    for (int j = 0; j < 32; j++) v[j] = xr[from[j]] * rv;
+#pragma unroll
+                    for (int j = 0; j < 32; j++) v[j] = k0 + j < a.k ? v[j] : 0.0f;
+                    f6_order(v, ev, od);
+#pragma unroll
+                    for (int d = 0; d < kF6Digits; d++) (void)f6_digit(ev, od, __uint_as_float(((e & (kF6DeepBit - 1)) - kF6Shift[d]) << 23));
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 16; j++) ev[j] = od[j] = 0.0f;
+                }
+#pragma unroll
+                for (int d = 0; d < kF6Deep; d++) {
+                    // (unmarked: zeros in any unit)
+                    const v6u code = f6_digit(ev, od, marked ? __uint_as_float(((e & (kF6DeepBit - 1)) - kF6Shift[kF6Digits + d]) << 23) : 1.0f);
+                    *reinterpret_cast<uint4*>(to + d * 1536 + ln * 16) = make_uint4(code[0], code[1], code[2], code[3]);
+                    *reinterpret_cast<uint2*>(to + d * 1536 + 1024 + ln * 8) = make_uint2(code[4], code[5]);
+                }
+            }
+            const F6Floats<TN> sc = scales_of(s / a.steps_per_group);
+            RUMUS_F6_WAIT(0);
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const int ea = (int)(exps_next[i] >> e_shift & (kF6DeepBit - 1));
+                const uint8_t* const pa = lds + (wm * 2 + i) * DTILE;
+                v8i da[kF6Deep];
+#pragma unroll
+                for (int d = 0; d < kF6Deep; d++) da[d] = f6_operand(read6(pa + d * 1536, pa + d * 1536 + 1024));
+#pragma unroll
+                for (int j = 0; j < TN; j++) {
+                    const uint8_t* const pb = lds_b + (wn * TN + j) * kF6BTile;
+                    const v8i fb = f6_operand(read6(pb, pb + 1024));
+                    v16f t;
+#pragma unroll
+                    for (int r = 0; r < 16; r++) t[r] = 0.0f;
+                    t = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(da[0], fb, t, 2, 2, 0, ea, 0, 130 - kF6Shift[kF6Digits]);
+                    t = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(da[1], fb, t, 2, 2, 0, ea, 0, 130 - kF6Shift[kF6Digits + 1]);
+                    t = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(da[2], fb, t, 2, 2, 0, ea, 0, 130 - kF6Shift[kF6Digits + 2]);
+                    const float ratio_s = nonzero(sc.v[j]) / sc_cur.v[j];
+#pragma unroll
+                    for (int r = 0; r < 16; r++) acc[i][j][r] = fmaf(t[r], ratio_s, acc[i][j][r]);
+                }
+            }
+            __syncthreads();                                       // before the next step's codes
+        }
+    }
+
+    // ---- what integer zero-points left over: - sum over g of scale (zp - z) (sum of x over the group) ----------------
+    if constexpr (!ZP4) {
+        if (__builtin_amdgcn_ballot_w64((zflag.x | zflag.y | zflag.z | zflag.w) != 0) != 0) {   // the same in every wave
+            // A product of two f32 tables over the groups, exact to 24 bits on the bf16 matrix cores: both factors split into
+            // three bf16 parts, eight of the nine products; the 16 k slots of an instruction are two groups of eight
+            // products, lane half h carries group g + h.  The tables go through LDS, GROUPS groups at a time: read from
+            // memory by every wave for itself, one trip per few groups, they cost 17 us a launch instead of 12.
+            constexpr uint32_t GROUPS = 32;
+            static_assert(GROUPS * (BN + kF6BM) * 4 <= 2 * (kF6Step + BBYTES), "the tables fit the LDS");
+            float* const t_y = reinterpret_cast<float*>(lds);          // [GROUPS][BN], in the accumulators' unit
+            float* const t_x = t_y + GROUPS * BN;                      // [GROUPS][kF6BM]
+            auto parts = [](float v, short (&p)[3]) __attribute__((always_inline)) {
+#pragma unroll
+                for (int q = 0; q < 3; q++) {
+                    const uint32_t hi = __float_as_uint(v) & 0xffff0000u;
+                    p[q] = (short)(hi >> 16);
+                    v -= __uint_as_float(hi);
+                }
+            };
+            const uint32_t spg = a.steps_per_group, gb = a.num_groups - 1;
+            const uint32_t t_col = min(n0 + tid, a.n - 1);             // BN <= 512: a column per thread
+            const float t_unit = 1.0f / nonzero(a.scales[(uint64_t)gb * a.n + t_col]);
+            for (uint32_t g0 = 0; g0 <= gb; g0 += GROUPS) {
+                const uint32_t count = min(GROUPS, gb - g0 + 1);
+                if (tid < BN) {
+                    for (uint32_t g = 0; g < GROUPS; g += 8) {
+                        float sv[8], zv[8];
+#pragma unroll
+                        for (int u = 0; u < 8; u++) {
+                            const uint32_t at = min(g0 + g + u, gb) * a.n + t_col;
+                            sv[u] = a.scales[at];
+                            zv[u] = a.zp[at];
+                        }
+#pragma unroll
+                        for (int u = 0; u < 8; u++) {
+                            const float z = fminf(fmaxf(rintf(zv[u]), 0.0f), 15.0f);
+                            t_y[(g + u) * BN + tid] = g + u < count ? -(zv[u] - z) * sv[u] * t_unit : 0.0f;
+                        }
+                    }
+                }
+                for (uint32_t e = tid; e < GROUPS * kF6BM; e += 512) {
+                    const uint32_t g = min(g0 + e / kF6BM, gb), sa = g * spg, sb = min(g * spg + spg, a.steps);
+                    const float* p = a.sums + ((uint64_t)blk * a.steps + sa) * kF6BM + e % kF6BM;
+                    float v = p[0] + (sb - sa > 1 ? p[kF6BM] : 0.0f);
+                    for (uint32_t s = sa + 2; s < sb; s++) v += p[(s - sa) * kF6BM];
+                    t_x[e] = e / kF6BM < count ? v : 0.0f;
+                }
+                __syncthreads();
+                for (uint32_t g2 = 0; g2 < count; g2 += 2) {
+                    const uint32_t g = g2 + kb;                        // (rows past count hold zeros)
+                    v8s fb[TN];
+                    short p[3];
+#pragma unroll
+                    for (int j = 0; j < TN; j++) {
+                        parts(t_y[g * BN + wn * (32 * TN) + TN * l32 + j], p);
+                        fb[j] = v8s{p[0], p[1], p[2], p[0], p[1], p[0], p[2], p[1]};
+                    }
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        parts(t_x[g * kF6BM + (wm * 2 + i) * 32 + l32], p);
+                        const v8s fa = v8s{p[0], p[0], p[0], p[1], p[1], p[2], p[1], p[2]};
+#pragma unroll
+                        for (int j = 0; j < TN; j++)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, fa), __builtin_bit_cast(v8bf, fb[j]), acc[i][j], 0, 0, 0);
+                    }
+                }
+                __syncthreads();
+            }
+        }
+    }
+
+    // ---- store -------------------------------------------------------------------------------------------------
+    float bv[TN];
+#pragma unroll
+    for (int j = 0; j < TN; j++) bv[j] = a.bias && my_col + j < a.n ? a.bias[my_col + j] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        if (my_col < a.n) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const uint32_t row = m0 + (wm * 2 + i) * 32 + 8 * (r / 4) + 4 * kb + (r % 4);
+                if (row >= a.m) continue;
+                const float rf = a.rfac[row];                     // back to the row's own scale: exact, a power of two
+                F6Floats<TN> o;
+#pragma unroll
+                for (int j = 0; j < TN; j++) o.v[j] = fmaf(acc[i][j][r] * rf, sc_cur.v[j], bv[j]);
+                float* p = a.y + (uint64_t)row * a.n + my_col;
+                if (TN != 3 || my_col + TN <= a.n) {
+                    f6_cols_store<TN>(p, o);
+                } else {                                             // the right edge: n % 4 == 0
+#pragma unroll
+                    for (int j = 0; j < TN; j++)
+                        if (my_col + j < a.n) p[j] = o.v[j];
+                }
+            }
+        }
+    }
+}
+
+// Columns per workgroup / 128, and the time of a call in microseconds: workgroups run one per compute unit, in rounds of
+// 256.  A round's steps (of 64 k) take L at least, and from about 170 workgroups on power limits them: a launch as a whole
+// cannot beat P per 256 workgroup-steps.  16 is a round's start and end, the rest the preparation.  Fitted to 252 timings
+// (130 .. 4096 rows; seven weights, 1024 -> 5504 to 8192 -> 8192 and 4096 -> 22016; 2, 3 and 4 forced): within 3 % rms, and the width chosen by
+// it costs 0.01 % against the best of the three, 1 % at worst.
+static int f6_pick(uint32_t m, uint32_t k, uint32_t n, double* us) {
+    static const double L[3] = {1.22, 1.55, 1.82}, P[3] = {1.29, 1.95, 2.50};
+    const double steps = ceil_div(k, 64);
+    int best = 4;
+    *us = 1e30;
+    for (int tn = 4; tn >= 2; tn--) {
+        const double wgs = (double)ceil_div(m, kF6BM) * ceil_div(n, 128 * tn), rounds = std::ceil(wgs / 256.0);
+        const double chain = rounds * (steps * L[tn - 2] + 16.0), power = wgs / 256.0 * steps * P[tn - 2];
+        const double t = std::sqrt(std::sqrt(chain * chain * chain * chain + power * power * power * power)) + 3.0 + 1.6e-6 * m * k;
+        if (t < *us) { *us = t; best = tn; }
+    }
+    return best;
+}
+
+static size_t f6_up(size_t v) { return (v + 255) & ~size_t(255); }
+
+struct F6Workspace {
+    uint32_t blocks, steps;
+    size_t planes, exps, sums, rfac, flags, total;   // bytes
+    F6Workspace(uint32_t m, uint32_t padded_k) : blocks(ceil_div(m, kF6BM)), steps(padded_k / 64) {
+        // (never less than the f16 tiles park, 4 bytes per element: what a caller reserved or a fixed buffer holds, and what it
+        // refuses, does not depend on the kernel)
+        planes = std::max((size_t)blocks * steps * kF6Step, (size_t)ceil_div(m, 32) * 32 * padded_k * 4);
+        exps = f6_up((size_t)blocks * ((steps + 1) / 2) * kF6Tiles * 64 * 2);
+        sums = (size_t)blocks * steps * kF6BM * 4;
+        rfac = (size_t)blocks * kF6BM * 4;
+        flags = kF6Flags * 4;
+        total = planes + exps + sums + rfac + flags;
+    }
+};
+
+// More than 256 rows (blocks of 128 rows: up to there the integer kernel's blocks of 64 fit as well or better, and K would have to be
+// shared over workgroups), where its time is below what the other two kernels are expected to take.  The two estimates of
+// those are loosest upwards for the integer kernel (8192 -> 8192 at 640 rows: 201 us expected, 164 measured, 185 here), hence its
+// margin.  Over the 60 cases above 256 rows the choice is 0.05 % off the better one and takes 17.5 % less time than
+// before on average: 2048 rows 4096 -> 11008 374 -> 287 us, 4096 -> 4096 146 -> 120, 4096 rows 4096 -> 22016 1448 -> 1022,
+// 1024 rows 1024 -> 5504 41.9 -> 41.9.
+bool w4_gemm_f6_chosen(const W4Args& a) {
+    const uintptr_t bits = reinterpret_cast<uintptr_t>(a.packed) | reinterpret_cast<uintptr_t>(a.scales) |
+                           reinterpret_cast<uintptr_t>(a.zp) | reinterpret_cast<uintptr_t>(a.y) |
+                           reinterpret_cast<uintptr_t>(a.perm) | reinterpret_cast<uintptr_t>(a.bias);
+    if (!(a.m > 256 && a.m <= 65535u * kF6BM && a.n % 4 == 0 && (bits & 15) == 0 && !a.g_idx && !a.tiled && !a.glu &&
+          a.group_size % 64 == 0 && (!a.zp4 || a.n % 8 == 0) && a.k >= 1024 && a.k <= 16384 &&    // (what the estimates were fitted to; a row of x in LDS, and 512 units of 32 k)
+          (uint64_t)a.padded_k / 8 * a.n * 4 < (1ull << 32) && (uint64_t)a.m * a.n < (1ull << 32)))
+        return false;
+    double us = 0.0, other = 0.0;
+    f6_pick(a.m, a.k, a.n, &us);
+    const bool i8 = w4_gemm_i8_supported(a, &other);
+    // what the integer kernel runs within the fixed scratch array (w4_gemv.hip) has to go on running there
+    if (i8 && F6Workspace(a.m, a.padded_k).total > (size_t(32) << 20)) return false;
+    return us < (i8 ? 0.92 : 1.0) * other;
+}
+
+template <int TN, int FOLD, bool ZP4>
+static int launch_f6(const F6Args& f, uint32_t blocks, hipStream_t s) {
+    constexpr size_t lds_bytes = 2 * (size_t)(kF6Step + 4 * TN * kF6BTile);
+    static_assert(lds_bytes <= 160 * 1024, "two steps fit the LDS");
+    static bool attr_set = false;   // benign race: setting the attribute is idempotent
+    if (!attr_set) {
+        if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&w4_gemm_f6_kernel<TN, FOLD, ZP4>),
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes),
+                               "hipFuncSetAttribute"))
+            return rc;
+        attr_set = true;
+    }
+    hipLaunchKernelGGL((w4_gemm_f6_kernel<TN, FOLD, ZP4>), dim3(ceil_div(f.n, 128 * TN), blocks), dim3(512), lds_bytes, s, f);
+    return check_launch("w4_gemm_f6_kernel");
+}
+
+template <int TN>
+static int launch_f6_groups(const F6Args& f, const W4Args& a, uint32_t blocks, hipStream_t s) {
+    if (a.group_size % 128 == 0) return a.zp4 ? launch_f6<TN, 2, true>(f, blocks, s) : launch_f6<TN, 2, false>(f, blocks, s);
+    return a.zp4 ? launch_f6<TN, 1, true>(f, blocks, s) : launch_f6<TN, 1, false>(f, blocks, s);
+}
+
+int w4_launch_gemm_f6(const W4Args& a, hipStream_t s) {
+    const F6Workspace w(a.m, a.padded_k);
+    void* ws = nullptr;
+    WorkspaceLease lease;                                    // until the last kernel of this call is queued
+    if (int rc = workspace_get(s, w.total, &ws, lease)) return rc;
+    uint8_t* p = static_cast<uint8_t*>(ws);
+    uint8_t* const planes = p; p += w.planes;
+    uint8_t* const exps = p; p += w.exps;
+    float* const sums = reinterpret_cast<float*>(p); p += w.sums;
+    float* const rfac = reinterpret_cast<float*>(p); p += w.rfac;
+    uint32_t* const zflags = reinterpret_cast<uint32_t*>(p);
+    // rows per workgroup of the preparation: at most 512 units and 80 KB of LDS (two workgroups per compute unit), and enough workgroups
+    const uint32_t units = 2 * w.steps, pitch = units * 36 + 4, rows_pad = w.blocks * kF6BM;
+    uint32_t rows = 8;
+    while (rows > 1 && ((size_t)rows * pitch * 4 > 80 * 1024 || rows * units > 512 || rows_pad / rows < 256)) rows /= 2;
+    static bool attr_set = false;   // benign race: setting the attribute is idempotent
+    if (!attr_set) {
+        for (const void* f : {reinterpret_cast<const void*>(&w4_f6_prepare_kernel<false>), reinterpret_cast<const void*>(&w4_f6_prepare_kernel<true>)})
+            if (int rc = check_hip(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024), "hipFuncSetAttribute"))
+                return rc;
+        attr_set = true;
+    }
+    const dim3 pgrid(rows_pad / rows + (a.zp4 ? 0 : kF6Flags));
+#define RUMUS_F6_PREPARE(PERM)                                                                                             \
+    hipLaunchKernelGGL(w4_f6_prepare_kernel<PERM>, pgrid, dim3(512), (size_t)rows * pitch * 4, s, a.x, a.perm, planes, exps, sums, \
+                       rfac, a.m, a.k, w.steps, rows, pitch, reinterpret_cast<const float4*>(a.zp),                        \
+                       (uint32_t)((uint64_t)a.num_groups * a.n / 4), zflags, rows_pad / rows)
+    if (a.perm) RUMUS_F6_PREPARE(true);
+    else RUMUS_F6_PREPARE(false);
+#undef RUMUS_F6_PREPARE
+    if (int rc = check_launch("w4_f6_prepare_kernel")) return rc;
+    const F6Args f{a.packed, a.scales, a.zp, a.zp4, a.bias, planes, reinterpret_cast<const uint16_t*>(exps), sums, a.x, a.perm, rfac,
+                   zflags, a.y, a.m, a.k, a.n, w.steps, a.group_size / 64, a.num_groups};
+    double us;
+    switch (f6_pick(a.m, a.k, a.n, &us)) {
+        case 2: return launch_f6_groups<2>(f, a, w.blocks, s);
+        case 3: return launch_f6_groups<3>(f, a, w.blocks, s);
+        default: return launch_f6_groups<4>(f, a, w.blocks, s);
+    }
+}
+
+}  // namespace rumus

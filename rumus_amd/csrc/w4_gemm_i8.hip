@@ -562,35 +562,39 @@ static bool i8_rounds_filled(uint32_t m, uint32_t n, bool zp4) {
 //   f16 tiles: from 192 tiles of 64 x 512 on, rounds as w4_launch_gemm prices its two shapes, 109 per round; below,
 //       K is split over the workgroups and the time follows the tile count.
 // Both scale with K; 16 and 24 are what a call costs besides (activation planes, launches).
-static bool i8_beats_f16_estimate(uint32_t m, uint32_t k, uint32_t n, bool zp4) {
+struct W4Estimates { double i8, f16; };
+static W4Estimates w4_estimates(uint32_t m, uint32_t k, uint32_t n, bool zp4) {
     const uint32_t row_blocks = ceil_div(m, 64);
     const uint32_t q = (uint32_t)pick_q(n, row_blocks, zp4);
     const double kf = (double)k / 4096.0;
     const double wgs = (double)ceil_div(n, 16 * q) * row_blocks;
-    const double est_i8 = (wgs / 256.0 - 0.14) * (3.4 + 3.9 * q) * kf + 16.0;
+    W4Estimates e;
+    e.i8 = (wgs / 256.0 - 0.14) * (3.4 + 3.9 * q) * kf + 16.0;
     const uint64_t tiles = (uint64_t)row_blocks * ceil_div(n, 512), full = (tiles + 255) / 256;
     const uint64_t halves = ((uint64_t)row_blocks * ceil_div(n, 256) + 255) / 256;
-    double est_f16;
     if (tiles >= 192) {
         double units = 0.97 * (double)full;
         units = std::min(units, (double)(halves / 2) * 1.05 + (double)(halves % 2) * 0.75);
-        est_f16 = units * 109.0 * kf + 24.0;
+        e.f16 = units * 109.0 * kf + 24.0;
     } else {
-        est_f16 = (156.0 * (double)tiles / 256.0 - 3.0) * kf + 24.0;
+        e.f16 = (156.0 * (double)tiles / 256.0 - 3.0) * kf + 24.0;
     }
-    return est_i8 < 0.97 * est_f16;                           // ties go to the f16 tiles (slightly fewer wrong choices on the fitted cases)
+    return e;
 }
 
-bool w4_gemm_i8_supported(const W4Args& a) {
+bool w4_gemm_i8_supported(const W4Args& a, double* us) {
     const uintptr_t bits = reinterpret_cast<uintptr_t>(a.packed) | reinterpret_cast<uintptr_t>(a.scales) |
                            reinterpret_cast<uintptr_t>(a.zp) | reinterpret_cast<uintptr_t>(a.y) |
                            (a.bias ? reinterpret_cast<uintptr_t>(a.bias) : 0);
-    if (!(a.m > 0 && a.m <= kI8MaxRows && a.group_size % 64 == 0 && a.n % 4 == 0 && a.n >= 4 && (bits & 15) == 0 &&
-          !a.g_idx && !a.tiled && !a.glu && (!a.zp4 || a.n % 8 == 0)))
-        return false;
-    if (a.m <= kI8AlwaysRows) return true;
-    if (a.n >= 4096 && a.k >= 2048) return i8_beats_f16_estimate(a.m, a.k, a.n, a.zp4 != nullptr);
-    return a.m <= kI8FilledRows && i8_rounds_filled(a.m, a.n, a.zp4 != nullptr);
+    const bool takes = a.m > 0 && a.m <= kI8MaxRows && a.group_size % 64 == 0 && a.n % 4 == 0 && a.n >= 4 && (bits & 15) == 0 &&
+                       !a.g_idx && !a.tiled && !a.glu && (!a.zp4 || a.n % 8 == 0);
+    if (takes && a.m <= kI8AlwaysRows && !us) return true;
+    const W4Estimates e = w4_estimates(a.m, a.k, a.n, a.zp4 != nullptr);
+    const bool chosen = takes && (a.m <= kI8AlwaysRows ? true
+                                  : a.n >= 4096 && a.k >= 2048 ? e.i8 < 0.97 * e.f16   // ties go to the f16 tiles (slightly fewer wrong choices on the fitted cases)
+                                                               : a.m <= kI8FilledRows && i8_rounds_filled(a.m, a.n, a.zp4 != nullptr));
+    if (us) *us = chosen ? e.i8 : e.f16;
+    return chosen;
 }
 
 template <int Q, int RT, int CS, int U>

@@ -1,0 +1,73 @@
+"""W4 forward on the six-bit-float matrix cores (large batches; qmatmul_int4.wgsl:40-87) at the edges of its tiles, against
+the float64 product."""
+import numpy as np
+import pytest
+
+import oracle
+from gpu_util import dev, host, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from rumus_amd import ops as o
+    return o
+
+
+# All of these are taken by that kernel.  Rows: blocks of 128 (last one of 1, 77 or 60 rows, or full); columns: tiles of
+# 256 (first two), 384 and 512, with a right edge inside a lane's columns or none; K: an even and an odd number of steps of
+# 64, padded (1500 -> 1536, 1028 and 1090 -> 1152) or not.
+@pytest.mark.parametrize("m,k,n,g,act_order,zeros", [
+    (1409, 1500, 2820, 64, False, "fractional"), (1408, 1024, 2816, 128, True, "integer"),
+    (1100, 1024, 6144, 128, True, "u4"), (1357, 1090, 6148, 64, False, "fractional"), (1400, 1152, 6144, 192, True, "fractional"),
+    (3516, 1028, 4100, 128, False, "fractional"), (3500, 1088, 4096, 64, True, "u4"), (3584, 1024, 4096, 256, False, "integer")])
+def test_six_bit_kernel_at_its_edges(ops, m, k, n, g, act_order, zeros):
+    say(f"w4 forward, six-bit kernel m={m} k={k} n={n} g={g} act_order={act_order} zero-points {zeros}")
+    rng = np.random.default_rng(m + k + n)
+    padded = -(-k // g) * g
+    w = rng.normal(0, 0.02, (k, n)).astype(np.float32)
+    packed, scales, zp = oracle.w4_from_f32(w, g)
+    if zeros != "fractional":
+        zp = np.clip(np.rint(zp), 0, 15).astype(np.float32)
+    scales[0, 3] = 0.0
+    x = rng.normal(0, 1, (m, k)).astype(np.float32)
+    x *= (10.0 ** rng.uniform(-12, 12, (m, 1))).astype(np.float32)
+    # elements that tower over their neighbours; one of them, 2^18 larger, meets weights of exactly zero where zero-points are
+    # integers: what is left of those rows is their small elements
+    perm_np = rng.permutation(k).astype(np.int32) if act_order else np.arange(k, dtype=np.int32)
+    x[5:9, perm_np[700]] *= 1000.0
+    x[m - 1, perm_np[k - 1]] *= 3000.0
+    if zeros != "fractional":
+        z = zp[40 // g].astype(np.uint32)
+        packed[40 // 8] = (packed[40 // 8] & ~np.uint32(15)) | z
+        x[7:11, perm_np[40]] *= np.float32(2.0 ** 18)
+    x[2, 9] = np.inf
+    bias = np.zeros(n, np.float32)
+    d = [dev(packed), dev(scales)]
+    if zeros == "u4":
+        q = np.rint(zp).astype(np.uint32).reshape(zp.shape[0], n // 8, 8)
+        qzeros = (q << (4 * np.arange(8, dtype=np.uint32))).sum(axis=2, dtype=np.uint32).view(np.int32)
+        got = host(ops.qmatmul_int4_zp4(dev(x), *d, dev(qzeros), k, g, bias=dev(bias), perm=dev(perm_np) if act_order else None))
+    elif act_order:
+        got = host(ops.qmatmul_int4_perm(dev(x), *d, dev(zp), k, g, bias=dev(bias), perm=dev(perm_np)))
+    else:
+        got = host(ops.qmatmul_int4(dev(x), *d, dev(zp), k, g, bias=dev(bias)))
+    assert np.isnan(got[2]).all()
+    rows = np.r_[0:2, 3:40, 120:140, m // 2:m // 2 + 30, m - 40:m]
+    xs = x[rows][:, perm_np].astype(np.float64)
+    groups = np.repeat(np.arange(scales.shape[0]), g)[:k]
+    q = oracle.w4_unpack(packed, k).astype(np.float64)
+    z = np.clip(np.rint(zp), 0, 15)[groups].astype(np.float64)
+    rest = zp[groups] - z
+    s = scales[groups].astype(np.float64)
+    exact = xs @ ((q - z - rest) * s)
+    terms = np.abs(xs) @ ((np.abs(q - z) + np.abs(rest)) * np.abs(s))
+    # sums: five additions and one change of scale per step of 64, two additions per group for the zero-points' rest, each within
+    # 2^-23 of what has been added up; values within 2^-24 of the largest of 32 (2^-39 where one of them towers), under
+    # 4 2^-23 of ordinary terms, and their bf16 thirds in the rest's products another 2^-23
+    steps = padded // 64
+    bound = (6 * steps + 2 * scales.shape[0] + 8) * 2.0 ** -23
+    err = np.abs(got[rows] - exact) / (terms + 1e-300)
+    say(f"    worst error / bound {err.max() / bound:.3f}")
+    assert (err <= bound).all()
