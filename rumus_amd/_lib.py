@@ -11,6 +11,7 @@ import subprocess
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "librumus_hip.so")
+HOST_PATH = os.path.join(_HERE, "_host_calls.so")
 CSRC = os.path.join(_HERE, "csrc")
 
 OK, EINVAL, EHIP = 0, 1, 2
@@ -25,11 +26,12 @@ class RumusError(RuntimeError):
 
 
 def build(jobs: int = 8) -> str:
-    """Compile every HIP source into ``librumus_hip.so`` (always recompiles)."""
+    """Compile every HIP source into ``librumus_hip.so`` and the native host calls beside it (always recompiles)."""
     subprocess.check_call(["make", "-C", CSRC, "clean"], stdout=subprocess.DEVNULL)
     subprocess.check_call(["make", "-C", CSRC, f"-j{jobs}"], stdout=subprocess.DEVNULL)
-    if not os.path.exists(LIB_PATH):
-        raise RuntimeError("hipcc did not produce librumus_hip.so")
+    for path in (LIB_PATH, HOST_PATH):
+        if not os.path.exists(path):
+            raise RuntimeError(f"make did not produce {os.path.basename(path)}")
     return LIB_PATH
 
 
@@ -105,6 +107,23 @@ def lib() -> C.CDLL:
             fn.restype, fn.argtypes = res, args
         _lib = handle
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The native side of the most frequent calls (csrc/host_calls.cpp): checks, result tensor, stream and the call in one
+    C++ function each, ``None`` where the general path in ``ops`` is to be taken."""
+    global _host
+    if _host is None:
+        lib()
+        if not os.path.exists(HOST_PATH):
+            raise ImportError(f"{HOST_PATH} is missing: `make -C rumus_amd/csrc` builds it; there is no fallback path")
+        import torch  # noqa: F401  (its libraries have to be loaded first)
+        from . import _host_calls
+        _host = _host_calls
+    return _host
 
 
 def check(status: int) -> None:

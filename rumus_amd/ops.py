@@ -37,6 +37,11 @@ def _opt(t, dtype, name):
     return None if t is None else _dev(t, dtype, name)
 
 
+def _native(name: str, *args):
+    """The call through its native front end, or None: then the general path below checks, allocates and calls."""
+    return getattr(_lib._host or _lib.host(), name)(*args)
+
+
 def w4_geometry(k: int, group_size: int):
     padded_k = ((k + group_size - 1) // group_size) * group_size
     return padded_k, padded_k // group_size
@@ -77,6 +82,8 @@ def q8_dequantize_kn(words: torch.Tensor, k: int, n: int, block_size: int) -> to
 
 
 def matmul_q8(a: torch.Tensor, words: torch.Tensor, k: int, n: int, block_size: int, out=None) -> torch.Tensor:
+    if out is None and (y := _native("matmul_q8", a, words, k, n, block_size)) is not None:
+        return y
     m = a.shape[0]
     if a.dim() != 2 or a.shape[1] != k:
         raise ValueError("matmul: inner dimension mismatch")
@@ -95,6 +102,8 @@ def matmul_q8(a: torch.Tensor, words: torch.Tensor, k: int, n: int, block_size: 
 def matmul_q8_f16(a: torch.Tensor, words: torch.Tensor, k: int, n: int, block_size: int, out=None) -> torch.Tensor:
     """:func:`matmul_q8` on half-precision activations: ``a`` and the result are ``torch.float16``; the product runs in
     the f32 kernels and is rounded to f16 once."""
+    if out is None and (y := _native("matmul_q8_f16", a, words, k, n, block_size)) is not None:
+        return y
     m = a.shape[0]
     if a.dim() != 2 or a.shape[1] != k:
         raise ValueError("matmul: inner dimension mismatch")
@@ -180,6 +189,14 @@ def i8_quantize_cols_t(w: torch.Tensor):
     call("rumus_hip_i8_quantize_cols_t", _dev(w, torch.float32, "w"), wq.data_ptr(), sw.data_ptr(),
          k, n, _stream())
     return wq, sw
+
+
+def i8_linear(x, wq, sw, bias=None):
+    """``i8_quantize_rows`` and ``i8_gemm`` on its result: the W8A8 layer's forward pass."""
+    if (y := _native("int8_linear", x, wq, sw, bias)) is not None:
+        return y
+    xq, sx = i8_quantize_rows(x.contiguous())
+    return i8_gemm(xq, wq, sx, sw, bias)[0]
 
 
 def i8_gemm(xq, wq, sx=None, sw=None, bias=None, want_acc=False, want_y=True, out=None):
@@ -314,6 +331,10 @@ def qmatmul_int4_decode_block(x, packed_t, scales_t, zp_t, k, group_size, norm_w
     """The decode projection with a decoder block's neighbours folded in: ``x`` through RMSNorm with
     ``norm_weight`` (or, ``swiglu``, ``x`` = gate | up rows of ``2k``), ``residual`` ``[m, n]`` added to the result
     (it may be ``out``); one launch."""
+    y = _native("qmatmul_int4_decode_block", x, packed_t, scales_t, zp_t, k, group_size, norm_weight, eps, swiglu, bias,
+                residual, out)
+    if y is not None:
+        return y
     m = x.shape[0]
     n = packed_t.shape[1]
     if x.dim() != 2 or x.shape[1] != (2 * k if swiglu else k):
@@ -370,6 +391,8 @@ def _w4_sizes(who, packed, scales, zp, k, group_size, rows, bias=None, index=Non
 
 
 def _w4_call(name, x, packed, scales, zp, bias, extra, k, group_size, out=None, act=torch.float32):
+    if (y := _native(name, x, packed, scales, zp, bias, extra, k, group_size, out)) is not None:
+        return y
     m = x.shape[0]
     n = packed.shape[1]
     if x.dim() != 2 or x.shape[1] != k:
@@ -408,6 +431,8 @@ def qmatmul_int4_perm_static(x, packed_sorted, scales, zp, k, group_size, bias=N
 
 
 def qmatmul_int4_t(a, packed, scales, zp, k, group_size, out=None):
+    if (y := _native("qmatmul_int4_t", a, packed, scales, zp, k, group_size, out)) is not None:
+        return y
     m, n = a.shape
     if packed.shape[1] != n:
         raise ValueError("qmatmul_int4_t: a must be [m, n]")
@@ -517,6 +542,8 @@ def attention_decode_append(q, k_new, v_new, k_cache, v_cache, pos: int, out=Non
     """``kv_append`` of one new token per sequence at ``pos`` and ``attention`` of its query over positions
     ``0..pos``, without the launch for the append.  ``q``, ``k_new``, ``v_new`` ``[B, 1, H, 128]``, caches
     ``[B, T, H, 128]`` (any strides with the last dim contiguous); returns ``[B, 1, H, 128]``."""
+    if out is None and (y := _native("attention_decode_append", q, k_new, v_new, k_cache, v_cache, pos)) is not None:
+        return y
     import ctypes
     b, n, h, d = q.shape
     if n != 1 or tuple(k_new.shape) != (b, 1, h, d) or tuple(v_new.shape) != (b, 1, h, d):
