@@ -47,6 +47,11 @@ int i8_launch_resident(const int8_t* xq, const int8_t* wq, const float* sx, cons
 int i8_launch_stream(const int8_t* xq, const int8_t* wq, const float* sx, const float* sw, const float* bias, int32_t* acc,
                      float* y, uint32_t m, uint32_t k, uint32_t n, hipStream_t s);
 
+// Whether the f32 x Q8 product takes the f16 kernel with 128 x 128 tiles (q8_gemm.hip), whose activations lie in blocks of
+// kQ8TallRows rows, per block and 64 k: [pair of 32 k][hi, lo][row][four 16-byte pieces, swizzled like an LDS row].
+constexpr uint32_t kQ8TallRows = 128;
+bool q8_gemm_tall(uint32_t m, uint32_t k, uint32_t n, uint32_t bs, uint32_t stride, uint32_t bpc, uint32_t max_shares);
+
 // chunk swizzle of an LDS row: bit0 = b1 ^ b3, bit1 = b2 of the row index
 __device__ __forceinline__ uint32_t row_swizzle(uint32_t row) {
     return (((row >> 1) ^ (row >> 3)) & 1u) | ((row >> 1) & 2u);

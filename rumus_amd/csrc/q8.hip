@@ -583,10 +583,13 @@ static int matmul_q8_mfma(const float* a, const uint32_t* b, float* c, uint32_t 
 
 // Activations for the f16 variant of the block-scale kernel: x f = hi + lo, two f16 planes [2][m][k]
 // (22 bits of every element), f a power of two per row with |x f| < 2^15; sx[row] = 1 / f.
+// TALL: in the order of q8_gemm_tall's kernel instead (i8_gemm.h), k % 64 == 0.
+template <bool TALL>
 __global__ __launch_bounds__(256) void q8_split_rows_f16_kernel(const float* __restrict__ a, _Float16* __restrict__ planes,
                                                                 float* __restrict__ sx, uint32_t m, uint32_t k) {
     __shared__ uint32_t red[4];
-    const uint32_t row = blockIdx.x, tid = threadIdx.x;
+    // TALL: neighbouring rows share cache lines of the planes, so they go to one die's L2
+    const uint32_t row = TALL ? xcd_contiguous(blockIdx.x, m) : blockIdx.x, tid = threadIdx.x;
     const float* ar = a + (uint64_t)row * k;                   // k % 4 == 0
     const bool cached = k <= 1024u * kSplitCache;
     float4 cache[kSplitCache];
@@ -599,6 +602,7 @@ __global__ __launch_bounds__(256) void q8_split_rows_f16_kernel(const float* __r
         sx[row] = poisoned ? __uint_as_float(0x7FC00000u) : nothing ? 0.0f : __uint_as_float((ebits - 14u) << 23);
     _Float16* hi = planes + (uint64_t)row * k;
     _Float16* lo = planes + ((uint64_t)m + row) * k;
+    const uint32_t in = row % kQ8TallRows, m0 = row - in, rows = min(kQ8TallRows, m - m0), swizzle = row_swizzle(in);
     typedef _Float16 v4h __attribute__((ext_vector_type(4)));
     auto emit = [&](uint32_t j, const float4& v) {
         const float xv[4] = {v.x, v.y, v.z, v.w};
@@ -609,8 +613,16 @@ __global__ __launch_bounds__(256) void q8_split_rows_f16_kernel(const float* __r
             h[e] = (_Float16)t;
             l[e] = (_Float16)(t - (float)h[e]);
         }
-        *reinterpret_cast<v4h*>(hi + j) = v4h{h[0], h[1], h[2], h[3]};
-        *reinterpret_cast<v4h*>(lo + j) = v4h{l[0], l[1], l[2], l[3]};
+        if constexpr (TALL) {
+            // f16 elements: the block's start, the step, the pair, the row, the piece and the place in it
+            _Float16* at = planes + (uint64_t)m0 * k * 2 + (uint64_t)(j / 64) * rows * 128 + (j / 32 % 2) * rows * 64 + in * 32 +
+                           (((j / 8) ^ swizzle) & 3) * 8 + j % 8;
+            *reinterpret_cast<v4h*>(at) = v4h{h[0], h[1], h[2], h[3]};
+            *reinterpret_cast<v4h*>(at + rows * 32) = v4h{l[0], l[1], l[2], l[3]};
+        } else {
+            *reinterpret_cast<v4h*>(hi + j) = v4h{h[0], h[1], h[2], h[3]};
+            *reinterpret_cast<v4h*>(lo + j) = v4h{l[0], l[1], l[2], l[3]};
+        }
     };
     if (cached) {
 #pragma unroll
@@ -647,7 +659,9 @@ static int matmul_q8_mfma_blocks(const float* a, const uint32_t* b, float* c, ui
     // exact digit planes on the int8 matrix cores
     if (bs <= 64 || m > 64) {
         _Float16* halves = reinterpret_cast<_Float16*>(ws);    // the same 4 m k bytes
-        hipLaunchKernelGGL(q8_split_rows_f16_kernel, dim3(m), dim3(256), 0, s, a, halves, sxp, m, k);
+        if (q8_gemm_tall(m, k, n, bs, stride, bpc, max_shares))
+            hipLaunchKernelGGL(q8_split_rows_f16_kernel<true>, dim3(m), dim3(256), 0, s, a, halves, sxp, m, k);
+        else hipLaunchKernelGGL(q8_split_rows_f16_kernel<false>, dim3(m), dim3(256), 0, s, a, halves, sxp, m, k);
         if (int rc = check_launch("q8_split_rows_f16_kernel")) return rc;
         return q8_gemm_blocks_f16(halves, sxp, b, c, m, k, n, bs, stride, bpc, part, max_shares, s);
     }

@@ -31,6 +31,40 @@ namespace rumus {
 
 constexpr int kQ8GemmPlanes = 4;
 
+// Results of a wave's TM x TN tiles of 32 x 32 back to their rows' scale: register r of lane l is row 8 (r/4) + 4 (l/32) +
+// r%4, column l%32.  The row factors come first, all in flight at once: a load in front of every store costs a trip to
+// memory per row (a load's wait includes the stores before it).
+template <int TM, int TN>
+__device__ __forceinline__ void q8_store_tiles(const float (&out)[TM][TN][16], const float* __restrict__ sx, float* __restrict__ c,
+                                               uint32_t M, uint32_t N, uint32_t m0, uint32_t n0, uint32_t lane) {
+    const uint32_t col_l = lane & 31, row_l = (lane >> 5) * 4;
+    float f[TM][16];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) f[i][r] = sx[min(m0 + i * 32 + 8 * (r / 4) + row_l + (r % 4), M - 1)];
+    const bool whole = m0 + 32 * TM <= M;
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        const uint32_t col = n0 + j * 32 + col_l;
+        if (col >= N) continue;
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            if (whole) {
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    c[(uint64_t)(m0 + i * 32 + 8 * (r / 4) + row_l + (r % 4)) * N + col] = out[i][j][r] * f[i][r];
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const uint32_t row = m0 + i * 32 + 8 * (r / 4) + row_l + (r % 4);
+                    if (row < M) c[(uint64_t)row * N + col] = out[i][j][r] * f[i][r];
+                }
+            }
+        }
+    }
+}
+
 template <int WM, int WN, int TN, int NS>
 __global__ __launch_bounds__(64 * WM * WN, 2) void q8_gemm_blocks_kernel(
     const int8_t* __restrict__ planes, const float* __restrict__ sx, const uint8_t* __restrict__ b,
@@ -121,11 +155,11 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void q8_gemm_blocks_kernel(
     const uint32_t s_off = A_BYTES + B_BYTES + (wn * TN * 32 + fr) * 4;
 
     v16i acc[P][TN];
-    float out[TN][16];
+    float out[1][TN][16];
 #pragma unroll
     for (int j = 0; j < TN; j++) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) out[j][r] = 0.0f;
+        for (int r = 0; r < 16; r++) out[0][j][r] = 0.0f;
 #pragma unroll
         for (int p = 0; p < P; p++)
 #pragma unroll
@@ -173,8 +207,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void q8_gemm_blocks_kernel(
                     for (int r = 0; r < 16; r++) {
                         const int lo = acc[1][j][r] * 128 + acc[0][j][r];
                         const int hi = acc[3][j][r] * 128 + acc[2][j][r];
-                        out[j][r] = fmaf((float)hi, s_hi, out[j][r]);
-                        out[j][r] = fmaf((float)lo, s_lo, out[j][r]);
+                        out[0][j][r] = fmaf((float)hi, s_hi, out[0][j][r]);
+                        out[0][j][r] = fmaf((float)lo, s_lo, out[0][j][r]);
 #pragma unroll
                         for (int p = 0; p < P; p++) acc[p][j][r] = 0;
                     }
@@ -185,19 +219,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void q8_gemm_blocks_kernel(
     }
     RUMUS_WAIT_VMCNT(0);         // no LDS-DMA write may outlive the workgroup
 
-    // ---- rows back to their scale: register r of lane l is row 8 (r/4) + 4 (l/32) + r%4, column l%32 ----
-    const uint32_t col_l = lane & 31, row_l = (lane >> 5) * 4;
-    c += (uint64_t)blockIdx.y * M * N;                         // partial sums of K share y when K is split
-#pragma unroll
-    for (int j = 0; j < TN; j++) {
-        const uint32_t col = n0 + (wn * TN + j) * 32 + col_l;
-        if (col >= N) continue;
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const uint32_t row = m0 + wm * 32 + 8 * (r / 4) + row_l + (r % 4);
-            if (row < M) c[(uint64_t)row * N + col] = out[j][r] * sx[row];
-        }
-    }
+    // partial sums of K share y when K is split
+    q8_store_tiles<1, TN>(out, sx, c + (uint64_t)blockIdx.y * M * N, M, N, m0 + wm * 32, n0 + wn * TN * 32, lane);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -229,6 +252,19 @@ __device__ __forceinline__ void q8_bytes_to_f16(const v4i& w, v8h& first, v8h& s
     }
     first = v8h{h[0][0], h[0][1], h[1][0], h[1][1], h[2][0], h[2][1], h[3][0], h[3][1]};
     second = v8h{h[4][0], h[4][1], h[5][0], h[5][1], h[6][0], h[6][1], h[7][0], h[7][1]};
+}
+
+// 8 int8 (two words) -> one B operand
+__device__ __forceinline__ v8h q8_half_to_f16(uint32_t w0, uint32_t w1) {
+    const v2h off = {(_Float16)1152.0f, (_Float16)1152.0f};
+    const uint32_t w[2] = {w0 ^ 0x80808080u, w1 ^ 0x80808080u};           // q + 128 in every byte
+    v2h h[4];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        h[2 * i] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, w[i], 0x04010400u)) - off;
+        h[2 * i + 1] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, w[i], 0x04030402u)) - off;
+    }
+    return v8h{h[0][0], h[0][1], h[1][0], h[1][1], h[2][0], h[2][1], h[3][0], h[3][1]};
 }
 
 template <int WM, int WN, int TN, int NS, bool EVERY>
@@ -322,12 +358,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void q8_gemm_blocks_f16_kernel(
     const uint32_t s_off = A_BYTES + B_BYTES + (wn * TN * 32 + fr) * 4;
 
     v16f acc[TN];
-    float out[TN][16];
+    float out[1][TN][16];
 #pragma unroll
     for (int j = 0; j < TN; j++)
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-            out[j][r] = 0.0f;
+            out[0][j][r] = 0.0f;
             acc[j][r] = 0.0f;
         }
     const v16f zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -394,7 +430,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void q8_gemm_blocks_f16_kernel(
                     const float sc = live ? __half2float(__ushort_as_half((unsigned short)(header & 0xFFFFu))) : 0.0f;
 #pragma unroll
                     for (int r = 0; r < 16; r++) {
-                        out[j][r] = fmaf(acc[j][r], sc, out[j][r]);
+                        out[0][j][r] = fmaf(acc[j][r], sc, out[0][j][r]);
                         if (!EVERY) acc[j][r] = 0.0f;
                     }
                 }
@@ -404,18 +440,212 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void q8_gemm_blocks_f16_kernel(
     }
     RUMUS_WAIT_VMCNT(0);         // no LDS-DMA write may outlive the workgroup
 
-    const uint32_t col_l = lane & 31, row_l = (lane >> 5) * 4;
-    c += (uint64_t)blockIdx.y * M * N;                         // partial sums of K share y when K is split
+    // partial sums of K share y when K is split
+    q8_store_tiles<1, TN>(out, sx, c + (uint64_t)blockIdx.y * M * N, M, N, m0 + wm * 32, n0 + wn * TN * 32, lane);
+}
+
+// ---------------------------------------------------------------------------------------------------
+// The f16 variant for batches that fill the chip with 128 x 128 tiles: a wave owns 64 x 64 outputs instead of 32 x 64,
+// so that a converted B fragment (10 vector instructions) serves four MFMAs instead of two and an A fragment four
+// instead of two, and a step issues 40 vector instructions and 10 LDS reads per 16 MFMAs.  One wave per SIMD, so every
+// latency has to be hidden inside it: a step is one pair of 32 k, and while its 16 MFMAs run the wave reads the next
+// step's fragments into a second set of registers (the loop is unrolled over the two sets) and converts its bytes; NS
+// steps are on their way to LDS meanwhile.  Products and sums in the order of the kernel above: the same bits.
+// What bounds it is the address side of the loads: a wave's load that touches 64 cache lines (headers, 4 bytes each) costs
+// the compute unit eight times one that reads 1 KB in a row.  Hence steps of 64 k (64 bytes of a column at a time), headers
+// only with the last step of a block, and activations laid out by q8_split_rows_f16_kernel<true> as a step wants them.
+// LDS per step: A [pair][plane][128 rows][64 bytes], B [128 columns][64 bytes], headers [128] (blocks of 32: [pair][128]).
+__device__ __forceinline__ uint32_t q8_lds_offset(const void* p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p; }
+// Loads into LDS, spelled out: the compiler would make every LDS read wait for all of them (it cannot see that they go
+// to another stage); the barrier that publishes a stage waits for them explicitly.
+__device__ __forceinline__ void q8_lds_load16(uint32_t to, const void* from, uint32_t lane_bytes) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(lane_bytes), "s"(from) : "memory");
+}
+__device__ __forceinline__ void q8_lds_load4(uint32_t to, const void* from, uint32_t lane_bytes) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(to), "v"(lane_bytes), "s"(from) : "memory");
+}
+
+constexpr int kTallA = 4 * kQ8TallRows * 64, kTallB = 128 * 64, kTallStage = kTallA + kTallB + 2 * 128 * 4;
+constexpr int kTallStages = 3;
+
+template <bool EVERY>
+__global__ __launch_bounds__(256, 2) void q8_gemm_tall_f16_kernel(
+    const _Float16* __restrict__ planes, const float* __restrict__ sx, const uint8_t* __restrict__ b,
+    float* __restrict__ c, uint32_t M, uint32_t K, uint32_t N, uint32_t bs, uint32_t bs_magic,
+    uint32_t stride_bytes, uint32_t bpc, uint32_t tiles_m, uint32_t tiles_n) {
+    constexpr int NS = kTallStages, LOADS = 11;
+    static_assert(kQ8TallRows == 128, "two waves of 64 rows");
+    extern __shared__ __attribute__((aligned(16))) int8_t lds[];   // [NS][kTallStage]
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wm = wave >> 1, wn = wave & 1;
+    const uint32_t tile = xcd_contiguous(blockIdx.x, tiles_m * tiles_n);
+    const uint32_t m0 = (tile % tiles_m) * 128, n0 = (tile / tiles_m) * 128;
+    const uint32_t rows = min(128u, M - m0);
+
+    // ---- loads into LDS: wave w brings pair w / 2 of plane w % 2 (16 rows per load), 32 columns of B, 64 headers -----
+    const uint32_t lr = lane >> 2;
+    const uint8_t* const a_base = reinterpret_cast<const uint8_t*>(planes) + (uint64_t)m0 * K * 4;
+    uint32_t a_at[8];
 #pragma unroll
-    for (int j = 0; j < TN; j++) {
-        const uint32_t col = n0 + (wn * TN + j) * 32 + col_l;
-        if (col >= N) continue;
+    for (int i = 0; i < 8; i++) a_at[i] = (wave * rows + min(i * 16 + lr, rows - 1)) * 64 + (lane & 3) * 16;
+    const uint32_t lc = ((lane & 3) ^ row_swizzle(lr)) & 3;
+    uint32_t b_at[2];                                          // byte offsets; the caller keeps the weight below 4 GB
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const uint32_t row = m0 + wm * 32 + 8 * (r / 4) + row_l + (r % 4);
-            if (row < M) c[(uint64_t)row * N + col] = out[j][r] * sx[row];
+    for (int i = 0; i < 2; i++) b_at[i] = min(n0 + wave * 32 + i * 16 + lr, N - 1) * bpc * stride_bytes;
+    const uint32_t s_at = min(n0 + wn * 64 + lane, N - 1) * bpc * stride_bytes;
+    const uint32_t lds0 = q8_lds_offset(lds);
+    const uint32_t steps = K / 64;
+    // the loads of step `at`, in two parts of 8 and 3 per wave; past the end the last step again, into a stage nobody reads
+    auto issue_a = [&](uint32_t at, uint32_t stage, int i) {
+        const uint32_t kt = min(at, steps - 1);
+        q8_lds_load16(lds0 + stage * kTallStage + (8 * wave + i) * 1024, a_base + (uint64_t)kt * rows * 256, a_at[i]);
+    };
+    auto issue_b = [&](uint32_t at, uint32_t stage) {
+        const uint32_t k0 = min(at, steps - 1) * 64, to = lds0 + stage * kTallStage + kTallA;
+        const uint32_t blk = __umulhi(k0, bs_magic);
+        if (EVERY) {                                           // two blocks of 36 bytes
+            const uint32_t at_b = (lc >> 1) * 36 + (lc & 1) * 16 + 4;
+#pragma unroll
+            for (int i = 0; i < 2; i++) q8_lds_load16(to + (2 * wave + i) * 1024, b + (uint64_t)blk * 36, b_at[i] + at_b);
+            q8_lds_load4(to + kTallB + wave * 256, b + (uint64_t)(blk + wm) * 36, s_at);
+        } else {
+            const uint32_t in = k0 - blk * bs;
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                q8_lds_load16(to + (2 * wave + i) * 1024, b + (uint64_t)(blk * stride_bytes + 4 + in), b_at[i] + lc * 16);
+            // wanted with a block's last step, from the first two waves; otherwise every lane reads one and the same word
+            const bool wanted = in + 64 == bs && wm == 0;
+            q8_lds_load4(to + kTallB + wave * 256, b + (uint64_t)blk * stride_bytes, wanted ? s_at : 0u);
         }
+    };
+
+    // ---- fragments: lane (row or column fr, half fh); MFMA i of a pair takes k = 16 fh + 8 i .. + 7 of it ------------
+    const uint32_t fr = lane & 31, fh = lane >> 5, fsw = row_swizzle(fr);
+    uint32_t a_off[2], b_off[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) a_off[i] = (wm * 64 + fr) * 64 + (((2 * fh + i) ^ fsw) & 3) * 16;
+#pragma unroll
+    for (int p = 0; p < 2; p++) b_off[p] = kTallA + (wn * 64 + fr) * 64 + (((2 * p + fh) ^ fsw) & 3) * 16;
+    const uint32_t s_off = kTallA + kTallB + (wn * 64 + fr) * 4;
+
+    // Quad q of a pair: the four MFMAs of plane q / 2 and half q % 2.  The registers of a fragment are refilled with the
+    // next pair's as soon as its quad is issued, three quads before they are wanted again.
+    v8h fa[4][2];                                              // [quad][row tile]
+    v8h fb[2][2];                                              // [half][column tile]
+    v4i raw[2];                                                // the next pair's bytes
+    uint32_t header[2];
+    v16f acc[2][2];
+    float out[2][2][16];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                acc[i][j][r] = 0.0f;
+                out[i][j][r] = 0.0f;
+            }
+    const v16f zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+
+    auto read_a = [&](const int8_t* base, int p, int q) {
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+            fa[q][i] = *reinterpret_cast<const v8h*>(base + a_off[q & 1] + ((2 * p + (q >> 1)) * 128 + i * 32) * 64);
+    };
+    auto read_b = [&](const int8_t* base, int p) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) raw[j] = *reinterpret_cast<const v4i*>(base + b_off[p] + j * 32 * 64);
+    };
+    auto read_header = [&](const int8_t* base, int p) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) header[j] = *reinterpret_cast<const uint32_t*>(base + s_off + (EVERY ? p * 512 : 0) + j * 128);
+    };
+    auto convert = [&](int h) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) fb[h][j] = q8_half_to_f16((uint32_t)raw[j][2 * h], (uint32_t)raw[j][2 * h + 1]);
+    };
+    auto quad = [&](int q, bool first) {
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[q][i], fb[q & 1][j], first ? zero : acc[i][j], 0, 0, 0);
+    };
+    auto fold = [&]() {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const float sc = __half2float(__ushort_as_half((unsigned short)(header[j] & 0xFFFFu)));
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) out[i][j][r] = fmaf(acc[i][j][r], sc, out[i][j][r]);
+        }
+    };
+    // One pair.  `next` is where pair `np` after it lies; its share of the loads into `stage` goes out between the MFMAs.
+    auto pair = [&](const int8_t* next, int np, bool first, bool second, uint32_t at, uint32_t stage) {
+        quad(0, first);
+        convert(1);
+        read_a(next, np, 0);
+        if (second) { issue_a(at, stage, 0); issue_a(at, stage, 1); }
+        else issue_b(at, stage);
+        read_b(next, np);
+        __builtin_amdgcn_sched_barrier(0);
+        quad(1, false);
+        read_a(next, np, 1);
+        if (second) { issue_a(at, stage, 2); issue_a(at, stage, 3); }
+        __builtin_amdgcn_sched_barrier(0);
+        quad(2, false);
+        read_a(next, np, 2);
+        if (second) { issue_a(at, stage, 4); issue_a(at, stage, 5); }
+        __builtin_amdgcn_sched_barrier(0);
+        quad(3, false);
+        convert(0);
+        read_a(next, np, 3);
+        if (second) { issue_a(at, stage, 6); issue_a(at, stage, 7); }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) issue_a(s, s, i);
+        if (s + 1 < NS) issue_b(s, s);                         // (the last one's goes out with the first pair)
     }
+    // all loads of a step have arrived when only those of the younger steps are outstanding
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * LOADS - 3) : "memory");
+    __builtin_amdgcn_s_barrier();
+    read_b(lds, 0);
+#pragma unroll
+    for (int q = 0; q < 4; q++) read_a(lds, 0, q);
+    convert(0);
+    uint32_t stage = 0;
+    const uint32_t period = EVERY ? 1 : bs / 64;               // steps of a block
+    for (uint32_t kt = 0; kt < steps;) {
+        if (!EVERY)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) acc[i][j] = zero;
+        for (uint32_t left = period; left > 0; left--, kt++) {
+            const int8_t* base = lds + stage * kTallStage;
+            if (EVERY) read_header(base, 0);
+            pair(base, 1, EVERY, false, kt + NS - 1, stage == 0 ? NS - 1 : stage - 1);
+            if (EVERY) fold();
+            read_header(base, EVERY ? 1 : 0);
+            // The step's fragments are in registers (lgkmcnt 0), in every wave past the barrier: its stage takes step kt + NS.
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * LOADS) : "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            const uint32_t freed = stage;
+            stage = stage + 1 == NS ? 0 : stage + 1;
+            pair(lds + stage * kTallStage, 0, EVERY, true, kt + NS, freed);
+            if (EVERY) fold();
+        }
+        if (!EVERY) fold();
+    }
+    RUMUS_WAIT_VMCNT(0);         // no load into LDS may outlive the workgroup
+    q8_store_tiles<2, 2>(out, sx, c, M, N, m0 + wm * 64, n0 + wn * 64, lane);
 }
 
 // c = sum over the K shares of their partial results, in share order
@@ -426,6 +656,19 @@ __global__ __launch_bounds__(256) void q8_gemm_add_shares_kernel(const float* __
     float v = part[i];
     for (uint32_t z = 1; z < shares; z++) v += part[(uint64_t)z * count + i];
     c[i] = v;
+}
+
+// Too few tiles for the chip: K is shared out over workgroups as well, in whole fold periods of at least 8 steps of 64 k.
+struct Q8Shares { uint32_t shares, steps_per; };
+static Q8Shares q8_shares(uint32_t tiles, uint32_t ksteps, uint32_t period, uint32_t max_shares) {
+    Q8Shares z{1, ksteps};
+    if (max_shares && tiles < 256) {
+        const uint32_t unit = period * ceil_div(8, period);
+        z.shares = min(min(max_shares, 512 / tiles), max(1u, ksteps / unit));
+        z.steps_per = ceil_div(ceil_div(ksteps, z.shares), unit) * unit;
+        z.shares = ceil_div(ksteps, z.steps_per);
+    }
+    return z;
 }
 
 template <int WM, int WN, int TN, int NS>
@@ -444,15 +687,7 @@ static int launch_q8_gemm_blocks(const int8_t* planes, const float* sx, const ui
     }
     const uint32_t tm = ceil_div(m, 32 * WM), tn = ceil_div(n, 32 * TN * WN);
     const uint32_t magic = (uint32_t)((0x100000000ull + bs - 1) / bs);
-    // too few tiles for the chip: K is shared out as well, in whole fold periods of at least 8 steps
-    const uint32_t ksteps = ceil_div(k, kBK);
-    uint32_t shares = 1, steps_per = ksteps;
-    if (part && tm * tn < 256) {
-        const uint32_t unit = period * ceil_div(8, period);
-        shares = min(min(max_shares, 512 / (tm * tn)), max(1u, ksteps / unit));
-        steps_per = ceil_div(ceil_div(ksteps, shares), unit) * unit;
-        shares = ceil_div(ksteps, steps_per);
-    }
+    const auto [shares, steps_per] = q8_shares(tm * tn, ceil_div(k, kBK), period, part ? max_shares : 0);
     hipLaunchKernelGGL((q8_gemm_blocks_kernel<WM, WN, TN, NS>), dim3(tm * tn, shares), dim3(64 * WM * WN),
                        lds_bytes, s, planes, sx, reinterpret_cast<const uint8_t*>(b), shares > 1 ? part : c, m, k, n, bs,
                        magic, stride * 4, bpc, period, tm, tn, steps_per);
@@ -479,14 +714,7 @@ static int launch_q8_gemm_blocks_f16(const _Float16* planes, const float* sx, co
     const uint32_t tm = ceil_div(m, 32 * WM), tn = ceil_div(n, 32 * TN * WN);
     const uint32_t magic = (uint32_t)((0x100000000ull + bs - 1) / bs);
     const uint32_t period = bs / 32;                           // pairs of 32 k per block: f32 sums need no earlier fold
-    const uint32_t ksteps = ceil_div(k, 64);
-    uint32_t shares = 1, steps_per = ksteps;
-    if (part && tm * tn < 256) {
-        const uint32_t unit = period * ceil_div(8, period);
-        shares = min(min(max_shares, 512 / (tm * tn)), max(1u, ksteps / unit));
-        steps_per = ceil_div(ceil_div(ksteps, shares), unit) * unit;
-        shares = ceil_div(ksteps, steps_per);
-    }
+    const auto [shares, steps_per] = q8_shares(tm * tn, ceil_div(k, 64), period, part ? max_shares : 0);
     hipLaunchKernelGGL((q8_gemm_blocks_f16_kernel<WM, WN, TN, NS, EVERY>), dim3(tm * tn, shares), dim3(64 * WM * WN),
                        lds_bytes, s, planes, sx, reinterpret_cast<const uint8_t*>(b), shares > 1 ? part : c, m, k, n, bs,
                        magic, stride * 4, bpc, period, tm, tn, steps_per);
@@ -496,8 +724,44 @@ static int launch_q8_gemm_blocks_f16(const _Float16* planes, const float* sx, co
     return check_launch("q8_gemm_add_shares_kernel");
 }
 
+template <bool EVERY>
+static int launch_q8_gemm_tall_f16(const _Float16* planes, const float* sx, const uint32_t* b, float* c, uint32_t m, uint32_t k,
+                                   uint32_t n, uint32_t bs, uint32_t stride, uint32_t bpc, hipStream_t s) {
+    constexpr size_t lds_bytes = (size_t)kTallStages * kTallStage;
+    static_assert(lds_bytes <= 160 * 1024, "more LDS than a compute unit has");
+    static bool attr_set = false;   // benign race: setting the attribute is idempotent
+    if (!attr_set) {
+        if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_gemm_tall_f16_kernel<EVERY>),
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes), "hipFuncSetAttribute"))
+            return rc;
+        attr_set = true;
+    }
+    const uint32_t tm = ceil_div(m, 128), tn = ceil_div(n, 128);
+    hipLaunchKernelGGL(q8_gemm_tall_f16_kernel<EVERY>, dim3(tm * tn), dim3(256), lds_bytes, s, planes, sx,
+                       reinterpret_cast<const uint8_t*>(b), c, m, k, n, bs, (uint32_t)((0x100000000ull + bs - 1) / bs), stride * 4, bpc,
+                       tm, tn);
+    return check_launch("q8_gemm_tall_f16_kernel");
+}
+
 #define RUMUS_Q8_LAUNCH_F16(WM, WN, TN, NS, EV) \
     launch_q8_gemm_blocks_f16<WM, WN, TN, NS, EV>(planes, sx, b, c, m, k, n, bs, stride, bpc, part, max_shares, s)
+
+// More than 64 rows and k % 64 == 0, where the estimate of the 128 x 128 tiles (a round of 256 workgroups takes 0.95 to 1.15
+// us per 64 k, by how full it is) is below that of the 64 x 128 ones (a round of 512 takes 1.5 us per 64 k, up to 256 alone
+// 1.06; few of them share K and add up).  Both measured over 180 products of 65 to 2048 rows, blocks of 32 and 128: the
+// choice is 0.03 % off the better one on average and 2 % at worst, and where it takes these tiles they are 1.1 to 1.4 times
+// as fast (1000 x 4096 x 4096, blocks of 128: 103 -> 80 us; 2048 x 4096 x 11008, blocks of 128 558 -> 433, of 32 582 -> 478).
+bool q8_gemm_tall(uint32_t m, uint32_t k, uint32_t n, uint32_t bs, uint32_t stride, uint32_t bpc, uint32_t max_shares) {
+    if (!(m > 64 && k % 64 == 0 && (bs == 32 || bs % 64 == 0) && (uint64_t)n * bpc * stride * 4 < (1ull << 32))) return false;
+    const uint64_t tall = (uint64_t)ceil_div(m, kQ8TallRows) * ceil_div(n, 128), flat = (uint64_t)ceil_div(m, 64) * ceil_div(n, 128);
+    const uint32_t last = (uint32_t)(tall % 256), steps = k / 64;
+    const double tall_us = steps * ((double)(tall / 256) * 1.15 + (last == 0 ? 0.0 : last <= 128 ? 0.95 : 0.95 + 0.2 * (last - 128) / 128));
+    const Q8Shares z = flat < 256 ? q8_shares((uint32_t)flat, steps, bs / 32, max_shares) : Q8Shares{1, steps};
+    const uint64_t groups = flat * z.shares, rest = groups % 512;
+    double flat_us = z.steps_per * ((double)(groups / 512) * 1.5 + (rest == 0 ? 0.0 : rest <= 256 ? 1.06 : 1.5));
+    if (z.shares > 1) flat_us += 2.0 + (double)m * n * 4e-6 * (z.shares + 1) / 4;
+    return tall_us < flat_us;
+}
 
 // planes: [2][m][k] f16 (hi, lo), sx: [m] the rows' 1 / f.  Same preconditions as q8_gemm_blocks.
 // Measured at 4096 x 11008: up to 32 rows one 32-row tile per workgroup, beyond that 64 x 128 tiles,
@@ -507,6 +771,9 @@ static int launch_q8_gemm_blocks_f16(const _Float16* planes, const float* sx, co
 int q8_gemm_blocks_f16(const _Float16* planes, const float* sx, const uint32_t* b, float* c, uint32_t m, uint32_t k,
                        uint32_t n, uint32_t bs, uint32_t stride, uint32_t bpc, float* part, uint32_t max_shares,
                        hipStream_t s) {
+    if (q8_gemm_tall(m, k, n, bs, stride, bpc, part ? max_shares : 0))
+        return bs == 32 ? launch_q8_gemm_tall_f16<true>(planes, sx, b, c, m, k, n, bs, stride, bpc, s)
+                        : launch_q8_gemm_tall_f16<false>(planes, sx, b, c, m, k, n, bs, stride, bpc, s);
     if (bs == 32) return m <= 32 ? RUMUS_Q8_LAUNCH_F16(1, 4, 1, 4, true) : RUMUS_Q8_LAUNCH_F16(2, 2, 2, 3, true);
     return m <= 32 ? RUMUS_Q8_LAUNCH_F16(1, 4, 1, 4, false) : RUMUS_Q8_LAUNCH_F16(2, 2, 2, 3, false);
 }
