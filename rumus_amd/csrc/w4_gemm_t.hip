@@ -121,7 +121,7 @@ constexpr int kTSlots = 12;                                   // wave-wide loads
 // The raw tile of grad_y of step t is dead once it has been converted (during step t - 1), the weights and tables of
 // step t are read during step t: one slot fewer for grad_y than for the rest, at the same depth of loads in flight.
 constexpr size_t w4t_lds_bytes(int stages) {
-    return (size_t)(stages - 1) * kTRawGy + (size_t)stages * kTRawWt + 2 * kTAbuf + 64 * sizeof(float);
+    return (size_t)(stages - 1) * kTRawGy + (size_t)stages * kTRawWt + 2 * kTAbuf + 2 * 64 * sizeof(float);
 }
 
 // KW = waves per workgroup = 32-column slices of k per tile: 4 when groups are multiples of 128, 2 for
@@ -355,24 +355,38 @@ __global__ __launch_bounds__(64 * KW, 2) void w4t_gemm_kernel(
     // ---- c[row]: the KW conversion threads of a row are neighbours in a wave ---------------------------
     if (KW >= 2) csum += __shfl_xor(csum, 1);
     if (KW == 4) csum += __shfl_xor(csum, 2);
-    if (tid % KW == 0) lds_c[s_row] = csum;
+    // and 1 / f_row = 2^(e - 140), from the bits of f (f = 2^(140 - e), biased exponent 267 - e), fetched when the kernel began: a
+    // load in front of every store would cost a trip to memory per row (its wait includes the stores before it)
+    if (tid % KW == 0) {
+        lds_c[s_row] = csum;
+        lds_c[64 + s_row] = frow_raw != frow_raw ? frow_raw
+                            : frow_raw == 0.0f   ? 0.0f
+                                                 : __uint_as_float((254u - (__float_as_uint(frow_raw) >> 23)) << 23);
+    }
     __syncthreads();
 
     // ---- register r of lane l is row 8 (r/4) + 4 (l/32) + r%4, column l%32 of its 32 x 32 tile -------
-    float* dst_out = out + (uint64_t)blockIdx.z * m * k;
     const uint32_t col = k0 + 32 * wave + bc;
     const float s_big = sgrp[g];
-    if (col < k) {
+    if (col >= k) return;
+    float* const dst_out = out + (uint64_t)blockIdx.z * m * k + (uint64_t)m0 * k + col;
+    auto value = [&](int i, int r, uint32_t lr) { return ((acc[i][r] - lds_c[lr]) * lds_c[64 + lr]) * s_big; };
+    const uint32_t live = m - m0;
+    if (live >= 32u * RTILES) {
 #pragma unroll
         for (int i = 0; i < RTILES; i++)
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                const uint32_t lr = 32 * i + 8 * (r / 4) + 4 * fh + (r % 4), row = m0 + lr;
-                if (row >= m) continue;
-                const float f = rowf[row];
-                // 1 / f_row = 2^(e - 140): from the bits of f (f = 2^(140 - e), biased exponent 267 - e)
-                const float finv = f != f ? f : f == 0.0f ? 0.0f : __uint_as_float((254u - (__float_as_uint(f) >> 23)) << 23);
-                dst_out[(uint64_t)row * k + col] = ((acc[i][r] - lds_c[lr]) * finv) * s_big;
+                const uint32_t lr = 32 * i + 8 * (r / 4) + 4 * fh + (r % 4);
+                dst_out[(uint64_t)lr * k] = value(i, r, lr);
+            }
+    } else {
+#pragma unroll
+        for (int i = 0; i < RTILES; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const uint32_t lr = 32 * i + 8 * (r / 4) + 4 * fh + (r % 4);
+                if (lr < live) dst_out[(uint64_t)lr * k] = value(i, r, lr);
             }
     }
 }
