@@ -733,31 +733,41 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
     }
 
     // ---- store -------------------------------------------------------------------------------------------------
+    // All row factors first (rfac holds whole blocks of rows): a load in front of every store would cost a trip to memory per
+    // row, since its wait includes the stores before it.
+    float rf[2][16];                                              // back to the rows' own scale: exact, powers of two
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float4 f = *reinterpret_cast<const float4*>(a.rfac + m0 + (wm * 2 + i) * 32 + 8 * q + 4 * kb);
+            rf[i][4 * q] = f.x; rf[i][4 * q + 1] = f.y; rf[i][4 * q + 2] = f.z; rf[i][4 * q + 3] = f.w;
+        }
     float bv[TN];
 #pragma unroll
     for (int j = 0; j < TN; j++) bv[j] = a.bias && my_col + j < a.n ? a.bias[my_col + j] : 0.0f;
+    if (my_col >= a.n) return;
+    auto put = [&](int i, int r, uint32_t row) __attribute__((always_inline)) {
+        F6Floats<TN> o;
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-        if (my_col < a.n) {
+        for (int j = 0; j < TN; j++) o.v[j] = fmaf(acc[i][j][r] * rf[i][r], sc_cur.v[j], bv[j]);
+        float* p = a.y + (uint64_t)row * a.n + my_col;
+        if (TN != 3 || my_col + TN <= a.n) {
+            f6_cols_store<TN>(p, o);
+        } else {                                                  // the right edge: n % 4 == 0
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const uint32_t row = m0 + (wm * 2 + i) * 32 + 8 * (r / 4) + 4 * kb + (r % 4);
-                if (row >= a.m) continue;
-                const float rf = a.rfac[row];                     // back to the row's own scale: exact, a power of two
-                F6Floats<TN> o;
-#pragma unroll
-                for (int j = 0; j < TN; j++) o.v[j] = fmaf(acc[i][j][r] * rf, sc_cur.v[j], bv[j]);
-                float* p = a.y + (uint64_t)row * a.n + my_col;
-                if (TN != 3 || my_col + TN <= a.n) {
-                    f6_cols_store<TN>(p, o);
-                } else {                                             // the right edge: n % 4 == 0
-#pragma unroll
-                    for (int j = 0; j < TN; j++)
-                        if (my_col + j < a.n) p[j] = o.v[j];
-                }
-            }
+            for (int j = 0; j < TN; j++)
+                if (my_col + j < a.n) p[j] = o.v[j];
         }
-    }
+    };
+    const bool whole = m0 + kF6BM <= a.m;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const uint32_t row = m0 + (wm * 2 + i) * 32 + 8 * (r / 4) + 4 * kb + (r % 4);
+            if (whole || row < a.m) put(i, r, row);
+        }
 }
 
 // Columns per workgroup / 128, and the time of a call in microseconds: workgroups run one per compute unit, in rounds of
