@@ -422,6 +422,20 @@ int rumus_hip_qmatmul_int4_decode_block(const float* x, const float* norm_weight
                                         uint32_t group_size, uint32_t num_groups,
                                         rumus_hip_stream_t stream);
 
+/* EXTENSION: the same for a batch of prompt tokens, on the reference's own
+ * arrays: RMSNorm or SwiGLU on the way in, the residual on the way out, without
+ * kernels of their own.  Only where rumus_hip_qmatmul_int4_block_takes (host
+ * arithmetic) returns 1: large batches, group_size % 64 == 0, k % 8 == 0; EINVAL
+ * otherwise, and unless the buffers are 16-byte aligned and y != x.  Workspace:
+ * that of qmatmul_int4, and with norm_weight or swiglu 4 * m * k + 256 more. */
+int rumus_hip_qmatmul_int4_block_takes(uint32_t m, uint32_t k, uint32_t n, uint32_t group_size);
+int rumus_hip_qmatmul_int4_block(const float* x, const float* norm_weight, float eps, int swiglu,
+                                 const uint32_t* packed, const float* scales,
+                                 const float* zero_points, const float* bias, const float* residual,
+                                 float* y, uint32_t m, uint32_t k, uint32_t n, uint32_t padded_k,
+                                 uint32_t group_size, uint32_t num_groups,
+                                 rumus_hip_stream_t stream);
+
 /* EXTENSION: qmatmul_int4_perm on AWQ storage: zero-points come as qzeros
  * (layout above) instead of f32.  perm may be NULL (plain k order).
  * EINVAL also unless n % 8 == 0. */

@@ -24,7 +24,7 @@ struct W4Args {
     // decode layout (w4_gemv_dot8 only): packed, scales and zp are tile-major copies, tile = 16
     // columns: packed_t[(c*word_rows + r)*16 + j] = packed[r*n + 16*c + j], likewise the metadata
     bool tiled = false;
-    // w4_gemv_dot8 only: x holds rows of 2k floats, gate | up; the activations are silu(gate) * up
+    // w4_gemv_dot8 and w4_gemm_f6 only: x holds rows of 2k floats, gate | up; the activations are silu(gate) * up
     bool glu = false;
     // w4_gemm_tile only (set by its launcher): activations split into hi and lo f16 planes in
     // A-fragment order, block (row tile of 32, step of 16 k) = 64 lanes x 16 bytes, and the f32
@@ -87,7 +87,14 @@ int w4_launch_gemm_i8(const W4Args& a, hipStream_t s);
 // six-bit-float matrix cores for large batches (w4_gemm_f6.hip): whether they take the call (more than 256 rows, group_size % 64 == 0,
 // n % 4 == 0, 16-byte aligned buffers, no g_idx, and the faster kernel by estimate).
 bool w4_gemm_f6_chosen(const W4Args& a);
-int w4_launch_gemm_f6(const W4Args& a, hipStream_t s);
+// a decoder block's operators around the projection: input through RMSNorm with `norm_w` (a.glu: through SwiGLU), `residual`
+// [m][n] added to the result (x and norm_w 16-byte aligned, k % 4 == 0, no perm)
+struct W4BlockArgs {
+    const float* norm_w = nullptr;
+    float eps = 0.0f;
+    const float* residual = nullptr;
+};
+int w4_launch_gemm_f6(const W4Args& a, hipStream_t s, const W4BlockArgs& block = {});
 
 // grad_x on the f16 matrix cores (w4_gemm_t.hip): group_size 32, 64 or a multiple of 128, n % 4 == 0, k % 4 == 0,
 // 16-byte aligned buffers.

@@ -76,6 +76,7 @@ struct F6Args {
     const uint32_t* zflags;    // kF6Flags words, nonzero where a part of the zero-point table holds a value that is no integer in 0..15
     float* y;
     uint32_t m, k, n, steps, steps_per_group, num_groups;
+    const float* residual;     // [m][n], added to the result, or null; may be y
 };
 
 __device__ __forceinline__ v8i f6_operand(const v6u& a) {
@@ -115,15 +116,25 @@ __device__ __forceinline__ v6u f6_digit(v16f& ev, v16f& od, float unit) {
 // Beyond the row groups, kF6Flags more workgroups look at the zero-points.
 __device__ __forceinline__ uint32_t f6_padded(uint32_t j) { return j + (j >> 5) * 4; }
 
-template <bool PERM>
+// What the rows of x go through on their way into LDS (a decoder block's operators in front of a projection; k % 4 == 0 and
+// 16-byte aligned then): RMSNorm with `norm_w`, or SwiGLU of rows gate | up of 2 k floats.  Their results are written
+// nowhere else but for the marked runs, which the matmul wants once more in f32 (`marked` [m][k]).
+// 4096 rows: SwiGLU of 2 x 11008 125 + 113 us as two kernels, 163 as one; RMSNorm of 4096 25 + 27 us, 35 as one.
+enum F6In { kF6Plain, kF6Perm, kF6Norm, kF6Glu };
+
+template <F6In IN>
 __global__ __launch_bounds__(512) void w4_f6_prepare_kernel(const float* __restrict__ x, const int32_t* __restrict__ perm,
                                                             uint8_t* __restrict__ planes, uint8_t* __restrict__ exps,
                                                             float* __restrict__ sums, float* __restrict__ rfac,
                                                             uint32_t m, uint32_t k, uint32_t steps, uint32_t rows,
                                                             uint32_t pitch, const float4* __restrict__ zp, uint32_t zp_count4,
-                                                            uint32_t* __restrict__ zflags, uint32_t row_groups) {
+                                                            uint32_t* __restrict__ zflags, uint32_t row_groups,
+                                                            const float* __restrict__ norm_w, float eps,
+                                                            float* __restrict__ marked) {
+    constexpr bool PERM = IN == kF6Perm;
     extern __shared__ __attribute__((aligned(16))) float lds_x[];
     __shared__ uint32_t rowmax[8];
+    __shared__ float squares[8];
     constexpr uint32_t T = 512;
     const uint32_t tid = threadIdx.x;
     if (blockIdx.x >= row_groups) {
@@ -155,11 +166,64 @@ __global__ __launch_bounds__(512) void w4_f6_prepare_kernel(const float* __restr
     const uint32_t per_row = T / rows, r1 = tid / per_row, t1 = tid % per_row;   // (a wave's threads share a row)
     {
         uint32_t am = 0;
-        if (r1 < live) {
-            const float* src = x + (uint64_t)(row0 + r1) * k;
-            float* dst = lds_x + r1 * pitch;
+        auto look = [&](const float4& v) __attribute__((always_inline)) {
+            am = max(max(am, __float_as_uint(v.x) & 0x7fffffffu), __float_as_uint(v.y) & 0x7fffffffu);
+            am = max(max(am, __float_as_uint(v.z) & 0x7fffffffu), __float_as_uint(v.w) & 0x7fffffffu);
+        };
+        const float* const src = x + (uint64_t)(row0 + r1) * k * (IN == kF6Glu ? 2 : 1);
+        float* const dst = lds_x + r1 * pitch;
+        const uint32_t last = k / 4 - 1;
+        if constexpr (IN == kF6Glu) {
+            if (r1 < live) {
+                for (uint32_t i0 = t1; i0 <= last; i0 += 8 * per_row) {
+                    float4 g[8], v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        g[u] = reinterpret_cast<const float4*>(src)[min(i0 + u * per_row, last)];
+                        v[u] = reinterpret_cast<const float4*>(src + k)[min(i0 + u * per_row, last)];
+                    }
+                    auto glu = [](float a, float b) { return a / (1.0f + expf(-a)) * b; };
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        const float4 y = make_float4(glu(g[u].x, v[u].x), glu(g[u].y, v[u].y), glu(g[u].z, v[u].z), glu(g[u].w, v[u].w));
+                        *reinterpret_cast<float4*>(dst + f6_padded(4 * min(i0 + u * per_row, last))) = y;
+                        look(y);
+                    }
+                }
+            }
+        } else if constexpr (IN == kF6Norm) {
+            float ss = 0.0f;
+            if (r1 < live) {
+                for (uint32_t i0 = t1; i0 <= last; i0 += 8 * per_row) {
+                    float4 v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) v[u] = reinterpret_cast<const float4*>(src)[min(i0 + u * per_row, last)];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        if (i0 + u * per_row > last) continue;
+                        *reinterpret_cast<float4*>(dst + f6_padded(4 * (i0 + u * per_row))) = v[u];
+                        ss = fmaf(v[u].x, v[u].x, fmaf(v[u].y, v[u].y, fmaf(v[u].z, v[u].z, fmaf(v[u].w, v[u].w, ss))));
+                    }
+                }
+            }
+            ss = wave_sum(ss);
+            if ((tid & 63) == 0) squares[tid >> 6] = ss;
+            __syncthreads();
+            const uint32_t waves = per_row / 64;                     // of a row, neighbours
+            float total = 0.0f;
+            for (uint32_t w = 0; w < waves; w++) total += squares[r1 * waves + w];
+            const float inv = 1.0f / sqrtf(total / (float)k + eps);
+            if (r1 < live) {
+                for (uint32_t i = t1; i <= last; i += per_row) {     // every thread's own elements
+                    const float4 w = reinterpret_cast<const float4*>(norm_w)[i];
+                    float4* const at = reinterpret_cast<float4*>(dst + f6_padded(4 * i));
+                    const float4 v = *at, y = make_float4(v.x * inv * w.x, v.y * inv * w.y, v.z * inv * w.z, v.w * inv * w.w);
+                    *at = y;
+                    look(y);
+                }
+            }
+        } else if (r1 < live) {
             if (vec) {
-                const uint32_t last = k / 4 - 1;
                 for (uint32_t i0 = t1; i0 <= last; i0 += 8 * per_row) {
                     float4 v[8];
 #pragma unroll
@@ -167,8 +231,7 @@ __global__ __launch_bounds__(512) void w4_f6_prepare_kernel(const float* __restr
 #pragma unroll
                     for (int u = 0; u < 8; u++) {
                         *reinterpret_cast<float4*>(dst + f6_padded(4 * min(i0 + u * per_row, last))) = v[u];
-                        am = max(max(am, __float_as_uint(v[u].x) & 0x7fffffffu), __float_as_uint(v[u].y) & 0x7fffffffu);
-                        am = max(max(am, __float_as_uint(v[u].z) & 0x7fffffffu), __float_as_uint(v[u].w) & 0x7fffffffu);
+                        look(v[u]);
                     }
                 }
             } else {
@@ -219,6 +282,13 @@ __global__ __launch_bounds__(512) void w4_f6_prepare_kernel(const float* __restr
     }
     const bool is_deep = low < top * 0.00390625f;
     if (!mine) return;                                           // whole waves or the tail of one: no barrier follows
+    if constexpr (IN == kF6Norm || IN == kF6Glu) {
+        if (is_deep) {                                           // (only rows below m have such runs)
+            for (uint32_t j = 0; j < 32 && 32 * unit + j < k; j += 4)
+                *reinterpret_cast<float4*>(marked + (uint64_t)row * k + 32 * unit + j) =
+                    *reinterpret_cast<const float4*>(lds_x + r * pitch + unit * 36 + j);
+        }
+    }
     float sum = 0.0f;
 #pragma unroll
     for (int j = 0; j < 32; j++) sum += v[j];
@@ -747,27 +817,48 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
 #pragma unroll
     for (int j = 0; j < TN; j++) bv[j] = a.bias && my_col + j < a.n ? a.bias[my_col + j] : 0.0f;
     if (my_col >= a.n) return;
-    auto put = [&](int i, int r, uint32_t row) __attribute__((always_inline)) {
+    const bool whole = m0 + kF6BM <= a.m, inside = TN != 3 || my_col + TN <= a.n;   // (otherwise the right edge: n % 4 == 0)
+    auto row_of = [&](int i, int r) { return m0 + (wm * 2 + i) * 32 + 8 * (r / 4) + 4 * kb + (r % 4); };
+    auto put = [&](int i, int r, const F6Floats<TN>& add) __attribute__((always_inline)) {
         F6Floats<TN> o;
 #pragma unroll
         for (int j = 0; j < TN; j++) o.v[j] = fmaf(acc[i][j][r] * rf[i][r], sc_cur.v[j], bv[j]);
-        float* p = a.y + (uint64_t)row * a.n + my_col;
-        if (TN != 3 || my_col + TN <= a.n) {
+        if (a.residual)
+#pragma unroll
+            for (int j = 0; j < TN; j++) o.v[j] += add.v[j];
+        float* p = a.y + (uint64_t)row_of(i, r) * a.n + my_col;
+        if (inside) {
             f6_cols_store<TN>(p, o);
-        } else {                                                  // the right edge: n % 4 == 0
+        } else {
 #pragma unroll
             for (int j = 0; j < TN; j++)
                 if (my_col + j < a.n) p[j] = o.v[j];
         }
     };
-    const bool whole = m0 + kF6BM <= a.m;
+    if (a.residual) {
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {                         // four rows at a time: their loads, then their stores
+                F6Floats<TN> add[4];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float* p = a.residual + (uint64_t)min(row_of(i, 4 * q + r), a.m - 1) * a.n + my_col;
+#pragma unroll
+                    for (int j = 0; j < TN; j++) add[r].v[j] = p[inside || my_col + j < a.n ? j : 0];
+                }
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (whole || row_of(i, 4 * q + r) < a.m) put(i, 4 * q + r, add[r]);
+            }
+        return;
+    }
+    const F6Floats<TN> none = {};
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const uint32_t row = m0 + (wm * 2 + i) * 32 + 8 * (r / 4) + 4 * kb + (r % 4);
-            if (whole || row < a.m) put(i, r, row);
-        }
+        for (int r = 0; r < 16; r++)
+            if (whole || row_of(i, r) < a.m) put(i, r, none);
 }
 
 // Columns per workgroup / 128, and the time of a call in microseconds: workgroups run one per compute unit, in rounds of
@@ -816,7 +907,7 @@ bool w4_gemm_f6_chosen(const W4Args& a) {
     const uintptr_t bits = reinterpret_cast<uintptr_t>(a.packed) | reinterpret_cast<uintptr_t>(a.scales) |
                            reinterpret_cast<uintptr_t>(a.zp) | reinterpret_cast<uintptr_t>(a.y) |
                            reinterpret_cast<uintptr_t>(a.perm) | reinterpret_cast<uintptr_t>(a.bias);
-    if (!(a.m > 256 && a.m <= 65535u * kF6BM && a.n % 4 == 0 && (bits & 15) == 0 && !a.g_idx && !a.tiled && !a.glu &&
+    if (!(a.m > 256 && a.m <= 65535u * kF6BM && a.n % 4 == 0 && (bits & 15) == 0 && !a.g_idx && !a.tiled &&
           a.group_size % 64 == 0 && (!a.zp4 || a.n % 8 == 0) && a.k >= 1024 && a.k <= 16384 &&    // (what the estimates were fitted to; a row of x in LDS, and 512 units of 32 k)
           (uint64_t)a.padded_k / 8 * a.n * 4 < (1ull << 32) && (uint64_t)a.m * a.n < (1ull << 32)))
         return false;
@@ -850,11 +941,13 @@ static int launch_f6_groups(const F6Args& f, const W4Args& a, uint32_t blocks, h
     return a.zp4 ? launch_f6<TN, 1, true>(f, blocks, s) : launch_f6<TN, 1, false>(f, blocks, s);
 }
 
-int w4_launch_gemm_f6(const W4Args& a, hipStream_t s) {
+int w4_launch_gemm_f6(const W4Args& a, hipStream_t s, const W4BlockArgs& block) {
     const F6Workspace w(a.m, a.padded_k);
     void* ws = nullptr;
     WorkspaceLease lease;                                    // until the last kernel of this call is queued
-    if (int rc = workspace_get(s, w.total, &ws, lease)) return rc;
+    const bool folded = block.norm_w || a.glu;
+    if (int rc = workspace_get(s, folded ? f6_up(w.total) + (size_t)a.m * a.k * 4 : w.total, &ws, lease)) return rc;
+    float* const marked = folded ? reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + f6_up(w.total)) : nullptr;
     uint8_t* p = static_cast<uint8_t*>(ws);
     uint8_t* const planes = p; p += w.planes;
     uint8_t* const exps = p; p += w.exps;
@@ -867,22 +960,25 @@ int w4_launch_gemm_f6(const W4Args& a, hipStream_t s) {
     while (rows > 1 && ((size_t)rows * pitch * 4 > 80 * 1024 || rows * units > 512 || rows_pad / rows < 256)) rows /= 2;
     static bool attr_set = false;   // benign race: setting the attribute is idempotent
     if (!attr_set) {
-        for (const void* f : {reinterpret_cast<const void*>(&w4_f6_prepare_kernel<false>), reinterpret_cast<const void*>(&w4_f6_prepare_kernel<true>)})
+        for (const void* f : {reinterpret_cast<const void*>(&w4_f6_prepare_kernel<kF6Plain>), reinterpret_cast<const void*>(&w4_f6_prepare_kernel<kF6Perm>),
+                              reinterpret_cast<const void*>(&w4_f6_prepare_kernel<kF6Norm>), reinterpret_cast<const void*>(&w4_f6_prepare_kernel<kF6Glu>)})
             if (int rc = check_hip(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024), "hipFuncSetAttribute"))
                 return rc;
         attr_set = true;
     }
     const dim3 pgrid(rows_pad / rows + (a.zp4 ? 0 : kF6Flags));
-#define RUMUS_F6_PREPARE(PERM)                                                                                             \
-    hipLaunchKernelGGL(w4_f6_prepare_kernel<PERM>, pgrid, dim3(512), (size_t)rows * pitch * 4, s, a.x, a.perm, planes, exps, sums, \
+#define RUMUS_F6_PREPARE(IN)                                                                                             \
+    hipLaunchKernelGGL(w4_f6_prepare_kernel<IN>, pgrid, dim3(512), (size_t)rows * pitch * 4, s, a.x, a.perm, planes, exps, sums, \
                        rfac, a.m, a.k, w.steps, rows, pitch, reinterpret_cast<const float4*>(a.zp),                        \
-                       (uint32_t)((uint64_t)a.num_groups * a.n / 4), zflags, rows_pad / rows)
-    if (a.perm) RUMUS_F6_PREPARE(true);
-    else RUMUS_F6_PREPARE(false);
+                       (uint32_t)((uint64_t)a.num_groups * a.n / 4), zflags, rows_pad / rows, block.norm_w, block.eps, marked)
+    if (a.perm) RUMUS_F6_PREPARE(kF6Perm);
+    else if (block.norm_w) RUMUS_F6_PREPARE(kF6Norm);
+    else if (a.glu) RUMUS_F6_PREPARE(kF6Glu);
+    else RUMUS_F6_PREPARE(kF6Plain);
 #undef RUMUS_F6_PREPARE
     if (int rc = check_launch("w4_f6_prepare_kernel")) return rc;
-    const F6Args f{a.packed, a.scales, a.zp, a.zp4, a.bias, planes, reinterpret_cast<const uint16_t*>(exps), sums, a.x, a.perm, rfac,
-                   zflags, a.y, a.m, a.k, a.n, w.steps, a.group_size / 64, a.num_groups};
+    const F6Args f{a.packed, a.scales, a.zp, a.zp4, a.bias, planes, reinterpret_cast<const uint16_t*>(exps), sums, folded ? marked : a.x, a.perm,
+                   rfac, zflags, a.y, a.m, a.k, a.n, w.steps, a.group_size / 64, a.num_groups, block.residual};
     double us;
     switch (f6_pick(a.m, a.k, a.n, &us)) {
         case 2: return launch_f6_groups<2>(f, a, w.blocks, s);

@@ -572,6 +572,31 @@ int rumus_hip_qmatmul_int4_decode_block(const float* x, const float* norm_weight
     return w4_launch_gemv_dot8_block(a, norm_weight, eps, residual, as_stream(stream));
 }
 
+int rumus_hip_qmatmul_int4_block_takes(uint32_t m, uint32_t k, uint32_t n, uint32_t group_size) {
+    if (group_size == 0 || k == 0 || k % 8 != 0) return 0;
+    const uint64_t groups = ((uint64_t)k + group_size - 1) / group_size;
+    if (groups * group_size > 0xffffffffull) return 0;
+    const W4Args a{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, m, k, n, (uint32_t)(groups * group_size),
+                   group_size, (uint32_t)groups};
+    return w4_gemm_f6_chosen(a) ? 1 : 0;
+}
+
+int rumus_hip_qmatmul_int4_block(const float* x, const float* norm_weight, float eps, int swiglu, const uint32_t* packed,
+                                 const float* scales, const float* zero_points, const float* bias, const float* residual, float* y,
+                                 uint32_t m, uint32_t k, uint32_t n, uint32_t padded_k, uint32_t group_size, uint32_t num_groups,
+                                 rumus_hip_stream_t stream) {
+    W4Args a{x, packed, scales, zero_points, bias, nullptr, nullptr, y, m, k, n, padded_k, group_size, num_groups, nullptr, false, swiglu != 0};
+    if (int rc = validate(a, "qmatmul_int4_block")) return rc;
+    RUMUS_REQUIRE(!(swiglu && norm_weight), "qmatmul_int4_block: RMSNorm and SwiGLU inputs exclude each other");
+    if (m == 0 || n == 0) return RUMUS_HIP_OK;
+    RUMUS_REQUIRE(((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(norm_weight)) & 15) == 0,
+                  "qmatmul_int4_block: x and norm_weight must be 16-byte aligned");
+    RUMUS_REQUIRE(y != x, "qmatmul_int4_block: y must not be x (residual may be y)");
+    RUMUS_REQUIRE(k % 8 == 0 && w4_gemm_f6_chosen(a),
+                  "qmatmul_int4_block: rumus_hip_qmatmul_int4_block_takes says no, or a buffer is not 16-byte aligned");
+    return w4_launch_gemm_f6(a, as_stream(stream), W4BlockArgs{norm_weight, eps, residual});
+}
+
 int rumus_hip_qmatmul_int4_zp4(const float* x, const uint32_t* packed, const float* scales,
                                const uint32_t* qzeros, const float* bias, const int32_t* perm, float* y,
                                uint32_t m, uint32_t k, uint32_t n, uint32_t padded_k, uint32_t group_size,

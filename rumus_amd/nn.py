@@ -309,8 +309,16 @@ class DecoderBlockW4:
         x2 = x.reshape(b * n, d)
         if k_cache is not None and n == 1 and self._folds(b):
             return self._decode_folded(x2, b, k_cache, v_cache, pos)
-        hn = ops.rmsnorm(x2, self.norm1, self.eps)
-        qkv = self.qkv(hn).view(b, n, 3, h, 128)
+        # Where a projection takes the kernel of large batches, the operators beside it are folded into it
+        # (``qmatmul_int4_block``); each of the four is asked for itself.
+        folds = self._folds_rows
+        if folds(self.qkv, x2, self.norm1):
+            qkv = self._block(self.qkv, x2, norm_weight=self.norm1, eps=self.eps)
+            hn = None
+        else:
+            hn = ops.rmsnorm(x2, self.norm1, self.eps)
+            qkv = self.qkv(hn)
+        qkv = qkv.view(b, n, 3, h, 128)
         q, k, v = qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2]
         if k_cache is None:
             att = ops.attention(q, k, v, causal=True)
@@ -320,18 +328,47 @@ class DecoderBlockW4:
                 raise ValueError("DecoderBlockW4: decode takes one token per sequence")
             att = ops.attention_decode_append(q, k, v, k_cache, v_cache, pos)
             k_out, v_out = k_cache, v_cache
-        o = self.proj["o"](att.view(b * n, d))
-        x1, h2 = ops.add_rmsnorm(x2, o, self.norm2, self.eps, sum_out=o, out=hn)
-        gu = self.gate_up(h2)
-        dw = self.proj["down"]
-        if b * n <= dw.weight.decode_rows and dw.weight.perm is None:
-            # decode rows: the SwiGLU happens while the down projection reads its input
-            down = ops.qmatmul_int4_decode_swiglu(gu, *dw.weight.decode, dw.weight.k, dw.weight.group_size,
-                                                  bias=dw.bias)
+        att = att.view(b * n, d)
+        x1 = o = None
+        if folds(self.proj["o"], att, x2):
+            x1 = self._block(self.proj["o"], att, residual=x2)
         else:
-            down = dw(ops.swiglu_rows(gu))
-        y = ops.add(x1, down, out=down)
+            o = self.proj["o"](att)
+        if folds(self.gate_up, x2 if x1 is None else x1, self.norm2):
+            if x1 is None:
+                x1 = ops.add(x2, o, out=o)
+            gu = self._block(self.gate_up, x1, norm_weight=self.norm2, eps=self.eps)
+        else:
+            if x1 is None:
+                x1, h2 = ops.add_rmsnorm(x2, o, self.norm2, self.eps, sum_out=o, out=hn)
+            else:
+                h2 = ops.rmsnorm(x1, self.norm2, self.eps, out=hn)
+            gu = self.gate_up(h2)
+        dw = self.proj["down"]
+        if folds(dw, gu, x1):
+            y = self._block(dw, gu, swiglu=True, residual=x1, out=x1)
+        else:
+            if b * n <= dw.weight.decode_rows and dw.weight.perm is None:
+                # decode rows: the SwiGLU happens while the down projection reads its input
+                down = ops.qmatmul_int4_decode_swiglu(gu, *dw.weight.decode, dw.weight.k, dw.weight.group_size,
+                                                      bias=dw.bias)
+            else:
+                down = dw(ops.swiglu_rows(gu))
+            y = ops.add(x1, down, out=down)
         return y.view(b, n, d), k_out, v_out
+
+    @staticmethod
+    def _folds_rows(lin, x, *beside) -> bool:
+        """Whether this projection of ``x`` takes ``qmatmul_int4_block``, operands included."""
+        w = lin.weight
+        arrays = (x, w.packed_tensor, w.scales_tensor, w.zp_tensor) + beside + ((lin.bias,) if lin.bias is not None else ())
+        return w.perm is None and ops.qmatmul_int4_block_takes(x.shape[0], w.k, w.n, w.group_size) and \
+            all(t.data_ptr() % 16 == 0 for t in arrays)
+
+    @staticmethod
+    def _block(lin, x, **kw):
+        w = lin.weight
+        return ops.qmatmul_int4_block(x, w.packed_tensor, w.scales_tensor, w.zp_tensor, w.k, w.group_size, bias=lin.bias, **kw)
 
     def _folds(self, rows: int) -> bool:
         """A decode step of few enough rows for every projection's decode kernel, plain weights: the norms, the

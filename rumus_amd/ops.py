@@ -354,6 +354,34 @@ def qmatmul_int4_decode_block(x, packed_t, scales_t, zp_t, k, group_size, norm_w
     return y
 
 
+def qmatmul_int4_block(x, packed, scales, zp, k, group_size, norm_weight=None, eps: float = 1e-6,
+                       swiglu: bool = False, bias=None, residual=None, out=None):
+    """:func:`qmatmul_int4_decode_block` for a batch of prompt tokens on the weight's own arrays, where
+    :func:`qmatmul_int4_block_takes` says so."""
+    m = x.shape[0]
+    n = packed.shape[1]
+    if x.dim() != 2 or x.shape[1] != (2 * k if swiglu else k):
+        raise ValueError("qmatmul_int4_block: x must be [m, k] (gate | up: [m, 2k])")
+    if norm_weight is not None and norm_weight.numel() < k:
+        raise ValueError("qmatmul_int4_block: norm_weight must hold k values")
+    if residual is not None and (residual.dim() != 2 or tuple(residual.shape) != (m, n) or not residual.is_contiguous()):
+        raise ValueError("qmatmul_int4_block: residual must be a contiguous [m, n] tensor")
+    _w4_sizes("qmatmul_int4_block", packed, scales, zp, k, group_size, m, bias, None, out)
+    padded_k, groups = w4_geometry(k, group_size) if group_size > 0 else (k, 0)
+    y = out if out is not None else torch.empty((m, n), dtype=torch.float32, device=x.device)
+    call("rumus_hip_qmatmul_int4_block", _dev(x, torch.float32, "x"), _opt(norm_weight, torch.float32, "norm_weight"),
+         float(eps), 1 if swiglu else 0, _dev(packed, torch.int32, "packed"), _dev(scales, torch.float32, "scales"),
+         _dev(zp, torch.float32, "zero_points"), _opt(bias, torch.float32, "bias"),
+         _opt(residual, torch.float32, "residual"), _dev(y, torch.float32, "y"), m, k, n, padded_k, group_size, groups,
+         _stream())
+    return y
+
+
+def qmatmul_int4_block_takes(m: int, k: int, n: int, group_size: int) -> bool:
+    """Whether :func:`qmatmul_int4_block` takes this shape (large batches)."""
+    return bool(_lib.lib().rumus_hip_qmatmul_int4_block_takes(m, k, n, group_size))
+
+
 def qmatmul_int4_zp4(x, packed, scales, qzeros, k, group_size, bias=None, perm=None, out=None):
     m = x.shape[0]
     n = packed.shape[1]
