@@ -17,7 +17,7 @@
 //     hi + lo f16 (22 bits), written to LDS in A-fragment rows of 64 bytes; c accumulates in f32;
 //   * every wave owns 32 of the 128 k: lane (k = lane % 32, half = lane / 32) reads the 8 consecutive
 //     words of word row k / 8 that hold its 8 values of n, takes nibble k % 8 of each, and splices them
-//     under the mantissa of 1024 (minus 1024, two at a time): 20 instructions per B fragment, which
+//     under the mantissa of 1024 (minus 1024, two at a time): 16 instructions per B fragment, which
 //     serves 4 MFMAs (two row tiles x hi, lo);
 //   * v_mfma_f32_32x32x16_f16 accumulates in f32; the epilogue subtracts c and undoes f_row and S.
 // Few tiles: n is shared out over blockIdx.z as well and the partial results are added in a fixed order.
@@ -124,6 +124,21 @@ constexpr size_t w4t_lds_bytes(int stages) {
     return (size_t)(stages - 1) * kTRawGy + (size_t)stages * kTRawWt + 2 * kTAbuf + 2 * 64 * sizeof(float);
 }
 
+// Direct-to-LDS loads and the barrier that publishes a step, spelled out.  With the compiler's own loads every LDS read that
+// follows waits for all of them (it cannot see that they go to another slot): the two steps meant to be in flight were waited
+// for within the step that had asked for them.  The barrier waits for the step it publishes, and for the wave's LDS writes.
+__device__ __forceinline__ uint32_t w4t_lds_offset(const void* p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p; }
+__device__ __forceinline__ void w4t_load16(uint32_t to, const void* from, uint32_t lane_bytes) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(lane_bytes), "s"(from) : "memory");
+}
+__device__ __forceinline__ void w4t_load4(uint32_t to, const void* from, uint32_t lane_bytes) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(to), "v"(lane_bytes), "s"(from) : "memory");
+}
+template <int LOADS>
+__device__ __forceinline__ void w4t_publish() {               // all but the youngest LOADS loads of the wave have landed
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LOADS) : "memory");
+}
+
 // KW = waves per workgroup = 32-column slices of k per tile: 4 when groups are multiples of 128, 2 for
 // groups of 64, 1 for groups of 32 (a tile must lie inside one group, since the activations are re-scaled
 // per group; the smaller workgroups convert the same 64 x 32 activations for fewer output columns).
@@ -196,28 +211,27 @@ __global__ __launch_bounds__(64 * KW, 2) void w4t_gemm_kernel(
             voff[i] = colw[i] * 2;
         }
     }
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(w4t_lds_offset(lds));
     auto issue = [&](uint32_t st, uint32_t gslot, uint32_t wslot) {
-        uint8_t* const gbase = raw_gy + gslot * kTRawGy;
-        uint8_t* const wbase = raw_wt + wslot * kTRawWt;
+        const uint32_t gbase = lds0 + gslot * kTRawGy, wbase = lds0 + (kTStages - 1) * kTRawGy + wslot * kTRawWt;
         const uint32_t c0 = min(st, st1 - 1) * 32;
-        if (c0 + 32 <= n) {
+        const bool inside = c0 + 32 <= n;
 #pragma unroll
-            for (int i = 0; i < kTLoads; i++) {
-                uint8_t* const base = is_gy[i] ? gbase : wbase;
-                const uint8_t* const sb = ubase[i] + (uint64_t)c0 * esz[i];
-                if (wide[i]) __builtin_amdgcn_global_load_lds((gptr_t)(sb + voff[i]), (lptr_t)(base + dst[i]), 16, 0, 0);
-                else __builtin_amdgcn_global_load_lds((gptr_t)(sb + voff[i]), (lptr_t)(base + dst[i]), 4, 0, 0);
-            }
-        } else {
-            // columns past n are fetched from column 0: the conversion turns them into zeros
-#pragma unroll
-            for (int i = 0; i < kTLoads; i++) {
-                uint8_t* const base = is_gy[i] ? gbase : wbase;
+        for (int i = 0; i < kTLoads; i++) {
+            constexpr int skip = HALF ? 4 : 0;
+            const bool all_wide = KW * (i + 1) - 1 + skip < 8 + WS;    // whatever the wave
+            const uint32_t to = (is_gy[i] ? gbase : wbase) + dst[i];
+            const uint8_t* from = ubase[i];
+            uint32_t at = voff[i];
+            if (inside) {
+                from += (uint64_t)c0 * esz[i];
+            } else {
+                // columns past n are fetched from column 0: the conversion turns them into zeros
                 const uint32_t col = c0 + colw[i] < n ? c0 + colw[i] : 0;
-                const uint8_t* const p = ubase[i] + (voff[i] - colw[i] * esz[i]) + (uint64_t)col * esz[i];
-                if (wide[i]) __builtin_amdgcn_global_load_lds((gptr_t)p, (lptr_t)(base + dst[i]), 16, 0, 0);
-                else __builtin_amdgcn_global_load_lds((gptr_t)p, (lptr_t)(base + dst[i]), 4, 0, 0);
+                at += (col - colw[i]) * esz[i];
             }
+            if (all_wide || wide[i]) w4t_load16(to, from, at);
+            else w4t_load4(to, from, at);
         }
     };
 
@@ -226,6 +240,7 @@ __global__ __launch_bounds__(64 * KW, 2) void w4t_gemm_kernel(
     const uint32_t s_row = tid / KW, s_ch0 = (tid % KW) * CPT;
     const float frow_raw = rowf[min(m0 + s_row, m - 1)];
     const float frow = frow_raw != frow_raw ? 0.0f : frow_raw; // inf / nan in the row: NaN times 0 poisons it below
+    const uint32_t n_end = min(n, st1 * 32);
     float csum = 0.0f;
     auto convert_chunk = [&](uint32_t st, uint32_t gslot, uint32_t wslot, int buf, uint32_t s_ch) {
         const uint32_t s_lds = s_row * 64 + ((s_ch ^ row_swizzle(s_row)) & 3) * 16;
@@ -238,9 +253,9 @@ __global__ __launch_bounds__(64 * KW, 2) void w4t_gemm_kernel(
         const float4 s1 = *reinterpret_cast<const float4*>(tbase + s_ch * 32 + 16);
         const float4 z0 = *reinterpret_cast<const float4*>(tbase + 128 + s_ch * 32);
         const float4 z1 = *reinterpret_cast<const float4*>(tbase + 128 + s_ch * 32 + 16);
-        const uint32_t c0 = st * 32 + s_ch * 8;
+        const uint32_t c0 = st * 32 + s_ch * 8;                // (and past the workgroup's share nothing is added to its sum)
         // n % 4 == 0: four columns are all-in or all-out; the columns past n hold values of column 0
-        const float f0 = c0 < n ? frow : 0.0f, f1 = c0 + 4 < n ? frow : 0.0f;
+        const float f0 = c0 < n_end ? frow : 0.0f, f1 = c0 + 4 < n_end ? frow : 0.0f;
         // powers of two first: gy f is exact, the product with s / S is rounded once
         const float a[8] = {(g0.x * f0) * s0.x, (g0.y * f0) * s0.y, (g0.z * f0) * s0.z, (g0.w * f0) * s0.w,
                             (g1.x * f1) * s1.x, (g1.y * f1) * s1.y, (g1.z * f1) * s1.z, (g1.w * f1) * s1.w};
@@ -277,20 +292,35 @@ __global__ __launch_bounds__(64 * KW, 2) void w4t_gemm_kernel(
 
     // ---- B role: lane (k = 32 wave + lane % 32, half = lane / 32): 8 words of word row 4 wave + k / 8 ----
     const uint32_t bc = lane & 31, bh = lane >> 5;
-    const uint32_t shift = 4 * (bc & 7);
+    // Nibble k % 8 lies in byte k % 8 / 2 of its word: one v_perm_b32 puts that byte of two words into the halves of a third,
+    // one shift (by 0 or 4) brings the nibbles down, one v_and_or_b32 masks them and adds the mantissa of 1024: four instructions
+    // for two values with the subtraction, where a field extract per word, a shift-or and an or took five (111 -> 103 vector
+    // instructions per step).  Mask and constant sit in vector registers: the instruction reads one scalar operand only.
+    const uint32_t shift = 4 * (bc & 1), pick = (0x0C040C00u) + ((bc & 7) >> 1) * 0x00010001u;
+    uint32_t mask = 0x000F000Fu, magic = 0x64006400u;
+    asm("" : "+v"(mask), "+v"(magic));
     const uint32_t b_off = (4 * wave + (bc >> 3)) * 128 + bh * 32;
-    auto b_frag = [&](int t, uint32_t wslot) {
+    uint4 bw[4];
+    t8h boff[2];                                               // 1024 + z0
+    auto b_read = [&](uint32_t wslot) {
         const uint8_t* sb = raw_wt + wslot * kTRawWt;
-        const uint4 w0 = *reinterpret_cast<const uint4*>(sb + b_off + t * 64), w1 = *reinterpret_cast<const uint4*>(sb + b_off + t * 64 + 16);
-        const uint32_t w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-        const t8h off = *reinterpret_cast<const t8h*>(sb + kTRawW + kTRawSz + 32 * t + 16 * bh);   // 1024 + z0
-        t2h h[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t q0 = (w[2 * i] >> shift) & 0xFu, q1 = (w[2 * i + 1] >> shift) & 0xFu;
-            h[i] = __builtin_bit_cast(t2h, (q1 << 16) | q0 | 0x64006400u) - t2h{off[2 * i], off[2 * i + 1]};   // (1024 + q) - (1024 + z0): exact
+        for (int t = 0; t < 2; t++) {
+            bw[2 * t] = *reinterpret_cast<const uint4*>(sb + b_off + t * 64);
+            bw[2 * t + 1] = *reinterpret_cast<const uint4*>(sb + b_off + t * 64 + 16);
+            boff[t] = *reinterpret_cast<const t8h*>(sb + kTRawW + kTRawSz + 32 * t + 16 * bh);
         }
-        return t8h{h[0][0], h[0][1], h[1][0], h[1][1], h[2][0], h[2][1], h[3][0], h[3][1]};
+    };
+    auto b_cut = [&](int j, t8h (&to)[2]) {                    // the four values of word quad j, j = 0 .. 3
+        const uint32_t w[4] = {bw[j].x, bw[j].y, bw[j].z, bw[j].w};
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const uint32_t q = ((__builtin_amdgcn_perm(w[2 * i + 1], w[2 * i], pick) >> shift) & mask) | magic;
+            const int e = 4 * (j & 1) + 2 * i;
+            const t2h h = __builtin_bit_cast(t2h, q) - t2h{boff[j >> 1][e], boff[j >> 1][e + 1]};   // (1024 + q) - (1024 + z0): exact
+            to[j >> 1][e] = h[0];
+            to[j >> 1][e + 1] = h[1];
+        }
     };
 
     // ---- A fragment reads: lane (row fr, half fh), MFMA step t: logical chunk 2 t + fh -----------------
@@ -310,13 +340,16 @@ __global__ __launch_bounds__(64 * KW, 2) void w4t_gemm_kernel(
     // stage nobody reads any more), so the counter arithmetic has no tail cases.
 #pragma unroll
     for (int s = 0; s < kTStages - 1; s++) issue(st0 + s, s, s);
-    RUMUS_WAIT_VMCNT((kTStages - 2) * kTLoads);               // step st0 has landed
-    __builtin_amdgcn_s_barrier();
+    w4t_publish<(kTStages - 2) * kTLoads>();                  // step st0 has landed
     convert(st0, 0, 0, 0);
     // The B fragments of a step are cut out of its words while the MFMAs of the step before run (a wave issues
     // nothing while it waits to issue an MFMA: fragments and MFMAs of the same step one after the other leave the
     // vector ALU idle during the MFMAs and the matrix cores idle during the cutting).
-    t8h b0 = b_frag(0, 0), b1 = b_frag(1, 0);
+    t8h first[2];
+    b_read(0);
+#pragma unroll
+    for (int j = 0; j < 4; j++) b_cut(j, first);
+    t8h b0 = first[0], b1 = first[1];
     uint32_t cur = 0, gcur = 0;                                // slots of step st: weights and tables, grad_y
     for (uint32_t st = st0; st < st1; st++) {
         const int ab = (st - st0) & 1;
@@ -325,32 +358,53 @@ __global__ __launch_bounds__(64 * KW, 2) void w4t_gemm_kernel(
         // step st+1 has landed once only the kTStages-3 younger steps are outstanding; past the barrier
         // the A fragments of step st are visible, the weight slot of step st-1 is free and so is the grad_y
         // slot of step st itself (converted during step st-1)
-        RUMUS_WAIT_VMCNT((kTStages - 3) * kTLoads);
-        __builtin_amdgcn_s_barrier();
+        w4t_publish<(kTStages - 3) * kTLoads>();
         issue(st + (kTStages - 1), gcur, prv);
-        const t8h nb0 = b_frag(0, nxt), nb1 = b_frag(1, nxt);   // step st+1 has landed (after the last step: that step's words again, unused)
+        // Tile by tile: the fragments of a tile are read in one go, and between its MFMAs stand a share of the next step's B
+        // fragments (first tile; after the last step: that step's words again, unused) and of its A fragments (after the last
+        // step: zeros that nobody reads), held there by the scheduling barriers.
         const uint8_t* abp = abuf + ab * kTAbuf;
+        t8h nb[2];
 #pragma unroll
         for (int i = 0; i < RTILES; i++) {
             const uint8_t* hi = abp + i * 32 * 64;
             const uint8_t* lo = abp + 64 * 64 + i * 32 * 64;
-            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const t8h*>(hi + a_off[0]), b0, acc[i], 0, 0, 0);
-            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const t8h*>(lo + a_off[0]), b0, acc[i], 0, 0, 0);
-            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const t8h*>(hi + a_off[1]), b1, acc[i], 0, 0, 0);
-            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const t8h*>(lo + a_off[1]), b1, acc[i], 0, 0, 0);
-        }
+            const t8h f[4] = {*reinterpret_cast<const t8h*>(hi + a_off[0]), *reinterpret_cast<const t8h*>(lo + a_off[0]),
+                              *reinterpret_cast<const t8h*>(hi + a_off[1]), *reinterpret_cast<const t8h*>(lo + a_off[1])};
+            if (i == 0) {
+                b_read(nxt);
+            } else {
+                convert(st + 1, gnxt, nxt, ab ^ 1);
+            }
 #pragma unroll
-        for (int i = 0; i < 4 * RTILES; i++) {                 // an MFMA, then its share of the 40 instructions of the next fragments
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, 40 / (4 * RTILES), 0);
+            for (int j = 0; j < 4; j++) {
+                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[j], j < 2 ? b0 : b1, acc[i], 0, 0, 0);
+                if (i == 0) b_cut(j, nb);
+            }
+            if (i == 0) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 10, 0);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+                }
+            } else {
+                __builtin_amdgcn_sched_group_barrier(0x100, 10, 0);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 13, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        if (st + 1 < st1) convert(st + 1, gnxt, nxt, ab ^ 1);
-        b0 = nb0;
-        b1 = nb1;
+        if (RTILES == 1) convert(st + 1, gnxt, nxt, ab ^ 1);
+        b0 = nb[0];
+        b1 = nb[1];
         cur = nxt;
         gcur = gnxt;
     }
-    RUMUS_WAIT_VMCNT(0);         // no direct-to-LDS write may outlive the workgroup
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no direct-to-LDS write may outlive the workgroup
 
     // ---- c[row]: the KW conversion threads of a row are neighbours in a wave ---------------------------
     if (KW >= 2) csum += __shfl_xor(csum, 1);
