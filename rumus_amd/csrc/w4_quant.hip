@@ -39,6 +39,28 @@ struct GroupReader {
     }
 };
 
+// v / scale, rounded as the division rounds, for the many v of a group: with y = RN(1 / scale), q = RN(v y) and the exact
+// remainder r = v - q scale, RN(q + r y) is the correctly rounded quotient (Markstein, "Computation of elementary functions on
+// the IBM RISC System/6000 processor", 1990) while nothing under- or overflows: three instructions per element instead of
+// the ten of the general division, which bounded the quantizers.  Held to groups whose scale and elements are within 2^+-60; quotients
+// below 2^-40, whose remainder may underflow, are off by an ulp at most and vanish in the sum with the zero-point or its
+// rounding to an integer all the same.  Other groups divide.
+// 4096 x 11008: groups of 128 42.4 -> 36.5 us (4.9 -> 5.7 TB/s), of 64 34.8 -> 33.8, of 32 34.6 -> 33.2; 4096 x 4096 g128 27.3 -> 23.7.
+struct GroupDivide {
+    float scale, y;
+    __device__ __forceinline__ float operator()(float v) const {
+        const float q = __fmul_rn(v, y);
+        return __fmaf_rn(__fmaf_rn(-q, scale, v), y, q);
+    }
+    static __device__ __forceinline__ bool holds(float scale, float top) {
+        return scale >= 0x1p-60f && scale <= 0x1p60f && top <= 0x1p60f;
+    }
+};
+struct PlainDivide {
+    float scale;
+    __device__ __forceinline__ float operator()(float v) const { return __fdiv_rn(v, scale); }
+};
+
 template <bool SYM, int GS>
 __global__ __launch_bounds__(256) void w4_quantize_pack_kernel(
     const float* __restrict__ w, uint32_t k, uint32_t n, uint32_t gs_arg,
@@ -50,13 +72,14 @@ __global__ __launch_bounds__(256) void w4_quantize_pack_kernel(
     const uint32_t r0 = g * gs;
     const GroupReader<GS> group(w, k, n, col, r0);
 
-    float scale, zp;
+    float scale, zp, top;                                       // top: the largest magnitude
     if (SYM) {
         float amax = 0.0f;
 #pragma unroll
         for (uint32_t i = 0; i < gs; i++) amax = fmaxf(amax, fabsf(group[i]));
         scale = amax > 0.0f ? __fdiv_rn(amax, 7.0f) : 1.0f;
         zp = 8.0f;
+        top = amax;
     } else {
         // quant.rs:66-74
         float mn = 3.402823466e+38f, mx = -3.402823466e+38f;
@@ -70,27 +93,32 @@ __global__ __launch_bounds__(256) void w4_quantize_pack_kernel(
         const bool live = range > 1e-10f;                       // quant.rs:77-79
         scale = live ? __fdiv_rn(range, 15.0f) : 1.0f;
         zp = live ? __fdiv_rn(-mn, scale) : 0.0f;
+        top = fmaxf(fabsf(mn), fabsf(mx));
     }
     scales[(uint64_t)g * n + col] = scale;
     if (zps) zps[(uint64_t)g * n + col] = zp;
 
+    auto emit = [&](auto divide) {
 #pragma unroll
-    for (uint32_t wr = 0; wr < gs / 8; wr++) {
-        uint32_t word = 0;
+        for (uint32_t wr = 0; wr < gs / 8; wr++) {
+            uint32_t word = 0;
 #pragma unroll
-        for (uint32_t j = 0; j < 8; j++) {
-            const float v = group[wr * 8 + j];
-            float t;
-            if (SYM) {
-                t = __fadd_rn(roundf(__fdiv_rn(v, scale)), 8.0f);
-            } else {
-                t = roundf(__fadd_rn(__fdiv_rn(v, scale), zp));  // quant.rs:96, half away
+            for (uint32_t j = 0; j < 8; j++) {
+                const float v = group[wr * 8 + j];
+                float t;
+                if (SYM) {
+                    t = __fadd_rn(roundf(divide(v)), 8.0f);
+                } else {
+                    t = roundf(__fadd_rn(divide(v), zp));        // quant.rs:96, half away
+                }
+                t = fminf(fmaxf(t, 0.0f), 15.0f);                // NaN -> 0 like `as i32`
+                word |= (uint32_t)t << (4 * j);
             }
-            t = fminf(fmaxf(t, 0.0f), 15.0f);                    // NaN -> 0 like `as i32`
-            word |= (uint32_t)t << (4 * j);
+            packed[(uint64_t)(r0 / 8 + wr) * n + col] = word;
         }
-        packed[(uint64_t)(r0 / 8 + wr) * n + col] = word;
-    }
+    };
+    if (GroupDivide::holds(scale, top)) emit(GroupDivide{scale, __fdiv_rn(1.0f, scale)});
+    else emit(PlainDivide{scale});
 }
 
 // AWQ storage: integer zero-points packed eight per word along n.
@@ -125,18 +153,22 @@ __global__ __launch_bounds__(256) void w4_quantize_pack_awq_kernel(
     zw |= __shfl_xor(zw, 2);
     zw |= __shfl_xor(zw, 4);
     if ((col & 7) == 0) qzeros[(uint64_t)g * (n / 8) + col / 8] = zw;
+    auto emit = [&](auto divide) {
 #pragma unroll
-    for (uint32_t wr = 0; wr < gs / 8; wr++) {
-        uint32_t word = 0;
+        for (uint32_t wr = 0; wr < gs / 8; wr++) {
+            uint32_t word = 0;
 #pragma unroll
-        for (uint32_t j = 0; j < 8; j++) {
-            const float v = group[wr * 8 + j];
-            float t = __fadd_rn(rintf(__fdiv_rn(v, scale)), zf);
-            t = fminf(fmaxf(t, 0.0f), 15.0f);
-            word |= (uint32_t)t << (4 * j);
+            for (uint32_t j = 0; j < 8; j++) {
+                const float v = group[wr * 8 + j];
+                float t = __fadd_rn(rintf(divide(v)), zf);
+                t = fminf(fmaxf(t, 0.0f), 15.0f);
+                word |= (uint32_t)t << (4 * j);
+            }
+            packed[(uint64_t)(r0 / 8 + wr) * n + col] = word;
         }
-        packed[(uint64_t)(r0 / 8 + wr) * n + col] = word;
-    }
+    };
+    if (GroupDivide::holds(scale, fmaxf(fabsf(mn), fabsf(mx)))) emit(GroupDivide{scale, __fdiv_rn(1.0f, scale)});
+    else emit(PlainDivide{scale});
 }
 
 // Decode layout: tile-major copies of [rows, n] arrays of 32-bit words, tile = 16 columns:
