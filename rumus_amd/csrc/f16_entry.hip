@@ -8,6 +8,7 @@
 // (finite values beyond 65504 become infinities, as any f16 store would make them).  That is at least as
 // accurate as an f16 running sum and deterministic.  The weights' metadata (scales, zero-points, bias) stays
 // f32: it is converted once when a checkpoint is loaded (rumus_hip_f16_to_f32), not per call.
+// Where a batch comes to the integer matrix-core kernel (w4_gemm_i8.hip) that kernel does both conversions itself.
 #include "common.h"
 
 namespace rumus {
@@ -87,7 +88,12 @@ int rumus_hip_matmul_q8_f16(const uint16_t* a, const uint32_t* b, uint16_t* c, u
     return f16_finish(st, c, (uint64_t)m * n, as_stream(stream));
 }
 
-int rumus_hip_qmatmul_int4_f16(const uint16_t* x, const uint32_t* packed, const float* scales, const float* zero_points,
+}  // extern "C"
+
+namespace rumus {
+
+// through f32 copies of activations and result
+int w4_f16_staged(const uint16_t* x, const uint32_t* packed, const float* scales, const float* zero_points,
                                const float* bias, const int32_t* g_idx, uint16_t* y, uint32_t m, uint32_t k, uint32_t n,
                                uint32_t padded_k, uint32_t group_size, uint32_t num_groups, rumus_hip_stream_t stream) {
     if (m == 0 || n == 0 || !x || !y)
@@ -101,4 +107,4 @@ int rumus_hip_qmatmul_int4_f16(const uint16_t* x, const uint32_t* packed, const 
     return f16_finish(st, y, (uint64_t)m * n, as_stream(stream));
 }
 
-}  // extern "C"
+}  // namespace rumus

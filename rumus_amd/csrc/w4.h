@@ -40,6 +40,9 @@ struct W4Args {
     // w4_gemm_tile only (set by its launcher; f32 zero-points): kZpFlagWords words, nonzero where a part of the
     // zero-point table holds a value that is no integer (w4_zp_scan_kernel)
     const uint32_t* zflags = nullptr;
+    // w4_gemm_i8 only, without perm: f16 activations and result instead of x and y (f16_entry.hip)
+    const _Float16* x16 = nullptr;
+    _Float16* y16 = nullptr;
 };
 
 // zero-points of 4 (col % 4 == 0) or 2 (col % 2 == 0) adjacent columns from the packed form
@@ -83,6 +86,12 @@ int w4_launch_gemm(const W4Args& a, hipStream_t s);
 // buffers, no g_idx.  Larger batches where an estimate says that it beats the f16 tiles; us: the faster one's estimate.
 bool w4_gemm_i8_supported(const W4Args& a, double* us = nullptr);
 int w4_launch_gemm_i8(const W4Args& a, hipStream_t s);
+// rumus_hip_qmatmul_int4_f16 by way of f32 copies (f16_entry.hip)
+int w4_f16_staged(const uint16_t* x, const uint32_t* packed, const float* scales, const float* zero_points, const float* bias,
+                  const int32_t* g_idx, uint16_t* y, uint32_t m, uint32_t k, uint32_t n, uint32_t padded_k, uint32_t group_size,
+                  uint32_t num_groups, rumus_hip_stream_t stream);
+// whether a checked call of this shape, f32 x and y aligned, comes to w4_launch_gemm_i8 (w4_gemv.hip)
+bool w4_routes_to_i8(const W4Args& a);
 
 // six-bit-float matrix cores for large batches (w4_gemm_f6.hip): whether they take the call (more than 256 rows, group_size % 64 == 0,
 // n % 4 == 0, 16-byte aligned buffers, no g_idx, and the faster kernel by estimate).

@@ -55,6 +55,7 @@ struct W4I8Args {
     const int32_t* out_k;     // [row][share][kI8Outliers]: their positions (rows of the packed matrix) ...
     const float* out_x;       // ... and values
     float* y;
+    _Float16* y16;            // instead of y, or null
     uint32_t m, n, steps, chunks, steps_per_group, per;   // per: chunks per share
 };
 
@@ -94,9 +95,9 @@ __device__ __forceinline__ int group_sum(int v) {
 // STAGED (act-order, x[row][perm[j]]): the eight waves of a row are one workgroup that first copies the row
 // into LDS (k floats of dynamic LDS) with contiguous reads and gathers from there; gathered from global
 // memory a wave instruction touches 64 cache lines for 256 bytes, behind the load of perm itself.
-template <int CS, bool VEC, bool STAGED>
+template <int CS, bool VEC, bool STAGED, typename T>
 __global__ __launch_bounds__(STAGED ? 64 * kI8WK : 64) void w4_i8_prepare_kernel(
-    const float* __restrict__ x, const int32_t* __restrict__ perm, uint8_t* __restrict__ planes,
+    const T* __restrict__ x, const int32_t* __restrict__ perm, uint8_t* __restrict__ planes,
     float* __restrict__ rscale, int32_t* __restrict__ csum, uint8_t* __restrict__ out_n, int32_t* __restrict__ out_k,
     float* __restrict__ out_x, uint32_t m, uint32_t k, uint32_t steps, uint32_t chunks, uint32_t per) {
     static_assert(!(VEC && STAGED), "staging is for the gather");
@@ -107,7 +108,7 @@ __global__ __launch_bounds__(STAGED ? 64 * kI8WK : 64) void w4_i8_prepare_kernel
     const uint32_t row = STAGED ? blockIdx.x : blockIdx.y, rt = row >> 4, row_l = row & 15;
     const uint32_t k_begin = min(share * per, chunks) * CS * 64, k_end = min((share + 1) * per, chunks) * CS * 64;
     const bool live = row < m;
-    const float* xr = x + (uint64_t)(live ? row : 0) * k;
+    const T* xr = x + (uint64_t)(live ? row : 0) * k;
     // STAGED (the launcher sends k % 8 == 0 and 16-byte aligned x and perm here): where a lane's 8 values come
     // from, then the values themselves.  Straight-line code with clamped addresses: a load under a branch
     // would make the wave wait for it at the end of the branch, one trip to memory after the other.
@@ -133,17 +134,17 @@ __global__ __launch_bounds__(STAGED ? 64 * kI8WK : 64) void w4_i8_prepare_kernel
     if (STAGED) {
 #pragma unroll
         for (int i = 0; i < CACHE; i++) cin[i] = index8(k_begin + (lane + 64 * i) * 8, cix[i]);
-        constexpr uint32_t T = 64 * kI8WK;
+        constexpr uint32_t threads = 64 * kI8WK;
         const uint32_t vecs = k / 4;
         const float4* src = reinterpret_cast<const float4*>(xr);
-        for (uint32_t i0 = threadIdx.x; i0 < vecs; i0 += 4 * T) {      // four loads in flight: one trip up to 8192 k
+        for (uint32_t i0 = threadIdx.x; i0 < vecs; i0 += 4 * threads) {      // four loads in flight: one trip up to 8192 k
             float4 t[4];
 #pragma unroll
-            for (int u = 0; u < 4; u++) t[u] = src[min(i0 + u * T, vecs - 1)];
+            for (int u = 0; u < 4; u++) t[u] = src[min(i0 + u * threads, vecs - 1)];
             __builtin_amdgcn_sched_barrier(0);                     // all issued before the first is waited for
 #pragma unroll
             for (int u = 0; u < 4; u++)
-                if (i0 + u * T < vecs) reinterpret_cast<float4*>(lds_row)[i0 + u * T] = t[u];
+                if (i0 + u * threads < vecs) reinterpret_cast<float4*>(lds_row)[i0 + u * threads] = t[u];
         }
         __syncthreads();
     }
@@ -152,7 +153,13 @@ __global__ __launch_bounds__(STAGED ? 64 * kI8WK : 64) void w4_i8_prepare_kernel
 #pragma unroll
         for (int j4 = 0; j4 < 2; j4++) {
             const uint32_t kk = k0 + 4 * j4;
-            if (VEC) {                                             // k % 4 == 0: a float4 is all in or all out
+            if constexpr (VEC && sizeof(T) == 2) {                 // f16, widened exactly
+                typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+                h4 f = {0, 0, 0, 0};
+                if (live && k0 < k_end && kk < k) f = *reinterpret_cast<const h4*>(xr + kk);
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[4 * j4 + j] = (float)f[j];
+            } else if constexpr (VEC) {                            // k % 4 == 0: a float4 is all in or all out
                 float4 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                 if (live && k0 < k_end && kk < k) f = *reinterpret_cast<const float4*>(xr + kk);
                 v[4 * j4] = f.x; v[4 * j4 + 1] = f.y; v[4 * j4 + 2] = f.z; v[4 * j4 + 3] = f.w;
@@ -167,7 +174,7 @@ __global__ __launch_bounds__(STAGED ? 64 * kI8WK : 64) void w4_i8_prepare_kernel
                 for (int j = 0; j < 4; j++) {
                     const bool in = live && k0 < k_end && kk + j < k;
                     const uint32_t src = in ? (perm ? (uint32_t)perm[kk + j] : kk + j) : 0;
-                    const float f = xr[src];
+                    const float f = (float)xr[src];
                     v[4 * j4 + j] = in ? f : 0.0f;
                 }
             }
@@ -527,6 +534,20 @@ __global__ __launch_bounds__(512) void w4_gemm_i8_kernel(W4I8Args a) {
                 if (a.bias) v += a.bias[colc + q];
                 o[q] = v;
             }
+            if (a.y16) {                                       // rounded to f16 once
+                _Float16* d16 = a.y16 + (uint64_t)row * a.n + colc;
+                typedef _Float16 hq __attribute__((ext_vector_type(Q == 3 ? 4 : Q)));
+                if constexpr (Q == 4 || Q == 2) {
+                    hq h;
+#pragma unroll
+                    for (int q = 0; q < Q; q++) h[q] = (_Float16)o[q];
+                    *reinterpret_cast<hq*>(d16) = h;
+                } else {
+#pragma unroll
+                    for (int q = 0; q < Q; q++) d16[q] = (_Float16)o[q];
+                }
+                continue;
+            }
             if constexpr (Q == 4) *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
             else if constexpr (Q == 2) *reinterpret_cast<float2*>(dst) = make_float2(o[0], o[1]);
             else {
@@ -661,21 +682,27 @@ int w4_launch_gemm_i8(const W4Args& a, hipStream_t s) {
     const size_t row_bytes = (size_t)a.k * sizeof(float);
 #define RUMUS_I8_PREPARE(CS)                                                                                           \
     do {                                                                                                               \
-        if (staged)                                                                                                    \
-            hipLaunchKernelGGL((w4_i8_prepare_kernel<CS, false, true>), dim3(rts * 16), dim3(64 * kI8WK), row_bytes, s, \
+        if (a.x16 && a.k % 4 == 0)   /* 8-byte aligned */                                                              \
+            hipLaunchKernelGGL((w4_i8_prepare_kernel<CS, true, false, _Float16>), pgrid, dim3(64), 0, s, a.x16, nullptr, planes, \
+                               rscale, csum, out_n, out_k, out_x, a.m, a.k, steps, chunks, per);                      \
+        else if (a.x16)                                                                                                \
+            hipLaunchKernelGGL((w4_i8_prepare_kernel<CS, false, false, _Float16>), pgrid, dim3(64), 0, s, a.x16, nullptr, planes, \
+                               rscale, csum, out_n, out_k, out_x, a.m, a.k, steps, chunks, per);                      \
+        else if (staged)                                                                                               \
+            hipLaunchKernelGGL((w4_i8_prepare_kernel<CS, false, true, float>), dim3(rts * 16), dim3(64 * kI8WK), row_bytes, s, \
                                a.x, a.perm, planes, rscale, csum, out_n, out_k, out_x, a.m, a.k, steps, chunks, per); \
         else if (vec)                                                                                                  \
-            hipLaunchKernelGGL((w4_i8_prepare_kernel<CS, true, false>), pgrid, dim3(64), 0, s, a.x, a.perm, planes,    \
+            hipLaunchKernelGGL((w4_i8_prepare_kernel<CS, true, false, float>), pgrid, dim3(64), 0, s, a.x, a.perm, planes,    \
                                rscale, csum, out_n, out_k, out_x, a.m, a.k, steps, chunks, per);                      \
         else                                                                                                           \
-            hipLaunchKernelGGL((w4_i8_prepare_kernel<CS, false, false>), pgrid, dim3(64), 0, s, a.x, a.perm, planes,   \
+            hipLaunchKernelGGL((w4_i8_prepare_kernel<CS, false, false, float>), pgrid, dim3(64), 0, s, a.x, a.perm, planes,   \
                                rscale, csum, out_n, out_k, out_x, a.m, a.k, steps, chunks, per);                      \
     } while (0)
     if (cs == 2) RUMUS_I8_PREPARE(2);
     else RUMUS_I8_PREPARE(1);
 #undef RUMUS_I8_PREPARE
     if (int rc = check_launch("w4_i8_prepare_kernel")) return rc;
-    const W4I8Args k{a.packed, a.scales, a.zp, a.zp4, a.bias, planes, rscale, csum, out_n, out_k, out_x, a.y,
+    const W4I8Args k{a.packed, a.scales, a.zp, a.zp4, a.bias, planes, rscale, csum, out_n, out_k, out_x, a.y, a.y16,
                      a.m, a.n, steps, chunks, a.group_size / 64, per};
     const bool zp4 = a.zp4 != nullptr;
     // a wave's whole share in flight when it is up to four chunks (two for two row tiles: registers)
