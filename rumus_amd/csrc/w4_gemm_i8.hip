@@ -55,8 +55,8 @@ struct W4I8Args {
     const int32_t* out_k;     // [row][share][kI8Outliers]: their positions (rows of the packed matrix) ...
     const float* out_x;       // ... and values
     float* y;
-    _Float16* y16;            // instead of y, or null
     uint32_t m, n, steps, chunks, steps_per_group, per;   // per: chunks per share
+    _Float16* y16;            // F16 only, instead of y
 };
 
 
@@ -320,7 +320,7 @@ __device__ __forceinline__ void load_q(const uint32_t* p, uint32_t (&o)[Q]) {
 
 // Q: columns per lane (16*Q per workgroup).  RT: row tiles of 16 per workgroup.  CS: steps of 64 k per
 // chunk (1 or 2).  U: chunks per round = chunks of weight loads in flight per lane.
-template <int Q, int RT, int CS, int U, bool ZP4>
+template <int Q, int RT, int CS, int U, bool ZP4, bool F16>
 __global__ __launch_bounds__(512) void w4_gemm_i8_kernel(W4I8Args a) {
     constexpr int WK = kI8WK;
     static_assert((U * RT) % 2 == 0, "the two activation slots alternate with a fixed phase per unrolled position");
@@ -534,7 +534,7 @@ __global__ __launch_bounds__(512) void w4_gemm_i8_kernel(W4I8Args a) {
                 if (a.bias) v += a.bias[colc + q];
                 o[q] = v;
             }
-            if (a.y16) {                                       // rounded to f16 once
+            if constexpr (F16) {                               // rounded to f16 once (asked for at run time the f32 form loses 0.2 us of 13.6)
                 _Float16* d16 = a.y16 + (uint64_t)row * a.n + colc;
                 typedef _Float16 hq __attribute__((ext_vector_type(Q == 3 ? 4 : Q)));
                 if constexpr (Q == 4 || Q == 2) {
@@ -621,8 +621,9 @@ bool w4_gemm_i8_supported(const W4Args& a, double* us) {
 template <int Q, int RT, int CS, int U>
 static int launch_i8(const W4I8Args& k, bool zp4, uint32_t row_blocks, hipStream_t s) {
     const dim3 grid(ceil_div(k.n, 16 * Q), row_blocks);
-    if (zp4) hipLaunchKernelGGL((w4_gemm_i8_kernel<Q, RT, CS, U, true>), grid, dim3(512), 0, s, k);
-    else hipLaunchKernelGGL((w4_gemm_i8_kernel<Q, RT, CS, U, false>), grid, dim3(512), 0, s, k);
+    if (k.y16) hipLaunchKernelGGL((w4_gemm_i8_kernel<Q, RT, CS, U, false, true>), grid, dim3(512), 0, s, k);
+    else if (zp4) hipLaunchKernelGGL((w4_gemm_i8_kernel<Q, RT, CS, U, true, false>), grid, dim3(512), 0, s, k);
+    else hipLaunchKernelGGL((w4_gemm_i8_kernel<Q, RT, CS, U, false, false>), grid, dim3(512), 0, s, k);
     return check_launch("w4_gemm_i8_kernel");
 }
 
@@ -702,8 +703,8 @@ int w4_launch_gemm_i8(const W4Args& a, hipStream_t s) {
     else RUMUS_I8_PREPARE(1);
 #undef RUMUS_I8_PREPARE
     if (int rc = check_launch("w4_i8_prepare_kernel")) return rc;
-    const W4I8Args k{a.packed, a.scales, a.zp, a.zp4, a.bias, planes, rscale, csum, out_n, out_k, out_x, a.y, a.y16,
-                     a.m, a.n, steps, chunks, a.group_size / 64, per};
+    const W4I8Args k{a.packed, a.scales, a.zp, a.zp4, a.bias, planes, rscale, csum, out_n, out_k, out_x, a.y,
+                     a.m, a.n, steps, chunks, a.group_size / 64, per, a.y16};
     const bool zp4 = a.zp4 != nullptr;
     // a wave's whole share in flight when it is up to four chunks (two for two row tiles: registers)
     if (rt_per == 1) return cs == 2 ? launch_i8_q<1, 2, 4>(k, zp4, row_blocks, s) : launch_i8_q<1, 1, 4>(k, zp4, row_blocks, s);
