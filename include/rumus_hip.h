@@ -250,7 +250,7 @@ int rumus_hip_f16_to_f32(const uint16_t* in, float* out, uint64_t numel,
  * sigma keep the tolerance.  The u4-zero-point decode entry point
  * (rumus_hip_qmatmul_int4_decode_zp4) does not make that exception and keeps
  * the plain bound.  Batches of more than 256 rows that the six-bit-float
- * kernel takes (group_size % 64 == 0, k from 1024 to 16384, where it is the faster one)
+ * kernel takes (group_size % 64 == 0, k from 1024, padded_k to 16384, where it is the faster one)
  * keep 24 bits below the largest of 32 consecutive k, and 39 where an
  * eighth of those lies 2^8 or more below it.  The others, which the f16 tile
  * kernel takes, keep 22 bits of every element and add in f32.  Both are

@@ -55,6 +55,7 @@ constexpr int kF6Tile = kF6Digits * 1536;       // bytes of one row tile and one
 constexpr int kF6Step = kF6Tiles * kF6Tile;     // 30 KB
 constexpr int kF6Lo = kF6Digits * 1024;         // inside a tile: the lanes' first 16 bytes of every digit, then their last 8
 constexpr int kF6BTile = 1024 + 512 + 32;       // the same for 32 columns of weights; 32 bytes of skew against bank conflicts
+constexpr uint32_t kF6MaxK = 16384;             // padded to whole groups: a thread of the preparation per 32 k of a row, a row in LDS
 constexpr uint32_t kF6Flags = 256;              // parts of the zero-point table, one flag word each
 constexpr int kF6Deep = 3;                      // further digits where a run of 32 k spans many binades
 constexpr uint32_t kF6DeepBit = 0x80;           // of an exponent byte: the run needs them (the exponents themselves stay below 128)
@@ -908,7 +909,8 @@ bool w4_gemm_f6_chosen(const W4Args& a) {
                            reinterpret_cast<uintptr_t>(a.zp) | reinterpret_cast<uintptr_t>(a.y) |
                            reinterpret_cast<uintptr_t>(a.perm) | reinterpret_cast<uintptr_t>(a.bias);
     if (!(a.m > 256 && a.m <= 65535u * kF6BM && a.n % 4 == 0 && (bits & 15) == 0 && !a.g_idx && !a.tiled &&
-          a.group_size % 64 == 0 && (!a.zp4 || a.n % 8 == 0) && a.k >= 1024 && a.k <= 16384 &&    // (what the estimates were fitted to; a row of x in LDS, and 512 units of 32 k)
+          a.group_size % 64 == 0 && (!a.zp4 || a.n % 8 == 0) && a.k >= 1024 &&                    // (what the estimates were fitted to)
+          a.padded_k <= kF6MaxK &&
           (uint64_t)a.padded_k / 8 * a.n * 4 < (1ull << 32) && (uint64_t)a.m * a.n < (1ull << 32)))
         return false;
     double us = 0.0, other = 0.0;
@@ -942,6 +944,7 @@ static int launch_f6_groups(const F6Args& f, const W4Args& a, uint32_t blocks, h
 }
 
 int w4_launch_gemm_f6(const W4Args& a, hipStream_t s, const W4BlockArgs& block) {
+    RUMUS_REQUIRE(a.padded_k <= kF6MaxK, "qmatmul_int4: padded_k %u is beyond the six-bit kernel's %u", a.padded_k, kF6MaxK);
     const F6Workspace w(a.m, a.padded_k);
     void* ws = nullptr;
     WorkspaceLease lease;                                    // until the last kernel of this call is queued

@@ -2,6 +2,7 @@
 the float64 product."""
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from gpu_util import dev, host, say
@@ -71,3 +72,35 @@ def test_six_bit_kernel_at_its_edges(ops, m, k, n, g, act_order, zeros):
     err = np.abs(got[rows] - exact) / (terms + 1e-300)
     say(f"    worst error / bound {err.max() / bound:.3f}")
     assert (err <= bound).all()
+
+
+# Long rows, where the preparation takes two rows or one per workgroup, and groups that pad K beyond what it takes (then
+# another kernel runs).  The stream's workspace holds another call's digits, exponents and sums, every run of 32 marked
+# there, and the padding nibbles are 15: what a kernel reads without having written it shows.
+@pytest.mark.parametrize("k,g,taken", [(4096, 128, True), (7000, 192, True), (11008, 64, True), (16384, 128, True), (16320, 192, True),
+                                       (16384, 192, False), (16384, 384, False), (16136, 384, False), (14336, 6144, False), (9224, 9216, False)])
+def test_long_rows(ops, k, g, taken):
+    m, n = 1500, 4096
+    say(f"w4 forward m={m} k={k} n={n} g={g}, six-bit kernel: {taken}")
+    assert ops.qmatmul_int4_block_takes(m, k, n, g) == taken
+    gen = torch.Generator(device="cuda").manual_seed(k + g)
+    normal = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    packed, scales, zp = ops.w4_quantize_pack(normal(k, n) * 0.02, g)
+    other = normal(2000, 4096)
+    other[:, ::32] *= 1e5
+    ops.qmatmul_int4(other, *ops.w4_quantize_pack(normal(4096, n) * 0.02, 64), 4096, 64)
+    packed[k // 8:] = -1
+    x = normal(m, k)
+    x[5:9, k - 30] *= 1000.0
+    x[m - 1, 100] *= 3000.0
+    got = ops.qmatmul_int4(x, packed, scales, zp, k, g)
+    rows = torch.cat([torch.arange(40), torch.arange(700, 740), torch.arange(m - 40, m)]).cuda()
+    q = torch.stack([(packed[:k // 8] >> (4 * i)) & 15 for i in range(8)], 1).reshape(k, n).double()
+    expand = lambda t: t.double().repeat_interleave(g, 0)[:k]
+    z, s, xs = expand(zp), expand(scales), x[rows].double()
+    exact = xs @ ((q - z) * s)
+    near = z.round().clamp(0, 15)
+    terms = xs.abs() @ (((q - near).abs() + (z - near).abs()) * s.abs())
+    padded, groups = ops.w4_geometry(k, g)
+    bound = (6 * padded // 64 + 2 * groups + 8) * 2.0 ** -23                 # as above
+    assert ((got[rows].double() - exact).abs() <= bound * terms).all()
