@@ -394,7 +394,7 @@ template <int TN, int FOLD, bool ZP4>
 __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
     constexpr int BN = 128 * TN, CPT = TN == 2 ? 1 : 2;          // columns per workgroup; columns each thread converts per step
     constexpr int BBYTES = 4 * TN * kF6BTile;
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // A[2][kF6Step], B[2][BBYTES]
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // A[2][kF6Step], B[2][BBYTES], 16 bytes per thread
     uint8_t* const lds_b = lds + 2 * kF6Step;
 
     const uint32_t tid = threadIdx.x, lane = tid & 63;
@@ -519,10 +519,33 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
     auto scales_of = [&](uint32_t g) __attribute__((always_inline)) {
         return f6_cols_at<TN>(b_scales, my_col_c * 4, min(g, a.num_groups - 1) * row_bytes);
     };
-    auto nonzero = [](float s) { return s == 0.0f ? 1e-30f : s; };
-    F6Floats<TN> sc_cur, sc_next, ratio;
+    // The accumulators are kept in units of the current group's scale.  A scale far below those before it would take them out of
+    // f32's range (and a zero or a subnormal its reciprocal): the unit is 2^-60 of the column's largest scale so far at
+    // least, and such a group counts with that.  The largest so far lie in LDS, a slot per lane (no registers are left).
+    float* const top_slot = reinterpret_cast<float*>(lds + 2 * (kF6Step + BBYTES)) + tid * 4;
+    auto unit_of = [](float s, float top) __attribute__((always_inline)) {
+        const float least = fmaxf(top * 0x1p-60f, 0x1p-149f);
+        return fabsf(s) < least ? copysignf(least, s) : s;          // (a NaN stays)
+    };
+    auto tops = [&]() __attribute__((always_inline)) {
+        const float4 t = *reinterpret_cast<const float4*>(top_slot);
+        const float v[4] = {t.x, t.y, t.z, t.w};
+        F6Floats<TN> o;
 #pragma unroll
-    for (int j = 0; j < TN; j++) ratio.v[j] = 1.0f;
+        for (int j = 0; j < TN; j++) o.v[j] = v[j];
+        return o;
+    };
+    auto tops_store = [&](const F6Floats<TN>& f) __attribute__((always_inline)) {
+        *reinterpret_cast<float4*>(top_slot) = make_float4(f.v[0], f.v[1], TN > 2 ? f.v[TN > 2 ? 2 : 0] : 0.0f, TN > 3 ? f.v[TN > 3 ? 3 : 0] : 0.0f);
+    };
+    F6Floats<TN> sc_cur, sc_next, top, ratio;
+    sc_cur = scales_of(0);
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        ratio.v[j] = 1.0f;
+        top.v[j] = fabsf(sc_cur.v[j]);
+    }
+    tops_store(top);
 
     constexpr int kB0 = 130 | (126 << 8) | (121 << 16) | (116 << 24), kB1 = 111;   // 2^3 / 2^shift of every digit
 
@@ -574,14 +597,19 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
                 sc_cur = scales_of(min(s, a.steps - 1) / a.steps_per_group);
                 sc_next = scales_of(min(s + 1, a.steps - 1) / a.steps_per_group);
             }
+            if (ENDS && t == 4) top = tops();
             if (ENDS && t == 5) {
 #pragma unroll
                 for (int j = 0; j < TN; j++) {
-                    const float sc = nonzero(sc_cur.v[j]), sn = nonzero(sc_next.v[j]);
-                    const float rc = __builtin_amdgcn_rcpf(sn);
+                    const float now = unit_of(sc_cur.v[j], top.v[j]);
+                    top.v[j] = fmaxf(top.v[j], fabsf(sc_next.v[j]));
+                    const float next = unit_of(sc_next.v[j], top.v[j]);
+                    const float up = fabsf(next) < 0x1p-64f ? 0x1p64f : 1.0f;   // (the reciprocal of a normal number)
+                    const float sc = now * up, sn = next * up, rc = __builtin_amdgcn_rcpf(sn);
                     const float q = sc * rc;
                     ratio.v[j] = fmaf(fmaf(-q, sn, sc), rc, q);   // one correction step: within an ulp of the quotient, and 1 for the same group
                 }
+                tops_store(top);
             }
             if (ENDS && t >= 6 && t < 6 + TN) {
 #pragma unroll
@@ -643,9 +671,12 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
     RUMUS_F6_WAIT(0);                                              // the loads past the last step have landed: the LDS is free
     __syncthreads();
 
+    // the last unit of every column; the slots hold these from now on
     sc_cur = scales_of(a.num_groups - 1);
+    top = tops();
 #pragma unroll
-    for (int j = 0; j < TN; j++) sc_cur.v[j] = nonzero(sc_cur.v[j]);
+    for (int j = 0; j < TN; j++) sc_cur.v[j] = unit_of(sc_cur.v[j], top.v[j]);
+    tops_store(sc_cur);
 
     // ---- the further digits of marked runs; ordinary data has none --------------------------------------------------
     if (__syncthreads_or((deep & (0x0101u * kF6DeepBit)) != 0)) {
@@ -723,7 +754,7 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
                     t = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(da[0], fb, t, 2, 2, 0, ea, 0, 130 - kF6Shift[kF6Digits]);
                     t = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(da[1], fb, t, 2, 2, 0, ea, 0, 130 - kF6Shift[kF6Digits + 1]);
                     t = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(da[2], fb, t, 2, 2, 0, ea, 0, 130 - kF6Shift[kF6Digits + 2]);
-                    const float ratio_s = nonzero(sc.v[j]) / sc_cur.v[j];
+                    const float ratio_s = sc.v[j] / sc_cur.v[j];
 #pragma unroll
                     for (int r = 0; r < 16; r++) acc[i][j][r] = fmaf(t[r], ratio_s, acc[i][j][r]);
                 }
@@ -753,7 +784,10 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
             };
             const uint32_t spg = a.steps_per_group, gb = a.num_groups - 1;
             const uint32_t t_col = min(n0 + tid, a.n - 1);             // BN <= 512: a column per thread
-            const float t_unit = 1.0f / nonzero(a.scales[(uint64_t)gb * a.n + t_col]);
+            __syncthreads();
+            const uint32_t t_c = min(tid, (uint32_t)BN - 1);
+            const float last = reinterpret_cast<const float*>(lds + 2 * (kF6Step + BBYTES))[(t_c / (32 * TN) * 64 + t_c % (32 * TN) / TN) * 4 + t_c % TN];
+            const float up = fabsf(last) < 0x1p-64f ? 0x1p64f : 1.0f, t_unit = 1.0f / (last * up);
             for (uint32_t g0 = 0; g0 <= gb; g0 += GROUPS) {
                 const uint32_t count = min(GROUPS, gb - g0 + 1);
                 if (tid < BN) {
@@ -768,7 +802,7 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
 #pragma unroll
                         for (int u = 0; u < 8; u++) {
                             const float z = fminf(fmaxf(rintf(zv[u]), 0.0f), 15.0f);
-                            t_y[(g + u) * BN + tid] = g + u < count ? -(zv[u] - z) * sv[u] * t_unit : 0.0f;
+                            t_y[(g + u) * BN + tid] = g + u < count ? -(zv[u] - z) * (sv[u] * up) * t_unit : 0.0f;
                         }
                     }
                 }
@@ -923,7 +957,7 @@ bool w4_gemm_f6_chosen(const W4Args& a) {
 
 template <int TN, int FOLD, bool ZP4>
 static int launch_f6(const F6Args& f, uint32_t blocks, hipStream_t s) {
-    constexpr size_t lds_bytes = 2 * (size_t)(kF6Step + 4 * TN * kF6BTile);
+    constexpr size_t lds_bytes = 2 * (size_t)(kF6Step + 4 * TN * kF6BTile) + 512 * 16;
     static_assert(lds_bytes <= 160 * 1024, "two steps fit the LDS");
     static bool attr_set = false;   // benign race: setting the attribute is idempotent
     if (!attr_set) {

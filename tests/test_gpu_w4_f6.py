@@ -104,3 +104,44 @@ def test_long_rows(ops, k, g, taken):
     padded, groups = ops.w4_geometry(k, g)
     bound = (6 * padded // 64 + 2 * groups + 8) * 2.0 ** -23                 # as above
     assert ((got[rows].double() - exact).abs() <= bound * terms).all()
+
+
+# The accumulators are kept in units of the current group's scale: scales that are zero, subnormal or tiny beside others, in
+# the first, a middle and the last group, in all but one and in all of a column; signs that change; and large ones.
+@pytest.mark.parametrize("k,g,zeros", [(1024, 64, "fractional"), (1152, 128, "integer"), (1536, 256, "fractional"), (1024, 128, "u4")])
+def test_scales_far_apart(ops, k, g, zeros):
+    m, n = 1409, 6144 if zeros == "u4" else 2820
+    say(f"w4 forward, six-bit kernel, scales far apart: m={m} k={k} n={n} g={g} zero-points {zeros}")
+    if zeros != "u4":
+        assert ops.qmatmul_int4_block_takes(m, k, n, g)
+    gen = torch.Generator(device="cuda").manual_seed(k + n)
+    packed, scales, zp = ops.w4_quantize_pack(torch.randn(k, n, device="cuda", generator=gen) * 0.02, g)
+    if zeros != "fractional":
+        zp = zp.round().clamp(0, 15)
+    col, last = 0, scales.shape[0] - 1
+    for value in (1e-40, 1.4e-45, 1e-37, 1e-30, 0.0, -1e-39, -0.02, 1e25):
+        for at in ([0], [last // 2], [last], [0, last], list(range(1, last)), list(range(last)), list(range(1, last + 1)), list(range(last + 1))):
+            scales[at, col:col + 3] = value
+            col += 5
+    scales[::2, col:col + 40] *= 1e-33                   # back and forth
+    scales[1::3, col + 20:col + 40] *= 1e-12
+    x = torch.randn(m, k, device="cuda", generator=gen)
+    x[m - 3] *= 1e8
+    if zeros == "u4":
+        shifts = 4 * torch.arange(8, device="cuda", dtype=torch.int32)
+        qzeros = (zp.to(torch.int32).reshape(-1, n // 8, 8) << shifts).sum(2).to(torch.int32)
+        got = ops.qmatmul_int4_zp4(x, packed, scales, qzeros, k, g)
+    else:
+        got = ops.qmatmul_int4(x, packed, scales, zp, k, g)
+    rows = torch.cat([torch.arange(40), torch.arange(700, 740), torch.arange(m - 40, m)]).cuda()
+    q = torch.stack([(packed >> (4 * i)) & 15 for i in range(8)], 1).reshape(-1, n)[:k].double()
+    expand = lambda t: t.double().repeat_interleave(g, 0)[:k]
+    z, s, xs = expand(zp), expand(scales), x[rows].double()
+    exact = xs @ ((q - z) * s)
+    near = z.round().clamp(0, 15)
+    levels = xs.abs() @ ((q - near).abs() + (z - near).abs())
+    terms = xs.abs() @ (((q - near).abs() + (z - near).abs()) * s.abs())
+    # as above; a group far below the column's largest scale counts with 2^-60 of that, and a result is a multiple of 2^-149
+    steps = -(-k // 64)
+    bound = (6 * steps + 2 * scales.shape[0] + 8) * 2.0 ** -23 * terms + levels * (s.abs().amax(0) * 2.0 ** -59 + 2.0 ** -148) + 2.0 ** -148
+    assert torch.isfinite(got).all() and ((got[rows].double() - exact).abs() <= bound).all()
