@@ -74,6 +74,7 @@ struct F6Args {
     const float* x;            // for the further digits of marked runs, with its gather and width
     const int32_t* perm;
     const float* rfac;         // [row]: back to the row's own scale (NaN: the row holds a NaN or an infinity)
+    const float* least;        // [column]: the smallest unit of its accumulators (NaN: a scale is)
     const uint32_t* zflags;    // kF6Flags words, nonzero where a part of the zero-point table holds a value that is no integer in 0..15
     float* y;
     uint32_t m, k, n, steps, steps_per_group, num_groups;
@@ -114,7 +115,7 @@ __device__ __forceinline__ v6u f6_digit(v16f& ev, v16f& od, float unit) {
 // instruction would touch 64 cache lines for 256 bytes.  Memory bound: 2048 x 4096 reads 33.5 and writes 32 MB in 14 us.
 // LDS: row r at r * pitch floats, 4 floats of padding after every 32, so that the 16-byte reads of threads 32 floats
 // apart fall on different banks (likewise rows: pitch / 4 is odd).
-// Beyond the row groups, kF6Flags more workgroups look at the zero-points.
+// Beyond the row groups, more workgroups look at the columns' scales, 64 columns each, and kF6Flags at f32 zero-points.
 __device__ __forceinline__ uint32_t f6_padded(uint32_t j) { return j + (j >> 5) * 4; }
 
 // What the rows of x go through on their way into LDS (a decoder block's operators in front of a projection; k % 4 == 0 and
@@ -129,7 +130,9 @@ __global__ __launch_bounds__(512) void w4_f6_prepare_kernel(const float* __restr
                                                             float* __restrict__ sums, float* __restrict__ rfac,
                                                             uint32_t m, uint32_t k, uint32_t steps, uint32_t rows,
                                                             uint32_t pitch, const float4* __restrict__ zp, uint32_t zp_count4,
-                                                            uint32_t* __restrict__ zflags, uint32_t row_groups,
+                                                            uint32_t* __restrict__ zflags, const float* __restrict__ scales,
+                                                            uint32_t num_groups, uint32_t n, float* __restrict__ least,
+                                                            uint32_t row_groups,
                                                             const float* __restrict__ norm_w, float eps,
                                                             float* __restrict__ marked) {
     constexpr bool PERM = IN == kF6Perm;
@@ -139,7 +142,29 @@ __global__ __launch_bounds__(512) void w4_f6_prepare_kernel(const float* __restr
     constexpr uint32_t T = 512;
     const uint32_t tid = threadIdx.x;
     if (blockIdx.x >= row_groups) {
-        const uint32_t part = blockIdx.x - row_groups;
+        uint32_t part = blockIdx.x - row_groups;
+        if (part < (n + 63) / 64) {                            // eight waves share the groups
+            const uint32_t col = part * 64 + (tid & 63), at = min(col, n - 1);
+            uint32_t top = 0;                                    // bit patterns without their sign: a NaN sorts highest
+            for (uint32_t g = tid >> 6; g < num_groups; g += 64) {
+                uint32_t v[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) v[u] = __float_as_uint(scales[(uint64_t)min(g + 8 * u, num_groups - 1) * n + at]);
+#pragma unroll
+                for (int u = 0; u < 8; u++) top = max(top, v[u] & 0x7fffffffu);
+            }
+            uint32_t* const tops = reinterpret_cast<uint32_t*>(lds_x);   // [8][64]
+            tops[tid] = top;
+            __syncthreads();
+            if (tid < 64 && col < n) {
+#pragma unroll
+                for (int w = 1; w < 8; w++) top = max(top, tops[64 * w + tid]);
+                const float t = __uint_as_float(top);
+                least[col] = t != t ? t : fmaxf(t * 0x1p-60f, 0x1p-126f);
+            }
+            return;
+        }
+        part -= (n + 63) / 64;
         bool mine = false;
         for (uint32_t i = part * T + tid; i < zp_count4; i += kF6Flags * T) {
             const float4 z = zp[i];
@@ -519,33 +544,24 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
     auto scales_of = [&](uint32_t g) __attribute__((always_inline)) {
         return f6_cols_at<TN>(b_scales, my_col_c * 4, min(g, a.num_groups - 1) * row_bytes);
     };
-    // The accumulators are kept in units of the current group's scale.  A scale far below those before it would take them out of
-    // f32's range (and a zero or a subnormal its reciprocal): the unit is 2^-60 of the column's largest scale so far at
-    // least, and such a group counts with that.  The largest so far lie in LDS, a slot per lane (no registers are left).
-    float* const top_slot = reinterpret_cast<float*>(lds + 2 * (kF6Step + BBYTES)) + tid * 4;
-    auto unit_of = [](float s, float top) __attribute__((always_inline)) {
-        const float least = fmaxf(top * 0x1p-60f, 0x1p-149f);
-        return fabsf(s) < least ? copysignf(least, s) : s;          // (a NaN stays)
-    };
-    auto tops = [&]() __attribute__((always_inline)) {
-        const float4 t = *reinterpret_cast<const float4*>(top_slot);
-        const float v[4] = {t.x, t.y, t.z, t.w};
+    // The accumulators are kept in units of the current group's scale.  A scale far below the column's others would take them
+    // out of f32's range (and a zero or a subnormal its reciprocal): the unit is 2^-60 of the column's largest scale, and
+    // 2^-126, at least (w4_f6_prepare_kernel finds it), and a smaller group counts with that.  It lies in LDS, a slot per lane
+    // (no registers are left): with the largest scale so far kept there from group to group a call took 2 to 3 % longer.
+    float* const unit_slot = reinterpret_cast<float*>(lds + 2 * (kF6Step + BBYTES)) + tid * 4;
+    auto units_read = [&]() __attribute__((always_inline)) {
         F6Floats<TN> o;
 #pragma unroll
-        for (int j = 0; j < TN; j++) o.v[j] = v[j];
+        for (int j = 0; j < TN; j++) o.v[j] = unit_slot[j];
         return o;
     };
-    auto tops_store = [&](const F6Floats<TN>& f) __attribute__((always_inline)) {
-        *reinterpret_cast<float4*>(top_slot) = make_float4(f.v[0], f.v[1], TN > 2 ? f.v[TN > 2 ? 2 : 0] : 0.0f, TN > 3 ? f.v[TN > 3 ? 3 : 0] : 0.0f);
-    };
-    F6Floats<TN> sc_cur, sc_next, top, ratio;
-    sc_cur = scales_of(0);
+    auto unit_of = [](float s, float least) __attribute__((always_inline)) { return copysignf(fmaxf(fabsf(s), least), s); };
+    F6Floats<TN> sc_cur, sc_next, least, ratio;
 #pragma unroll
     for (int j = 0; j < TN; j++) {
         ratio.v[j] = 1.0f;
-        top.v[j] = fabsf(sc_cur.v[j]);
+        unit_slot[j] = a.least[min(my_col_c + j, a.n - 1)];
     }
-    tops_store(top);
 
     constexpr int kB0 = 130 | (126 << 8) | (121 << 16) | (116 << 24), kB1 = 111;   // 2^3 / 2^shift of every digit
 
@@ -597,19 +613,15 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
                 sc_cur = scales_of(min(s, a.steps - 1) / a.steps_per_group);
                 sc_next = scales_of(min(s + 1, a.steps - 1) / a.steps_per_group);
             }
-            if (ENDS && t == 4) top = tops();
+            if (ENDS && t == 4) least = units_read();
             if (ENDS && t == 5) {
 #pragma unroll
                 for (int j = 0; j < TN; j++) {
-                    const float now = unit_of(sc_cur.v[j], top.v[j]);
-                    top.v[j] = fmaxf(top.v[j], fabsf(sc_next.v[j]));
-                    const float next = unit_of(sc_next.v[j], top.v[j]);
-                    const float up = fabsf(next) < 0x1p-64f ? 0x1p64f : 1.0f;   // (the reciprocal of a normal number)
-                    const float sc = now * up, sn = next * up, rc = __builtin_amdgcn_rcpf(sn);
+                    const float sc = unit_of(sc_cur.v[j], least.v[j]), sn = unit_of(sc_next.v[j], least.v[j]);
+                    const float rc = __builtin_amdgcn_rcpf(sn);
                     const float q = sc * rc;
                     ratio.v[j] = fmaf(fmaf(-q, sn, sc), rc, q);   // one correction step: within an ulp of the quotient, and 1 for the same group
                 }
-                tops_store(top);
             }
             if (ENDS && t >= 6 && t < 6 + TN) {
 #pragma unroll
@@ -673,10 +685,12 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
 
     // the last unit of every column; the slots hold these from now on
     sc_cur = scales_of(a.num_groups - 1);
-    top = tops();
+    least = units_read();
 #pragma unroll
-    for (int j = 0; j < TN; j++) sc_cur.v[j] = unit_of(sc_cur.v[j], top.v[j]);
-    tops_store(sc_cur);
+    for (int j = 0; j < TN; j++) {
+        sc_cur.v[j] = least.v[j] != least.v[j] ? least.v[j] : unit_of(sc_cur.v[j], least.v[j]);   // (the column holds a NaN)
+        unit_slot[j] = sc_cur.v[j];
+    }
 
     // ---- the further digits of marked runs; ordinary data has none --------------------------------------------------
     if (__syncthreads_or((deep & (0x0101u * kF6DeepBit)) != 0)) {
@@ -787,7 +801,7 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
             __syncthreads();
             const uint32_t t_c = min(tid, (uint32_t)BN - 1);
             const float last = reinterpret_cast<const float*>(lds + 2 * (kF6Step + BBYTES))[(t_c / (32 * TN) * 64 + t_c % (32 * TN) / TN) * 4 + t_c % TN];
-            const float up = fabsf(last) < 0x1p-64f ? 0x1p64f : 1.0f, t_unit = 1.0f / (last * up);
+            const float t_unit = 1.0f / last;
             for (uint32_t g0 = 0; g0 <= gb; g0 += GROUPS) {
                 const uint32_t count = min(GROUPS, gb - g0 + 1);
                 if (tid < BN) {
@@ -802,7 +816,7 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
 #pragma unroll
                         for (int u = 0; u < 8; u++) {
                             const float z = fminf(fmaxf(rintf(zv[u]), 0.0f), 15.0f);
-                            t_y[(g + u) * BN + tid] = g + u < count ? -(zv[u] - z) * (sv[u] * up) * t_unit : 0.0f;
+                            t_y[(g + u) * BN + tid] = g + u < count ? -(zv[u] - z) * sv[u] * t_unit : 0.0f;
                         }
                     }
                 }
@@ -919,16 +933,17 @@ static size_t f6_up(size_t v) { return (v + 255) & ~size_t(255); }
 
 struct F6Workspace {
     uint32_t blocks, steps;
-    size_t planes, exps, sums, rfac, flags, total;   // bytes
-    F6Workspace(uint32_t m, uint32_t padded_k) : blocks(ceil_div(m, kF6BM)), steps(padded_k / 64) {
+    size_t planes, exps, sums, rfac, least, flags, total;   // bytes
+    F6Workspace(uint32_t m, uint32_t padded_k, uint32_t n) : blocks(ceil_div(m, kF6BM)), steps(padded_k / 64) {
         // (never less than the f16 tiles park, 4 bytes per element: what a caller reserved or a fixed buffer holds, and what it
         // refuses, does not depend on the kernel)
         planes = std::max((size_t)blocks * steps * kF6Step, (size_t)ceil_div(m, 32) * 32 * padded_k * 4);
         exps = f6_up((size_t)blocks * ((steps + 1) / 2) * kF6Tiles * 64 * 2);
         sums = (size_t)blocks * steps * kF6BM * 4;
         rfac = (size_t)blocks * kF6BM * 4;
+        least = f6_up((size_t)n * 4);
         flags = kF6Flags * 4;
-        total = planes + exps + sums + rfac + flags;
+        total = planes + exps + sums + rfac + least + flags;
     }
 };
 
@@ -951,7 +966,7 @@ bool w4_gemm_f6_chosen(const W4Args& a) {
     f6_pick(a.m, a.k, a.n, &us);
     const bool i8 = w4_gemm_i8_supported(a, &other);
     // what the integer kernel runs within the fixed scratch array (w4_gemv.hip) has to go on running there
-    if (i8 && F6Workspace(a.m, a.padded_k).total > (size_t(32) << 20)) return false;
+    if (i8 && F6Workspace(a.m, a.padded_k, a.n).total > (size_t(32) << 20)) return false;
     return us < (i8 ? 0.92 : 1.0) * other;
 }
 
@@ -979,7 +994,7 @@ static int launch_f6_groups(const F6Args& f, const W4Args& a, uint32_t blocks, h
 
 int w4_launch_gemm_f6(const W4Args& a, hipStream_t s, const W4BlockArgs& block) {
     RUMUS_REQUIRE(a.padded_k <= kF6MaxK, "qmatmul_int4: padded_k %u is beyond the six-bit kernel's %u", a.padded_k, kF6MaxK);
-    const F6Workspace w(a.m, a.padded_k);
+    const F6Workspace w(a.m, a.padded_k, a.n);
     void* ws = nullptr;
     WorkspaceLease lease;                                    // until the last kernel of this call is queued
     const bool folded = block.norm_w || a.glu;
@@ -990,6 +1005,7 @@ int w4_launch_gemm_f6(const W4Args& a, hipStream_t s, const W4BlockArgs& block) 
     uint8_t* const exps = p; p += w.exps;
     float* const sums = reinterpret_cast<float*>(p); p += w.sums;
     float* const rfac = reinterpret_cast<float*>(p); p += w.rfac;
+    float* const least = reinterpret_cast<float*>(p); p += w.least;
     uint32_t* const zflags = reinterpret_cast<uint32_t*>(p);
     // rows per workgroup of the preparation: at most 512 units and 80 KB of LDS (two workgroups per compute unit), and enough workgroups
     const uint32_t units = 2 * w.steps, pitch = units * 36 + 4, rows_pad = w.blocks * kF6BM;
@@ -1003,11 +1019,11 @@ int w4_launch_gemm_f6(const W4Args& a, hipStream_t s, const W4BlockArgs& block) 
                 return rc;
         attr_set = true;
     }
-    const dim3 pgrid(rows_pad / rows + (a.zp4 ? 0 : kF6Flags));
+    const dim3 pgrid(rows_pad / rows + ceil_div(a.n, 64) + (a.zp4 ? 0 : kF6Flags));
 #define RUMUS_F6_PREPARE(IN)                                                                                             \
     hipLaunchKernelGGL(w4_f6_prepare_kernel<IN>, pgrid, dim3(512), (size_t)rows * pitch * 4, s, a.x, a.perm, planes, exps, sums, \
                        rfac, a.m, a.k, w.steps, rows, pitch, reinterpret_cast<const float4*>(a.zp),                        \
-                       (uint32_t)((uint64_t)a.num_groups * a.n / 4), zflags, rows_pad / rows, block.norm_w, block.eps, marked)
+                       (uint32_t)((uint64_t)a.num_groups * a.n / 4), zflags, a.scales, a.num_groups, a.n, least, rows_pad / rows, block.norm_w, block.eps, marked)
     if (a.perm) RUMUS_F6_PREPARE(kF6Perm);
     else if (block.norm_w) RUMUS_F6_PREPARE(kF6Norm);
     else if (a.glu) RUMUS_F6_PREPARE(kF6Glu);
@@ -1015,7 +1031,7 @@ int w4_launch_gemm_f6(const W4Args& a, hipStream_t s, const W4BlockArgs& block) 
 #undef RUMUS_F6_PREPARE
     if (int rc = check_launch("w4_f6_prepare_kernel")) return rc;
     const F6Args f{a.packed, a.scales, a.zp, a.zp4, a.bias, planes, reinterpret_cast<const uint16_t*>(exps), sums, folded ? marked : a.x, a.perm,
-                   rfac, zflags, a.y, a.m, a.k, a.n, w.steps, a.group_size / 64, a.num_groups, block.residual};
+                   rfac, least, zflags, a.y, a.m, a.k, a.n, w.steps, a.group_size / 64, a.num_groups, block.residual};
     double us;
     switch (f6_pick(a.m, a.k, a.n, &us)) {
         case 2: return launch_f6_groups<2>(f, a, w.blocks, s);
