@@ -69,7 +69,7 @@ int rumus_hip_sync(rumus_hip_stream_t stream);
  * inside the call that needs it.  A caller that must not allocate later
  * (graph capture, serving loop) reserves the largest size up front.  Upper
  * bounds per call, in bytes:
- *   qmatmul_int4 / _perm / _zp4, m > 5: 5 * (m + 64) * (padded_k + 128) (activations
+ *   qmatmul_int4 / _perm / _zp4 / _block, m > 5: 5 * (m + 64) * (padded_k + 128) (activations
  *       in matrix-core order and a scale factor per row) + 64 * m * n (partial
  *       sums, only while the output has fewer than 192 tiles of 64 x 512) + 1280
  *       (the last kilobyte: flags of the look at the zero-point table);
@@ -427,7 +427,7 @@ int rumus_hip_qmatmul_int4_decode_block(const float* x, const float* norm_weight
  * kernels of their own.  Only where rumus_hip_qmatmul_int4_block_takes (host
  * arithmetic) returns 1: large batches, group_size % 64 == 0, k % 8 == 0; EINVAL
  * otherwise, and unless the buffers are 16-byte aligned and y != x.  Workspace:
- * that of qmatmul_int4, and with norm_weight or swiglu 4 * m * k + 256 more. */
+ * that of qmatmul_int4. */
 int rumus_hip_qmatmul_int4_block_takes(uint32_t m, uint32_t k, uint32_t n, uint32_t group_size);
 int rumus_hip_qmatmul_int4_block(const float* x, const float* norm_weight, float eps, int swiglu,
                                  const uint32_t* packed, const float* scales,

@@ -71,8 +71,11 @@ struct F6Args {
     const uint8_t* planes;     // [row block][step][kF6Step]
     const uint16_t* exps;      // [row block][pair of steps][row tile][64 lanes]: two E8M0 bytes
     const float* sums;         // [row block][step][kF6BM rows]: sum of x over the step's 64 k
-    const float* x;            // for the further digits of marked runs, with its gather and width
+    const float* x;            // for the further digits of marked runs, with what the preparation does to its rows
     const int32_t* perm;
+    const float* norm_w;
+    bool glu;
+    const float* rinv;         // [row], RMSNorm: 1 / rms
     const float* rfac;         // [row]: back to the row's own scale (NaN: the row holds a NaN or an infinity)
     const float* least;        // [column]: the smallest unit of its accumulators (NaN: a scale is)
     const uint32_t* zflags;    // kF6Flags words, nonzero where a part of the zero-point table holds a value that is no integer in 0..15
@@ -120,9 +123,11 @@ __device__ __forceinline__ uint32_t f6_padded(uint32_t j) { return j + (j >> 5) 
 
 // What the rows of x go through on their way into LDS (a decoder block's operators in front of a projection; k % 4 == 0 and
 // 16-byte aligned then): RMSNorm with `norm_w`, or SwiGLU of rows gate | up of 2 k floats.  Their results are written
-// nowhere else but for the marked runs, which the matmul wants once more in f32 (`marked` [m][k]).
+// nowhere: for marked runs the matmul computes them once more, in the same operations.
 // 4096 rows: SwiGLU of 2 x 11008 125 + 113 us as two kernels, 163 as one; RMSNorm of 4096 25 + 27 us, 35 as one.
 enum F6In { kF6Plain, kF6Perm, kF6Norm, kF6Glu };
+__device__ __forceinline__ float f6_norm(float v, float inv, float w) { return v * inv * w; }
+__device__ __forceinline__ float f6_glu(float a, float b) { return a / (1.0f + expf(-a)) * b; }
 
 template <F6In IN>
 __global__ __launch_bounds__(512) void w4_f6_prepare_kernel(const float* __restrict__ x, const int32_t* __restrict__ perm,
@@ -134,7 +139,7 @@ __global__ __launch_bounds__(512) void w4_f6_prepare_kernel(const float* __restr
                                                             uint32_t num_groups, uint32_t n, float* __restrict__ least,
                                                             uint32_t row_groups,
                                                             const float* __restrict__ norm_w, float eps,
-                                                            float* __restrict__ marked) {
+                                                            float* __restrict__ rinv) {
     constexpr bool PERM = IN == kF6Perm;
     extern __shared__ __attribute__((aligned(16))) float lds_x[];
     __shared__ uint32_t rowmax[8];
@@ -208,10 +213,9 @@ __global__ __launch_bounds__(512) void w4_f6_prepare_kernel(const float* __restr
                         g[u] = reinterpret_cast<const float4*>(src)[min(i0 + u * per_row, last)];
                         v[u] = reinterpret_cast<const float4*>(src + k)[min(i0 + u * per_row, last)];
                     }
-                    auto glu = [](float a, float b) { return a / (1.0f + expf(-a)) * b; };
 #pragma unroll
                     for (int u = 0; u < 8; u++) {
-                        const float4 y = make_float4(glu(g[u].x, v[u].x), glu(g[u].y, v[u].y), glu(g[u].z, v[u].z), glu(g[u].w, v[u].w));
+                        const float4 y = make_float4(f6_glu(g[u].x, v[u].x), f6_glu(g[u].y, v[u].y), f6_glu(g[u].z, v[u].z), f6_glu(g[u].w, v[u].w));
                         *reinterpret_cast<float4*>(dst + f6_padded(4 * min(i0 + u * per_row, last))) = y;
                         look(y);
                     }
@@ -240,10 +244,11 @@ __global__ __launch_bounds__(512) void w4_f6_prepare_kernel(const float* __restr
             for (uint32_t w = 0; w < waves; w++) total += squares[r1 * waves + w];
             const float inv = 1.0f / sqrtf(total / (float)k + eps);
             if (r1 < live) {
+                if (t1 == 0) rinv[row0 + r1] = inv;
                 for (uint32_t i = t1; i <= last; i += per_row) {     // every thread's own elements
                     const float4 w = reinterpret_cast<const float4*>(norm_w)[i];
                     float4* const at = reinterpret_cast<float4*>(dst + f6_padded(4 * i));
-                    const float4 v = *at, y = make_float4(v.x * inv * w.x, v.y * inv * w.y, v.z * inv * w.z, v.w * inv * w.w);
+                    const float4 v = *at, y = make_float4(f6_norm(v.x, inv, w.x), f6_norm(v.y, inv, w.y), f6_norm(v.z, inv, w.z), f6_norm(v.w, inv, w.w));
                     *at = y;
                     look(y);
                 }
@@ -308,13 +313,6 @@ __global__ __launch_bounds__(512) void w4_f6_prepare_kernel(const float* __restr
     }
     const bool is_deep = low < top * 0.00390625f;
     if (!mine) return;                                           // whole waves or the tail of one: no barrier follows
-    if constexpr (IN == kF6Norm || IN == kF6Glu) {
-        if (is_deep) {                                           // (only rows below m have such runs)
-            for (uint32_t j = 0; j < 32 && 32 * unit + j < k; j += 4)
-                *reinterpret_cast<float4*>(marked + (uint64_t)row * k + 32 * unit + j) =
-                    *reinterpret_cast<const float4*>(lds_x + r * pitch + unit * 36 + j);
-        }
-    }
     float sum = 0.0f;
 #pragma unroll
     for (int j = 0; j < 32; j++) sum += v[j];
@@ -694,14 +692,54 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
 
     // ---- the further digits of marked runs; ordinary data has none --------------------------------------------------
     if (__syncthreads_or((deep & (0x0101u * kF6DeepBit)) != 0)) {
+        // LDS: the codes of the further digits, the step's values of x and RMSNorm weights, and which steps have marks
+        constexpr int DTILE = kF6Deep * 1536;
+        constexpr uint32_t PITCH = 64 + 4;
+        static_assert(kF6Tiles * DTILE + (kF6BM * PITCH + 64 + kF6MaxK / 64) * 4 <= 2 * kF6Step, "they fit the buffers of the planes");
+        float* const values = reinterpret_cast<float*>(lds + kF6Tiles * DTILE);
+        float* const weights = values + kF6BM * PITCH;
+        uint32_t* const has_marks = reinterpret_cast<uint32_t*>(weights + 64);
+        if (tid < kF6MaxK / 64) has_marks[tid] = 0;
+        __syncthreads();
+        {
+            const uint32_t* const e2 = reinterpret_cast<const uint32_t*>(a.exps) + (uint64_t)blk * e_pairs * (kF6Tiles * 32);
+            for (uint32_t i = tid; i < e_pairs * (kF6Tiles * 32); i += 512) {   // two lanes of a pair of steps
+                const uint32_t e = e2[i];
+                if (e & 0x00010001u * kF6DeepBit) has_marks[i / (kF6Tiles * 32) * 2] = 1;
+                if (e & 0x01000100u * kF6DeepBit) has_marks[i / (kF6Tiles * 32) * 2 + 1] = 1;
+            }
+        }
+        __syncthreads();
+        // a thread per run: its row's factors
+        const uint32_t d_row = m0 + tid % kF6BM, d_half = tid / kF6BM, d_tile = tid % kF6BM / 32, d_lane = d_half * 32 + (tid & 31);
+        const uint32_t d_rowc = min(d_row, a.m - 1);
+        const float d_rv = __uint_as_float((254u - (__float_as_uint(a.rfac[d_rowc]) >> 23)) << 23), d_inv = a.norm_w ? a.rinv[d_rowc] : 0.0f;
         for (uint32_t s = 0; s < a.steps; s++) {
-            if ((s & 1) == 0) exps_load(s);
+            if (!has_marks[s]) continue;
             const uint32_t e_shift = 8 * (s & 1);
-            if (!__syncthreads_or(((exps_next[0] | exps_next[1]) >> e_shift & kF6DeepBit) != 0)) continue;
-            // this step's weights once more
+            // everything that the step reads from memory at once: its weights and values once more, exponents, scales
+            const uint32_t kk = 64 * s + lane, from = kk >= a.k ? 0 : a.perm ? (uint32_t)a.perm[kk] : kk;
 #pragma unroll
             for (int i = 0; i < 4; i++) word_load(s, 0, i);
             zp_load(s, 0);
+            exps_load(s);
+            const uint32_t e = a.exps[(((uint64_t)blk * e_pairs + s / 2) * kF6Tiles + d_tile % kF6Tiles) * 64 + d_lane % 64] >> e_shift & 0xffu;
+            const F6Floats<TN> sc = scales_of(s / a.steps_per_group);
+            constexpr int ROWS = kF6BM / 8;                        // of a wave, 64 values each
+            const uint32_t width = a.glu ? 2 * a.k : a.k;
+            float xv[ROWS];
+#pragma unroll
+            for (int i = 0; i < ROWS; i++) xv[i] = a.x[(uint64_t)min(m0 + wave + 8 * i, a.m - 1) * width + from];
+            if (a.glu) {
+                float up[ROWS];
+#pragma unroll
+                for (int i = 0; i < ROWS; i++) up[i] = a.x[(uint64_t)min(m0 + wave + 8 * i, a.m - 1) * width + a.k + from];
+#pragma unroll
+                for (int i = 0; i < ROWS; i++) xv[i] = f6_glu(xv[i], up[i]);
+            }
+            if (a.norm_w && wave == 0) weights[lane] = kk < a.k ? a.norm_w[from] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < ROWS; i++) values[(wave + 8 * i) * PITCH + lane] = kk < a.k ? xv[i] : 0.0f;
             zero_points(0);
 #pragma unroll
             for (int c = 0; c < CPT; c++) {
@@ -709,30 +747,23 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
                 convert_words(0, c, 2);
                 column_store(c, std::integral_constant<int, 0>{});
             }
-            // and the runs: a thread each, from x itself, past the digits that the planes hold
-            constexpr int DTILE = kF6Deep * 1536;
+            __syncthreads();
+            // the runs' digits past those that the planes hold
             if (tid < 2 * kF6BM) {
-                const uint32_t r = tid % kF6BM, half = tid / kF6BM, rt = r / 32, ln = half * 32 + (r & 31), row = m0 + r;
-                const uint32_t e = a.exps[(((uint64_t)blk * e_pairs + s / 2) * kF6Tiles + rt) * 64 + ln] >> e_shift & 0xffu;
                 const bool marked = (e & kF6DeepBit) != 0;        // (rows past m are not)
+                const uint32_t rt = d_tile, ln = d_lane;
                 uint8_t* const to = lds + rt * DTILE;
                 v16f ev, od;
                 if (marked) {
-                    const float rv = __uint_as_float((254u - (__float_as_uint(a.rfac[row]) >> 23)) << 23);
-                    const float* const xr = a.x + (uint64_t)row * a.k;
-                    const uint32_t k0 = 64 * s + 32 * half;
-                    uint32_t from[32];
                     float v[32];
 #pragma unroll
-                    for (int j = 0; j < 32; j++) from[j] = min(k0 + j, a.k - 1);
-                    if (a.perm) {
+                    for (int j = 0; j < 32; j++) v[j] = values[tid % kF6BM * PITCH + 32 * d_half + j];
+                    if (a.norm_w) {
 #pragma unroll
-                        for (int j = 0; j < 32; j++) from[j] = (uint32_t)a.perm[from[j]];
+                        for (int j = 0; j < 32; j++) v[j] = f6_norm(v[j], d_inv, weights[32 * d_half + j]);
                     }
 #pragma unroll
-                    for (int j = 0; j < 32; j++) v[j] = xr[from[j]] * rv;
-#pragma unroll
-                    for (int j = 0; j < 32; j++) v[j] = k0 + j < a.k ? v[j] : 0.0f;
+                    for (int j = 0; j < 32; j++) v[j] *= d_rv;
                     f6_order(v, ev, od);
 #pragma unroll
                     for (int d = 0; d < kF6Digits; d++) (void)f6_digit(ev, od, __uint_as_float(((e & (kF6DeepBit - 1)) - kF6Shift[d]) << 23));
@@ -748,7 +779,6 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
                     *reinterpret_cast<uint2*>(to + d * 1536 + 1024 + ln * 8) = make_uint2(code[4], code[5]);
                 }
             }
-            const F6Floats<TN> sc = scales_of(s / a.steps_per_group);
             RUMUS_F6_WAIT(0);
             __syncthreads();
 #pragma unroll
@@ -933,7 +963,7 @@ static size_t f6_up(size_t v) { return (v + 255) & ~size_t(255); }
 
 struct F6Workspace {
     uint32_t blocks, steps;
-    size_t planes, exps, sums, rfac, least, flags, total;   // bytes
+    size_t planes, exps, sums, rfac, rinv, least, flags, total;   // bytes
     F6Workspace(uint32_t m, uint32_t padded_k, uint32_t n) : blocks(ceil_div(m, kF6BM)), steps(padded_k / 64) {
         // (never less than the f16 tiles park, 4 bytes per element: what a caller reserved or a fixed buffer holds, and what it
         // refuses, does not depend on the kernel)
@@ -941,9 +971,10 @@ struct F6Workspace {
         exps = f6_up((size_t)blocks * ((steps + 1) / 2) * kF6Tiles * 64 * 2);
         sums = (size_t)blocks * steps * kF6BM * 4;
         rfac = (size_t)blocks * kF6BM * 4;
+        rinv = rfac;
         least = f6_up((size_t)n * 4);
         flags = kF6Flags * 4;
-        total = planes + exps + sums + rfac + least + flags;
+        total = planes + exps + sums + rfac + rinv + least + flags;
     }
 };
 
@@ -997,14 +1028,13 @@ int w4_launch_gemm_f6(const W4Args& a, hipStream_t s, const W4BlockArgs& block) 
     const F6Workspace w(a.m, a.padded_k, a.n);
     void* ws = nullptr;
     WorkspaceLease lease;                                    // until the last kernel of this call is queued
-    const bool folded = block.norm_w || a.glu;
-    if (int rc = workspace_get(s, folded ? f6_up(w.total) + (size_t)a.m * a.k * 4 : w.total, &ws, lease)) return rc;
-    float* const marked = folded ? reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + f6_up(w.total)) : nullptr;
+    if (int rc = workspace_get(s, w.total, &ws, lease)) return rc;
     uint8_t* p = static_cast<uint8_t*>(ws);
     uint8_t* const planes = p; p += w.planes;
     uint8_t* const exps = p; p += w.exps;
     float* const sums = reinterpret_cast<float*>(p); p += w.sums;
     float* const rfac = reinterpret_cast<float*>(p); p += w.rfac;
+    float* const rinv = reinterpret_cast<float*>(p); p += w.rinv;
     float* const least = reinterpret_cast<float*>(p); p += w.least;
     uint32_t* const zflags = reinterpret_cast<uint32_t*>(p);
     // rows per workgroup of the preparation: at most 512 units and 80 KB of LDS (two workgroups per compute unit), and enough workgroups
@@ -1023,14 +1053,14 @@ int w4_launch_gemm_f6(const W4Args& a, hipStream_t s, const W4BlockArgs& block) 
 #define RUMUS_F6_PREPARE(IN)                                                                                             \
     hipLaunchKernelGGL(w4_f6_prepare_kernel<IN>, pgrid, dim3(512), (size_t)rows * pitch * 4, s, a.x, a.perm, planes, exps, sums, \
                        rfac, a.m, a.k, w.steps, rows, pitch, reinterpret_cast<const float4*>(a.zp),                        \
-                       (uint32_t)((uint64_t)a.num_groups * a.n / 4), zflags, a.scales, a.num_groups, a.n, least, rows_pad / rows, block.norm_w, block.eps, marked)
+                       (uint32_t)((uint64_t)a.num_groups * a.n / 4), zflags, a.scales, a.num_groups, a.n, least, rows_pad / rows, block.norm_w, block.eps, rinv)
     if (a.perm) RUMUS_F6_PREPARE(kF6Perm);
     else if (block.norm_w) RUMUS_F6_PREPARE(kF6Norm);
     else if (a.glu) RUMUS_F6_PREPARE(kF6Glu);
     else RUMUS_F6_PREPARE(kF6Plain);
 #undef RUMUS_F6_PREPARE
     if (int rc = check_launch("w4_f6_prepare_kernel")) return rc;
-    const F6Args f{a.packed, a.scales, a.zp, a.zp4, a.bias, planes, reinterpret_cast<const uint16_t*>(exps), sums, folded ? marked : a.x, a.perm,
+    const F6Args f{a.packed, a.scales, a.zp, a.zp4, a.bias, planes, reinterpret_cast<const uint16_t*>(exps), sums, a.x, a.perm, block.norm_w, a.glu, rinv,
                    rfac, least, zflags, a.y, a.m, a.k, a.n, w.steps, a.group_size / 64, a.num_groups, block.residual};
     double us;
     switch (f6_pick(a.m, a.k, a.n, &us)) {

@@ -76,3 +76,31 @@ def test_prompt_block_equals_the_separate_operators(monkeypatch, heads, f, b, n,
     for one, other in zip(got, block(x)):
         # two norms, each off by a few roundings of 2^-24, ahead of f32 sums
         assert one.shape == other.shape and (one - other).norm() <= 64 * 2.0 ** -24 * other.norm()
+
+
+def test_captured_within_the_documented_workspace():
+    m, k, n, g = 1500, 4096, 4096, 128
+    say("qmatmul_int4_block captured in a graph, workspace of qmatmul_int4 reserved")
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    packed, scales, zp = ops.w4_quantize_pack(rand(k, n) * 0.02, g)
+    w, x, res = 1.0 + 0.1 * rand(k), rand(m, 2 * k), rand(m, n)
+    x[3:7, 33] *= 5000.0
+    x1 = x[:, :k].contiguous()
+    calls = (lambda out: ops.qmatmul_int4_block(x, packed, scales, zp, k, g, swiglu=True, residual=res, out=out),
+             lambda out: ops.qmatmul_int4_block(x1, packed, scales, zp, k, g, norm_weight=w, out=out))
+    want = [call(None) for call in calls]
+    side = torch.cuda.Stream()
+    _lib.call("rumus_hip_workspace_reserve", side.cuda_stream, 5 * (m + 64) * (k + 128) + 1280)
+    got = [torch.empty_like(t) for t in want]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        for call, out in zip(calls, got):
+            call(out)
+    for _ in range(3):
+        for out in got:
+            out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
