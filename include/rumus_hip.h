@@ -251,8 +251,8 @@ int rumus_hip_f16_to_f32(const uint16_t* in, float* out, uint64_t numel,
  * (rumus_hip_qmatmul_int4_decode_zp4) does not make that exception and keeps
  * the plain bound.  Batches of more than 256 rows that the six-bit-float
  * kernel takes (group_size % 64 == 0, k from 1024, padded_k to 16384, where it is the faster one)
- * keep 24 bits below the largest of 32 consecutive k, and 39 where an
- * eighth of those lies 2^8 or more below it.  The others, which the f16 tile
+ * keep 29 bits below the largest of 32 consecutive k, and 39 where a
+ * quarter of those lies 2^8 or more below it, or twelve of them 2^9.  The others, which the f16 tile
  * kernel takes, keep 22 bits of every element and add in f32.  Both are
  * faster on tables of integer zero-points (what AWQ and GPTQ checkpoints hold;
  * they look first): part of the work exists only for their fractional part. */

@@ -5,25 +5,28 @@
 // with z the zero-point's nearest integer (within 0..15) and rest = zp - z.  v_mfma_scale_f32_32x32x64_f8f6f4 runs
 // operands of six bits (e2m3: sign, 0 .. 7.5, integers up to 16 in units of 1/8 .. 1/2) at four times the f16 rate:
 //   - q - z is -15 .. 15: exact as (q - z) / 8;
-//   - x becomes five six-bit digits.  Per row and 32 consecutive k, x 2^-e (largest magnitude below 7.5) is rounded to
+//   - x becomes six six-bit digits.  Per row and 32 consecutive k, x 2^-e (largest magnitude below 7.5) is rounded to
 //     the nearest e2m3, the exact remainder, at most 1/4, is rounded again in units of 2^-4, the remainder of that, at
-//     most 2^-7, in units of 2^-9, then 2^-14 and 2^-19: what is left is below 2^-22, i.e. 24 bits below the largest of
+//     most 2^-7, in units of 2^-9, then 2^-14, 2^-19 and 2^-24: what is left is below 2^-27, i.e. 29 bits below the largest of
 //     the 32 values.  The exponent e is the MFMA's own block scale (one E8M0 byte per row and 32 k), and the
-//     digits' constant offsets ride on the block scale of the weight operand, so all five products add up in one f32
+//     digits' constant offsets ride on the block scale of the weight operand, so all six products add up in one f32
 //     accumulator.
-// Five products at four times the rate take 5/8 of the two f16 products of the hi/lo split (w4_gemm_tile.hip), and what a
-// launch can issue is limited by the board's power: from registers, on digits of N(0,1) activations against quantized
-// normal weights, 1275 useful TFLOP/s (at 1.63 GHz) against 961 (at 1.94 GHz).
-// What bounds the whole call: power.  2048 x 4096 -> 11008 takes 265 us with integer zero-points, 284 with fractional ones (f16
-// tiles: 344 and 365), of which the preparation is 14 and the tables of fractional zero-points 12; a step of 64 k takes 3938 clocks at
-// 1.71 GHz where its 80 MFMAs per wave pair alone take 2680.  The conversion of the weights draws about 12 % of the loop's
-// energy, the loads into LDS 7 %, the change of scale from group to group 5 %.  Other sizes, before -> after (fractional
-// zero-points): 4096 x 4096 -> 22016 1430 -> 1002 us, 4096 x 11008 -> 4096 751 -> 553, 4096 x 4096 -> 4096 285 -> 198;
-// groups of 64: 2048 x 4096 -> 11008 426 -> 328.
+// Why six: the f16 tiles (w4_gemm_tile.hip) keep 22 bits of every element, and so does this down to 2^-7 of the largest of the
+// 32.  Five digits, 24 bits below the largest, are about 6 % faster and were further off than those: the split's own error against
+// float64, as a share of the result, with some channels 20 times as large 5.5e-8 (f16 tiles 4.3e-8, six digits 1.0e-9), with
+// SwiGLU outputs 5.4e-8 (4.4e-8, 0.9e-9), with every eighth channel 2^4 as large and met by weights of zero 3.4e-7 (4.4e-8, 0.7e-8).
+// Whole calls, 2048 x 4096 -> 11008 on such inputs, sums included: 3.4e-7 (f16 tiles 4.7e-7 to 5.8e-7).
+// Six products at four times the rate are 3/4 of the matrix work of the two f16 products of the hi/lo split.  One box in turn, f16
+// tiles -> this (us): 2048 x 4096 -> 11008 344 -> 298 with integer zero-points, 370 -> 325 with fractional ones, groups of 64
+// 383 -> 332; 4096 x 4096 -> 22016 1312 -> 1086, 4096 x 11008 -> 4096 707 -> 610, 4096 x 4096 -> 4096 267 -> 219.
 //
-// Elements that tower over some of their 32 neighbours would cost those their low bits: where an octet of the 32 lies 2^8
-// or more below the largest, the run of 32 is marked, and a second pass over such steps, after the main loop, multiplies
-// three more digits (2^-24, 2^-29, 2^-34: 39 bits below the largest).
+// Elements that tower over some of their 32 neighbours would still cost those their low bits: where an octet of the 32 lies 2^8
+// or more below the largest, or kF6Small of the 32 (not counting zeros) 2^9 or more, the run is marked, and a second pass over such
+// steps, after the main loop, multiplies two more digits (2^-29, 2^-34: 39 bits below the largest).  N(0,1) marks no run in
+// 10^7, SwiGLU outputs of gates N(0,4) fewer than one in 10^4, of gates N(0,16) one in 200; a call in which every step has marks takes
+// 2.4 times as long.  The split's error with every second, eighth or 32nd channel 2^p as large and met by weights of zero, p = 2 to 16: at
+// most 1.6e-7 of the result.  The whole call's is larger there, up to 1.5e-6, where the small elements come to about half a unit of a digit
+// (p = 6, 10 and 16); most likely the instruction aligns its sum to the operands' exponents, those of products with zero among them.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -50,14 +53,15 @@ typedef void __attribute__((address_space(3)))* lptr_t;
 
 constexpr int kF6BM = 128;                      // rows per workgroup
 constexpr int kF6Tiles = kF6BM / 32;            // row tiles of 32 per workgroup
-constexpr int kF6Digits = 5;
+constexpr int kF6Digits = 6;
 constexpr int kF6Tile = kF6Digits * 1536;       // bytes of one row tile and one step of 64 k: 64 lanes x 24 bytes per digit
-constexpr int kF6Step = kF6Tiles * kF6Tile;     // 30 KB
+constexpr int kF6Step = kF6Tiles * kF6Tile;     // 36 KB
 constexpr int kF6Lo = kF6Digits * 1024;         // inside a tile: the lanes' first 16 bytes of every digit, then their last 8
 constexpr int kF6BTile = 1024 + 512 + 32;       // the same for 32 columns of weights; 32 bytes of skew against bank conflicts
 constexpr uint32_t kF6MaxK = 16384;             // padded to whole groups: a thread of the preparation per 32 k of a row, a row in LDS
 constexpr uint32_t kF6Flags = 256;              // parts of the zero-point table, one flag word each
-constexpr int kF6Deep = 3;                      // further digits where a run of 32 k spans many binades
+constexpr int kF6Deep = 2;                      // further digits where a run of 32 k spans many binades
+constexpr uint32_t kF6Small = 12;               // elements 2^9 or more below the largest of a run that mark it
 constexpr uint32_t kF6DeepBit = 0x80;           // of an exponent byte: the run needs them (the exponents themselves stay below 128)
 // digit d counts in units of 2^-shift
 constexpr int kF6Shift[kF6Digits + kF6Deep] = {0, 4, 9, 14, 19, 24, 29, 34};
@@ -113,9 +117,9 @@ __device__ __forceinline__ v6u f6_digit(v16f& ev, v16f& od, float unit) {
 
 // ---- activations -> digits ---------------------------------------------------------------------------
 // A workgroup takes `rows` rows (a power of two up to 8): copies them into LDS with contiguous reads, finding each row's
-// largest magnitude on the way, and then every thread turns one unit, 32 consecutive k of one row, into five digits
+// largest magnitude on the way, and then every thread turns one unit, 32 consecutive k of one row, into six digits
 // (rows * units <= 512 threads).  The gather of act-order weights happens on the way out of LDS: from global memory a wave
-// instruction would touch 64 cache lines for 256 bytes.  Memory bound: 2048 x 4096 reads 33.5 and writes 32 MB in 14 us.
+// instruction would touch 64 cache lines for 256 bytes.  Memory bound: 2048 x 4096 reads 33.5 and writes 38 MB.
 // LDS: row r at r * pitch floats, 4 floats of padding after every 32, so that the 16-byte reads of threads 32 floats
 // apart fall on different banks (likewise rows: pitch / 4 is odd).
 // Beyond the row groups, more workgroups look at the columns' scales, 64 columns each, and kF6Flags at f32 zero-points.
@@ -311,7 +315,10 @@ __global__ __launch_bounds__(512) void w4_f6_prepare_kernel(const float* __restr
         top = fmaxf(top, o4[o]);
         low = o4[o] > 0.0f ? fminf(low, o4[o]) : low;            // (octets of zeros have nothing to lose)
     }
-    const bool is_deep = low < top * 0.00390625f;
+    uint32_t small = 0;
+#pragma unroll
+    for (int j = 0; j < 32; j++) small += v[j] != 0.0f && fabsf(v[j]) < top * 0x1p-9f ? 1u : 0u;
+    const bool is_deep = low < top * 0x1p-8f || small >= kF6Small;
     if (!mine) return;                                           // whole waves or the tail of one: no barrier follows
     float sum = 0.0f;
 #pragma unroll
@@ -411,8 +418,8 @@ __device__ __forceinline__ void lds_write24(uint32_t hi_at, uint32_t lo_at, cons
 
 // Eight waves as 2 (rows) x 4 (columns); a wave owns 64 rows (two row tiles) and 32 TN columns, lane l's columns being
 // TN adjacent ones per tile set.  The accumulators (32 TN registers) set the tile: with 128 TN columns by 128 rows every
-// converted weight serves two row tiles and every activation digit TN column tiles, two steps of both fill the LDS
-// (156 KB at TN = 4), and one workgroup runs per compute unit; w4_launch_gemm_f6 picks TN.
+// converted weight serves two row tiles and every activation digit TN column tiles, two steps of both take 129 KB
+// of LDS at TN = 4, and one workgroup runs per compute unit; w4_launch_gemm_f6 picks TN.
 template <int TN, int FOLD, bool ZP4>
 __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
     constexpr int BN = 128 * TN, CPT = TN == 2 ? 1 : 2;          // columns per workgroup; columns each thread converts per step
@@ -500,15 +507,15 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
         lds_write24<OFF>(c_hi[c], c_lo[c], code);
     };
 
-    // ---- activations: a step is 30 KB, straight into LDS; wave w takes KB w, w + 8, w + 16, w + 24 (the last two waves
-    // repeat one: same bytes to the same place, so that every wave counts the same loads) ------------------
+    // ---- activations: a step is 36 KB, straight into LDS; wave w takes KB w, w + 8, w + 16, w + 24, w + 32 (the last four waves
+    // repeat the last: same bytes to the same place, so that every wave counts the same loads) ------------------
     const uint8_t* const a_blk = a.planes + (uint64_t)blk * a.steps * kF6Step;
     const uint32_t a_lds = lds_offset(lds), a_lane = lane * 16;
     auto digits_load = [&](uint32_t s, uint32_t buf) __attribute__((always_inline)) {
         const uint8_t* src = a_blk + (uint64_t)min(s, a.steps - 1) * kF6Step;
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint32_t c = min(wave + 8 * q, 29u) * 1024;
+        for (uint32_t q = 0; q < (kF6Step / 1024 + 7) / 8; q++) {
+            const uint32_t c = min(wave + 8 * q, kF6Step / 1024 - 1u) * 1024;
             lds_load16(a_lds + buf * kF6Step + c, src + c, a_lane);
         }
     };
@@ -561,7 +568,7 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
         unit_slot[j] = a.least[min(my_col_c + j, a.n - 1)];
     }
 
-    constexpr int kB0 = 130 | (126 << 8) | (121 << 16) | (116 << 24), kB1 = 111;   // 2^3 / 2^shift of every digit
+    constexpr int kB0 = 130 | (126 << 8) | (121 << 16) | (116 << 24), kB1 = 111 | (106 << 8);   // 2^3 / 2^shift of every digit
 
     auto read6 = [&](const uint8_t* hi, const uint8_t* lo) __attribute__((always_inline)) {
         const uint4 h = *reinterpret_cast<const uint4*>(hi + lane * 16);
@@ -569,14 +576,14 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
         return v6u{h.x, h.y, h.z, h.w, l.x, l.y};
     };
 
-    // Step s from buffer P, in ten sections of TN MFMAs (row tile i, digit d): a section's A fragment is read one section
+    // Step s from buffer P, in twelve sections of TN MFMAs (row tile i, digit d): a section's A fragment is read one section
     // ahead, and the vector work of a step is dealt out over its sections so that every MFMA has its share: the change of
     // the accumulators from one group's scale to the next (a row tile undergoes it while the other one multiplies, in the
     // second half of an odd step and the first half of an even one), and in the other halves the next step's weights.
     auto step = [&](uint32_t s, auto p_tag) __attribute__((always_inline)) {
         constexpr int P = decltype(p_tag)::value;
         constexpr bool ENDS = P == 1 || FOLD == 1, STARTS = P == 0 || FOLD == 1;   // a group may end / start with this step
-        constexpr int C0 = P == 0 ? 5 : 0;                       // first section of the conversion
+        constexpr int D = kF6Digits, C0 = P == 0 ? D : 0;                       // first section of the conversion
         constexpr int SET = P ^ 1;                               // of step s + 1
         typedef std::integral_constant<int, P ^ 1> other;
         const uint8_t* const pa = lds + P * kF6Step + wm * 2 * kF6Tile;
@@ -586,10 +593,10 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
 #pragma unroll
         for (int j = 0; j < TN; j++) bf[j] = read6(pb + j * kF6BTile, pb + j * kF6BTile + 1024);
 #pragma unroll
-        for (int t = 0; t < 10; t++) {
-            const int i = t / 5, d = t % 5;
-            if (t + 1 < 10) {
-                const int i2 = (t + 1) / 5, d2 = (t + 1) % 5;
+        for (int t = 0; t < 2 * D; t++) {
+            const int i = t / D, d = t % D;
+            if (t + 1 < 2 * D) {
+                const int i2 = (t + 1) / D, d2 = (t + 1) % D;
                 af[(t + 1) & 1] = read6(pa + i2 * kF6Tile + d2 * 1024, pa + i2 * kF6Tile + kF6Lo + d2 * 512);
             }
             if (t == 0) digits_load(s + 1, P ^ 1);
@@ -611,8 +618,8 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
                 sc_cur = scales_of(min(s, a.steps - 1) / a.steps_per_group);
                 sc_next = scales_of(min(s + 1, a.steps - 1) / a.steps_per_group);
             }
-            if (ENDS && t == 4) least = units_read();
-            if (ENDS && t == 5) {
+            if (ENDS && t == D - 1) least = units_read();
+            if (ENDS && t == D) {
 #pragma unroll
                 for (int j = 0; j < TN; j++) {
                     const float sc = unit_of(sc_cur.v[j], least.v[j]), sn = unit_of(sc_next.v[j], least.v[j]);
@@ -621,9 +628,9 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
                     ratio.v[j] = fmaf(fmaf(-q, sn, sc), rc, q);   // one correction step: within an ulp of the quotient, and 1 for the same group
                 }
             }
-            if (ENDS && t >= 6 && t < 6 + TN) {
+            if (ENDS && t > D && t <= D + TN) {
 #pragma unroll
-                for (int r = 0; r < 16; r++) acc[0][t - 6][r] *= ratio.v[t - 6];
+                for (int r = 0; r < 16; r++) acc[0][t - D - 1][r] *= ratio.v[t - D - 1];
             }
 #pragma unroll
             for (int j = 0; j < TN; j++) {
@@ -634,9 +641,10 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
                 if (d == 2) acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa, fb, acc[i][j], 2, 2, P, (int)exps[i], 2, kB0);
                 if (d == 3) acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa, fb, acc[i][j], 2, 2, P, (int)exps[i], 3, kB0);
                 if (d == 4) acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa, fb, acc[i][j], 2, 2, P, (int)exps[i], 0, kB1);
+                if (d == 5) acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa, fb, acc[i][j], 2, 2, P, (int)exps[i], 1, kB1);
             }
             // the reads of the next section, then MFMAs with a share of the vector work behind each
-            if (t + 1 < 10) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            if (t + 1 < 2 * D) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
 #pragma unroll
             for (int j = 0; j < TN; j++) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -797,7 +805,6 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
                     for (int r = 0; r < 16; r++) t[r] = 0.0f;
                     t = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(da[0], fb, t, 2, 2, 0, ea, 0, 130 - kF6Shift[kF6Digits]);
                     t = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(da[1], fb, t, 2, 2, 0, ea, 0, 130 - kF6Shift[kF6Digits + 1]);
-                    t = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(da[2], fb, t, 2, 2, 0, ea, 0, 130 - kF6Shift[kF6Digits + 2]);
                     const float ratio_s = sc.v[j] / sc_cur.v[j];
 #pragma unroll
                     for (int r = 0; r < 16; r++) acc[i][j][r] = fmaf(t[r], ratio_s, acc[i][j][r]);
@@ -941,19 +948,19 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
 }
 
 // Columns per workgroup / 128, and the time of a call in microseconds: workgroups run one per compute unit, in rounds of
-// 256.  A round's steps (of 64 k) take L at least, and from about 170 workgroups on power limits them: a launch as a whole
-// cannot beat P per 256 workgroup-steps.  16 is a round's start and end, the rest the preparation.  Fitted to 252 timings
-// (130 .. 4096 rows; seven weights, 1024 -> 5504 to 8192 -> 8192 and 4096 -> 22016; 2, 3 and 4 forced): within 3 % rms, and the width chosen by
-// it costs 0.01 % against the best of the three, 1 % at worst.
+// 256.  A round's steps (of 64 k) take L at least, and with more than about 170 workgroups at work each is slower: a launch as a whole
+// does not beat P per 256 workgroup-steps.  16 is a round's start and end, the rest the preparation.  The form was fitted to 252 timings
+// with five digits, each width forced (130 .. 4096 rows; seven weights), L, P and the preparation then to 50 calls with six (512 to 4096
+// rows, 1024 -> 2816 to 8192 -> 8192 and 4096 -> 22016): within 5 %, up to 10 % too low at k = 11008.
 static int f6_pick(uint32_t m, uint32_t k, uint32_t n, double* us) {
-    static const double L[3] = {1.22, 1.55, 1.82}, P[3] = {1.29, 1.95, 2.50};
+    static const double L[3] = {1.24, 1.59, 1.87}, P[3] = {1.31, 2.00, 2.58};
     const double steps = ceil_div(k, 64);
     int best = 4;
     *us = 1e30;
     for (int tn = 4; tn >= 2; tn--) {
         const double wgs = (double)ceil_div(m, kF6BM) * ceil_div(n, 128 * tn), rounds = std::ceil(wgs / 256.0);
         const double chain = rounds * (steps * L[tn - 2] + 16.0), power = wgs / 256.0 * steps * P[tn - 2];
-        const double t = std::sqrt(std::sqrt(chain * chain * chain * chain + power * power * power * power)) + 3.0 + 1.6e-6 * m * k;
+        const double t = std::sqrt(std::sqrt(chain * chain * chain * chain + power * power * power * power)) + 3.0 + 2.0e-6 * m * k;
         if (t < *us) { *us = t; best = tn; }
     }
     return best;
@@ -965,9 +972,7 @@ struct F6Workspace {
     uint32_t blocks, steps;
     size_t planes, exps, sums, rfac, rinv, least, flags, total;   // bytes
     F6Workspace(uint32_t m, uint32_t padded_k, uint32_t n) : blocks(ceil_div(m, kF6BM)), steps(padded_k / 64) {
-        // (never less than the f16 tiles park, 4 bytes per element: what a caller reserved or a fixed buffer holds, and what it
-        // refuses, does not depend on the kernel)
-        planes = std::max((size_t)blocks * steps * kF6Step, (size_t)ceil_div(m, 32) * 32 * padded_k * 4);
+        planes = (size_t)blocks * steps * kF6Step;
         exps = f6_up((size_t)blocks * ((steps + 1) / 2) * kF6Tiles * 64 * 2);
         sums = (size_t)blocks * steps * kF6BM * 4;
         rfac = (size_t)blocks * kF6BM * 4;
@@ -978,12 +983,22 @@ struct F6Workspace {
     }
 };
 
+// Six digits park 4.6 bytes per element of x, the f16 tiles 4.25.  What those run within the fixed scratch array (w4_gemv.hip),
+// and what a caller reserved by the documented bound, has to do for this kernel too: such a call runs as two halves of its rows.
+constexpr uint64_t kF6Array = uint64_t(32) << 20;
+static bool f6_array_fits(uint32_t m, uint32_t padded_k) { return (uint64_t)m * padded_k * 17 / 4 <= kF6Array; }
+static uint32_t f6_rows_at_once(uint32_t m, uint32_t padded_k, uint32_t n) {
+    const F6Workspace w(m, padded_k, n);
+    uint64_t limit = (uint64_t)5 * (m + 64) * (padded_k + 128);
+    if (f6_array_fits(m, padded_k)) limit = std::min(limit, kF6Array);
+    return w.total <= limit ? m : ceil_div(w.blocks, 2) * kF6BM;
+}
+
 // More than 256 rows (blocks of 128 rows: up to there the integer kernel's blocks of 64 fit as well or better, and K would have to be
 // shared over workgroups), where its time is below what the other two kernels are expected to take.  The two estimates of
 // those are loosest upwards for the integer kernel (8192 -> 8192 at 640 rows: 201 us expected, 164 measured, 185 here), hence its
-// margin.  Over the 60 cases above 256 rows the choice is 0.05 % off the better one and takes 17.5 % less time than
-// before on average: 2048 rows 4096 -> 11008 374 -> 287 us, 4096 -> 4096 146 -> 120, 4096 rows 4096 -> 22016 1448 -> 1022,
-// 1024 rows 1024 -> 5504 41.9 -> 41.9.
+// margin.  Over 45 calls above 512 rows the choice takes 10 % less time than the older kernels alone, 24 % at best (1000 rows
+// 4096 -> 11008 199 -> 152 us), and 6 % more at worst (1400 rows 11008 -> 4096 283 -> 293).
 bool w4_gemm_f6_chosen(const W4Args& a) {
     const uintptr_t bits = reinterpret_cast<uintptr_t>(a.packed) | reinterpret_cast<uintptr_t>(a.scales) |
                            reinterpret_cast<uintptr_t>(a.zp) | reinterpret_cast<uintptr_t>(a.y) |
@@ -991,13 +1006,14 @@ bool w4_gemm_f6_chosen(const W4Args& a) {
     if (!(a.m > 256 && a.m <= 65535u * kF6BM && a.n % 4 == 0 && (bits & 15) == 0 && !a.g_idx && !a.tiled &&
           a.group_size % 64 == 0 && (!a.zp4 || a.n % 8 == 0) && a.k >= 1024 &&                    // (what the estimates were fitted to)
           a.padded_k <= kF6MaxK &&
+          (a.x != a.y || !a.x) &&                              // (marked runs read x again while other workgroups store)
           (uint64_t)a.padded_k / 8 * a.n * 4 < (1ull << 32) && (uint64_t)a.m * a.n < (1ull << 32)))
         return false;
     double us = 0.0, other = 0.0;
     f6_pick(a.m, a.k, a.n, &us);
     const bool i8 = w4_gemm_i8_supported(a, &other);
-    // what the integer kernel runs within the fixed scratch array (w4_gemv.hip) has to go on running there
-    if (i8 && F6Workspace(a.m, a.padded_k, a.n).total > (size_t(32) << 20)) return false;
+    // what the integer kernel runs within the fixed scratch array (w4_gemv.hip), 3.1 bytes per element of x, has to go on running there
+    if (i8 && !f6_array_fits(a.m, a.padded_k)) return false;
     return us < (i8 ? 0.92 : 1.0) * other;
 }
 
@@ -1023,8 +1039,7 @@ static int launch_f6_groups(const F6Args& f, const W4Args& a, uint32_t blocks, h
     return a.zp4 ? launch_f6<TN, 1, true>(f, blocks, s) : launch_f6<TN, 1, false>(f, blocks, s);
 }
 
-int w4_launch_gemm_f6(const W4Args& a, hipStream_t s, const W4BlockArgs& block) {
-    RUMUS_REQUIRE(a.padded_k <= kF6MaxK, "qmatmul_int4: padded_k %u is beyond the six-bit kernel's %u", a.padded_k, kF6MaxK);
+static int launch_f6_rows(const W4Args& a, hipStream_t s, const W4BlockArgs& block) {
     const F6Workspace w(a.m, a.padded_k, a.n);
     void* ws = nullptr;
     WorkspaceLease lease;                                    // until the last kernel of this call is queued
@@ -1068,6 +1083,21 @@ int w4_launch_gemm_f6(const W4Args& a, hipStream_t s, const W4BlockArgs& block) 
         case 3: return launch_f6_groups<3>(f, a, w.blocks, s);
         default: return launch_f6_groups<4>(f, a, w.blocks, s);
     }
+}
+
+int w4_launch_gemm_f6(const W4Args& a, hipStream_t s, const W4BlockArgs& block) {
+    RUMUS_REQUIRE(a.padded_k <= kF6MaxK, "qmatmul_int4: padded_k %u is beyond the six-bit kernel's %u", a.padded_k, kF6MaxK);
+    const uint32_t rows = f6_rows_at_once(a.m, a.padded_k, a.n);
+    for (uint32_t r0 = 0; r0 < a.m; r0 += rows) {
+        W4Args part = a;
+        W4BlockArgs around = block;
+        part.m = min(rows, a.m - r0);
+        part.x = a.x + (uint64_t)r0 * a.k * (a.glu ? 2 : 1);
+        part.y = a.y + (uint64_t)r0 * a.n;
+        if (block.residual) around.residual = block.residual + (uint64_t)r0 * a.n;
+        if (int rc = launch_f6_rows(part, s, around)) return rc;
+    }
+    return RUMUS_HIP_OK;
 }
 
 }  // namespace rumus

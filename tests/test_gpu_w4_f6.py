@@ -25,6 +25,8 @@ def ops():
     (3516, 1028, 4100, 128, False, "fractional"), (3500, 1088, 4096, 64, True, "u4"), (3584, 1024, 4096, 256, False, "integer")])
 def test_six_bit_kernel_at_its_edges(ops, m, k, n, g, act_order, zeros):
     say(f"w4 forward, six-bit kernel m={m} k={k} n={n} g={g} act_order={act_order} zero-points {zeros}")
+    if zeros != "u4":                          # (asked for whole words of eight k)
+        assert ops.qmatmul_int4_block_takes(m, k // 8 * 8, n, g)
     rng = np.random.default_rng(m + k + n)
     padded = -(-k // g) * g
     w = rng.normal(0, 0.02, (k, n)).astype(np.float32)
@@ -64,8 +66,8 @@ def test_six_bit_kernel_at_its_edges(ops, m, k, n, g, act_order, zeros):
     s = scales[groups].astype(np.float64)
     exact = xs @ ((q - z - rest) * s)
     terms = np.abs(xs) @ ((np.abs(q - z) + np.abs(rest)) * np.abs(s))
-    # sums: five additions and one change of scale per step of 64, two additions per group for the zero-points' rest, each within
-    # 2^-23 of what has been added up; values within 2^-24 of the largest of 32 (2^-39 where one of them towers), under
+    # sums: six additions and one change of scale per step of 64, 7 2^-24 of what has been added up, two additions per group for the
+    # zero-points' rest, each within 2^-23 of that; values within 2^-29 of the largest of 32 (2^-39 where one of them towers), under
     # 4 2^-23 of ordinary terms, and their bf16 thirds in the rest's products another 2^-23
     steps = padded // 64
     bound = (6 * steps + 2 * scales.shape[0] + 8) * 2.0 ** -23
@@ -148,3 +150,30 @@ def test_scales_far_apart(ops, k, g, zeros):
     whole = torch.arange(n, device="cuda") != n - 7
     assert torch.equal(torch.isfinite(got), whole.expand(m, n))
     assert ((got[rows].double() - exact).abs() <= bound)[:, whole].all()
+
+
+# Every st-th channel 2^p as large and met by weights of zero: the result is made of the small elements alone, whose bits must
+# not suffer from their neighbours' size.  Error of the result as a whole.
+@pytest.mark.parametrize("st", [2, 8, 32])
+def test_small_elements_beside_large_channels(ops, st):
+    m, k, n, g = 1500, 4096, 4096, 128
+    assert ops.qmatmul_int4_block_takes(m, k, n, g)
+    gen = torch.Generator(device="cuda").manual_seed(st)
+    packed, scales, zp = ops.w4_quantize_pack(torch.randn(k, n, device="cuda", generator=gen) * 0.02, g)
+    zp = zp.round().clamp(0, 15)
+    expand = lambda t: t.double().repeat_interleave(g, 0)
+    q = torch.stack([(packed >> (4 * i)) & 15 for i in range(8)], 1).reshape(k, n)
+    q[::st] = expand(zp)[::st].to(torch.int32)
+    shifts = (4 * torch.arange(8, device="cuda")).reshape(1, 8, 1)
+    words = (q.reshape(k // 8, 8, n).long() << shifts).sum(1)
+    packed = torch.where(words >= 2 ** 31, words - 2 ** 32, words).to(torch.int32)
+    w = (q.double() - expand(zp)) * expand(scales)
+    for p in (0, 3, 5, 6, 7, 8, 9, 10, 12, 16):
+        say(f"w4 forward, six-bit kernel: every {st}. channel 2^{p} as large, weights of zero")
+        x = torch.randn(m, k, device="cuda", generator=gen)
+        x[:, ::st] *= 2.0 ** p
+        exact = x.double() @ w
+        err = ((ops.qmatmul_int4(x, packed, scales, zp, k, g).double() - exact).norm() / exact.norm()).item()
+        say(f"    {err:.2e} of the result")
+        # 22 bits of every element, and six additions per step of 64, each within 2^-23 of the result, independent of each other
+        assert err <= 2.0 ** -22 + (6 * k / 64) ** 0.5 * 2.0 ** -23
