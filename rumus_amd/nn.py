@@ -359,7 +359,10 @@ class DecoderBlockW4:
 
     @staticmethod
     def _folds_rows(lin, x, *beside) -> bool:
-        """Whether this projection of ``x`` takes ``qmatmul_int4_block``, operands included."""
+        """Whether this projection of ``x`` takes ``qmatmul_int4_block``, operands included.  One of another type than
+        ``QLinear`` (a subclass, a wrapper, any callable) is called as it is."""
+        if type(lin) is not QLinear:
+            return False
         w = lin.weight
         arrays = (x, w.packed_tensor, w.scales_tensor, w.zp_tensor) + beside + ((lin.bias,) if lin.bias is not None else ())
         return w.perm is None and ops.qmatmul_int4_block_takes(x.shape[0], w.k, w.n, w.group_size) and \
