@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes as C
 import os
 import subprocess
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "librumus_hip.so")
@@ -111,20 +112,32 @@ def lib() -> C.CDLL:
     return _lib
 
 
+class _GeneralPath:
+    """In the place of the native host calls where they cannot be loaded: every call takes the general path in ``ops``
+    (the same kernels of librumus_hip.so, some microseconds later)."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 _host = None
 
 
 def host():
     """The native side of the most frequent calls (csrc/host_calls.cpp): checks, result tensor, stream and the call in one
-    C++ function each, ``None`` where the general path in ``ops`` is to be taken."""
+    C++ function each, ``None`` where the general path in ``ops`` is to be taken.  Built against one version of torch; the
+    library itself does not need it."""
     global _host
     if _host is None:
         lib()
-        if not os.path.exists(HOST_PATH):
-            raise ImportError(f"{HOST_PATH} is missing: `make -C rumus_amd/csrc` builds it; there is no fallback path")
         import torch  # noqa: F401  (its libraries have to be loaded first)
-        from . import _host_calls
-        _host = _host_calls
+        try:
+            from . import _host_calls
+            _host = _host_calls
+        except ImportError as e:
+            warnings.warn(f"rumus_amd: calls go through Python, the native host side did not load ({e}); "
+                          "`make -C rumus_amd/csrc` builds it", RuntimeWarning, stacklevel=3)
+            _host = _GeneralPath()
     return _host
 
 
