@@ -1,4 +1,5 @@
 """The native host calls are an addition: without them every call takes the general path."""
+import subprocess
 import sys
 
 import pytest
@@ -18,3 +19,8 @@ def test_without_the_native_host_calls(monkeypatch):
 
 def test_they_load_here():
     assert _lib.host().__name__ == "rumus_amd._host_calls"
+
+
+def test_the_library_alone_builds_without_torch():
+    plan = subprocess.run(["make", "-n", "-B", "-C", _lib.CSRC, "lib", "PYTHON=/nonexistent"], capture_output=True, text=True, check=True)
+    assert "librumus_hip.so" in plan.stdout and "host_calls" not in plan.stdout and not plan.stderr
