@@ -12,7 +12,7 @@
 //     digits' constant offsets ride on the block scale of the weight operand, so all six products add up in one f32
 //     accumulator.
 // Why six: the f16 tiles (w4_gemm_tile.hip) keep 22 bits of every element, and so does this down to 2^-7 of the largest of the
-// 32.  Five digits, 24 bits below the largest, are about 6 % faster and were further off than those: the split's own error against
+// 32.  Five digits, 24 bits below the largest, took 12 % less time and were further off than those: the split's own error against
 // float64, as a share of the result, with some channels 20 times as large 5.5e-8 (f16 tiles 4.3e-8, six digits 1.0e-9), with
 // SwiGLU outputs 5.4e-8 (4.4e-8, 0.9e-9), with every eighth channel 2^4 as large and met by weights of zero 3.4e-7 (4.4e-8, 0.7e-8).
 // Whole calls, 2048 x 4096 -> 11008 on such inputs, sums included: 3.4e-7 (f16 tiles 4.7e-7 to 5.8e-7).
