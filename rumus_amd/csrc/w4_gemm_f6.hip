@@ -4,7 +4,7 @@
 //
 // with z the zero-point's nearest integer (within 0..15) and rest = zp - z.  v_mfma_scale_f32_32x32x64_f8f6f4 runs
 // operands of six bits (e2m3: sign, 0 .. 7.5, integers up to 16 in units of 1/8 .. 1/2) at four times the f16 rate:
-//   - q - z is -15 .. 15: exact as (q - z) / 8;
+//   - q - z is -15 .. 15: exact as (q - z) / 2;
 //   - x becomes six six-bit digits.  Per row and 32 consecutive k, x 2^-e (largest magnitude below 7.5) is rounded to
 //     the nearest e2m3, the exact remainder, at most 1/4, is rounded again in units of 2^-4, the remainder of that, at
 //     most 2^-7, in units of 2^-9, then 2^-14, 2^-19 and 2^-24: what is left is below 2^-27, i.e. 29 bits below the largest of
@@ -25,8 +25,11 @@
 // steps, after the main loop, multiplies two more digits (2^-29, 2^-34: 39 bits below the largest).  N(0,1) marks no run in
 // 10^7, SwiGLU outputs of gates N(0,4) fewer than one in 10^4, of gates N(0,16) one in 200; a call in which every step has marks takes
 // 2.4 times as long.  The split's error with every second, eighth or 32nd channel 2^p as large and met by weights of zero, p = 2 to 16: at
-// most 1.6e-7 of the result.  The whole call's is larger there, up to 1.5e-6, where the small elements come to about half a unit of a digit
-// (p = 6, 10 and 16); most likely the instruction aligns its sum to the operands' exponents, those of products with zero among them.
+// most 1.6e-7 of the result.
+// Why q - z in halves: codes below 1 have no leading bit, and the instruction seems to align its sum as if they had one.  With
+// q - z in eighths, most of them such codes, a sum of few small products lost low bits of the accumulator: 1.5e-6 of the result
+// where the small elements of those inputs come to half a unit of a digit (p = 6, 10 and 16), in halves 4.7e-7, f16 tiles 4.5e-7 to
+// 4.8e-7 throughout.  It costs 1.5 % of a call (2048 x 4096 -> 11008 307 -> 312 us); quarters 6.2e-7 and nothing.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -503,7 +506,7 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
     };
     auto column_store = [&](int c, auto buf_tag) __attribute__((always_inline)) {
         constexpr int OFF = decltype(buf_tag)::value * BBYTES;
-        const v6u code = __builtin_amdgcn_cvt_scalef32_pk32_fp6_f16(halves, 8.0f);
+        const v6u code = __builtin_amdgcn_cvt_scalef32_pk32_fp6_f16(halves, 2.0f);
         lds_write24<OFF>(c_hi[c], c_lo[c], code);
     };
 
@@ -568,7 +571,7 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
         unit_slot[j] = a.least[min(my_col_c + j, a.n - 1)];
     }
 
-    constexpr int kB0 = 130 | (126 << 8) | (121 << 16) | (116 << 24), kB1 = 111 | (106 << 8);   // 2^3 / 2^shift of every digit
+    constexpr int kB0 = 128 | (124 << 8) | (119 << 16) | (114 << 24), kB1 = 109 | (104 << 8);   // 2 / 2^shift of every digit
 
     auto read6 = [&](const uint8_t* hi, const uint8_t* lo) __attribute__((always_inline)) {
         const uint4 h = *reinterpret_cast<const uint4*>(hi + lane * 16);
@@ -803,8 +806,8 @@ __global__ __launch_bounds__(512, 2) void w4_gemm_f6_kernel(F6Args a) {
                     v16f t;
 #pragma unroll
                     for (int r = 0; r < 16; r++) t[r] = 0.0f;
-                    t = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(da[0], fb, t, 2, 2, 0, ea, 0, 130 - kF6Shift[kF6Digits]);
-                    t = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(da[1], fb, t, 2, 2, 0, ea, 0, 130 - kF6Shift[kF6Digits + 1]);
+                    t = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(da[0], fb, t, 2, 2, 0, ea, 0, 128 - kF6Shift[kF6Digits]);
+                    t = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(da[1], fb, t, 2, 2, 0, ea, 0, 128 - kF6Shift[kF6Digits + 1]);
                     const float ratio_s = sc.v[j] / sc_cur.v[j];
 #pragma unroll
                     for (int r = 0; r < 16; r++) acc[i][j][r] = fmaf(t[r], ratio_s, acc[i][j][r]);

@@ -176,5 +176,5 @@ def test_small_elements_beside_large_channels(ops, st):
         exact = x.double() @ w
         err = ((ops.qmatmul_int4(x, packed, scales, zp, k, g).double() - exact).norm() / exact.norm()).item()
         say(f"    {err:.2e} of the result")
-        # 22 bits of every element, and six additions per step of 64, each within 2^-23 of the result, independent of each other
-        assert err <= 2.0 ** -22 + (6 * k / 64) ** 0.5 * 2.0 ** -23
+        # 22 bits of every element, and six additions per step of 64, each within 2^-24 of the result, independent of each other
+        assert err <= 2.0 ** -22 + (6 * k / 64) ** 0.5 * 2.0 ** -24
