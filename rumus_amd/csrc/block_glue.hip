@@ -152,7 +152,7 @@ constexpr uint32_t kAttnRows = 128;             // queries per workgroup
 // LDS rows with padding against bank conflicts: a fragment read takes 16 bytes of 32 adjacent rows
 constexpr uint32_t kAttnKPitch = 136;           // bf16 per key (128 dims)
 constexpr uint32_t kAttnVPitch = 40;            // bf16 per dim (32 keys)
-constexpr uint32_t kAttnHuge = 0x7f7f8000u;     // magnitudes from here on round to an infinite bf16
+constexpr float kAttnHuge = 0x1p60f;            // magnitudes from here on: a product of parts, or a sum of 128, might leave f32
 
 struct AttnPair { uint32_t part[kAttnParts]; }; // two floats' parts, packed
 __device__ __forceinline__ uint32_t attn_pack(float x, float y) {
@@ -172,15 +172,16 @@ __device__ __forceinline__ attn_v8b attn_operand(const AttnPair (&p)[4], int par
     return __builtin_bit_cast(attn_v8b, attn_v4u{p[0].part[part], p[1].part[part], p[2].part[part], p[3].part[part]});
 }
 __device__ __forceinline__ bool attn_any_huge(const float4& v) {
-    return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))) >= __uint_as_float(kAttnHuge);
+    return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))) >= kAttnHuge;
 }
 __device__ __forceinline__ float attn_other_half_max(float v) {
     const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return fmaxf(__uint_as_float(t[0]), __uint_as_float(t[1]));
 }
 
-// The same on v_mfma_f32_32x32x2_f32, for workgroups that meet an infinity or a value beyond the largest bf16: parts would
-// make NaNs of them (0 * infinity).  The 128 dims of the S^T product are walked as d = 64 * (lane / 32) + step, so that a lane's Q
+// The same on v_mfma_f32_32x32x2_f32, for workgroups that meet an infinity or a value of 2^60 and more: where the product of two
+// first parts leaves f32, the small products leave it with either sign, and a score of -infinity (a key without weight) would become
+// NaN (below 2^60 all 128 products of a score add up to less than 2^128).  The 128 dims of the S^T product are walked as d = 64 * (lane / 32) + step, so that a lane's Q
 // and K fragments are contiguous floats.  LDS tiles are [32 rows][33 chunks of 16 bytes]: the odd row stride spreads a
 // column of chunks (the K fragment read, one row per lane) over all banks, a row (the V fragment read) stays contiguous,
 // and every address is one per-lane base plus a compile-time offset.

@@ -75,3 +75,23 @@ def test_scores_near_the_lowest_value(ops):
     q[0, 2, 0, 5] = np.nan
     got = host(ops.attention(dev(q), dev(k), dev(v), False))
     assert np.isnan(got[0, 2]).all() and np.isfinite(got[0, [0, 1, 3, 4]]).all()
+
+
+@pytest.mark.parametrize("nq,nkv,causal", [(40, 90, False), (150, 150, False), (150, 300, True)])
+def test_scores_that_leave_f32(ops, nq, nkv, causal):
+    """Finite operands whose product is below the lowest f32: a score of -infinity, a key without weight."""
+    say(f"attention, scores of -1e45, {nq} queries of {nkv} keys")
+    for large in (1e22, 1e20, 3e37):
+        q, k, v = _operands(1, nq, nkv, 2, nq + 1)
+        k[..., 7] = 0.0
+        q[:, :, 0, 7] = large * (1.0 + 0.3 * np.abs(q[:, :, 0, 7]))    # all bits of it in use
+        k[0, [2, 33, nkv - 4], 0, 7] = -1e45 / large if large < 1e30 else -1e9
+        got = host(ops.attention(dev(q), dev(k), dev(v), causal))
+        k64 = k.astype(np.float64)
+        score = np.einsum("bqhd,bkhd->bhqk", q.astype(np.float64), k64) / np.sqrt(128.0)
+        if causal:
+            score = np.where(np.arange(nkv) <= np.arange(nq)[:, None] + nkv - nq, score, -np.inf)
+        weight = np.exp(score - score.max(-1, keepdims=True))
+        want = np.einsum("bhqk,bkhd->bqhd", weight / weight.sum(-1, keepdims=True), v.astype(np.float64))
+        assert np.isfinite(got).all()
+        np.testing.assert_allclose(got, want, rtol=1e-3, atol=2e-5)
