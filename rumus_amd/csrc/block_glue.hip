@@ -136,7 +136,7 @@ constexpr int kHeadDim = 128;
 // product 1.29).  f32 matrix cores (32 rows at a time; fewer than 64 rows on the vector units) -> this, us: 8 x 32 heads x 512 causal
 // 207 -> 149, without mask 309 -> 221, 2 x 16 x 1377 causal 252 -> 162, 8 x 32 x 63 30 -> 13, 32 heads, 16 rows behind 2048 keys
 // 762 -> 194.  Error against float64, as a share of the result: 512 causal rows 3.3e-7 -> 1.9e-7, operands four times as large
-// 1.7e-6 -> 0.6e-6, 4096 keys 1.2e-6 -> 1.0e-6 (values below 2^-108, whose last parts have no bf16, keep fewer bits).
+// 1.7e-6 -> 0.6e-6, 4096 keys 1.2e-6 -> 1.0e-6.
 // Measured slower: the split of the next tile between the MFMAs of this one (150 -> 170 us, registers), fragments read
 // ahead of their step (171), one sum for all six products of S (error 2.9e-7).
 typedef float attn_v16f __attribute__((ext_vector_type(16)));
@@ -153,6 +153,8 @@ constexpr uint32_t kAttnRows = 128;             // queries per workgroup
 constexpr uint32_t kAttnKPitch = 136;           // bf16 per key (128 dims)
 constexpr uint32_t kAttnVPitch = 40;            // bf16 per dim (32 keys)
 constexpr float kAttnHuge = 0x1p60f;            // magnitudes from here on: a product of parts, or a sum of 128, might leave f32
+constexpr float kAttnLeast = 0x1p-110f;         // magnitudes below: the last bits of their parts, 2^-23 of them, are below the least bf16
+constexpr float kAttnWeight = 0x1p23f;          // weights, 1 to 2^-126, are split as this many times themselves: parts of all of them
 
 struct AttnPair { uint32_t part[kAttnParts]; }; // two floats' parts, packed
 __device__ __forceinline__ uint32_t attn_pack(float x, float y) {
@@ -174,14 +176,22 @@ __device__ __forceinline__ attn_v8b attn_operand(const AttnPair (&p)[4], int par
 __device__ __forceinline__ bool attn_any_huge(const float4& v) {
     return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))) >= kAttnHuge;
 }
+__device__ __forceinline__ float attn_least(float least, const float4& v) {
+    return fminf(fminf(least, fminf(fabsf(v.x), fabsf(v.y))), fminf(fabsf(v.z), fabsf(v.w)));
+}
+__device__ __forceinline__ bool attn_any_small(const float4& v) {
+    auto small = [](float x) { return x != 0.0f && fabsf(x) < kAttnLeast; };
+    return small(v.x) || small(v.y) || small(v.z) || small(v.w);
+}
 __device__ __forceinline__ float attn_other_half_max(float v) {
     const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return fmaxf(__uint_as_float(t[0]), __uint_as_float(t[1]));
 }
 
-// The same on v_mfma_f32_32x32x2_f32, for workgroups that meet an infinity or a value of 2^60 and more: where the product of two
-// first parts leaves f32, the small products leave it with either sign, and a score of -infinity (a key without weight) would become
-// NaN (below 2^60 all 128 products of a score add up to less than 2^128).  The 128 dims of the S^T product are walked as d = 64 * (lane / 32) + step, so that a lane's Q
+// The same on v_mfma_f32_32x32x2_f32, for workgroups that meet an operand without parts.  From 2^60 on, infinities among them: where
+// the product of two first parts leaves f32, the small products leave it with either sign, and a score of -infinity (a key without
+// weight) would become NaN (below 2^60 all 128 products of a score add up to less than 2^128).  Values of V below 2^-110 (of 2^-118 the
+// parts lose 2^-16); queries and keys that small make scores of nothing, whatever they lose.  The 128 dims of the S^T product are walked as d = 64 * (lane / 32) + step, so that a lane's Q
 // and K fragments are contiguous floats.  LDS tiles are [32 rows][33 chunks of 16 bytes]: the odd row stride spreads a
 // column of chunks (the K fragment read, one row per lane) over all banks, a row (the V fragment read) stays contiguous,
 // and every address is one per-lane base plus a compile-time offset.
@@ -334,7 +344,7 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(AttnArgs a) {
     constexpr uint32_t kKPart = kAttnKeys * kAttnKPitch, kVPart = kHeadDim * kAttnVPitch;
     static_assert(kAttnParts * (kKPart + kVPart) * 2 >= 2 * kAttnKeys * kAttnRowChunks * 16, "the f32 tiles fit as well");
     __shared__ __attribute__((aligned(16))) uint16_t lds[kAttnParts * (kKPart + kVPart)];
-    __shared__ uint32_t huge;                                  // an operand that has no parts has been read
+    __shared__ uint32_t partless;                              // an operand that has no parts has been read
     uint16_t* const ks = lds;
     uint16_t* const vs = lds + kAttnParts * kKPart;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -391,7 +401,7 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(AttnArgs a) {
                 *reinterpret_cast<uint2*>(vput + p * kVPart + i * 32 * kAttnVPitch) = make_uint2(v0.part[p], v1.part[p]);
         }
     };
-    if (tid == 0) huge = 0;
+    if (tid == 0) partless = 0;
     fetch(0);
     __syncthreads();
 
@@ -415,7 +425,7 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(AttnArgs a) {
 #pragma unroll
             for (int i = 0; i < kAttnParts; i++) qf[s][i] = attn_operand(p, i);
         }
-        if (any) huge = 1;                                     // the parts are not looked at then
+        if (any) partless = 1;                                 // the parts are not looked at then
     }
     attn_v16f oacc[4];
 #pragma unroll
@@ -428,12 +438,20 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(AttnArgs a) {
     for (uint32_t j0 = 0; j0 < kv_end; j0 += kAttnKeys) {
         if (j0) __syncthreads();                               // the previous tile has been consumed
         bool any = false;
+        float least = kAttnLeast;
 #pragma unroll
-        for (int t = 0; t < 4; t++) any |= attn_any_huge(kreg[t]) | attn_any_huge(vreg[t]);
-        if (any) huge = 1;
+        for (int t = 0; t < 4; t++) {
+            any |= attn_any_huge(kreg[t]) | attn_any_huge(vreg[t]);
+            least = attn_least(least, vreg[t]);
+        }
+        if (any || least < kAttnLeast) {                       // (zeros come here too)
+#pragma unroll
+            for (int t = 0; t < 4; t++) any |= attn_any_small(vreg[t]);
+            if (any) partless = 1;
+        }
         store();
         __syncthreads();
-        in_f32 = __builtin_amdgcn_readfirstlane(huge) != 0;   // the same for the whole workgroup: written before the barrier
+        in_f32 = __builtin_amdgcn_readfirstlane(partless) != 0;   // the same for the whole workgroup: written before the barrier
         if (in_f32) break;
         if (!wave_live || j0 >= wave_end) {                    // wave-uniform: nothing visible in this tile
             fetch(j0 + kAttnKeys);
@@ -493,7 +511,7 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(AttnArgs a) {
             AttnPair pair[4];
             attn_v8b pf[kAttnParts];
 #pragma unroll
-            for (int i = 0; i < 4; i++) pair[i] = attn_split(sacc[8 * s + 2 * i], sacc[8 * s + 2 * i + 1]);
+            for (int i = 0; i < 4; i++) pair[i] = attn_split(sacc[8 * s + 2 * i] * kAttnWeight, sacc[8 * s + 2 * i + 1] * kAttnWeight);
 #pragma unroll
             for (int p = 0; p < kAttnParts; p++) pf[p] = attn_operand(pair, p);
 #pragma unroll
@@ -517,8 +535,8 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(AttnArgs a) {
     }
     lrun += __shfl_xor(lrun, 32);
     if (qrow >= a.q_len) return;
-    // oacc[i][r] = O[qrow][4 * ((r/4)*8 + kb*4 + r%4) + i]
-    const float inv = lrun > 0.0f ? 1.0f / lrun : 0.0f;
+    // oacc[i][r] / kAttnWeight = O[qrow][4 * ((r/4)*8 + kb*4 + r%4) + i]
+    const float inv = lrun > 0.0f ? 1.0f / (lrun * kAttnWeight) : 0.0f;
     float* op = a.o + b * a.o_sb + h * a.o_sh + (uint64_t)qrow * a.o_sr;
 #pragma unroll
     for (int r = 0; r < 16; r++)

@@ -95,3 +95,31 @@ def test_scores_that_leave_f32(ops, nq, nkv, causal):
         want = np.einsum("bhqk,bkhd->bqhd", weight / weight.sum(-1, keepdims=True), v.astype(np.float64))
         assert np.isfinite(got).all()
         np.testing.assert_allclose(got, want, rtol=1e-3, atol=2e-5)
+
+
+@pytest.mark.parametrize("nq,nkv", [(40, 90), (130, 200)])
+def test_small_operands_keep_their_bits(ops, nq, nkv):
+    """Values and weights so small that the last parts of them would have no bf16."""
+    say(f"attention, small values and weights, {nq} queries of {nkv} keys")
+    error = lambda got, want: np.linalg.norm(got.astype(np.float64) - want) / np.linalg.norm(want)
+    for power in (-99, -104, -112, -118):
+        q, k, v = _operands(1, nq, nkv, 2, nq)
+        v[:, :, 0] *= np.float32(2.0 ** power)
+        got = host(ops.attention(dev(q), dev(k), dev(v), False))
+        want = oracle.attention(q, k, v, False)
+        # a weight is up to 1 and down to 2^-15 here: sums of products of 2^(power - 15) and more, f32 down to 2^-149
+        bound = 128 * 2.0 ** -24 + np.sqrt(nkv) * 2.0 ** -24 + 2.0 ** -22
+        for head in (0, 1):
+            e = error(got[:, :, head], want[:, :, head])
+            say(f"    values of 2^{power if head == 0 else 0}: {e:.2e}")
+            assert e <= bound
+    # every key but the first has a weight of 2^-122 to 2^-117, and the first a value of zero
+    q, k, v = _operands(1, nq, nkv, 1, nq + 1)
+    q[:], k[:, :, :, 0], v[:, 0] = 0.0, -(118.0 + 0.5 * np.abs(k[:, :, :, 0]).clip(0, 4)) * np.log(2.0), 0.0
+    q[..., 0] = np.sqrt(128.0)
+    k[:, 0, :, 0] = 0.0
+    v *= 1e15
+    got = host(ops.attention(dev(q), dev(k), dev(v), False))
+    e = error(got, oracle.attention(q, k, v, False))
+    say(f"    weights of 2^-120: {e:.2e}")
+    assert e <= 122 * 3 * 2.0 ** -24                          # the score: three roundings of about 120 in f32
