@@ -1322,18 +1322,20 @@ static int launch_f6_rows(const W4Args& a, hipStream_t s, const W4BlockArgs& blo
 
 int w4_launch_gemm_f6(const W4Args& a, hipStream_t s, const W4BlockArgs& block) {
     RUMUS_REQUIRE(a.padded_k <= kF6MaxK, "qmatmul_int4: padded_k %u is beyond the six-bit kernel's %u", a.padded_k, kF6MaxK);
-    // With the weights converted where the workspace has room for that or may grow; the same bits without.
+    // With the weights converted where the workspace has room for that or may grow; the same bits without.  A size that the caller
+    // set holds what is taken without: the digits of `rows` rows, which may be half of all.
+    const uint32_t rows = f6_rows_at_once(a.m, a.padded_k, a.n);
     const F6Plan plan = f6_plan(a.m, a.padded_k, a.n, true);
     if (plan.codes) {
-        const size_t base = F6Workspace(a.m, a.padded_k, a.n).total;
-        if (workspace_has_or_grows(s, base, base + f6_codes_bytes(a.padded_k, a.n, plan.tn))) {
+        const size_t least = F6Workspace(min(rows, a.m), a.padded_k, a.n).total;
+        const size_t all = F6Workspace(a.m, a.padded_k, a.n).total + f6_codes_bytes(a.padded_k, a.n, plan.tn);
+        if (workspace_has_or_grows(s, least, all)) {
             bool lost = false;
             const int rc = launch_f6_rows(a, s, block, plan, &lost);
             if (!lost) return rc;
             (void)hipGetLastError();                         // the memory was not there: without
         }
     }
-    const uint32_t rows = f6_rows_at_once(a.m, a.padded_k, a.n);
     for (uint32_t r0 = 0; r0 < a.m; r0 += rows) {
         W4Args part = a;
         W4BlockArgs around = block;

@@ -1,0 +1,51 @@
+"""Calls that are faster with more workspace than they need: what they take, and what they leave alone."""
+import pytest
+
+from gpu_util import say
+
+pytestmark = pytest.mark.gpu
+
+MIB = 1 << 20
+
+
+def _weight(k, n, group, seed):
+    import torch
+    from rumus_amd import ops
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    return ops.w4_quantize_pack(torch.empty((k, n), device="cuda").normal_(0.0, 0.02, generator=gen), group)
+
+
+def _rows(m, k, seed):
+    import torch
+    return torch.empty((m, k), device="cuda").normal_(generator=torch.Generator(device="cuda").manual_seed(seed))
+
+
+def _no_workspaces():
+    """Frees every stream's workspace; the bytes of device memory that came back."""
+    import torch
+    from rumus_amd import _lib
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    _lib.call("rumus_hip_shutdown")
+    return torch.cuda.mem_get_info()[0] - before
+
+
+# digits of all rows at once (4.6 bytes per element) are more than the documented size for 385 x 3584, and more than the 32 MiB
+# in which the f16 tiles run 1500 x 5120: such calls take their rows in two halves and have no room for codes
+@pytest.mark.parametrize("m,k,n,reserve", [
+    (385, 3584, 14336, 5 * (385 + 64) * (3584 + 128) + 1280), (1500, 5120, 4096, 32 * MIB)])
+def test_reserved_size_is_kept(m, k, n, reserve):
+    import torch
+    from rumus_amd import _lib, ops
+    say(f"qmatmul_int4 {m} x {k} -> {n} on a stream whose workspace is reserved")
+    assert ops.qmatmul_int4_block_takes(m, k, n, 128)
+    weight, x, y = _weight(k, n, 128, 1), _rows(m, k, 2), torch.empty((m, n), device="cuda")
+    want = ops.qmatmul_int4(x, *weight, k, 128)
+    _no_workspaces()
+    stream = torch.cuda.Stream()
+    _lib.call("rumus_hip_workspace_reserve", stream.cuda_stream, reserve)
+    with torch.cuda.stream(stream):
+        ops.qmatmul_int4(x, *weight, k, 128, out=y)
+    stream.synchronize()
+    assert torch.equal(y, want)
+    assert _no_workspaces() <= reserve + 2 * MIB                 # whole MiB; the codes alone are 15 MB and more
