@@ -34,9 +34,11 @@ class WorkspaceLease {
 // Device workspace of at least `bytes` for work queued on `stream` (runtime.hip); `lease` then holds the
 // stream's workspace lock.
 int workspace_get(hipStream_t stream, size_t bytes, void** out, WorkspaceLease& lease);
-// Whether a call that can do with `least` bytes may ask workspace_get for `bytes`: they are there already, or the workspace can
-// grow and its size was not set by the caller (rumus_hip_workspace_reserve) at `least` or more.  It never shrinks, so a yes stands.
-bool workspace_has_or_grows(hipStream_t stream, size_t least, size_t bytes);
+// The same for a call that needs `least` bytes and is faster with `want`; `*got` is which of the two it has.  `want` is had where the
+// bytes are there already, or where the workspace may grow for speed alone: not while the stream is being captured, not under a
+// graph that was captured with it (growing frees what the graph's kernels use), not beyond a size of `least` or more that the caller
+// set (rumus_hip_workspace_reserve), and not when the memory cannot be had.
+int workspace_get_upto(hipStream_t stream, size_t least, size_t want, size_t* got, void** out, WorkspaceLease& lease);
 // A second buffer per (device, stream), for entry points that wrap another entry point between two conversions
 // (the half-precision ones): what they stage must outlive the inner call, whose workspace may grow - that is, be
 // freed - under it.  Never nested, never replaced by a fixed buffer.

@@ -396,11 +396,18 @@ static uint32_t mid_shares(uint32_t M, uint32_t K, uint32_t N, uint32_t* steps_p
 }
 
 // A K that is no multiple of 64 took no workspace before it came to the tiles that share K: where there is none (a capture, a
-// size the caller reserved) it is not shared.
-static uint32_t shares_with_room(uint32_t shares, uint32_t* steps_per, uint32_t M, uint32_t K, uint32_t N, hipStream_t s) {
-    if (shares == 1 || K % kBK == 0 || workspace_has_or_grows(s, 0, (size_t)shares * M * N * sizeof(int32_t))) return shares;
-    *steps_per = K / kBK;
-    return 1;
+// size the caller reserved) it is not shared.  `ws`: the partial sums, while `lease` lives.
+static int shares_with_room(uint32_t* shares, uint32_t* steps_per, uint32_t M, uint32_t K, uint32_t N, hipStream_t s, void** ws,
+                            WorkspaceLease& lease) {
+    if (*shares == 1) return RUMUS_HIP_OK;
+    const size_t want = (size_t)*shares * M * N * sizeof(int32_t);
+    size_t got = 0;
+    if (int rc = workspace_get_upto(s, K % kBK ? 0 : want, want, &got, ws, lease)) return rc;
+    if (got < want) {
+        *shares = 1;
+        *steps_per = K / kBK;
+    }
+    return RUMUS_HIP_OK;
 }
 
 // Few tiles: one wave per 64 x 64 tile, eight stages of direct-to-LDS loads deep, and K
@@ -412,16 +419,15 @@ static int launch_small(const int8_t* A, const int8_t* B, const float* sx, const
     constexpr int NS = 8;
     constexpr size_t lds_bytes = (size_t)NS * 128 * kBK;       // 64 KB
     const uint32_t tm = ceil_div(M, 64), tn = ceil_div(N, 64);
-    uint32_t steps_per = 0;
-    const uint32_t shares = shares_with_room(small_shares(M, K, N, &steps_per), &steps_per, M, K, N, s);
+    uint32_t steps_per = 0, shares = small_shares(M, K, N, &steps_per);
+    void* ws = nullptr;
+    WorkspaceLease lease;                                    // until both kernels are queued
+    if (int rc = shares_with_room(&shares, &steps_per, M, K, N, s, &ws, lease)) return rc;
     if (shares == 1) {
         hipLaunchKernelGGL((i8_gemm_dma_kernel<2, 2, 1, 1, NS>), dim3(tm * tn, 1), dim3(64), lds_bytes, s, A, B, sx, sw,
                            bias, acc, y, M, K, N, tm, tn, steps_per);
         return check_launch("i8_gemm_dma_kernel");
     }
-    void* ws = nullptr;
-    WorkspaceLease lease;                                    // until both kernels are queued
-    if (int rc = workspace_get(s, (size_t)shares * M * N * sizeof(int32_t), &ws, lease)) return rc;
     int32_t* part = static_cast<int32_t*>(ws);
     hipLaunchKernelGGL((i8_gemm_dma_kernel<2, 2, 1, 1, NS>), dim3(tm * tn, shares), dim3(64), lds_bytes, s, A, B,
                        (const float*)nullptr, (const float*)nullptr, (const float*)nullptr, part, (float*)nullptr, M, K, N,
@@ -439,16 +445,15 @@ static int launch_mid(const int8_t* A, const int8_t* B, const float* sx, const f
     constexpr int NS = 4;
     constexpr size_t lds_bytes = (size_t)NS * 256 * kBK;       // 64 KB
     const uint32_t tm = ceil_div(M, 128), tn = ceil_div(N, 128);
-    uint32_t steps_per = 0;
-    const uint32_t shares = shares_with_room(mid_shares(M, K, N, &steps_per), &steps_per, M, K, N, s);
+    uint32_t steps_per = 0, shares = mid_shares(M, K, N, &steps_per);
+    void* ws = nullptr;
+    WorkspaceLease lease;                                    // until both kernels are queued
+    if (int rc = shares_with_room(&shares, &steps_per, M, K, N, s, &ws, lease)) return rc;
     if (shares == 1) {
         hipLaunchKernelGGL((i8_gemm_dma_kernel<2, 2, 2, 2, NS>), dim3(tm * tn, 1), dim3(256), lds_bytes, s, A, B, sx, sw,
                            bias, acc, y, M, K, N, tm, tn, steps_per);
         return check_launch("i8_gemm_dma_kernel");
     }
-    void* ws = nullptr;
-    WorkspaceLease lease;                                    // until both kernels are queued
-    if (int rc = workspace_get(s, (size_t)shares * M * N * sizeof(int32_t), &ws, lease)) return rc;
     int32_t* part = static_cast<int32_t*>(ws);
     hipLaunchKernelGGL((i8_gemm_dma_kernel<2, 2, 2, 2, NS>), dim3(tm * tn, shares), dim3(256), lds_bytes, s, A, B,
                        (const float*)nullptr, (const float*)nullptr, (const float*)nullptr, part, (float*)nullptr, M, K, N,

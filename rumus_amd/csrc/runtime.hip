@@ -35,6 +35,7 @@ struct Arena {
     void* ptr = nullptr;
     size_t bytes = 0;
     bool reserved = false;           // the caller set the size
+    bool in_graph = false;           // it was handed out under a capture: a graph's kernels may use it
     std::recursive_mutex in_use;     // held by a WorkspaceLease
 };
 struct ArenaKey {
@@ -102,14 +103,35 @@ static int workspace_reserve(hipStream_t stream, size_t bytes, void** out, Works
     return rc;
 }
 
-bool workspace_has_or_grows(hipStream_t stream, size_t least, size_t bytes) {
-    if (g_fixed_ptr) return g_nest_offset + bytes <= g_fixed_bytes;
+static int arena_grow(Arena& a, hipStream_t stream, size_t bytes) {
+    const RelaxedCapture relaxed;
+    if (a.ptr) {
+        if (int rc = check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize")) return rc;
+        if (int rc = check_hip(hipFree(a.ptr), "hipFree(workspace)")) return rc;
+        a.ptr = nullptr;
+        a.bytes = 0;
+        a.in_graph = false;
+    }
+    const size_t want = (bytes + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);   // whole MiB
+    if (int rc = check_hip(hipMalloc(&a.ptr, want), "hipMalloc(workspace)")) return rc;
+    a.bytes = want;
+    return RUMUS_HIP_OK;
+}
+
+int workspace_get_upto(hipStream_t stream, size_t least, size_t want, size_t* got, void** out, WorkspaceLease& lease) {
     int device = 0;
-    if (hipGetDevice(&device) != hipSuccess) return false;
+    if (int rc = check_hip(hipGetDevice(&device), "hipGetDevice")) return rc;
     Arena& a = *arena_of(device, stream, 0);
     std::lock_guard<std::recursive_mutex> lock(a.in_use);
-    if (a.bytes >= g_nest_offset + bytes) return true;
-    return !g_nest_offset && !(a.reserved && a.bytes >= least) && !is_capturing(stream);
+    *got = want;
+    if ((g_fixed_ptr ? g_fixed_bytes : a.bytes) < g_nest_offset + want) {
+        const bool grows = !g_fixed_ptr && !g_nest_offset && !(a.reserved && a.bytes >= least) && !a.in_graph && !is_capturing(stream);
+        if (!grows || arena_grow(a, stream, want) != RUMUS_HIP_OK) {
+            if (grows) (void)hipGetLastError();              // the memory was not there
+            *got = least;
+        }
+    }
+    return arena_get(0, stream, *got, out, lease);
 }
 
 int staging_get(hipStream_t stream, size_t bytes, void** out, WorkspaceLease& lease) {
@@ -145,17 +167,9 @@ int arena_get(int kind, hipStream_t stream, size_t bytes, void** out, WorkspaceL
                              "%s of %zu bytes needed while the stream is capturing: call %s before the capture",
                              kind ? "staging memory" : "workspace", bytes,
                              kind ? "rumus_hip_f16_staging_reserve" : "rumus_hip_workspace_reserve");
-        const RelaxedCapture relaxed;
-        if (a.ptr) {
-            if (int rc = check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize")) return rc;
-            if (int rc = check_hip(hipFree(a.ptr), "hipFree(workspace)")) return rc;
-            a.ptr = nullptr;
-            a.bytes = 0;
-        }
-        const size_t want = (bytes + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);   // whole MiB
-        if (int rc = check_hip(hipMalloc(&a.ptr, want), "hipMalloc(workspace)")) return rc;
-        a.bytes = want;
+        if (int rc = arena_grow(a, stream, bytes)) return rc;
     }
+    if (bytes && !a.in_graph) a.in_graph = is_capturing(stream);
     *out = a.ptr;
     return RUMUS_HIP_OK;
 }

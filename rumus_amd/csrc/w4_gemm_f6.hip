@@ -1267,16 +1267,12 @@ static int launch_f6_groups(const F6Args& f, const W4Args& a, uint32_t blocks, u
     return wide ? launch_f6<TN, 2, ZP4, true>(f, blocks, s) : launch_f6<TN, 1, ZP4, true>(f, blocks, s);
 }
 
-// `plan.codes`: the workspace may be asked for the converted weights too; `lost` then says that it could not be had
-static int launch_f6_rows(const W4Args& a, hipStream_t s, const W4BlockArgs& block, const F6Plan& plan, bool* lost = nullptr) {
+static int launch_f6_rows(const W4Args& a, hipStream_t s, const W4BlockArgs& block, const F6Plan& plan) {
     const F6Workspace w(a.m, a.padded_k, a.n);
     const size_t codes_bytes = plan.codes ? f6_codes_bytes(a.padded_k, a.n, plan.tn) : 0;
     void* ws = nullptr;
     WorkspaceLease lease;                                    // until the last kernel of this call is queued
-    if (int rc = workspace_get(s, w.total + codes_bytes, &ws, lease)) {
-        if (lost) *lost = true;
-        return rc;
-    }
+    if (int rc = workspace_get(s, w.total + codes_bytes, &ws, lease)) return rc;
     uint8_t* p = static_cast<uint8_t*>(ws);
     uint8_t* const planes = p; p += w.planes;
     uint8_t* const exps = p; p += w.exps;
@@ -1329,12 +1325,11 @@ int w4_launch_gemm_f6(const W4Args& a, hipStream_t s, const W4BlockArgs& block) 
     if (plan.codes) {
         const size_t least = F6Workspace(min(rows, a.m), a.padded_k, a.n).total;
         const size_t all = F6Workspace(a.m, a.padded_k, a.n).total + f6_codes_bytes(a.padded_k, a.n, plan.tn);
-        if (workspace_has_or_grows(s, least, all)) {
-            bool lost = false;
-            const int rc = launch_f6_rows(a, s, block, plan, &lost);
-            if (!lost) return rc;
-            (void)hipGetLastError();                         // the memory was not there: without
-        }
+        size_t got = 0;
+        void* ws = nullptr;
+        WorkspaceLease lease;
+        if (int rc = workspace_get_upto(s, least, all, &got, &ws, lease)) return rc;
+        if (got == all) return launch_f6_rows(a, s, block, plan);
     }
     for (uint32_t r0 = 0; r0 < a.m; r0 += rows) {
         W4Args part = a;

@@ -49,3 +49,33 @@ def test_reserved_size_is_kept(m, k, n, reserve):
     stream.synchronize()
     assert torch.equal(y, want)
     assert _no_workspaces() <= reserve + 2 * MIB                 # whole MiB; the codes alone are 15 MB and more
+
+
+def test_a_graph_keeps_its_workspace():
+    """A call on a stream whose workspace a graph uses does without room that it could have: growing would free the graph's memory."""
+    import torch
+    from rumus_amd import ops
+    k = 4096
+    say("qmatmul_int4 1500 x 4096 -> 4096 in a graph, 1200 x 4096 -> 11008 beside it on the graph's stream")
+    small, large = _weight(k, 4096, 128, 1), _weight(k, 11008, 128, 2)
+    x, other = _rows(1500, k, 3), _rows(1200, k, 4)
+    want, beside = ops.qmatmul_int4(x, *small, k, 128), ops.qmatmul_int4(other, *large, k, 128)
+    _no_workspaces()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    y, got = torch.empty_like(want), torch.empty_like(beside)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        ops.qmatmul_int4(x, *small, k, 128, out=y)
+    stream.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        ops.qmatmul_int4(x, *small, k, 128, out=y)
+    with torch.cuda.stream(stream):
+        ops.qmatmul_int4(other, *large, k, 128, out=got)
+    stream.synchronize()
+    assert torch.equal(got, beside)
+    y.zero_()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(y, want)
+    # digits and sums of 1500 rows, 29 MB, with the codes of 4096 columns, 13 MB; what the other call would like is 58 MB
+    assert _no_workspaces() <= 44 * MIB
