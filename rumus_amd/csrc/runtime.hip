@@ -83,7 +83,8 @@ static bool is_capturing(hipStream_t stream) {
     return stream && hipStreamIsCapturing(stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
 }
 
-// While one of these lives, this thread may allocate and free although another stream is being captured.
+// While one of these lives, this thread may allocate and free although another stream is being captured.  For growing that a call
+// can do without (it ran beside captures before it had a use for more); one that has to allocate is refused there, as ever.
 struct RelaxedCapture {
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
@@ -104,7 +105,6 @@ static int workspace_reserve(hipStream_t stream, size_t bytes, void** out, Works
 }
 
 static int arena_grow(Arena& a, hipStream_t stream, size_t bytes) {
-    const RelaxedCapture relaxed;
     if (a.ptr) {
         if (int rc = check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize")) return rc;
         if (int rc = check_hip(hipFree(a.ptr), "hipFree(workspace)")) return rc;
@@ -126,7 +126,12 @@ int workspace_get_upto(hipStream_t stream, size_t least, size_t want, size_t* go
     *got = want;
     if ((g_fixed_ptr ? g_fixed_bytes : a.bytes) < g_nest_offset + want) {
         const bool grows = !g_fixed_ptr && !g_nest_offset && !(a.reserved && a.bytes >= least) && !a.in_graph && !is_capturing(stream);
-        if (!grows || arena_grow(a, stream, want) != RUMUS_HIP_OK) {
+        auto grow = [&] {
+            if (a.bytes < least) return arena_grow(a, stream, want);
+            const RelaxedCapture relaxed;
+            return arena_grow(a, stream, want);
+        };
+        if (!grows || grow() != RUMUS_HIP_OK) {
             if (grows) (void)hipGetLastError();              // the memory was not there
             *got = least;
         }

@@ -79,3 +79,33 @@ def test_a_graph_keeps_its_workspace():
     assert torch.equal(y, want)
     # digits and sums of 1500 rows, 29 MB, with the codes of 4096 columns, 13 MB; what the other call would like is 58 MB
     assert _no_workspaces() <= 44 * MIB
+
+
+def test_growing_beside_a_capture():
+    """While another stream is being captured a call may still let its workspace grow for speed."""
+    import torch
+    from rumus_amd import _lib, ops
+    k = 4096
+    say("qmatmul_int4 1200 x 4096 -> 11008 while another stream is captured")
+    small, large = _weight(k, 4096, 128, 1), _weight(k, 11008, 128, 2)
+    x, other = _rows(1500, k, 3), _rows(1200, k, 4)
+    beside = ops.qmatmul_int4(other, *large, k, 128)
+    _no_workspaces()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    got, doubled = torch.empty_like(beside), torch.empty_like(x)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        ops.qmatmul_int4(x, *small, k, 128, out=torch.empty((1500, 4096), device="cuda"))
+    stream.synchronize()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        torch.mul(x, 2.0, out=doubled)
+        with torch.cuda.stream(stream):
+            ops.qmatmul_int4(other, *large, k, 128, out=got)
+    stream.synchronize()
+    assert torch.equal(got, beside)
+    for _ in range(2):
+        doubled.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(doubled, 2.0 * x)
+    assert _no_workspaces() >= 50 * MIB                          # digits of 1200 rows, 24 MB, and the codes, 34 MB
