@@ -82,7 +82,8 @@ int rumus_hip_sync(rumus_hip_stream_t stream);
  *   qmatmul_int4_t, m >= 8: 64 * m * k (partial sums, only below 512 tiles of
  *       64 x 128) + 10 * num_groups * n + 4 * (m + num_groups) + 2048;
  *   i8_gemm: rumus_hip_i8_gemm_workspace_size(m, k, n) exactly; at most
- *       min(32 * m * n, 16 MiB);
+ *       min(32 * m * n, 16 MiB) (with k % 64 != 0 only where there is room, as
+ *       above; exact sums either way);
  *   matmul_q8, m >= 5: 4 * m * k * 4 (digit planes of a) + 4 * m * n * 4 + 32 MiB
  *       (partial sums of the int8 GEMM inside); with one block per column from
  *       384 rows on also k * n + 4 * n;

@@ -34,6 +34,8 @@ int i8_gemm_fold4(const int8_t* planes, const int8_t* wq, const float* sx4, cons
 // Workspace bytes rumus_hip_i8_gemm takes for an m x k x n product (i32 partial sums where K is shared over
 // workgroups); replays the dispatch, no device call.
 size_t i8_gemm_workspace_need(uint32_t m, uint32_t k, uint32_t n);
+// ... and those it cannot do without: the sums of a ragged K are only kept where there is room.
+size_t i8_gemm_workspace_least(uint32_t m, uint32_t k, uint32_t n);
 
 // Decode kernel for m <= 4 on v_dot4_i32_i8 (i8_gemv.hip).
 int i8_launch_gemv(const int8_t* xq, const int8_t* wq, const float* sx, const float* sw, const float* bias, int32_t* acc,

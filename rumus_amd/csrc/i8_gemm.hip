@@ -574,6 +574,8 @@ size_t i8_gemm_workspace_need(uint32_t m, uint32_t k, uint32_t n) {
     return shares > 1 ? (size_t)shares * m * n * sizeof(int32_t) : 0;
 }
 
+size_t i8_gemm_workspace_least(uint32_t m, uint32_t k, uint32_t n) { return k % kBK ? 0 : i8_gemm_workspace_need(m, k, n); }
+
 // Routes whose kernels have the plane-adding epilogue: the two kernels of large shapes, and row splits into them.
 bool i8_gemm_fold4_supported(uint32_t m4, uint32_t k, uint32_t n) {
     if (m4 == 0 || m4 % 4 != 0 || n == 0 || k == 0 || k % kBK != 0) return false;

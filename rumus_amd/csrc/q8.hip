@@ -531,8 +531,9 @@ static size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
 // c = a x (wq, sw): wq dense int8 [n, k], sw [n].  The planes are added in the GEMM's epilogue where the shape
 // has such a kernel (large ones), by a pass over the four partial outputs otherwise; both give the same bits.
-// `ws` holds q8_dense_workspace(m, k, n) bytes, the int8 GEMM's own partial sums behind `own` of them.
-struct Q8DenseWs { size_t planes, sx, y, own, total; bool fold; };
+// `ws` holds q8_dense_workspace(m, k, n) bytes, the int8 GEMM's own partial sums behind `own` of them: `total` where there is
+// room, `least` where not.
+struct Q8DenseWs { size_t planes, sx, y, own, least, total; bool fold; };
 
 static Q8DenseWs q8_dense_workspace(uint32_t m, uint32_t k, uint32_t n) {
     Q8DenseWs w;
@@ -542,6 +543,7 @@ static Q8DenseWs q8_dense_workspace(uint32_t m, uint32_t k, uint32_t n) {
     w.y = w.fold ? 0 : align256((size_t)kQ8Planes * m * n * sizeof(float));
     w.own = w.planes + w.sx + w.y;
     w.total = w.own + (w.fold ? 0 : i8_gemm_workspace_need(kQ8Planes * m, k, n));
+    w.least = w.own + (w.fold ? 0 : i8_gemm_workspace_least(kQ8Planes * m, k, n));
     return w;
 }
 
@@ -570,7 +572,8 @@ static int matmul_q8_mfma(const float* a, const uint32_t* b, float* c, uint32_t 
     const size_t wq_bytes = align256((size_t)n * k), sw_bytes = align256((size_t)n * sizeof(float));
     void* ws = nullptr;
     WorkspaceLease lease;                                    // until the last kernel of this call is queued
-    if (int rc = workspace_get(s, wq_bytes + sw_bytes + w.total, &ws, lease)) return rc;
+    size_t got = 0;
+    if (int rc = workspace_get_upto(s, wq_bytes + sw_bytes + w.least, wq_bytes + sw_bytes + w.total, &got, &ws, lease)) return rc;
     WorkspaceNest nest(wq_bytes + sw_bytes + w.own);
     uint8_t* base = static_cast<uint8_t*>(ws);
     int8_t* wq = reinterpret_cast<int8_t*>(base);
@@ -899,7 +902,8 @@ int rumus_hip_matmul_q8_dense(const float* a, const int8_t* wq, const float* sw,
     const Q8DenseWs w = q8_dense_workspace(m, k, n);
     void* ws = nullptr;
     WorkspaceLease lease;                                    // until the last kernel of this call is queued
-    if (int rc = workspace_get(s, w.total, &ws, lease)) return rc;
+    size_t got = 0;
+    if (int rc = workspace_get_upto(s, w.least, w.total, &got, &ws, lease)) return rc;
     WorkspaceNest nest(w.own);
     return matmul_q8_planes(a, wq, sw, c, m, k, n, w, static_cast<uint8_t*>(ws), s);
 }

@@ -109,3 +109,38 @@ def test_growing_beside_a_capture():
         torch.cuda.synchronize()
         assert torch.equal(doubled, 2.0 * x)
     assert _no_workspaces() >= 50 * MIB                          # digits of 1200 rows, 24 MB, and the codes, 34 MB
+
+
+def _captured_in(reserve, call, outs):
+    """The outputs of a call captured on a stream with a workspace of `reserve` bytes, after each of three replays."""
+    import torch
+    from rumus_amd import _lib
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    _lib.call("rumus_hip_workspace_reserve", stream.cuda_stream, reserve)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        call()
+    for _ in range(3):
+        outs.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        yield outs
+
+
+def test_q8_with_a_ragged_k_needs_no_partial_sums():
+    """One block per column: the int8 GEMM inside has no room for shares of K, in a capture on a workspace of what the call keeps there."""
+    import torch
+    from rumus_amd import ops
+    m, k, n = 384, 2064, 500
+    say(f"matmul_q8 {m} x {k} x {n}, one block per column, captured without room for shares of K")
+    a, w = _rows(m, k, 3), _rows(n, k, 4)
+    words = ops.q8_quantize(w.reshape(-1), k)
+    wq, sw = ops.q8_dense_layout(words, k, n, k)
+    up = lambda v: -(-v // 256) * 256
+    own = up(4 * m * k) + up(16 * m) + up(16 * m * n)            # digit planes, their factors, the planes' products
+    c = torch.empty((m, n), device="cuda")
+    for room, call in ((own + up(n * k) + up(4 * n), lambda out: ops.matmul_q8(a, words, k, n, k, out=out)),
+                       (own, lambda out: ops.matmul_q8_dense(a, wq, sw, out=out))):
+        want = call(torch.empty_like(c))
+        for got in _captured_in(room, lambda: call(c), c):
+            assert torch.equal(got, want)
