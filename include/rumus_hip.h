@@ -80,7 +80,9 @@ int rumus_hip_sync(rumus_hip_stream_t stream);
  *       once per 128 rows.  Same bits without;
  *       to reserve for it: 3 * (padded_k + 64) * (n + 512) / 4 on top;
  *   qmatmul_int4_t, m >= 8: 64 * m * k (partial sums, only below 512 tiles of
- *       64 x 128) + 10 * num_groups * n + 4 * (m + num_groups) + 2048;
+ *       64 x 128; 32 * m * k do from 65 rows on where there is no room for more,
+ *       at some speed and with sums in another order) + 10 * num_groups * n +
+ *       4 * (m + num_groups) + 2048;
  *   i8_gemm: rumus_hip_i8_gemm_workspace_size(m, k, n) exactly; at most
  *       min(32 * m * n, 16 MiB) (with k % 64 != 0 only where there is room, as
  *       above; exact sums either way);

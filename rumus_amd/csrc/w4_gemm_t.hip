@@ -817,13 +817,12 @@ int w4_launch_gemm_t(const float* gy, const uint32_t* packed, const float* scale
     const uint32_t ktiles = padded_k / (32 * kw), mtiles = ceil_div(m, 64), nsteps = ceil_div(n, 32);
     RUMUS_REQUIRE(mtiles <= 65535, "qmatmul_int4_t: m %u is beyond the grid limit", m);
     // fewer tiles than two per compute unit: n is shared out too, in shares of at least 16 steps
-    uint32_t shares = 1, steps_per = nsteps;
+    uint32_t shares = 1, steps_per = nsteps, wide_shares = 1;
     const uint64_t tiles = (uint64_t)ktiles * mtiles;
     // Up to 32 rows half of the wide kernel's rows would be empty (11008 x 4096 at 16 rows 24.1 us above, 24.6 there).
     const bool wide = kw == 4 && n % 16 == 0 && m > 32;
-    if (wide) {
-        if (tiles < 512) shares = w4t_wide_shares((uint32_t)tiles, m, k, n);
-    } else if (tiles < 512) {
+    if (wide && tiles < 512) wide_shares = w4t_wide_shares((uint32_t)tiles, m, k, n);
+    if (tiles < 512) {
         shares = (uint32_t)(1024 / tiles);
         // one row tile: up to 16 shares (46 us instead of 60 for up to 64 rows); beyond, the partial results
         // of more than 8 shares cost more than the shares gain (128 rows: 84 us against 72)
@@ -838,10 +837,18 @@ int w4_launch_gemm_t(const float* gy, const uint32_t* packed, const float* scale
     const size_t gn = (size_t)num_groups * n;
     const size_t rowf_bytes = up((size_t)m * sizeof(float)), sgrp_bytes = up((size_t)num_groups * sizeof(float));
     const size_t sp_bytes = up(gn * sizeof(float)), zo_bytes = up(gn * sizeof(_Float16) + 64);
-    const size_t part_bytes = shares > 1 ? (size_t)shares * m * k * sizeof(float) : 0;
+    auto bytes = [&](uint32_t parts) {
+        return rowf_bytes + sgrp_bytes + 2 * sp_bytes + zo_bytes + (parts > 1 ? (size_t)parts * m * k * sizeof(float) : 0);
+    };
+    // The wide kernel's shares may be more than the narrow one's: it takes them where there is room for their partial results
+    // (100 rows, 11008 -> 512: 16 shares, 8), and no more than those where not, so that a capture runs in what it ran in.
+    const uint32_t fewest = wide ? min(shares, wide_shares) : shares;
+    if (wide) shares = wide_shares;
     void* ws = nullptr;
+    size_t got = 0;
     WorkspaceLease lease;                                    // until the last kernel of this call is queued
-    if (int rc = workspace_get(s, rowf_bytes + sgrp_bytes + 2 * sp_bytes + zo_bytes + part_bytes, &ws, lease)) return rc;
+    if (int rc = workspace_get_upto(s, bytes(fewest), bytes(shares), &got, &ws, lease)) return rc;
+    if (got < bytes(shares)) shares = fewest;
     uint8_t* b = static_cast<uint8_t*>(ws);
     float* rowf = reinterpret_cast<float*>(b);
     float* sgrp = reinterpret_cast<float*>(b + rowf_bytes);

@@ -144,3 +144,24 @@ def test_q8_with_a_ragged_k_needs_no_partial_sums():
         want = call(torch.empty_like(c))
         for got in _captured_in(room, lambda: call(c), c):
             assert torch.equal(got, want)
+
+
+# 100 rows: eight shares of n fit, sixteen would be faster; 40 rows with a short n: four fit
+@pytest.mark.parametrize("m,k,n,shares", [(100, 512, 11008, 8), (40, 512, 2048, 4)])
+def test_grad_x_with_room_for_fewer_shares(m, k, n, shares):
+    import torch
+    from rumus_amd import ops
+    say(f"qmatmul_int4_t {m} rows of {n} -> {k}, captured with room for {shares} shares of n")
+    packed, scales, zp = _weight(k, n, 128, 5)
+    gy = _rows(m, n, 6)
+    out = torch.empty((m, k), device="cuda")
+    up = lambda v: -(-v // 256) * 256
+    entries = k // 128 * n
+    room = up(4 * m) + up(4 * (k // 128)) + 2 * up(4 * entries) + up(2 * entries + 64) + shares * m * k * 4
+    q = torch.stack([(packed.view(torch.int32) >> (4 * i)) & 15 for i in range(8)], 1).reshape(k, n).double()
+    each = lambda t: t.double().repeat_interleave(128, 0)
+    w = ((q - each(zp)) * each(scales)).t().contiguous()
+    want, size = gy.double() @ w, gy.double().abs() @ w.abs()
+    for got in _captured_in(room, lambda: ops.qmatmul_int4_t(gy, packed, scales, zp, k, 128, out=out), out):
+        # test_gpu_w4_t_wide.py's bound of an ordinary sum, far above both share counts' rounding
+        assert float(((got.double() - want).abs() / size).max()) < 2e-6
