@@ -31,3 +31,12 @@ def host_u32(t: torch.Tensor) -> np.ndarray:
 
 def assert_close(got, want, what=""):
     np.testing.assert_allclose(got, want, rtol=RTOL, atol=ATOL, err_msg=what)
+
+
+def free_workspaces() -> int:
+    """Frees every stream's workspace (no launch may be in flight); the bytes of device memory that came back."""
+    from rumus_amd import _lib
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    _lib.call("rumus_hip_shutdown")
+    return torch.cuda.mem_get_info()[0] - before

@@ -1,7 +1,7 @@
 """INT8 GEMM with K that ends in one to three chunks of 16: every tile size, exact i32 sums."""
 import pytest
 
-from gpu_util import say
+from gpu_util import free_workspaces, say
 
 pytestmark = pytest.mark.gpu
 
@@ -34,15 +34,16 @@ def test_tail_without_room_for_shares():
     gen = torch.Generator(device="cuda").manual_seed(3)
     x, w = (torch.randint(-128, 128, (r, 4144), generator=gen, device="cuda", dtype=torch.int32).to(torch.int8) for r in (60, 520))
     _, want = ops.i8_gemm(x, w, want_acc=True, want_y=False)
-    torch.cuda.synchronize()
-    _lib.call("rumus_hip_shutdown")                              # no stream has a workspace now
+    big, wide = torch.cat([x] * 2), torch.cat([w] * 4)
+    assert _lib.lib().rumus_hip_i8_gemm_workspace_size(120, 4144, 2080) >= 3 << 20
+    free_workspaces()
     sized, captured = torch.cuda.Stream(), torch.cuda.Stream()
-    _lib.call("rumus_hip_workspace_reserve", sized.cuda_stream, 256)   # a mebibyte; eight shares take one of 998400 bytes
-    big = torch.cat([x] * 2)
+    _lib.call("rumus_hip_workspace_reserve", sized.cuda_stream, 256)   # a mebibyte
     with torch.cuda.stream(sized):
-        _, got = ops.i8_gemm(big, w, want_acc=True, want_y=False)
+        _, got = ops.i8_gemm(big, wide, want_acc=True, want_y=False)
     sized.synchronize()
-    assert torch.equal(got, torch.cat([want] * 2))
+    assert torch.equal(got, torch.cat([torch.cat([want] * 4, 1)] * 2))
+    assert free_workspaces() <= 2 << 20                          # (memory comes in 2 MiB)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=captured):
         _, got = ops.i8_gemm(x, w, want_acc=True, want_y=False)

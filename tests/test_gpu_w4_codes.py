@@ -2,9 +2,11 @@
 of the caller's own size, with no room for the codes): the same bits, and the product in float64."""
 import pytest
 
-from gpu_util import say
+from gpu_util import free_workspaces, say
 
 pytestmark = pytest.mark.gpu
+
+MIB = 1 << 20
 
 
 # every width of the workgroups' columns, groups of one, two and three steps of 64 k, an odd number of steps, K no multiple of the
@@ -23,18 +25,21 @@ def test_codes_once_or_by_every_block(m, k, n, group, packed_zero):
     x = torch.empty((m, k), device="cuda").normal_(generator=gen)
     x[::7, ::37] *= 3000.0                                       # marked runs in some rows
     call = ops.qmatmul_int4_zp4 if packed_zero else ops.qmatmul_int4
-    torch.cuda.synchronize()
-    _lib.call("rumus_hip_shutdown")                              # no stream has a workspace now
-    grows, sized = torch.cuda.Stream(), torch.cuda.Stream()
     padded, groups = ops.w4_geometry(k, group)
     blocks, steps = -(-m // 128), padded // 64                   # digits, exponents, sums, row factors, column scales, flags
-    _lib.call("rumus_hip_workspace_reserve", sized.cuda_stream,
-              blocks * (steps * (36864 + 512) + -(-steps // 2) * 512 + 1024) + 4 * n + 1024 + 512)
+    digits = blocks * (steps * (36864 + 512) + -(-steps // 2) * 512 + 1024) + 4 * n + 1024 + 512
+    codes = 48 * n * steps                                       # and more where the last block of columns is not full
     outs = []
-    for stream in (grows, sized):
+    for sized in (False, True):
+        free_workspaces()
+        stream = torch.cuda.Stream()
+        if sized:
+            _lib.call("rumus_hip_workspace_reserve", stream.cuda_stream, digits)
         with torch.cuda.stream(stream):
             outs.append(call(x, packed, scales, zp, k, group))
         stream.synchronize()
+        took = free_workspaces()
+        assert took <= -(-digits // (2 * MIB)) * 2 * MIB if sized else took >= digits - 512 + codes   # (memory comes in 2 MiB)
     assert torch.equal(outs[0].view(torch.int32), outs[1].view(torch.int32))
     q = torch.stack([(packed.view(torch.int32) >> (4 * i)) & 15 for i in range(8)], 1).reshape(padded, n).double()
     if packed_zero:

@@ -78,8 +78,8 @@ def test_six_bit_kernel_at_its_edges(ops, m, k, n, g, act_order, zeros):
 
 # Long rows, where the preparation takes two rows or one per workgroup, and groups that pad K beyond what it takes (then
 # another kernel runs).  The stream's workspace holds another call's digits, exponents and sums, every run of 32 marked
-# there, and the padding nibbles are 15: what a kernel reads without having written it shows.  At k = 5120 the rows go in two halves
-# (32 MiB hold what the f16 tiles would park, not the six digits).
+# there, and the padding nibbles are 15: what a kernel reads without having written it shows.  (At k = 5120 the rows go in two halves
+# where the workspace cannot grow: test_gpu_workspace_room.py.)
 @pytest.mark.parametrize("k,g,taken", [(4096, 128, True), (5120, 128, True), (7000, 192, True), (11008, 64, True), (16384, 128, True), (16320, 192, True),
                                        (16384, 192, False), (16384, 384, False), (16136, 384, False), (14336, 6144, False), (9224, 9216, False)])
 def test_long_rows(ops, k, g, taken):

@@ -1,7 +1,7 @@
 """Calls that are faster with more workspace than they need: what they take, and what they leave alone."""
 import pytest
 
-from gpu_util import say
+from gpu_util import free_workspaces, say
 
 pytestmark = pytest.mark.gpu
 
@@ -20,16 +20,6 @@ def _rows(m, k, seed):
     return torch.empty((m, k), device="cuda").normal_(generator=torch.Generator(device="cuda").manual_seed(seed))
 
 
-def _no_workspaces():
-    """Frees every stream's workspace; the bytes of device memory that came back."""
-    import torch
-    from rumus_amd import _lib
-    torch.cuda.synchronize()
-    before = torch.cuda.mem_get_info()[0]
-    _lib.call("rumus_hip_shutdown")
-    return torch.cuda.mem_get_info()[0] - before
-
-
 # digits of all rows at once (4.6 bytes per element) are more than the documented size for 385 x 3584, and more than the 32 MiB
 # in which the f16 tiles run 1500 x 5120: such calls take their rows in two halves and have no room for codes
 @pytest.mark.parametrize("m,k,n,reserve", [
@@ -41,14 +31,19 @@ def test_reserved_size_is_kept(m, k, n, reserve):
     assert ops.qmatmul_int4_block_takes(m, k, n, 128)
     weight, x, y = _weight(k, n, 128, 1), _rows(m, k, 2), torch.empty((m, n), device="cuda")
     want = ops.qmatmul_int4(x, *weight, k, 128)
-    _no_workspaces()
+    # and with a block's operators around it, which have to find the second half's rows of the gate, the values and the residual
+    gate, res, z = _rows(m, 2 * k, 3), _rows(m, n, 4), torch.empty_like(y)
+    folded = lambda out: ops.qmatmul_int4_block(gate, *weight, k, 128, swiglu=True, residual=res, out=out)
+    want_folded = folded(None)
+    free_workspaces()
     stream = torch.cuda.Stream()
     _lib.call("rumus_hip_workspace_reserve", stream.cuda_stream, reserve)
     with torch.cuda.stream(stream):
         ops.qmatmul_int4(x, *weight, k, 128, out=y)
+        folded(z)
     stream.synchronize()
-    assert torch.equal(y, want)
-    assert _no_workspaces() <= reserve + 2 * MIB                 # whole MiB; the codes alone are 15 MB and more
+    assert torch.equal(y, want) and torch.equal(z, want_folded)
+    assert free_workspaces() <= reserve + 2 * MIB                 # whole MiB; the codes alone are 15 MB and more
 
 
 def test_a_graph_keeps_its_workspace():
@@ -60,7 +55,7 @@ def test_a_graph_keeps_its_workspace():
     small, large = _weight(k, 4096, 128, 1), _weight(k, 11008, 128, 2)
     x, other = _rows(1500, k, 3), _rows(1200, k, 4)
     want, beside = ops.qmatmul_int4(x, *small, k, 128), ops.qmatmul_int4(other, *large, k, 128)
-    _no_workspaces()
+    free_workspaces()
     stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
     y, got = torch.empty_like(want), torch.empty_like(beside)
     torch.cuda.synchronize()
@@ -78,7 +73,7 @@ def test_a_graph_keeps_its_workspace():
     torch.cuda.synchronize()
     assert torch.equal(y, want)
     # digits and sums of 1500 rows, 29 MB, with the codes of 4096 columns, 13 MB; what the other call would like is 58 MB
-    assert _no_workspaces() <= 44 * MIB
+    assert free_workspaces() <= 44 * MIB
 
 
 def test_growing_beside_a_capture():
@@ -90,7 +85,7 @@ def test_growing_beside_a_capture():
     small, large = _weight(k, 4096, 128, 1), _weight(k, 11008, 128, 2)
     x, other = _rows(1500, k, 3), _rows(1200, k, 4)
     beside = ops.qmatmul_int4(other, *large, k, 128)
-    _no_workspaces()
+    free_workspaces()
     stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
     got, doubled = torch.empty_like(beside), torch.empty_like(x)
     torch.cuda.synchronize()
@@ -108,7 +103,7 @@ def test_growing_beside_a_capture():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(doubled, 2.0 * x)
-    assert _no_workspaces() >= 50 * MIB                          # digits of 1200 rows, 24 MB, and the codes, 34 MB
+    assert free_workspaces() >= 50 * MIB                          # digits of 1200 rows, 24 MB, and the codes, 34 MB
 
 
 def _captured_in(reserve, call, outs):
