@@ -74,10 +74,12 @@ int rumus_hip_sync(rumus_hip_stream_t stream);
  *       sums, only while the output has fewer than 192 tiles of 64 x 512) + 1280
  *       (the last kilobyte: flags of the look at the zero-point table).  Large
  *       batches take up to 3/4 of a byte per weight more, at most 256 MiB, where
- *       the workspace has room for it or can grow (not while capturing, not once a
- *       graph was captured with it, and not beyond a size reserved here): the
- *       weights as the matrix cores read them, converted once per call instead of
- *       once per 128 rows.  Same bits without;
+ *       the workspace has room for it or can grow (not while capturing, and not
+ *       beyond a size reserved here; what it had before stays allocated until
+ *       rumus_hip_shutdown, for graphs that were captured with it, and beyond
+ *       256 MiB of that it grows no more): the weights as the matrix cores read
+ *       them, converted once per call instead of once per 128 rows.  Same bits
+ *       without;
  *       to reserve for it: 3 * (padded_k + 64) * (n + 512) / 4 on top;
  *   qmatmul_int4_t, m >= 8: 64 * m * k (partial sums, only below 512 tiles of
  *       64 x 128; 32 * m * k do from 65 rows on where there is no room for more,

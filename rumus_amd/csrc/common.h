@@ -35,9 +35,9 @@ class WorkspaceLease {
 // stream's workspace lock.
 int workspace_get(hipStream_t stream, size_t bytes, void** out, WorkspaceLease& lease);
 // The same for a call that needs `least` bytes and is faster with `want`; `*got` is which of the two it has.  `want` is had where the
-// bytes are there already, or where the workspace may grow for speed alone: not while the stream is being captured, not under a
-// graph that was captured with it (growing frees what the graph's kernels use), not beyond a size of `least` or more that the caller
-// set (rumus_hip_workspace_reserve), and not when the memory cannot be had.
+// bytes are there already, or where the workspace may grow for speed alone: not while the stream is being captured, not beyond a
+// size of `least` or more that the caller set (rumus_hip_workspace_reserve), and not when the memory cannot be had.  What graphs may
+// have been captured with then stays allocated beside the new memory.
 int workspace_get_upto(hipStream_t stream, size_t least, size_t want, size_t* got, void** out, WorkspaceLease& lease);
 // A second buffer per (device, stream), for entry points that wrap another entry point between two conversions
 // (the half-precision ones): what they stage must outlive the inner call, whose workspace may grow - that is, be

@@ -5,6 +5,7 @@
 
 #include <mutex>
 #include <unordered_map>
+#include <vector>
 
 #include "common.h"
 
@@ -35,7 +36,8 @@ struct Arena {
     void* ptr = nullptr;
     size_t bytes = 0;
     bool reserved = false;           // the caller set the size
-    bool in_graph = false;           // it was handed out under a capture: a graph's kernels may use it
+    std::vector<void*> kept;         // smaller ones before it, where it grew for speed alone: a graph's kernels may use them
+    size_t kept_bytes = 0;
     std::recursive_mutex in_use;     // held by a WorkspaceLease
 };
 struct ArenaKey {
@@ -104,18 +106,43 @@ static int workspace_reserve(hipStream_t stream, size_t bytes, void** out, Works
     return rc;
 }
 
+static size_t whole_mib(size_t bytes) { return (bytes + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1); }
+
 static int arena_grow(Arena& a, hipStream_t stream, size_t bytes) {
     if (a.ptr) {
         if (int rc = check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize")) return rc;
         if (int rc = check_hip(hipFree(a.ptr), "hipFree(workspace)")) return rc;
         a.ptr = nullptr;
         a.bytes = 0;
-        a.in_graph = false;
     }
-    const size_t want = (bytes + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);   // whole MiB
+    const size_t want = whole_mib(bytes);
     if (int rc = check_hip(hipMalloc(&a.ptr, want), "hipMalloc(workspace)")) return rc;
     a.bytes = want;
     return RUMUS_HIP_OK;
+}
+
+// Growing for speed alone: graphs that were captured with the old memory have to go on running, so it is kept, up to kMostKept a
+// stream.  (The null stream cannot be captured.  Asking the runtime in every call whether it is being captured, to free what no
+// graph uses, costs 0.15 us of a call.)
+constexpr size_t kMostKept = size_t(256) << 20;
+static bool arena_grow_beside(Arena& a, hipStream_t stream, size_t bytes) {
+    if (stream && a.kept_bytes + a.bytes > kMostKept) return false;
+    const RelaxedCapture relaxed;
+    void* ptr = nullptr;
+    if (hipMalloc(&ptr, whole_mib(bytes)) != hipSuccess) {
+        (void)hipGetLastError();                             // the memory is not there
+        return false;
+    }
+    if (a.ptr && stream) {
+        a.kept.push_back(a.ptr);
+        a.kept_bytes += a.bytes;
+    } else if (a.ptr) {
+        (void)hipStreamSynchronize(stream);
+        (void)hipFree(a.ptr);
+    }
+    a.ptr = ptr;
+    a.bytes = whole_mib(bytes);
+    return true;
 }
 
 int workspace_get_upto(hipStream_t stream, size_t least, size_t want, size_t* got, void** out, WorkspaceLease& lease) {
@@ -125,16 +152,14 @@ int workspace_get_upto(hipStream_t stream, size_t least, size_t want, size_t* go
     std::lock_guard<std::recursive_mutex> lock(a.in_use);
     *got = want;
     if ((g_fixed_ptr ? g_fixed_bytes : a.bytes) < g_nest_offset + want) {
-        const bool grows = !g_fixed_ptr && !g_nest_offset && !(a.reserved && a.bytes >= least) && !a.in_graph && !is_capturing(stream);
-        auto grow = [&] {
-            if (a.bytes < least) return arena_grow(a, stream, want);
-            const RelaxedCapture relaxed;
-            return arena_grow(a, stream, want);
-        };
-        if (!grows || grow() != RUMUS_HIP_OK) {
-            if (grows) (void)hipGetLastError();              // the memory was not there
-            *got = least;
+        bool grown = false;
+        if (g_fixed_ptr || g_nest_offset || is_capturing(stream)) {
+        } else if (a.bytes >= least) {
+            grown = !a.reserved && arena_grow_beside(a, stream, want);
+        } else if (!(grown = arena_grow(a, stream, want) == RUMUS_HIP_OK)) {
+            (void)hipGetLastError();                         // the memory is not there
         }
+        if (!grown) *got = least;
     }
     return arena_get(0, stream, *got, out, lease);
 }
@@ -174,7 +199,6 @@ int arena_get(int kind, hipStream_t stream, size_t bytes, void** out, WorkspaceL
                              kind ? "rumus_hip_f16_staging_reserve" : "rumus_hip_workspace_reserve");
         if (int rc = arena_grow(a, stream, bytes)) return rc;
     }
-    if (bytes && !a.in_graph) a.in_graph = is_capturing(stream);
     *out = a.ptr;
     return RUMUS_HIP_OK;
 }
@@ -183,11 +207,13 @@ static int workspace_release_all() {
     std::lock_guard<std::mutex> lock(g_arena_mutex);
     int rc = RUMUS_HIP_OK;
     for (auto& kv : g_arenas) {
-        if (!kv.second.ptr) continue;
+        if (!kv.second.ptr && kv.second.kept.empty()) continue;
         int cur = 0;
         (void)hipGetDevice(&cur);
         (void)hipSetDevice(kv.first.device);
-        if (int e = check_hip(hipFree(kv.second.ptr), "hipFree(workspace)")) rc = e;
+        kv.second.kept.push_back(kv.second.ptr);
+        for (void* ptr : kv.second.kept)
+            if (int e = check_hip(hipFree(ptr), "hipFree(workspace)")) rc = e;
         (void)hipSetDevice(cur);
     }
     g_arenas.clear();

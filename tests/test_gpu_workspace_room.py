@@ -43,11 +43,11 @@ def test_reserved_size_is_kept(m, k, n, reserve):
         folded(z)
     stream.synchronize()
     assert torch.equal(y, want) and torch.equal(z, want_folded)
-    assert free_workspaces() <= reserve + 2 * MIB                 # whole MiB; the codes alone are 15 MB and more
+    assert free_workspaces() <= reserve + 4 * MIB                 # (memory comes in 2 MiB, give or take as much); the codes are 15 MB and more
 
 
 def test_a_graph_keeps_its_workspace():
-    """A call on a stream whose workspace a graph uses does without room that it could have: growing would free the graph's memory."""
+    """A call that lets the workspace grow for speed leaves the memory of a graph that was captured on the stream before."""
     import torch
     from rumus_amd import ops
     k = 4096
@@ -68,12 +68,36 @@ def test_a_graph_keeps_its_workspace():
         ops.qmatmul_int4(other, *large, k, 128, out=got)
     stream.synchronize()
     assert torch.equal(got, beside)
-    y.zero_()
-    graph.replay()
-    torch.cuda.synchronize()
-    assert torch.equal(y, want)
-    # digits and sums of 1500 rows, 29 MB, with the codes of 4096 columns, 13 MB; what the other call would like is 58 MB
-    assert free_workspaces() <= 44 * MIB
+    for _ in range(2):
+        y.zero_()
+        graph.replay()
+        with torch.cuda.stream(stream):
+            got.zero_()
+            ops.qmatmul_int4(other, *large, k, 128, out=got)
+        torch.cuda.synchronize()
+        assert torch.equal(y, want) and torch.equal(got, beside)
+    # 1500 rows: digits and sums, 29 MB, and the codes of 4096 columns, 13 MB; beside that 23 MB and 34 MB for the other call
+    assert free_workspaces() >= 92 * MIB
+
+
+def test_growing_for_speed_is_bounded():
+    """Streams do not keep more than 256 MiB of earlier workspaces: then a call does without."""
+    import torch
+    from rumus_amd import ops
+    m, k = 8192, 4096
+    say("qmatmul_int4 8192 x 4096 -> 4096 and on to 14336 columns on one stream")
+    x = _rows(m, k, 3)
+    stream = torch.cuda.Stream()
+    weights = [_weight(k, n, 128, n) for n in (4096, 8192, 11008, 14336)]
+    want = [ops.qmatmul_int4(x, *w, k, 128) for w in weights]
+    free_workspaces()
+    for w, y in zip(weights, want):
+        with torch.cuda.stream(stream):
+            got = ops.qmatmul_int4(x, *w, k, 128)
+        stream.synchronize()
+        assert torch.equal(got, y)
+    # digits and sums take 147 MiB, the codes 12, 24, 32 and 42: the first growth keeps 160 MiB beside 172, a second would keep 332
+    assert 320 * MIB <= free_workspaces() <= 356 * MIB
 
 
 def test_growing_beside_a_capture():
