@@ -520,7 +520,12 @@ static I8Choice i8_choose(uint32_t m, uint32_t k, uint32_t n) {
     // shared has, and the more steps it takes until that pays (whole layer, register-staged -> this, us: 60 x 10000 x 1024 82 -> 20, 10 x 6000 x 4096
     // 50 -> 17, 64 x 1552 x 1504 16.2 -> 13.5, 64 x 1040 x 4000 12.3 -> 13.6; 100 x 2032 x 3000 20.6 -> 16.8, 128 x 1040 x 4000 12.5 -> 15.0; 2000 x 4016 x
     // 11008 194 -> 183, 1000 x 2512 x 1500 30.1 -> 28.4, 512 x 1808 x 2000 21.3 -> 21.6, 700 x 1040 x 1000 15.4 -> 16.6).
-    const bool staged = k >= (m <= 64 ? 1408 : m <= 128 ? 1792 : 2048);
+    // Up to 64 rows, outputs of 64 x 11008 and more have that many partial sums that they come earlier only from 1744 on
+    // (weights from HBM, us: 64 x 1424 x 11008 18.5 -> 20.9, x 1680 21.4 -> 22.3, 64 x 1424 x 16384 19.1 -> 23.8, 56 x 1808 x 16384 24.9 -> 23.1,
+    // 48 x 1424 x 11008 20.1 -> 18.7).  All of this holds for weights from HBM, one layer after another (385 shapes of 9 to 512 rows, 1424 to 6000
+    // x 1000 to 16384: 1.5 times as fast on average, none 3 % slower); with one weight that stays in the caches the
+    // register-staged tiles would keep 70 of them, 64 x 1808 x 4000 10.5 -> 12.6, 128 x 2064 x 4000 11.9 -> 16.9.
+    const bool staged = k >= (m <= 64 ? (uint64_t)m * n < 690000 ? 1408 : 1744 : m <= 128 ? 1792 : 2048);
     if (big >= 256 && staged && k % kBK != 0) return {I8Route::Dma256, 0, 0};
     if (big >= 256 && k % kBK == 0) {
         // Workgroups of the large tiles run one per CU, in rounds of 256 that last the same full or not, so the

@@ -8,6 +8,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("m,k,n", [
     (9, 1424, 100), (32, 1568, 1000), (100, 1840, 64), (60, 4144, 520),    # one-wave tiles, whole K and K in shares
+    (64, 1728, 11008), (64, 1744, 11008), (64, 1728, 10752),               # to either side of the line for large outputs
     (130, 2064, 300), (300, 4128, 260), (257, 2096, 1000),                 # 128 x 128 tiles, the same
     (4096, 2064, 4100), (4090, 2080, 4224), (4096, 2096, 4128),            # 256 x 128 tiles
     (33, 1008, 70), (9, 1040, 100), (100, 1072, 64), (300, 1552, 200), (300, 80, 200), (2048, 208, 2304)])                    # shorter: register-staged tiles
