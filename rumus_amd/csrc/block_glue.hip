@@ -123,7 +123,7 @@ constexpr int kHeadDim = 128;
 // More than one query (prompts, and queries behind a cache): f32 attention on the bf16 matrix cores.
 // v_mfma_f32_32x32x16_bf16 does 16 times the work of v_mfma_f32_32x32x2_f32 in half its time, so every f32 operand enters
 // as three bf16 parts, x = x0 + x1 + x2 (each rounded to nearest from what the one before left: 24 bits, all of x), and a
-// product as the six of the nine part products that reach 2^-24 of it; x1 y2, x2 y1 and x2 y2 are below 2^-26.
+// product as six of the nine part products; x1 y2 and x2 y1, which are left out, are up to 2^-25 of it each, 2^-28 in the mean.
 // Workgroup = 128 query rows of one (batch, head), 32 per wave; K/V tiles of 32 keys are split by all of its threads and go
 // through LDS.  Everything is computed transposed so that no fragment ever has to be re-laid out:
 //   S^T = K Q^T   rows = keys (A operand, from LDS), columns = queries (B operand: the parts of the wave's Q rows, kept in
@@ -133,10 +133,10 @@ constexpr int kHeadDim = 128;
 //                 8 s .. 8 s + 7 of S^T, split, are the B operand of step s.
 // Causal: query row i sits at position kv_len - q_len + i and sees keys up to its position.
 // Bound by the matrix cores' power: without a mask, 8 x 32 heads x 512 rows, the six products run at 0.93 PFLOP/s (an 8192^3 bf16
-// product 1.29).  f32 matrix cores (32 rows at a time; fewer than 64 rows on the vector units) -> this, us: 8 x 32 heads x 512 causal
-// 207 -> 149, without mask 309 -> 221, 2 x 16 x 1377 causal 252 -> 162, 8 x 32 x 63 30 -> 13, 32 heads, 16 rows behind 2048 keys
-// 762 -> 194.  Error against float64, as a share of the result: 512 causal rows 3.3e-7 -> 1.9e-7, operands four times as large
-// 1.7e-6 -> 0.6e-6, 4096 keys 1.2e-6 -> 1.0e-6.
+// product 1.29).  f32 matrix cores (32 rows at a time; fewer than 64 rows on the vector units) -> this, one box in turn, us: 8 x 32 heads x 512
+// causal 183 -> 124, without mask 296 -> 202, 2 x 16 x 1377 causal 250 -> 149, 8 x 32 x 63 29.3 -> 12.4, 32 heads, 16 rows behind 2048
+// keys 776 -> 199, 32 heads x 4096 causal 1194 -> 760; 1 to 3 % of that is the look for operands without parts (below).  Error against float64, as a
+// share of the result: 512 causal rows 3.3e-7 -> 1.9e-7, operands four times as large 1.7e-6 -> 0.6e-6, 4096 keys 1.2e-6 -> 1.0e-6.
 // Measured slower: the split of the next tile between the MFMAs of this one (150 -> 170 us, registers), fragments read
 // ahead of their step (171), one sum for all six products of S (error 2.9e-7).
 typedef float attn_v16f __attribute__((ext_vector_type(16)));

@@ -753,8 +753,9 @@ static int launch_q8_gemm_tall_f16(const _Float16* planes, const float* sx, cons
 
 // More than 64 rows and k % 64 == 0, where the estimate of the 128 x 128 tiles (a round of 256 workgroups takes 0.95 to 1.15
 // us per 64 k, by how full it is) is below that of the 64 x 128 ones (a round of 512 takes 1.5 us per 64 k, up to 256 alone
-// 1.06; few of them share K and add up).  Both measured over 180 products of 65 to 2048 rows, blocks of 32 and 128: the
-// choice is 0.03 % off the better one on average and 2 % at worst, and where it takes these tiles they are 1.1 to 1.4 times
+// 1.06; few of them share K and add up).  Both measured over 180 products of 65 to 2048 rows, K and N of 768 to 11008, blocks of 32 and
+// 128: the choice is 0.6 % off the better one on average and 9 % at worst (384 x 768 x 3072: 18.8 us here, 17.3 on the others, whose shares
+// of K have become more even since the estimate was fitted), and where it takes these tiles they are 1.1 to 1.4 times
 // as fast (1000 x 4096 x 4096, blocks of 128: 103 -> 80 us; 2048 x 4096 x 11008, blocks of 128 558 -> 433, of 32 582 -> 478).
 bool q8_gemm_tall(uint32_t m, uint32_t k, uint32_t n, uint32_t bs, uint32_t stride, uint32_t bpc, uint32_t max_shares) {
     if (!(m > 64 && k % 64 == 0 && (bs == 32 || bs % 64 == 0) && (uint64_t)n * bpc * stride * 4 < (1ull << 32))) return false;

@@ -1235,7 +1235,9 @@ bool w4_gemm_f6_chosen(const W4Args& a) {
           (uint64_t)a.padded_k / 8 * a.n * 4 < (1ull << 32) && (uint64_t)a.m * a.n < (1ull << 32)))
         return false;
     double other = 0.0;
-    const double us = f6_plan(a.m, a.k, a.n, false).us;    // (whether there is room for the codes must not change a call's bits)
+    // (the time without codes, for every call: whether there is room for them must not change the kernel, that is the bits.  With
+    // them it is 6 to 10 % less, so where it is close the call goes to a slower kernel.)
+    const double us = f6_plan(a.m, a.k, a.n, false).us;
     const bool i8 = w4_gemm_i8_supported(a, &other);
     // what the integer kernel runs within the fixed scratch array (w4_gemv.hip), 3.1 bytes per element of x, has to go on running there
     if (i8 && !f6_array_fits(a.m, a.padded_k)) return false;
