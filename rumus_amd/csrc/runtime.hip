@@ -122,8 +122,8 @@ static int arena_grow(Arena& a, hipStream_t stream, size_t bytes) {
 }
 
 // Growing for speed alone: graphs that were captured with the old memory have to go on running, so it is kept, up to kMostKept a
-// stream.  (The null stream cannot be captured.  Asking the runtime in every call whether it is being captured, to free what no
-// graph uses, costs 0.15 us of a call.)
+// stream.  (The null stream cannot be captured.  Which memory a graph uses could only be known by asking in every call whether its
+// stream is being captured.)
 constexpr size_t kMostKept = size_t(256) << 20;
 static bool arena_grow_beside(Arena& a, hipStream_t stream, size_t bytes) {
     if (stream && a.kept_bytes + a.bytes > kMostKept) return false;
