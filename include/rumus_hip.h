@@ -252,14 +252,15 @@ int rumus_hip_f16_to_f32(const uint16_t* in, float* out, uint64_t numel,
  * any magnitude; a NaN or an infinity in x poisons its own row only.  Up to
  * 128 rows (up to 1024 where the integer matrix-core kernel is the faster one:
  * group_size % 64 == 0 and enough columns to fill the chip) x is held in fixed
- * point below the largest magnitude of a part of the row (20 bits per 32 k up
- * to decode_max_rows rows, 22 bits per eighth of K beyond):
- * |error| <= max|x| * 2^-19 * sum|w| over that part.  Elements
- * that tower over their part by 2^8 or more are multiplied in f32 on their
- * own (all of a chunk of 32 k in the few-row kernel; up to 16 elements per
- * row and eighth of K beyond), so single outlier channels of thousands of
- * sigma keep the tolerance.  The u4-zero-point decode entry point
- * (rumus_hip_qmatmul_int4_decode_zp4) does not make that exception and keeps
+ * point below the largest magnitude of a part of the row (20 bits per 32 k for
+ * one row, or two of a long K; 21 bits per 128 or 256 k up to decode_max_rows
+ * rows, 22 bits per eighth of K beyond):
+ * |error| <= max|x| * 2^-19 * sum|w| over that part.  Where elements
+ * tower over their part by 2^8 or more the small ones keep their bits (in the
+ * few-row kernels all of that part, in f32 or in further digits; beyond, up to 16
+ * towering elements per row and eighth of K are multiplied on their own), so single outlier channels of thousands of
+ * sigma keep the tolerance.  One or two rows on u4 zero-points
+ * (rumus_hip_qmatmul_int4_decode_zp4) do not make that exception and keep
  * the plain bound.  Batches of more than 256 rows that the six-bit-float
  * kernel takes (group_size % 64 == 0, k from 1024, padded_k to 16384, where it is the faster one)
  * keep 29 bits below the largest of 32 consecutive k, and 39 where a
@@ -388,6 +389,8 @@ int rumus_hip_qmatmul_int4_decode(const float* x, const uint32_t* packed_t,
  * rumus_hip_qmatmul_int4 takes the matrix cores).  The dispatch inside
  * rumus_hip_qmatmul_int4 uses the same number.  No counterpart in the reference. */
 uint32_t rumus_hip_qmatmul_int4_decode_max_rows(uint32_t padded_k, uint32_t n);
+/* the same for act-order weights (a `perm`): as many rows as the kernel gathers in one launch */
+uint32_t rumus_hip_qmatmul_int4_decode_max_rows_perm(uint32_t padded_k, uint32_t n);
 
 /* EXTENSION: the decode layout and its matmul for AWQ storage (u4 zero-points,
  * rumus_hip_w4_quantize_pack_awq): packed_t and scales_t as in

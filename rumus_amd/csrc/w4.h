@@ -68,18 +68,24 @@ int w4_launch_generic(const W4Args& a, hipStream_t s);
 bool w4_gemv_supported(const W4Args& a);
 int w4_launch_gemv(const W4Args& a, hipStream_t s);
 
-// Decode kernel on v_dot8_u32_u4 (m <= 8, group_size % 64 == 0, n % 4 == 0,
+// Decode kernels (m <= 8, group_size % 32 == 0, n % 4 == 0,
 // 16-byte aligned buffers, no g_idx); preferred over the f32 bandwidth kernel.
 bool w4_gemv_dot8_supported(const W4Args& a);
 int w4_launch_gemv_dot8(const W4Args& a, hipStream_t s);
 // the decoder block's forms (decode layout, f32 zero-points, no perm): input through RMSNorm with `norm_w` (or null),
 // or through SwiGLU (a.glu), `resid` (or null) added to the result
 int w4_launch_gemv_dot8_block(const W4Args& a, const float* norm_w, float eps, const float* resid, hipStream_t s);
+// the same calls for 2 to 8 rows, on the int8 matrix cores (w4_gemv_mfma.hip); f16 rows too (x16, y16: 8-byte aligned, k % 4 == 0, no perm)
+bool w4_gemv_mfma_reaches(const W4Args& a);
+// a few rows in f16 (x16, y16) by the kernels that take them in f32, row-major arrays
+bool w4_gemv_half_takes(const W4Args& a);
+int w4_launch_gemv_half(const W4Args& a, hipStream_t s);
+int w4_launch_gemv_mfma(const W4Args& a, const float* norm_w, float eps, const float* resid, hipStream_t s);
 
 // f16 MFMA kernel for larger m (needs group_size 32, 64 or a multiple of 128,
 // n % 4 == 0, 16-byte aligned buffers, no g_idx).
 bool w4_gemm_supported(const W4Args& a);
-uint32_t w4_decode_max_rows(uint32_t padded_k, uint32_t n);   // w4_gemv.hip
+uint32_t w4_decode_max_rows(uint32_t padded_k, uint32_t n, bool perm);   // w4_gemv.hip
 int w4_launch_gemm(const W4Args& a, hipStream_t s);
 
 // int8 matrix cores for up to 128 rows (w4_gemm_i8.hip): group_size % 64 == 0, n % 4 == 0, 16-byte aligned

@@ -400,28 +400,26 @@ static int validate(const W4Args& a, const char* who) {
     return RUMUS_HIP_OK;
 }
 
-// Rows of x up to which the decode kernels beat the matrix-core kernel.  Measured on 4096 x 4096
-// and 4096 x 11008 (g128): a decode launch costs 2.5 + 0.82 W us for one row and 0.45 W us per
-// further row, W = millions of packed words; the matrix-core kernel 8.8 + 0.94 W us for any m up
-// to 32.  The crossing is at 7 rows for 4096 x 4096 and 3 rows for 4096 x 11008; the decode
-// kernels take at most 8.
-uint32_t w4_decode_max_rows(uint32_t padded_k, uint32_t n) {
+// Rows of x up to which the decode kernels beat the two launches of the integer kernel (g128, from HBM, us, decode kernel / integer kernel):
+// 4 rows 4096 x 12288 12.2 / 14.4, 4096 x 22016 18.4 / 23.4, 11008 x 4096 11.1 / 17.8; 8 rows 4096 x 4096 7.6 / 9.2, 11008 x 4096 17.7 / 17.8, 4096 x
+// 12288 17.6 / 14.4: eight up to four million packed words, four beyond.  Act-order rows wait in LDS beside their digits, 128 KB in all, and
+// a call whose rows do not fit takes them in parts, a launch each (8 x 4096 x 4096 17.1 / 10.9): as many as fit at once.
+uint32_t w4_decode_max_rows(uint32_t padded_k, uint32_t n, bool perm) {
     const double mw = (double)(padded_k / 8) * n * 1e-6;
-    if (mw <= 0.0) return 8;
-    const double rows = 1.27 + 14.0 / mw;
-    return rows >= 8.0 ? 8u : rows < 1.0 ? 1u : (uint32_t)rows;
+    if (perm && padded_k > 2048) return padded_k <= 4096 ? 4 : 2;
+    return mw <= 4.0 ? 8 : 4;
 }
 
 bool w4_routes_to_i8(const W4Args& a) {
     if (a.m == 0 || a.n == 0 || a.k == 0) return false;
-    const bool few_rows = a.m <= w4_decode_max_rows(a.padded_k, a.n) || !w4_gemm_supported(a);
+    const bool few_rows = a.m <= w4_decode_max_rows(a.padded_k, a.n, a.perm) || !w4_gemm_supported(a);
     return !(few_rows && (w4_gemv_dot8_supported(a) || w4_gemv_supported(a))) && !w4_gemm_f6_chosen(a) && w4_gemm_i8_supported(a);
 }
 
 static int dispatch(const W4Args& a, hipStream_t s) {
     if (a.m == 0 || a.n == 0) return RUMUS_HIP_OK;
     RUMUS_REQUIRE(a.k > 0, "qmatmul_int4: k must be > 0");
-    const bool few_rows = a.m <= w4_decode_max_rows(a.padded_k, a.n) || !w4_gemm_supported(a);
+    const bool few_rows = a.m <= w4_decode_max_rows(a.padded_k, a.n, a.perm) || !w4_gemm_supported(a);
     if (few_rows && w4_gemv_dot8_supported(a)) return w4_launch_gemv_dot8(a, s);
     if (few_rows && w4_gemv_supported(a)) return w4_launch_gemv(a, s);
     if (w4_gemm_f6_chosen(a)) return w4_launch_gemm_f6(a, s);
@@ -495,8 +493,8 @@ int rumus_hip_qmatmul_int4(const float* x, const uint32_t* packed, const float* 
 int rumus_hip_qmatmul_int4_f16(const uint16_t* x, const uint32_t* packed, const float* scales, const float* zero_points,
                                const float* bias, const int32_t* g_idx, uint16_t* y, uint32_t m, uint32_t k, uint32_t n,
                                uint32_t padded_k, uint32_t group_size, uint32_t num_groups, rumus_hip_stream_t stream) {
-    // The integer matrix-core kernel turns every activation into digits and rounds every result once: it reads and writes f16
-    // itself where a f32 call would come to it (8-byte aligned: its stores of four), the same values without a launch on either
+    // The decode kernels and the integer matrix-core kernel turn every activation into digits and round every result once: they read and write f16
+    // themselves where a f32 call would come to them (8-byte aligned: stores of four), the same values without a launch on either
     // side: 100 x 2000 x 1000, groups of 64, 16.0 -> 11.6 us.  Every other kernel gets f32 copies.
     W4Args a{reinterpret_cast<const float*>(x), packed, scales, zero_points, bias, g_idx, nullptr, reinterpret_cast<float*>(y), m, k, n,
              padded_k, group_size, num_groups};
@@ -506,6 +504,7 @@ int rumus_hip_qmatmul_int4_f16(const uint16_t* x, const uint32_t* packed, const 
         a.y16 = reinterpret_cast<_Float16*>(y);
         a.x = nullptr;
         a.y = nullptr;
+        if (m <= w4_decode_max_rows(padded_k, n, false) && w4_gemv_half_takes(a)) return w4_launch_gemv_half(a, as_stream(stream));
         if (w4_routes_to_i8(a)) return w4_launch_gemm_i8(a, as_stream(stream));
     }
     return w4_f16_staged(x, packed, scales, zero_points, bias, g_idx, y, m, k, n, padded_k, group_size, num_groups, stream);
@@ -540,7 +539,11 @@ int rumus_hip_qmatmul_int4_decode(const float* x, const uint32_t* packed_t, cons
 }
 
 uint32_t rumus_hip_qmatmul_int4_decode_max_rows(uint32_t padded_k, uint32_t n) {
-    return w4_decode_max_rows(padded_k, n);
+    return w4_decode_max_rows(padded_k, n, false);
+}
+
+uint32_t rumus_hip_qmatmul_int4_decode_max_rows_perm(uint32_t padded_k, uint32_t n) {
+    return w4_decode_max_rows(padded_k, n, true);
 }
 
 int rumus_hip_qmatmul_int4_decode_zp4(const float* x, const uint32_t* packed_t, const float* scales_t,

@@ -1,4 +1,4 @@
-// INT4 engine: the decode-shape kernel (m <= 8, group_size % (8*OCT) == 0).
+// INT4 engine: the decode-shape kernel for one row, and two of a long K (group_size % (8*OCT) == 0); up to 8 rows go on to w4_gemv_mfma.hip.
 //
 // At 1 x 4096 x 4096 the whole problem is 9.4 MB: the launch lasts a few
 // microseconds and is bound by latencies (dispatch, first byte from HBM) as
@@ -100,9 +100,10 @@ __device__ __forceinline__ float* d8_sq_lds() {
 // the decoder block, in the epilogue.
 // `resid` may be the output itself (each element is read by the thread that then stores it), so neither of the
 // two pointers is declared restrict.
+// HALF (with FASTX): rows and result in f16, rounded once.
 // BLOCK: the kernel looks at norm_w / eps / resid at all; the plain kernels are launched with nulls there and
 // compile to what they were without these arguments.
-template <int M, int T, int OCT, bool FASTX, bool ZP4, bool TILED, bool GLU = false, bool NORM = false, bool BLOCK = false>
+template <int M, int T, int OCT, bool FASTX, bool ZP4, bool TILED, bool GLU = false, bool NORM = false, bool BLOCK = false, bool HALF = false>
 __global__ __launch_bounds__(T) void w4_gemv_dot8_kernel(
     const uint32_t* __restrict__ packed, const float* __restrict__ scales,
     const float* __restrict__ zps, const float* __restrict__ xin, float* yout,
@@ -169,8 +170,16 @@ __global__ __launch_bounds__(T) void w4_gemv_dot8_kernel(
                     const bool in = kt < k;              // k % 8 == 0: all 8 in or out
                     const uint32_t kc = in ? kt : 0;
                     const float* xrow = xin + (uint64_t)m * (GLU ? 2 * k : k) + kc;
-                    float4 lo = *reinterpret_cast<const float4*>(xrow);
-                    float4 hi = *reinterpret_cast<const float4*>(xrow + 4);
+                    float4 lo, hi;
+                    if constexpr (HALF) {
+                        typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+                        const h8 h = *reinterpret_cast<const h8*>(reinterpret_cast<const _Float16*>(xin) + (uint64_t)m * k + kc);
+                        lo = make_float4((float)h[0], (float)h[1], (float)h[2], (float)h[3]);
+                        hi = make_float4((float)h[4], (float)h[5], (float)h[6], (float)h[7]);
+                    } else {
+                        lo = *reinterpret_cast<const float4*>(xrow);
+                        hi = *reinterpret_cast<const float4*>(xrow + 4);
+                    }
                     if (GLU) {
                         const float4 ul = *reinterpret_cast<const float4*>(xrow + k);
                         const float4 uh = *reinterpret_cast<const float4*>(xrow + k + 4);
@@ -366,7 +375,9 @@ __global__ __launch_bounds__(T) void w4_gemv_dot8_kernel(
                         const bool in = kk < k;
                         const uint32_t kc = in ? kk : 0;
                         float xe;
-                        if (FASTX) {
+                        if constexpr (HALF) {
+                            xe = (float)reinterpret_cast<const _Float16*>(xin)[(uint64_t)m * k + kc];
+                        } else if (FASTX) {
                             const float* xrow = xin + (uint64_t)m * (GLU ? 2 * k : k) + kc;
                             xe = xrow[0];
                             if (GLU) xe = silu_mul(xe, xrow[k]);
@@ -426,7 +437,8 @@ __global__ __launch_bounds__(T) void w4_gemv_dot8_kernel(
             if constexpr (BLOCK) {
                 if (resid) v += resid[(uint64_t)m * n + oc];
             }
-            yout[(uint64_t)m * n + oc] = v;
+            if constexpr (HALF) reinterpret_cast<_Float16*>(yout)[(uint64_t)m * n + oc] = (_Float16)v;
+            else yout[(uint64_t)m * n + oc] = v;
         }
     }
 }
@@ -483,18 +495,42 @@ static int launch_m(const W4Args& a, hipStream_t s) {
     return check_launch("w4_gemv_dot8_kernel");
 }
 
-int w4_launch_gemv_dot8(const W4Args& a, hipStream_t s) {
-    switch (a.m) {
-        case 1: return launch_m<1>(a, s);
-        case 2: return launch_m<2>(a, s);
-        case 3: return launch_m<3>(a, s);
-        case 4: return launch_m<4>(a, s);
-        case 5: return launch_m<5>(a, s);
-        case 6: return launch_m<6>(a, s);
-        case 7: return launch_m<7>(a, s);
-        case 8: return launch_m<8>(a, s);
+// Two rows of a plain weight with a long K stay here: the conversion of four rows, half of it for rows that are not there, is longer than two planes.
+// 2 x 2048 x 2048 4.5 us here, 3.7 on the matrix cores; 2 x 6528 x 512 6.8 and 7.2, 2 x 4096 x 12288 10.9 and 12.2.
+static bool w4_two_rows_long(const W4Args& a) { return a.m == 2 && a.padded_k > 2048 && !a.perm; }
+// f16 rows and result, row-major arrays with f32 zero-points: a call that came here in f32, k % 8 == 0 and 16-byte aligned rows
+template <int M>
+static int launch_half_m(const W4Args& a, hipStream_t s) {
+    hipLaunchKernelGGL((w4_gemv_dot8_kernel<M, kD8Threads, kD8Oct, true, false, false, false, false, false, true>), dim3(ceil_div(a.n, kD8Cols)),
+                       dim3(kD8Threads), 0, s, a.packed, a.scales, a.zp, reinterpret_cast<const float*>(a.x16), reinterpret_cast<float*>(a.y16),
+                       a.n, a.k, a.padded_k, a.group_size, a.bias, static_cast<const int32_t*>(nullptr), nullptr, 0.0f, nullptr);
+    return check_launch("w4_gemv_dot8_kernel");
+}
+bool w4_gemv_half_takes(const W4Args& a) {
+    if (a.zp4 || a.tiled || a.perm || a.glu || !w4_gemv_dot8_supported(a) || !w4_gemv_mfma_reaches(a)) return false;
+    return a.m >= 2 && !w4_two_rows_long(a) ? a.k % 4 == 0 : a.m <= 2 && a.k % 8 == 0 && (reinterpret_cast<uintptr_t>(a.x16) & 15) == 0;
+}
+int w4_launch_gemv_half(const W4Args& a, hipStream_t s) {
+    if (a.m >= 2 && !w4_two_rows_long(a)) return w4_launch_gemv_mfma(a, nullptr, 0.0f, nullptr, s);
+    return a.m == 1 ? launch_half_m<1>(a, s) : launch_half_m<2>(a, s);
+}
+
+// one launch for two rows (or one) at a time
+template <typename F>
+static int w4_in_pairs(const W4Args& a, const float* resid, F launch) {
+    for (uint32_t r0 = 0; r0 < a.m; r0 += 2) {
+        W4Args p = a;
+        p.m = min(2u, a.m - r0);
+        p.x = a.x + (uint64_t)r0 * a.k * (a.glu ? 2 : 1);
+        p.y = a.y + (uint64_t)r0 * a.n;
+        if (int rc = launch(p, resid ? resid + (uint64_t)r0 * a.n : nullptr)) return rc;
     }
-    return set_error(RUMUS_HIP_EINVAL, "w4 gemv: m = %u out of range", a.m);
+    return RUMUS_HIP_OK;
+}
+
+int w4_launch_gemv_dot8(const W4Args& a, hipStream_t s) {
+    if (w4_gemv_mfma_reaches(a) && a.m >= 2 && !w4_two_rows_long(a)) return w4_launch_gemv_mfma(a, nullptr, 0.0f, nullptr, s);
+    return w4_in_pairs(a, nullptr, [&](const W4Args& p, const float* r) { return p.m == 1 ? launch_m<1>(p, s) : launch_m<2>(p, s); });
 }
 
 template <int M>
@@ -515,17 +551,8 @@ static int launch_block_m(const W4Args& a, const float* norm_w, float eps, const
 // (a.glu false, norm_w non-null), SwiGLU of gate | up rows (a.glu), or nothing.  The caller has checked the
 // shapes (w4_gemv_dot8_supported, a.tiled, no packed zero-points, no perm, k % 8 == 0, 16-byte aligned x).
 int w4_launch_gemv_dot8_block(const W4Args& a, const float* norm_w, float eps, const float* resid, hipStream_t s) {
-    switch (a.m) {
-        case 1: return launch_block_m<1>(a, norm_w, eps, resid, s);
-        case 2: return launch_block_m<2>(a, norm_w, eps, resid, s);
-        case 3: return launch_block_m<3>(a, norm_w, eps, resid, s);
-        case 4: return launch_block_m<4>(a, norm_w, eps, resid, s);
-        case 5: return launch_block_m<5>(a, norm_w, eps, resid, s);
-        case 6: return launch_block_m<6>(a, norm_w, eps, resid, s);
-        case 7: return launch_block_m<7>(a, norm_w, eps, resid, s);
-        case 8: return launch_block_m<8>(a, norm_w, eps, resid, s);
-    }
-    return set_error(RUMUS_HIP_EINVAL, "w4 gemv: m = %u out of range", a.m);
+    if (w4_gemv_mfma_reaches(a) && a.m >= 2 && !w4_two_rows_long(a)) return w4_launch_gemv_mfma(a, norm_w, eps, resid, s);
+    return w4_in_pairs(a, resid, [&](const W4Args& p, const float* r) { return p.m == 1 ? launch_block_m<1>(p, norm_w, eps, r, s) : launch_block_m<2>(p, norm_w, eps, r, s); });
 }
 
 }  // namespace rumus

@@ -59,7 +59,7 @@ class QuantizedTensor:
             self.decode = ops.w4_decode_layout(packed, scales, zp, group_size)
         # batches up to this many rows take the decode kernel (its cost grows with the rows, the
         # matrix-core kernel's hardly does; the library knows where they cross for this shape)
-        self.decode_rows = ops.qmatmul_int4_decode_max_rows(padded_k, n) if self.decode is not None else 0
+        self.decode_rows = ops.qmatmul_int4_decode_max_rows(padded_k, n, perm is not None) if self.decode is not None else 0
 
     @staticmethod
     def _has_decode_layout(n, group_size) -> bool:

@@ -289,9 +289,10 @@ def qmatmul_int4_decode(x, packed_t, scales_t, zp_t, k, group_size, bias=None, p
     return _w4_call("rumus_hip_qmatmul_int4_decode", x, packed_t, scales_t, zp_t, bias, perm, k, group_size, out)
 
 
-def qmatmul_int4_decode_max_rows(padded_k: int, n: int) -> int:
-    """Rows up to which the decode entry points beat the matrix-core kernel for this weight."""
-    return int(_lib.lib().rumus_hip_qmatmul_int4_decode_max_rows(padded_k, n))
+def qmatmul_int4_decode_max_rows(padded_k: int, n: int, perm: bool = False) -> int:
+    """Rows up to which the decode entry points beat the matrix-core kernel for this weight (``perm``: act-order)."""
+    name = "rumus_hip_qmatmul_int4_decode_max_rows_perm" if perm else "rumus_hip_qmatmul_int4_decode_max_rows"
+    return int(getattr(_lib.lib(), name)(padded_k, n))
 
 
 def w4_decode_layout_zp4(packed, scales, qzeros, group_size):

@@ -1,0 +1,118 @@
+"""INT4 forward for 2 to 8 rows on the int8 matrix cores (``w4_gemv_mfma.hip``): units of 128 and 256 k and their tails, groups of 32, 64 and
+128, column tiles, act-order rows in one launch and in parts, f16 rows, elements far apart in a unit, NaN and infinity.
+
+The bound, against float64: an activation is rounded to 2^-21 of the power of two above its unit's largest magnitude, so an output is off by at
+most max|x| 2^-20 sum|w|; the f32 sums around it lose less than 2^-20 of the summed magnitudes (up to K/128 + 8 additions of 2^-24 each)."""
+import numpy as np
+import pytest
+
+from gpu_util import dev, host, say
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from rumus_amd import ops
+    return ops
+
+
+def weights(rng, k, n, g, zero="float"):
+    packed, scales, zp = oracle.w4_from_f32(rng.normal(0, 0.02, (k, n)).astype(np.float32), g)
+    if zero == "integer":
+        zp = np.clip(np.rint(zp), 0, 15).astype(np.float32)
+    q = oracle.w4_unpack(packed, packed.shape[0] * 8).astype(np.float64)[:k]
+    rows = np.arange(k) // g
+    return packed, scales, zp, (q - zp[rows].astype(np.float64)) * scales[rows].astype(np.float64)
+
+
+def check(got, x, w, largest=None):
+    x = x.astype(np.float64)
+    want = x @ w
+    top = np.abs(x).max(axis=1, keepdims=True) if largest is None else largest
+    bound = 2.0 ** -20 * (top * np.abs(w).sum(axis=0) + np.abs(x) @ np.abs(w))
+    worst = float((np.abs(got - want) / bound).max())
+    assert worst <= 1.0, worst
+
+
+SHAPES = [(2, 32, 16, 32), (3, 96, 20, 32), (8, 160, 48, 32), (2, 1000, 52, 64), (5, 1088, 64, 64), (4, 128, 4, 128), (7, 1152, 36, 128),
+          (2, 2048, 80, 128), (6, 2176, 16, 128), (3, 4096, 64, 256), (8, 4224, 32, 128), (4, 8320, 32, 64), (4, 512, 8192, 128),
+          (8, 300, 8224, 32), (3, 1001, 16, 8 * 32)]
+
+
+@pytest.mark.parametrize("m,k,n,g", SHAPES)
+@pytest.mark.parametrize("tiled", [False, True])
+def test_few_rows_against_float64(ops, m, k, n, g, tiled):
+    if tiled and n % 16:
+        pytest.skip("the decode layout wants whole tiles")
+    say(f"few rows m={m} k={k} n={n} g={g} tiled={tiled}")
+    rng = np.random.default_rng(m * 7 + k + n)
+    packed, scales, zp, w = weights(rng, k, n, g)
+    x = rng.normal(0, 1, (m, k)).astype(np.float32)
+    d = [dev(a) for a in (packed, scales, zp)]
+    if tiled:
+        got = host(ops.qmatmul_int4_decode(dev(x), *ops.w4_decode_layout(*d, g), k, g))
+    else:
+        got = host(ops.qmatmul_int4(dev(x), *d, k, g))
+    check(got, x, w)
+    if not tiled and k % 4 == 0:             # a row does not depend on the others
+        one = host(ops.qmatmul_int4(dev(np.ascontiguousarray(np.concatenate([x[-1:], x[:1] * 3, x[:1]]))), *d, k, g))
+        if k <= 2048 or m > 2:
+            np.testing.assert_array_equal(one[0], got[-1])
+    if not tiled and k % 8 == 0:             # f16 rows: the same kernel, rounded once
+        xh = x.astype(np.float16)
+        f32 = host(ops.qmatmul_int4(dev(xh.astype(np.float32)), *d, k, g))
+        np.testing.assert_array_equal(host(ops.qmatmul_int4_f16(dev(xh), *d, k, g)), f32.astype(np.float16))
+
+
+@pytest.mark.parametrize("m,k", [(2, 256), (8, 2048), (4, 4096), (8, 4096), (3, 8192), (5, 12288), (2, 16384), (2, 32768)])
+def test_act_order_rows_in_parts(ops, m, k):
+    n, g = 48, 128
+    say(f"few rows act-order m={m} k={k}")
+    rng = np.random.default_rng(m + k)
+    packed, scales, zp, w = weights(rng, k, n, g)
+    perm = rng.permutation(k).astype(np.int32)
+    x = rng.normal(0, 1, (m, k)).astype(np.float32)
+    t = ops.w4_decode_layout(dev(packed), dev(scales), dev(zp), g)
+    got = host(ops.qmatmul_int4_decode(dev(x), *t, k, g, perm=dev(perm)))
+    check(got, x[:, perm], w)
+
+
+@pytest.mark.parametrize("m,k,g", [(3, 256, 128), (4, 1000, 64), (8, 4096, 128), (2, 992, 32)])
+@pytest.mark.parametrize("power", [7, 9, 20, 60])
+def test_elements_far_apart(ops, m, k, g, power):
+    """Channels 2^power as large that meet weights of zero: what the others add up to keeps its bits."""
+    say(f"few rows far apart m={m} k={k} g={g} power={power}")
+    n = 32
+    rng = np.random.default_rng(power + k)
+    packed, scales, zp, w = weights(rng, k, n, g, zero="integer")
+    loud = rng.permutation(k)[:max(1, k // 64)]
+    for c in loud:                                          # code = zero-point: a weight of zero
+        z = zp[c // g].astype(np.uint32)
+        shift = np.uint32(4 * (c % 8))
+        packed[c // 8] = (packed[c // 8] & ~(np.uint32(15) << shift)) | (z << shift)
+        w[c] = 0.0
+    x = rng.normal(0, 1, (m, k)).astype(np.float32)
+    x[1, loud] *= np.float32(2.0 ** power)                  # one row: its neighbours stay as they are
+    got = host(ops.qmatmul_int4(dev(x), dev(packed), dev(scales), dev(zp), k, g))
+    # up to 2^8 apart the plain bound; beyond, every element counts with its own bits and only sums round
+    largest = np.abs(x).max(axis=1, keepdims=True).astype(np.float64)
+    largest[1] = min(largest[1], 2.0 ** 10)
+    y = x.copy()
+    y[1, loud] = 0.0
+    check(got, y, w, largest)
+
+
+def test_not_finite_and_tiny(ops):
+    m, k, n, g = 4, 1024, 32, 128
+    rng = np.random.default_rng(5)
+    packed, scales, zp, w = weights(rng, k, n, g)
+    x = rng.normal(0, 1, (m, k)).astype(np.float32)
+    x[1, 77] = np.nan
+    x[2, 1000] = -np.inf
+    x[3] *= np.float32(2.0 ** -100)
+    got = host(ops.qmatmul_int4(dev(x), dev(packed), dev(scales), dev(zp), k, g))
+    assert not np.isfinite(got[1:3]).any()
+    check(got[[0, 3]], x[[0, 3]], w)
