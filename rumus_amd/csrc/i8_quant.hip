@@ -77,6 +77,69 @@ __global__ __launch_bounds__(256) void i8_quantize_rows_kernel(const float* __re
 
 // ---- per-output-channel weights: w[k,n] -> wq[n,k], sw[n] -----------------
 
+// One launch, w read once (n % 4 == 0, k % 4 == 0 up to 12288, 16-byte aligned w, 4-byte aligned wq).  A workgroup owns 4 QUADS columns over
+// all of K: thread = four adjacent columns of four consecutive rows, 4096 / QUADS rows a sweep.  All sweeps stay in registers between
+// the maximum and the digits, all their loads in flight at once.  A thread's four rows are four bytes of a column of wq: a wave
+// stores 64 (QUADS = 4) contiguous bytes of 16 columns, no trip through LDS.
+// What bounds it: HBM in segments of 64 bytes of w (the other half of a line belongs to the neighbour, on the same L2), and one
+// workgroup a compute unit from 3072 rows on, which loads and then stores; a small matrix the launch.
+// The four launches that it stands for (accumulators cleared, maxima per slice of 64 rows with atomics, digits, scales: below, for other
+// shapes) waited for one row after the other and read w twice.  us before -> now, from HBM: 656 x 2560 26.9 -> 11.2 (the call from
+// Python), 2048 x 2048 40.1 -> 11.5, 4096 x 4096 53.9 -> 22.6, 4096 x 11008 98.8 -> 65.5 (3.4 TB/s), 5504 x 11008 120 -> 82.
+// QUADS = 2, beyond 6144 rows, is half of such a segment and twice the rows in the same registers: 8192 x 1024 49.4 -> 30.1, 11008 x 4096 91.7 -> 76.7;
+// with QUADS = 4 and the rest of the rows read twice 44.6 and 86.4.  Up to 6144 rows it is slower (4096 x 4096 33.1, 1024 x 11008 19.8 against
+// 14.8).
+constexpr uint32_t kColsThreads = 1024, kColsMaxK = 12288;
+template <uint32_t QUADS, int SWEEPS>
+__global__ __launch_bounds__(kColsThreads) void quantize_cols_kernel(const float* __restrict__ w, int8_t* __restrict__ wq,
+                                                                     float* __restrict__ sw, uint32_t k, uint32_t n) {
+    constexpr uint32_t kColsRows = kColsThreads * 4 / QUADS;
+    __shared__ float4 red[kColsThreads / kWave][QUADS];
+    const uint32_t tid = threadIdx.x, tx = tid % QUADS, lane = tid & 63;
+    const uint32_t col = xcd_contiguous(blockIdx.x, gridDim.x) * (4 * QUADS) + 4 * tx, from = min(col, n - 4);
+    const uint32_t r0 = tid / QUADS * 4;                               // of a sweep
+    const float* const src = w + from;
+    auto load = [&](uint32_t base, float4 (&v)[4]) {               // rows base + r0 .. + 3; past the end: the last four (k % 4 == 0)
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = *reinterpret_cast<const float4*>(src + (uint64_t)(min(base + r0, k - 4) + i) * n);
+    };
+    auto largest = [](float4& top, const float4& v) {
+        top.x = fmaxf(top.x, fabsf(v.x)); top.y = fmaxf(top.y, fabsf(v.y));
+        top.z = fmaxf(top.z, fabsf(v.z)); top.w = fmaxf(top.w, fabsf(v.w));
+    };
+    float4 cache[SWEEPS][4], top = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int s = 0; s < SWEEPS; s++) load(s * kColsRows, cache[s]);
+#pragma unroll
+    for (int s = 0; s < SWEEPS; s++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) largest(top, cache[s][i]);
+#pragma unroll
+    for (int d = QUADS; d < 64; d *= 2)
+        largest(top, make_float4(__shfl_xor(top.x, d), __shfl_xor(top.y, d), __shfl_xor(top.z, d), __shfl_xor(top.w, d)));
+    if (lane < QUADS) red[tid / kWave][tx] = top;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < kColsThreads / kWave; i++) largest(top, red[i][tx]);
+    if (col >= n) return;
+    auto scale = [](float am) { return am == 0.0f ? 1.0f : __fdiv_rn(am, 127.0f); };
+    auto inverse = [](float am) { return am == 0.0f ? 0.0f : __fdiv_rn(127.0f, am); };
+    if (tid < QUADS) {
+        sw[col] = scale(top.x); sw[col + 1] = scale(top.y); sw[col + 2] = scale(top.z); sw[col + 3] = scale(top.w);
+    }
+    const float4 inv = make_float4(inverse(top.x), inverse(top.y), inverse(top.z), inverse(top.w));
+    auto store = [&](uint32_t base, const float4 (&v)[4]) {
+        if (base + r0 >= k) return;
+        uint32_t* const to = reinterpret_cast<uint32_t*>(wq + (uint64_t)col * k + base + r0);
+        to[0] = pack_i8x4(make_float4(v[0].x, v[1].x, v[2].x, v[3].x), inv.x);
+        to[k / 4] = pack_i8x4(make_float4(v[0].y, v[1].y, v[2].y, v[3].y), inv.y);
+        to[k / 4 * 2] = pack_i8x4(make_float4(v[0].z, v[1].z, v[2].z, v[3].z), inv.z);
+        to[(uint64_t)(k / 4) * 3] = pack_i8x4(make_float4(v[0].w, v[1].w, v[2].w, v[3].w), inv.w);
+    };
+#pragma unroll
+    for (int s = 0; s < SWEEPS; s++) store(s * kColsRows, cache[s]);
+}
+
 __global__ __launch_bounds__(256) void fill_zero_kernel(uint32_t* __restrict__ p, uint32_t n) {
     uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i < n) p[i] = 0u;
@@ -93,7 +156,8 @@ __global__ __launch_bounds__(256) void col_absmax_kernel(const float* __restrict
     const uint32_t k0 = blockIdx.y * kslice, k1 = min(k, k0 + kslice);
     float amax[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (n % 4 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0) {
-        for (uint32_t r = k0; r < k1; r++) {
+#pragma unroll 16
+        for (uint32_t r = k0; r < k1; r++) {          // (sixteen loads in flight)
             const float4 v = *reinterpret_cast<const float4*>(w + (uint64_t)r * n + col);
             amax[0] = fmaxf(amax[0], fabsf(v.x)); amax[1] = fmaxf(amax[1], fabsf(v.y));
             amax[2] = fmaxf(amax[2], fabsf(v.z)); amax[3] = fmaxf(amax[3], fabsf(v.w));
@@ -195,6 +259,19 @@ int rumus_hip_i8_quantize_cols_t(const float* w, int8_t* wq, float* sw, uint32_t
     if (n == 0) return RUMUS_HIP_OK;
     RUMUS_REQUIRE(k > 0, "i8_quantize_cols_t: k must be > 0");
     hipStream_t s = as_stream(stream);
+    if (n % 4 == 0 && k % 4 == 0 && k <= kColsMaxK && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && (reinterpret_cast<uintptr_t>(wq) & 3) == 0) {
+        const dim3 block(kColsThreads);
+#define RUMUS_COLS(QUADS, SWEEPS) \
+    hipLaunchKernelGGL((quantize_cols_kernel<QUADS, SWEEPS>), dim3(ceil_div(n, 4 * QUADS)), block, 0, s, w, wq, sw, k, n)
+        if (k > 8192) RUMUS_COLS(2, 6);
+        else if (k > 6144) RUMUS_COLS(2, 4);
+        else if (k > 4096) RUMUS_COLS(4, 6);
+        else if (k > 2048) RUMUS_COLS(4, 4);
+        else if (k > 1024) RUMUS_COLS(4, 2);
+        else RUMUS_COLS(4, 1);
+#undef RUMUS_COLS
+        return check_launch("quantize_cols_kernel");
+    }
     // sw doubles as the abs-max accumulator until pass 3 turns it into scales.
     hipLaunchKernelGGL(fill_zero_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, s,
                        reinterpret_cast<uint32_t*>(sw), n);

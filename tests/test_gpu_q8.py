@@ -303,13 +303,17 @@ def test_i8_quantize_rows_bit_exact(ops, rows, cols):
     np.testing.assert_array_equal(host(s), ws)
 
 
-@pytest.mark.parametrize("k,n", [(512, 512), (100, 37), (4096, 200), (64, 1), (208, 130), (72, 64), (1024, 2052)])
+@pytest.mark.parametrize("k,n", [(512, 512), (100, 37), (4096, 200), (64, 1), (208, 130), (72, 64), (1024, 2052),
+                                 # one launch, every number of sweeps at its ends, columns past the last tile
+                                 (4, 4), (1024, 16), (1028, 20), (2048, 36), (2052, 12), (4096, 20), (4100, 8), (6144, 28),
+                                 (6148, 4), (8192, 20), (8196, 12), (12288, 28), (12292, 16), (4097, 16)])
 def test_i8_quantize_cols_t_bit_exact(ops, k, n):
     say(f"i8_quantize_cols_t k={k} n={n}")
     rng = np.random.default_rng(k + n)
     w = rng.normal(0, 0.02, (k, n)).astype(np.float32)
     if n > 3:
         w[:, 2] = 0.0
+    w[-1, -1] = -1.0                                    # the largest magnitude in the last row
     want_q, want_s = oracle.i8_quantize_rows(np.ascontiguousarray(w.T))
     wq, sw = ops.i8_quantize_cols_t(dev(w))
     np.testing.assert_array_equal(host(wq), want_q)
