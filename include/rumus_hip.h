@@ -193,6 +193,16 @@ int rumus_hip_i8_gemm(const int8_t* xq, const int8_t* wq, const float* sx,
  * sizes temporaries inside the op, rumus/src/backend/gpu/pool.rs:34-75). */
 uint64_t rumus_hip_i8_gemm_workspace_size(uint32_t m, uint32_t k, uint32_t n);
 
+/* The W8A8 layer in one call: rumus_hip_i8_quantize_rows of x [m,k], then
+ * rumus_hip_i8_gemm, the same bits.  Few rows (16, fewer where k is long) take
+ * one launch and no scratch.  scratch: device memory of
+ * rumus_hip_i8_linear_scratch_size(m, k, n) bytes, 16-byte aligned, written by
+ * the call; NULL where that is 0.  bias may be NULL.  EINVAL unless k % 16 == 0. */
+int rumus_hip_i8_linear(const float* x, const int8_t* wq, const float* sw,
+                        const float* bias, void* scratch, float* y, uint32_t m,
+                        uint32_t k, uint32_t n, rumus_hip_stream_t stream);
+uint64_t rumus_hip_i8_linear_scratch_size(uint32_t m, uint32_t k, uint32_t n);
+
 /* ---- INT4 engine --------------------------------------------------------- */
 
 /* QuantizedTensor::from_f32 (rumus-vision/src/quant.rs:42-102) on the device:

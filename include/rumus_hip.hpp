@@ -341,12 +341,20 @@ struct Int8Linear {
                                 hipStream_t stream = nullptr) const {
         require(in_features && x.size() % in_features == 0, "Int8Linear::forward: x must be [m, in_features]");
         const uint32_t m = (uint32_t)(x.size() / in_features);
+        DeviceBuffer<float> y((size_t)m * out_features);
+        if (!acc) {
+            DeviceBuffer<int8_t> scratch(rumus_hip_i8_linear_scratch_size(m, in_features, out_features));
+            check(rumus_hip_i8_linear(x.data(), wq.data(), sw.data(), bias.size() ? bias.data() : nullptr,
+                                      scratch.size() ? scratch.data() : nullptr, y.data(), m, in_features, out_features, stream));
+            check(rumus_hip_sync(stream));   // scratch is released on return
+            return y;
+        }
         DeviceBuffer<int8_t> xq(x.size());
-        DeviceBuffer<float> sx(m), y((size_t)m * out_features);
+        DeviceBuffer<float> sx(m);
         check(rumus_hip_i8_quantize_rows(x.data(), xq.data(), sx.data(), m, in_features, stream));
-        if (acc) *acc = DeviceBuffer<int32_t>((size_t)m * out_features);
+        *acc = DeviceBuffer<int32_t>((size_t)m * out_features);
         check(rumus_hip_i8_gemm(xq.data(), wq.data(), sx.data(), sw.data(), bias.size() ? bias.data() : nullptr,
-                                acc ? acc->data() : nullptr, y.data(), m, in_features, out_features, stream));
+                                acc->data(), y.data(), m, in_features, out_features, stream));
         check(rumus_hip_sync(stream));   // xq / sx are released on return
         return y;
     }

@@ -225,17 +225,15 @@ PyObject* int8_linear(PyObject*, PyObject* const* a, Py_ssize_t count) {
     RUMUS_PLAIN(x->dim() == 2 && wq->dim() == 2 && x->size(1) == wq->size(1) && fits(x->size(0)) && fits(x->size(1)) && fits(wq->size(0)));
     const uint32_t m = (uint32_t)x->size(0), k = (uint32_t)x->size(1), n = (uint32_t)wq->size(0);
     RUMUS_PLAIN((uint64_t)sw->numel() >= n && plain_or_none(a[3], at::kFloat, n, bias));
-    // rows and their scales in one allocation
-    const int64_t rows = (((int64_t)m * k) + 255) & ~(int64_t)255;
-    const Tensor scratch = make({rows + 4 * (int64_t)m}, *x, at::kChar);
+    const uint64_t bytes = rumus_hip_i8_linear_scratch_size(m, k, n);
+    Tensor scratch;                                            // quantized rows, where they go through memory
+    if (bytes) scratch = make({(int64_t)bytes}, *x, at::kChar);
     const Tensor y = make({m, n}, *x, at::kFloat);
-    int8_t* xq = ptr<int8_t>(&scratch);
-    float* sx = reinterpret_cast<float*>(xq + rows);
+    void* const mem = bytes ? ptr<void>(&scratch) : nullptr;
     void* s = stream();
     const int rc = unlocked([&] {
-        const int quantized = rumus_hip_i8_quantize_rows(ptr<const float>(x), xq, sx, m, k, s);
-        return quantized ? quantized : rumus_hip_i8_gemm(xq, ptr<const int8_t>(wq), sx, ptr<const float>(sw), ptr<const float>(bias),
-                                                         nullptr, ptr<float>(&y), m, k, n, s);
+        return rumus_hip_i8_linear(ptr<const float>(x), ptr<const int8_t>(wq), ptr<const float>(sw), ptr<const float>(bias), mem, ptr<float>(&y), m,
+                                   k, n, s);
     });
     return result(rc, y);
     END_HANDLE_TH_ERRORS

@@ -43,6 +43,7 @@ int i8_launch_gemv(const int8_t* xq, const int8_t* wq, const float* sx, const fl
 
 // 5 to 32 rows, K % 256 == 0: MFMA tiles fed straight from global memory (i8_gemv.hip).
 // 5..64 rows with the activations resident in registers, where i8_resident_takes says so
+uint32_t i8_resident_grid(uint32_t n);
 bool i8_resident_takes(uint32_t m, uint32_t k, uint32_t n);
 int i8_launch_resident(const int8_t* xq, const int8_t* wq, const float* sx, const float* sw, const float* bias, int32_t* acc,
                        float* y, uint32_t m, uint32_t k, uint32_t n, hipStream_t s);
@@ -53,6 +54,17 @@ int i8_launch_stream(const int8_t* xq, const int8_t* wq, const float* sx, const 
 // kQ8TallRows rows, per block and 64 k: [pair of 32 k][hi, lo][row][four 16-byte pieces, swizzled like an LDS row].
 constexpr uint32_t kQ8TallRows = 128;
 bool q8_gemm_tall(uint32_t m, uint32_t k, uint32_t n, uint32_t bs, uint32_t stride, uint32_t bpc, uint32_t max_shares);
+
+// The rule of both W8A8 quantizers (i8_quant.hip)
+__device__ __forceinline__ int q_i8(float v, float inv) {
+    float t = rintf(__fmul_rn(v, inv));
+    return (int)fminf(fmaxf(t, -128.0f), 127.0f);
+}
+
+__device__ __forceinline__ uint32_t pack_i8x4(const float4& v, float inv) {
+    return ((uint32_t)q_i8(v.x, inv) & 0xFFu) | (((uint32_t)q_i8(v.y, inv) & 0xFFu) << 8) |
+           (((uint32_t)q_i8(v.z, inv) & 0xFFu) << 16) | (((uint32_t)q_i8(v.w, inv) & 0xFFu) << 24);
+}
 
 // chunk swizzle of an LDS row: bit0 = b1 ^ b3, bit1 = b2 of the row index
 __device__ __forceinline__ uint32_t row_swizzle(uint32_t row) {

@@ -3,25 +3,15 @@
 // rule (rumus/src/backend/gpu/shaders/quantize.wgsl:66-67,93) with the scale
 // kept in f32: scale = amax/127 (1 if amax == 0), inv = 127/amax (0 if
 // amax == 0), q = clamp(rint(v*inv), -128, 127).
-#include "common.h"
+#include "i8_gemm.h"
 
 namespace rumus {
 
 __device__ __forceinline__ float wave_max64(float v) { return wave_max(v); }
 
-__device__ __forceinline__ int q_i8(float v, float inv) {
-    float t = rintf(__fmul_rn(v, inv));
-    return (int)fminf(fmaxf(t, -128.0f), 127.0f);
-}
-
 // One workgroup per row.  A row of up to 1024 CACHE elements stays in registers between the two
 // passes (all of a thread's loads in flight at once, the row read once: 2048 x 11008 29 -> 18 us);
 // CACHE = 0 or longer rows: read twice (the second read hits L2).
-
-__device__ __forceinline__ uint32_t pack_i8x4(const float4& v, float inv) {
-    return ((uint32_t)q_i8(v.x, inv) & 0xFFu) | (((uint32_t)q_i8(v.y, inv) & 0xFFu) << 8) |
-           (((uint32_t)q_i8(v.z, inv) & 0xFFu) << 16) | (((uint32_t)q_i8(v.w, inv) & 0xFFu) << 24);
-}
 
 template <int CACHE>
 __global__ __launch_bounds__(256) void i8_quantize_rows_kernel(const float* __restrict__ x,

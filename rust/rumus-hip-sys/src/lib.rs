@@ -97,6 +97,9 @@ extern "C" {
                                      s: Stream) -> c_int;
     pub fn rumus_hip_matmul_q8_dense(a: *const f32, wq: *const i8, sw: *const f32, c: *mut f32, m: u32, k: u32,
                                      n: u32, s: Stream) -> c_int;
+    pub fn rumus_hip_i8_linear(x: *const f32, wq: *const i8, sw: *const f32, bias: *const f32, scratch: *mut core::ffi::c_void,
+                               y: *mut f32, m: u32, k: u32, n: u32, s: Stream) -> c_int;
+    pub fn rumus_hip_i8_linear_scratch_size(m: u32, k: u32, n: u32) -> u64;
     pub fn rumus_hip_i8_gemm_workspace_size(m: u32, k: u32, n: u32) -> u64;
     pub fn rumus_hip_qmatmul_int4_perm_static(x: *const f32, packed_sorted: *const u32, scales: *const f32,
                                               zp: *const f32, bias: *const f32, perm: *const i32, y: *mut f32,

@@ -104,6 +104,10 @@ def test_empty_calls_succeed_without_arrays_and_full_ones_need_them(library):
     assert L.rumus_hip_i8_quantize_rows(None, None, None, 3, 64, None) == _lib.EINVAL
     assert L.rumus_hip_i8_gemm(None, None, None, None, None, None, None, 0, 64, 8, None) == 0
     assert L.rumus_hip_i8_gemm(None, None, None, None, None, None, None, 0, 24, 8, None) == _lib.EINVAL
+    assert L.rumus_hip_i8_linear(None, None, None, None, None, None, 0, 64, 8, None) == 0
+    assert L.rumus_hip_i8_linear(None, None, None, None, None, None, 2, 24, 8, None) == _lib.EINVAL
+    assert L.rumus_hip_i8_linear(None, None, None, None, None, None, 2, 64, 8, None) == _lib.EINVAL
+    assert L.rumus_hip_i8_linear_scratch_size(16, 2048, 64) == 0 and L.rumus_hip_i8_linear_scratch_size(17, 64, 64) == 17 * 64 + 192 + 17 * 4
     assert L.rumus_hip_add_bias(None, None, None, 0, 8, None) == 0
     assert L.rumus_hip_transpose_f32(None, None, 0, 8, None) == 0
     assert L.rumus_hip_rmsnorm(None, None, None, 0, 64, 1e-6, None) == 0
