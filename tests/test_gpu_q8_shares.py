@@ -13,7 +13,10 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("m,k,n,bs", [
     (5, 1152, 100, 32), (13, 1152, 9632, 32), (30, 2048, 2048, 32), (32, 2080, 130, 32), (32, 1920, 260, 64), (17, 2880, 300, 96),
     (32, 2592, 128, 96), (9, 4096, 1000, 128), (24, 3072, 520, 1024), (6, 4096, 640, 4096), (16, 1152, 33000, 32), (32, 64, 100, 32),
-    (5, 128, 36, 64), (7, 192, 132, 32), (31, 96, 132, 96), (40, 2592, 256, 96), (64, 1152, 300, 32), (70, 2880, 130, 96)])
+    (5, 128, 36, 64), (7, 192, 132, 32), (31, 96, 132, 96), (40, 2592, 256, 96), (64, 1152, 300, 32), (70, 2880, 130, 96),
+    # one block per column beyond 64 rows: K is cut inside it, in periods of 32, 4, 2, 11, 31, 13 and 1 halves of a step
+    (70, 2048, 130, 2048), (66, 5248, 200, 5248), (250, 2752, 100, 2752), (100, 1056, 70, 1056), (66, 992, 64, 992), (130, 2080, 300, 2080),
+    (65, 1696, 40, 1696), (300, 4096, 1000, 2048)])
 def test_shares_of_k(m, k, n, bs):
     from rumus_amd import nn
     say(f"matmul_q8 m={m} k={k} n={n} block {bs}")
