@@ -41,6 +41,10 @@ __global__ __launch_bounds__(256) void f16_narrow_kernel(const float* __restrict
     for (uint64_t j = i; j < numel && j < i + 8; j++) out[j] = (_Float16)in[j];
 }
 
+// f32 x Q8 for a few f16 rows (q8.hip)
+bool q8_few_rows_take(uint32_t m, uint32_t k, uint32_t bs);
+int q8_few_rows_f16(const _Float16* a, const uint32_t* b, _Float16* c, uint32_t m, uint32_t k, uint32_t n, uint32_t bs, hipStream_t s);
+
 static inline size_t round_256(size_t b) { return (b + 255) & ~size_t(255); }
 
 // f32 copies of the activations and of the result, in the stream's staging buffer
@@ -82,6 +86,8 @@ int rumus_hip_matmul_q8_f16(const uint16_t* a, const uint32_t* b, uint16_t* c, u
                             uint32_t block_size, rumus_hip_stream_t stream) {
     // nothing to compute, or nothing to compute on: the f32 entry point's own checks give the answer
     if (m == 0 || n == 0 || !a || !c) return rumus_hip_matmul_q8(nullptr, b, nullptr, m, k, n, block_size, stream);
+    if (b && q8_few_rows_take(m, k, block_size))
+        return q8_few_rows_f16(reinterpret_cast<const _Float16*>(a), b, reinterpret_cast<_Float16*>(c), m, k, n, block_size, as_stream(stream));
     F16Stage st;
     if (int rc = f16_stage(a, (uint64_t)m * k, (uint64_t)m * n, as_stream(stream), st, "matmul_q8_f16")) return rc;
     if (int rc = rumus_hip_matmul_q8(st.a, b, st.c, m, k, n, block_size, stream)) return rc;

@@ -3,6 +3,8 @@
 //
 // Buffer format (rumus/src/tensor/core.rs:61-98): per block one header word
 // (f16 scale in the low half) followed by block_size signed bytes.
+#include <atomic>
+
 #include <hip/hip_fp16.h>
 
 #include "common.h"
@@ -248,18 +250,20 @@ struct __attribute__((packed, aligned(4))) Q8Words4 { uint32_t x, y, z, w; };
 // ONCE: one block per column.  The bytes of a column are then one unbroken run behind a single header and the
 // loads carry the non-temporal hint (1 x 4096 x 11008 from HBM: 14.5 -> 13.2 us; with smaller blocks the same
 // hint costs 0.4 to 1.2 us).
-template <int M, bool ONCE>
+// CW: columns per wave.  Fewer than four where four leave compute units without a workgroup; 8 / CW runs of a lane are then in flight, the first
+// of them while x is staged.
+// T: f32 or f16 rows, staged as f32 (exact), and result (rounded once).
+template <int M, int CW, bool ONCE, typename T>
 __global__ __launch_bounds__(512) void matmul_q8_rows_kernel(
-    const float* __restrict__ a, const uint32_t* __restrict__ b, float* __restrict__ c, uint32_t k,
+    const T* __restrict__ a, const uint32_t* __restrict__ b, T* __restrict__ c, uint32_t k,
     uint32_t n, uint32_t stride, uint32_t blocks_per_col, uint32_t kpad, uint32_t runs_per_block,
-    uint32_t run_magic) {
-    constexpr int CW = 4;                                     // columns per wave
+    uint32_t run_magic, uint32_t vec) {
     // x in LDS as [row][quarter of a run][run][4]: the lanes of a wave, one run each, then read
     // consecutive 16-byte pieces (run-major order would put them 64 bytes apart, 16 to a bank)
     extern __shared__ float xs[];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t nruns = kpad / 16;
-    const uint32_t col0 = blockIdx.x * 32 + wave * CW;
+    const uint32_t col0 = blockIdx.x * (8 * CW) + wave * CW;
     const uint32_t* colbase[CW];
 #pragma unroll
     for (int cc = 0; cc < CW; cc++)
@@ -286,16 +290,31 @@ __global__ __launch_bounds__(512) void matmul_q8_rows_kernel(
     // Blocks smaller than a column: the first two runs of every lane are on their way while the activations are
     // staged, and two stay in flight (1 x 4096 x 11008 from HBM, blocks of 32: 16.8 -> 16.0 us, of 128: 16.1 -> 15.4).
     // One block per column streams with the non-temporal hint and is faster in the plain loop (13.3 against 14.9 us).
-    Q8Words4 wa[CW], wb[CW];
-    uint32_t ha[CW], hb[CW];
-    if constexpr (!ONCE) {
+    constexpr int FLIGHT = CW < 4 ? 8 / CW : 1;
+    Q8Words4 wa[CW], wb[CW], wf[FLIGHT][CW];
+    uint32_t ha[CW], hb[CW], hf[FLIGHT][CW];
+    if constexpr (CW < 4) {
+#pragma unroll
+        for (int i = 0; i < FLIGHT; i++) fetch(lane + 64 * i, wf[i], hf[i]);
+        __builtin_amdgcn_sched_barrier(0);
+    } else if constexpr (!ONCE) {
         fetch(lane, wa, ha);
         fetch(lane + 64, wb, hb);
         __builtin_amdgcn_sched_barrier(0);
     }
-    for (uint32_t r = 0; r < M; r++)
-        for (uint32_t kk = tid; kk < kpad; kk += 512)
-            xs[((r * 4 + (kk % 16) / 4) * nruns + kk / 16) * 4 + kk % 4] = kk < k ? a[(uint64_t)r * k + kk] : 0.0f;
+    if (vec) {                                                // k % 16 == 0, rows aligned to four elements
+        typedef T T4 __attribute__((ext_vector_type(4)));
+        for (uint32_t r = 0; r < M; r++)
+#pragma unroll 4
+            for (uint32_t q = tid; q < kpad / 4; q += 512) {
+                const T4 v = *reinterpret_cast<const T4*>(a + (uint64_t)r * k + 4 * q);
+                *reinterpret_cast<float4*>(xs + ((r * 4 + q % 4) * nruns + q / 4) * 4) = make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
+            }
+    } else {
+        for (uint32_t r = 0; r < M; r++)
+            for (uint32_t kk = tid; kk < kpad; kk += 512)
+                xs[((r * 4 + (kk % 16) / 4) * nruns + kk / 16) * 4 + kk % 4] = kk < k ? (float)a[(uint64_t)r * k + kk] : 0.0f;
+    }
     __syncthreads();
     float acc[CW][M];
 #pragma unroll
@@ -335,14 +354,24 @@ __global__ __launch_bounds__(512) void matmul_q8_rows_kernel(
             for (int r = 0; r < M; r++) acc[cc][r] = fmaf(part[cc][r], sc, acc[cc][r]);
         }
     };
-    if constexpr (ONCE) {
+    if constexpr (CW < 4) {
+        for (uint32_t run = lane;;) {
+#pragma unroll
+            for (int i = 0; i < FLIGHT; i++)
+                if (run + 64 * i < nruns) multiply(run + 64 * i, wf[i], hf[i]);
+            run += 64 * FLIGHT;
+            if (run - lane >= nruns) break;                   // wave-uniform
+#pragma unroll
+            for (int i = 0; i < FLIGHT; i++) fetch(run + 64 * i, wf[i], hf[i]);
+        }
+    } else if constexpr (ONCE) {
         for (uint32_t run = lane; run < nruns; run += 64) {
             fetch(run, wa, ha);
             multiply(run, wa, ha);
         }
     }
     // two runs per lane in flight: the slot just multiplied is refilled two runs ahead
-    for (uint32_t run = lane; !ONCE && run < nruns; run += 128) {
+    for (uint32_t run = lane; CW == 4 && !ONCE && run < nruns; run += 128) {
         Q8Words4 w0[CW];
         uint32_t h0[CW];
 #pragma unroll
@@ -363,22 +392,76 @@ __global__ __launch_bounds__(512) void matmul_q8_rows_kernel(
 #pragma unroll
         for (int r = 0; r < M; r++) {
             const float v = wave_sum(acc[cc][r]);
-            if (lane == 0 && col0 + cc < n) c[(uint64_t)r * n + col0 + cc] = v;
+            if (lane == 0 && col0 + cc < n) c[(uint64_t)r * n + col0 + cc] = (T)v;
         }
 }
 
-template <int M>
-static int launch_q8_rows(const float* a, const uint32_t* b, float* c, uint32_t k, uint32_t n, uint32_t bs,
-                          uint32_t stride, uint32_t blocks_per_col, uint32_t kpad, hipStream_t s) {
+constexpr uint32_t kQ8RowsFloats = 32768;                     // of x in LDS: 128 KB
+
+template <int M, int CW, bool ONCE, typename T>
+static int launch_q8_rows_form(const T* a, const uint32_t* b, T* c, uint32_t k, uint32_t n, uint32_t bs, uint32_t stride, uint32_t blocks_per_col,
+                               uint32_t kpad, hipStream_t s) {
+    const size_t lds = (size_t)M * kpad * sizeof(float);
+    static std::atomic<bool> allowed{false};
+    if (lds > 64 * 1024 && !allowed.load(std::memory_order_relaxed)) {
+        if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&matmul_q8_rows_kernel<M, CW, ONCE, T>),
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, kQ8RowsFloats * 4), "hipFuncSetAttribute"))
+            return rc;
+        allowed.store(true, std::memory_order_relaxed);
+    }
     const uint32_t runs_per_block = bs / 16;
     const uint32_t run_magic = runs_per_block == 1 ? 0u : (uint32_t)((0x100000000ull + runs_per_block - 1) / runs_per_block);
-    if (blocks_per_col == 1)
-        hipLaunchKernelGGL((matmul_q8_rows_kernel<M, true>), dim3(ceil_div(n, 32)), dim3(512), (size_t)M * kpad * sizeof(float), s,
-                           a, b, c, k, n, stride, blocks_per_col, kpad, runs_per_block, run_magic);
-    else
-        hipLaunchKernelGGL((matmul_q8_rows_kernel<M, false>), dim3(ceil_div(n, 32)), dim3(512), (size_t)M * kpad * sizeof(float), s,
-                           a, b, c, k, n, stride, blocks_per_col, kpad, runs_per_block, run_magic);
+    const bool vec = k % 16 == 0 && reinterpret_cast<uintptr_t>(a) % (4 * sizeof(T)) == 0;
+    hipLaunchKernelGGL((matmul_q8_rows_kernel<M, CW, ONCE, T>), dim3(ceil_div(n, 8 * CW)), dim3(512), lds, s, a, b, c, k, n, stride, blocks_per_col,
+                       kpad, runs_per_block, run_magic, vec);
     return check_launch("matmul_q8_rows_kernel");
+}
+// The fewest columns a wave whose workgroups run in one round of 256.  From HBM, us with 1, 2 and 4 columns: 1 x 6400 x 764, blocks of 32, 6.1, 6.6, 9.1
+// (9.9 to 11.2 with four and x staged element by element, as until now), 4 x 2048 x 2048 7.4, 7.9, 10.1 (12.8), 2 x 4096 x 4096 12.7, 9.9, 10.6 (14.7),
+// 4 x 2048 x 6608 20.6, 13.1, 11.8 (16.0); one launch where two carried the rows: 4 x 8192 x 8192 25.5 (55.8), 3 x 6400 x 764 from f16 13.1 (32.3).
+template <int M, typename T>
+static int launch_q8_rows(const T* a, const uint32_t* b, T* c, uint32_t k, uint32_t n, uint32_t bs, uint32_t stride, uint32_t bpc, uint32_t kpad,
+                          hipStream_t s) {
+    if constexpr (M <= 4) {
+        if (n <= 2048)
+            return bpc == 1 ? launch_q8_rows_form<M, 1, true>(a, b, c, k, n, bs, stride, bpc, kpad, s)
+                            : launch_q8_rows_form<M, 1, false>(a, b, c, k, n, bs, stride, bpc, kpad, s);
+        if (n <= 4096)
+            return bpc == 1 ? launch_q8_rows_form<M, 2, true>(a, b, c, k, n, bs, stride, bpc, kpad, s)
+                            : launch_q8_rows_form<M, 2, false>(a, b, c, k, n, bs, stride, bpc, kpad, s);
+    }
+    return bpc == 1 ? launch_q8_rows_form<M, 4, true>(a, b, c, k, n, bs, stride, bpc, kpad, s)
+                    : launch_q8_rows_form<M, 4, false>(a, b, c, k, n, bs, stride, bpc, kpad, s);
+}
+
+// Rows that do not go to the matrix cores (block_size % 16 == 0, kpad <= 16384), in groups whose x fits the LDS.
+template <typename T>
+static int q8_rows(const T* a, const uint32_t* b, T* c, uint32_t m, uint32_t k, uint32_t n, uint32_t bs, uint32_t stride, uint32_t bpc,
+                   hipStream_t s) {
+    const uint32_t kpad = (k + 15) & ~15u, group = min(8u, kQ8RowsFloats / kpad);
+    for (uint32_t r0 = 0; r0 < m; r0 += group) {
+        const T* ar = a + (uint64_t)r0 * k;
+        T* cr = c + (uint64_t)r0 * n;
+        int rc;
+        switch (min(group, m - r0)) {
+            case 1: rc = launch_q8_rows<1>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
+            case 2: rc = launch_q8_rows<2>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
+            case 3: rc = launch_q8_rows<3>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
+            case 4: rc = launch_q8_rows<4>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
+            case 5: rc = launch_q8_rows<5>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
+            case 6: rc = launch_q8_rows<6>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
+            case 7: rc = launch_q8_rows<7>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
+            default: rc = launch_q8_rows<8>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
+        }
+        if (rc) return rc;
+    }
+    return RUMUS_HIP_OK;
+}
+
+// f16 rows, where the call above's f32 form comes here: up to four rows
+bool q8_few_rows_take(uint32_t m, uint32_t k, uint32_t bs) { return m <= 4 && k > 0 && bs > 0 && bs % 16 == 0 && k <= 16384; }
+int q8_few_rows_f16(const _Float16* a, const uint32_t* b, _Float16* c, uint32_t m, uint32_t k, uint32_t n, uint32_t bs, hipStream_t s) {
+    return q8_rows(a, b, c, m, k, n, bs, (4 + bs + 3) / 4, ceil_div(k, bs), s);
 }
 
 // Dequantize into the tensor's own [K, N] order: the buffer holds the transposed tensor ([N, K]
@@ -840,29 +923,7 @@ int rumus_hip_matmul_q8(const float* a, const uint32_t* b, float* c, uint32_t m,
     if (block_kernel)
         return matmul_q8_mfma_blocks(a, b, c, m, k, n, block_size, stride, blocks_per_col, as_stream(stream));
     const uint32_t kpad = (k + 15) & ~15u;
-    if (block_size % 16 == 0 && kpad <= 16384) {
-        // rows in groups whose x fits 64 KB of LDS: 4 rows at k = 4096, 1 at k = 11008, all 8 up to k = 2048
-        const uint32_t group = min(8u, 16384u / kpad);
-        hipStream_t s = as_stream(stream);
-        for (uint32_t r0 = 0; r0 < m; r0 += group) {
-            const uint32_t rows = min(group, m - r0);
-            const float* ar = a + (uint64_t)r0 * k;
-            float* cr = c + (uint64_t)r0 * n;
-            int rc;
-            switch (rows) {
-                case 1: rc = launch_q8_rows<1>(ar, b, cr, k, n, block_size, stride, blocks_per_col, kpad, s); break;
-                case 2: rc = launch_q8_rows<2>(ar, b, cr, k, n, block_size, stride, blocks_per_col, kpad, s); break;
-                case 3: rc = launch_q8_rows<3>(ar, b, cr, k, n, block_size, stride, blocks_per_col, kpad, s); break;
-                case 4: rc = launch_q8_rows<4>(ar, b, cr, k, n, block_size, stride, blocks_per_col, kpad, s); break;
-                case 5: rc = launch_q8_rows<5>(ar, b, cr, k, n, block_size, stride, blocks_per_col, kpad, s); break;
-                case 6: rc = launch_q8_rows<6>(ar, b, cr, k, n, block_size, stride, blocks_per_col, kpad, s); break;
-                case 7: rc = launch_q8_rows<7>(ar, b, cr, k, n, block_size, stride, blocks_per_col, kpad, s); break;
-                default: rc = launch_q8_rows<8>(ar, b, cr, k, n, block_size, stride, blocks_per_col, kpad, s); break;
-            }
-            if (rc) return rc;
-        }
-        return RUMUS_HIP_OK;
-    }
+    if (block_size % 16 == 0 && kpad <= 16384) return q8_rows(a, b, c, m, k, n, block_size, stride, blocks_per_col, as_stream(stream));
     if (block_size % 16 == 0) {
         dim3 grid(ceil_div(n, kQ8Tile), ceil_div(m, kQ8Tile));
         hipLaunchKernelGGL(matmul_q8_tiled_kernel, grid, dim3(256), 0, as_stream(stream), a, b, c,

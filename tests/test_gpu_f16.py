@@ -4,6 +4,7 @@ The oracle's f32 loops run on the f16-rounded activations (widening is exact); t
 result rounded to f16 once: within the f32 tolerance of the other tests plus half an f16 ulp."""
 import numpy as np
 import pytest
+import torch
 
 import oracle
 
@@ -28,6 +29,7 @@ def assert_close_f16(got16, want32, what=""):
 
 
 @pytest.mark.parametrize("m,k,n,bs", [(1, 512, 512, 512), (3, 256, 40, 64), (7, 96, 33, 12), (16, 1024, 352, 128),
+                                      (2, 64, 2050, 64), (4, 9232, 20, 9232), (3, 128, 4100, 32), (5, 128, 40, 32),
                                       (70, 480, 40, 96), (300, 512, 700, 512)])
 def test_matmul_q8_f16(ops, m, k, n, bs):
     say(f"matmul_q8_f16 m={m} k={k} n={n} bs={bs}")
@@ -41,6 +43,18 @@ def test_matmul_q8_f16(ops, m, k, n, bs):
     # the same bits as the f32 entry point's result rounded to f16
     f32 = host(ops.matmul_q8(dev(a16.astype(np.float32)), dev(words), k, n, bs))
     np.testing.assert_array_equal(got, f32.astype(np.float16))
+
+
+@pytest.mark.parametrize("half", [False, True])
+def test_matmul_q8_few_rows_of_any_alignment(ops, half):
+    say(f"matmul_q8, 3 rows at an odd element, half={half}")
+    rng = np.random.default_rng(11)
+    words = dev(oracle.tensor_quantize(rng.normal(0, 0.02, (320, 50)).astype(np.float32), 64))
+    x = dev(rng.normal(0, 1, (3, 320)).astype(np.float16 if half else np.float32))
+    odd = torch.empty(3 * 320 + 1, dtype=x.dtype, device="cuda")[1:].view(3, 320)
+    odd.copy_(x)
+    run = ops.matmul_q8_f16 if half else ops.matmul_q8
+    assert torch.equal(run(odd, words, 320, 50, 64), run(x, words, 320, 50, 64))
 
 
 @pytest.mark.parametrize("m,k,n,g,act_order", [(1, 4096, 4096, 128, False), (1, 100, 24, 32, False), (4, 512, 352, 64, True),

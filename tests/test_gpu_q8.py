@@ -92,6 +92,10 @@ def test_q8_rejects_bad_block_size(ops):
 
 
 @pytest.mark.parametrize("m,k,n,bs", [(32, 512, 512, 512), (4, 64, 10, 64), (3, 96, 7, 32),
+                                      # up to four rows: one, two and four columns a wave, one run a lane and several rounds of them, x beyond
+                                      # 64 KB of LDS and beyond one launch
+                                      (1, 1024, 2048, 32), (2, 1040, 2049, 1040), (4, 9232, 40, 9232), (3, 10016, 30, 32), (1, 16384, 9, 64),
+                                      (4, 8192, 33, 8192), (3, 4112, 4096, 16), (2, 2064, 4097, 48), (4, 528, 2056, 528), (1, 48, 17, 48),
                                       (2, 40, 5, 8), (70, 256, 130, 128), (5, 100, 9, 20),
                                       (1, 4096, 1100, 4096),   # few-rows kernel, per-channel blocks
                                       (4, 8192, 70, 128),      # two groups of two rows
