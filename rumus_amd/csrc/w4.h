@@ -38,7 +38,7 @@ struct W4Args {
     const float* rinv = nullptr;
     const float* rfac = nullptr;
     // w4_gemm_tile only (set by its launcher; f32 zero-points): kZpFlagWords words, nonzero where a part of the
-    // zero-point table holds a value that is no integer (w4_zp_scan_kernel)
+    // zero-point table holds a value that is no integer (w4_look_at_zero_points, w4_gemm_tile.hip)
     const uint32_t* zflags = nullptr;
     // w4_gemm_i8 only, without perm: f16 activations and result instead of x and y (f16_entry.hip)
     const _Float16* x16 = nullptr;

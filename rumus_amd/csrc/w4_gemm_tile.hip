@@ -60,7 +60,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int kTileCols = 512;   // columns per workgroup of eight waves
 constexpr int kStageK = 128;     // rows of K staged per barrier (8 MFMA steps of 16)
 constexpr int kMaxSplits = 16;
-constexpr uint32_t kZpFlagWords = 256;   // blocks of w4_zp_scan_kernel, one flag word each
+constexpr uint32_t kZpFlagWords = 256;   // blocks that look at the zero-points, one flag word each
 
 // one packed word -> B fragment, k order 0,4,1,5,2,6,3,7, with the column's integer zero-point z taken off on the way:
 // the magic-number conversion ends in a subtraction anyway (1024 + n - 1024, and (1024 + 16 n) / 16 - 64 for the nibbles
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void w4_gemm_tile_kernel(W4Args a, f
     const uint32_t k_end = min(a.padded_k, st_end * kStageK);
     if (tid < BM) lds_rf[tid] = a.rfac[min(m0 + tid, a.m - 1)];          // read after the stages' barriers
 
-    // Whether any zero-point of the table has a rest at all (found by w4_zp_scan_kernel before this launch):
+    // Whether any zero-point of the table has a rest at all (w4_look_at_zero_points, before this launch):
     // checkpoints store integers (as f32 here, or packed), and then the rank-1 updates - an eighth of the
     // matrix-core time at groups of 128 - are left out.  Requested here, looked at before the first stage.
     // (No flags - small batches, where the look costs more than it saves: the updates run.)
@@ -619,15 +619,21 @@ static uint32_t pick_splits(uint32_t tiles, uint32_t nstages, uint32_t* stages_p
 
 // flags[block] = 1 when the block's share of the zero-point table (count4 float4) holds a value that is no integer
 // within the range that the tile kernel takes off inside its f16 conversion, else 0.  Every word is written by every
-// launch: nothing to clear.
-__global__ __launch_bounds__(256) void w4_zp_scan_kernel(const float4* __restrict__ zp, uint32_t count4,
-                                                         uint32_t* __restrict__ flags) {
+// launch: nothing to clear.  The first kZpFlagWords blocks of the launch that prepares the activations do it (a launch of its own took 2.5 to 3 us of
+// every call: 515 x 1088 -> 704 19.7 -> 17.5 us, 196 x 5760 -> 1120 25.1 -> 21.8, 1533 x 768 -> 1856 34.5 -> 32.3); `blocks` is 0 where nobody looks.
+struct W4Look {
+    const float4* zp;
+    uint32_t count4, blocks;
+    uint32_t* flags;
+};
+__device__ __forceinline__ bool w4_look_at_zero_points(const W4Look& look) {
+    if (blockIdx.x >= look.blocks) return false;
     bool mine = false;
-    const uint32_t step = kZpFlagWords * 256;
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < count4; i += 4 * step) {
+    const uint32_t step = kZpFlagWords * blockDim.x;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < look.count4; i += 4 * step) {
         float4 z[4];
 #pragma unroll
-        for (uint32_t u = 0; u < 4; u++) z[u] = zp[min(i + u * step, count4 - 1)];
+        for (uint32_t u = 0; u < 4; u++) z[u] = look.zp[min(i + u * step, look.count4 - 1)];
 #pragma unroll
         for (uint32_t u = 0; u < 4; u++) {
             const float v[4] = {z[u].x, z[u].y, z[u].z, z[u].w};
@@ -636,12 +642,10 @@ __global__ __launch_bounds__(256) void w4_zp_scan_kernel(const float4* __restric
         }
     }
     const int any = __syncthreads_or(mine);
-    if (threadIdx.x == 0) flags[blockIdx.x] = any ? 1u : 0u;
+    if (threadIdx.x == 0) look.flags[blockIdx.x] = any ? 1u : 0u;
+    return true;
 }
 
-// xp[r][j] = x[r][perm[j]] (perm null: j) for j < k, 0 for k <= j < k4: the act-order column
-// gather done once per call instead of once per workgroup column, and the padding / alignment
-// of rows that the tile kernel's 128-bit loads need.
 // One workgroup per row of x: rinv[row] = 2^(141 - E) for a largest magnitude a * 2^(E - 127), 1 <= a < 2, so that
 // the scaled row lies in [2^14, 2^15) -- inside the range of f16 whatever the row's own size, and with its small
 // elements' low halves clear of f16's subnormals -- and rfac[row] = 1 / rinv[row].  Both are powers of two: scaling
@@ -655,41 +659,66 @@ __device__ __forceinline__ uint32_t w4_row_factor_exponent(uint32_t amax) {
     return e == 0 || e == 255 ? 127u : min(268u - e, 240u);
 }
 
-__global__ __launch_bounds__(256) void w4_row_factor_kernel(const float* __restrict__ x, uint32_t k,
-                                                            float* __restrict__ rinv, float* __restrict__ rfac) {
-    __shared__ uint32_t part[4];
-    const uint32_t tid = threadIdx.x, row = blockIdx.x;
+// xp (or null): xp[row][j] = x[row][perm[j]] (perm null: j) for j < k, 0 for k <= j < k4: the act-order column
+// gather done once per call instead of once per workgroup column, and the padding / alignment of rows that the tile kernel's
+// 128-bit loads need.  The order of up to 8192 columns is asked for ahead of the row, which the gather then finds in the caches.
+constexpr uint32_t kRowFactorThreads = 512;
+__global__ __launch_bounds__(kRowFactorThreads) void w4_row_factor_kernel(const float* __restrict__ x, uint32_t k,
+                                                                          float* __restrict__ rinv, float* __restrict__ rfac, W4Look look,
+                                                                          const int32_t* __restrict__ perm, float* __restrict__ xp, uint32_t k4) {
+    constexpr uint32_t T = kRowFactorThreads, G = 16;
+    __shared__ uint32_t part[T / 64];
+    if (w4_look_at_zero_points(look)) return;
+    const uint32_t tid = threadIdx.x, row = blockIdx.x - look.blocks;
     const float* xr = x + (uint64_t)row * k;
+    uint32_t at[G];
+    auto order = [&](uint32_t j0) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t u = 0; u < G; u++) {
+            at[u] = min(j0 + u * T, k - 1);
+            if (perm) at[u] = (uint32_t)perm[at[u]];
+        }
+    };
+    if (xp) order(tid);
     uint32_t amax = 0;                                       // bit patterns of |x| order like the values; NaN sorts last
     if (k % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
-        for (uint32_t i = tid; i < k / 4; i += 256) {
-            const float4 v = reinterpret_cast<const float4*>(xr)[i];
-            amax = max(max(amax, __float_as_uint(v.x) & 0x7FFFFFFFu), __float_as_uint(v.y) & 0x7FFFFFFFu);
-            amax = max(max(amax, __float_as_uint(v.z) & 0x7FFFFFFFu), __float_as_uint(v.w) & 0x7FFFFFFFu);
+        for (uint32_t i = tid; i < k / 4; i += 4 * T) {      // four loads in flight; past the end the last again
+            float4 v[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; u++) v[u] = reinterpret_cast<const float4*>(xr)[min(i + u * T, k / 4 - 1)];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; u++) {
+                amax = max(max(amax, __float_as_uint(v[u].x) & 0x7FFFFFFFu), __float_as_uint(v[u].y) & 0x7FFFFFFFu);
+                amax = max(max(amax, __float_as_uint(v[u].z) & 0x7FFFFFFFu), __float_as_uint(v[u].w) & 0x7FFFFFFFu);
+            }
         }
     } else {
-        for (uint32_t i = tid; i < k; i += 256) amax = max(amax, __float_as_uint(xr[i]) & 0x7FFFFFFFu);
+        for (uint32_t i = tid; i < k; i += T) amax = max(amax, __float_as_uint(xr[i]) & 0x7FFFFFFFu);
     }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) amax = max(amax, (uint32_t)__shfl_xor((int)amax, o));
+    amax = wave_max(amax);
     if ((tid & 63) == 0) part[tid >> 6] = amax;
     __syncthreads();
     if (tid == 0) {
-        amax = max(max(part[0], part[1]), max(part[2], part[3]));
+#pragma unroll
+        for (uint32_t w = 1; w < T / 64; w++) amax = max(amax, part[w]);
         const uint32_t b = w4_row_factor_exponent(amax);
         rinv[row] = __uint_as_float(b << 23);
         rfac[row] = __uint_as_float((254u - b) << 23);
     }
-}
-
-__global__ __launch_bounds__(256) void w4_prepare_x_kernel(const float* __restrict__ x,
-                                                           const int32_t* __restrict__ perm,
-                                                           float* __restrict__ xp, uint32_t k, uint32_t k4) {
-    const uint32_t j = blockIdx.x * 256 + threadIdx.x, row = blockIdx.y;
-    if (j >= k4) return;
-    float v = 0.0f;
-    if (j < k) v = x[(uint64_t)row * k + (perm ? (uint32_t)perm[j] : j)];
-    xp[(uint64_t)row * k4 + j] = v;
+    if (!xp) return;
+    for (uint32_t j0 = tid;;) {
+        float v[G];
+#pragma unroll
+        for (uint32_t u = 0; u < G; u++) v[u] = xr[at[u]];
+#pragma unroll
+        for (uint32_t u = 0; u < G; u++) {
+            const uint32_t j = j0 + u * T;
+            if (j < k4) xp[(uint64_t)row * k4 + j] = j < k ? v[u] : 0.0f;
+        }
+        j0 += G * T;
+        if (j0 - tid >= k4) return;
+        order(j0);
+    }
 }
 
 // Activations -> the form the PRE tile kernel copies into LDS.  Workgroup = one row tile of 32
@@ -752,12 +781,13 @@ __global__ __launch_bounds__(256) void w4_convert_x_rows_kernel(const float* __r
                                                                 uint8_t* __restrict__ xh, uint8_t* __restrict__ xl,
                                                                 float* __restrict__ xs, uint32_t m, uint32_t k,
                                                                 uint32_t xsteps, uint32_t rows, uint32_t kpad,
-                                                                float* __restrict__ rfac) {
+                                                                float* __restrict__ rfac, W4Look look) {
     extern __shared__ __attribute__((aligned(16))) float lds_rows[];
     __shared__ uint32_t rowmax[8];
+    if (w4_look_at_zero_points(look)) return;
     const uint32_t tid = threadIdx.x;
     if (tid < 8) rowmax[tid] = 0;
-    const uint32_t row0 = blockIdx.x * rows;                  // rows divides 32: a workgroup stays inside a row tile
+    const uint32_t row0 = (blockIdx.x - look.blocks) * rows;                  // rows divides 32: a workgroup stays inside a row tile
     const uint32_t live = row0 < m ? min(rows, m - row0) : 0;
     const float* src = x + (uint64_t)row0 * k;
     if ((k % 4 == 0) && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
@@ -838,10 +868,11 @@ template <int ITER>
 __global__ __launch_bounds__(256) void w4_convert_x_regs_kernel(const float* __restrict__ x, uint8_t* __restrict__ xh,
                                                                 uint8_t* __restrict__ xl, float* __restrict__ xs,
                                                                 float* __restrict__ rfac, uint32_t m, uint32_t k,
-                                                                uint32_t xsteps) {
+                                                                uint32_t xsteps, W4Look look) {
     __shared__ uint32_t rowmax[4];
+    if (w4_look_at_zero_points(look)) return;
     const uint32_t tid = threadIdx.x, r = tid & 3, s0 = tid >> 2;
-    const uint32_t grow = blockIdx.x * 4 + r, tile = grow >> 5, row = grow & 31;
+    const uint32_t grow = (blockIdx.x - look.blocks) * 4 + r, tile = grow >> 5, row = grow & 31;
     const bool live = grow < m;
     const float* xr = x + (uint64_t)(live ? grow : 0) * k;
     if (tid < 4) rowmax[tid] = 0;
@@ -933,13 +964,10 @@ static int launch_tile(const W4Args& a_in, hipStream_t s) {
         uint32_t* zflags = static_cast<uint32_t*>(ws);
         float* fac = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + flag_bytes);
         ws = static_cast<uint8_t*>(ws) + fac_bytes;
-        // the look at the zero-points takes 2.5 to 3 us: from 128 rows on the updates it may save cost more
-        if (!a.zp4 && a.m >= 128) {
-            hipLaunchKernelGGL(w4_zp_scan_kernel, dim3(kZpFlagWords), dim3(256), 0, s, reinterpret_cast<const float4*>(a.zp),
-                               (uint32_t)((uint64_t)a.num_groups * a.n / 4), zflags);
-            if (int rc = check_launch("w4_zp_scan_kernel")) return rc;
-            a.zflags = zflags;
-        }
+        // (fewer rows have the updates: what the look may save them is less than it costs)
+        const bool look_first = !a.zp4 && a.m >= 128;
+        const W4Look look{reinterpret_cast<const float4*>(a.zp), (uint32_t)((uint64_t)a.num_groups * a.n / 4), look_first ? kZpFlagWords : 0, zflags};
+        if (look_first) a.zflags = zflags;
         a.rinv = fac;
         a.rfac = fac + a.m;
         // the pre-converting kernels that hold whole rows (in LDS for the gather, in registers for plain x) find
@@ -948,8 +976,14 @@ static int launch_tile(const W4Args& a_in, hipStream_t s) {
         const uint32_t regs_iter = PRE && vec8 ? ceil_div(xsteps, 64u) : 0;   // steps of 16 k per thread
         const bool in_regs = regs_iter >= 1 && regs_iter <= 16;
         if (!(PRE && ((a.perm && convert_perm_rows(k4)) || in_regs))) {
-            hipLaunchKernelGGL(w4_row_factor_kernel, dim3(a.m), dim3(256), 0, s, a.x, a.k, fac, fac + a.m);
+            float* const xp = prepare ? static_cast<float*>(ws) : nullptr;
+            hipLaunchKernelGGL(w4_row_factor_kernel, dim3(a.m + look.blocks), dim3(kRowFactorThreads), 0, s, a.x, a.k, fac, fac + a.m, look, a.perm, xp, k4);
             if (int rc = check_launch("w4_row_factor_kernel")) return rc;
+            if (prepare) {
+                a.x = xp;
+                a.perm = nullptr;
+                a.k = k4;                                    // the added columns are zero
+            }
         }
         if (PRE) {
             uint8_t* base = static_cast<uint8_t*>(ws);
@@ -958,18 +992,18 @@ static int launch_tile(const W4Args& a_in, hipStream_t s) {
             float* sums = reinterpret_cast<float*>(base + 2 * plane_bytes);
             const uint32_t perm_rows = a.perm ? convert_perm_rows(k4) : 0;   // 0: a row does not fit LDS
             if (in_regs) {
-                const dim3 g4(xtiles * 8);                   // four rows each
+                const dim3 g4(xtiles * 8 + look.blocks);                   // four rows each
 #define RUMUS_W4_REGS(N) hipLaunchKernelGGL(w4_convert_x_regs_kernel<N>, g4, dim3(256), 0, s, a.x, base, base + plane_bytes, \
-                                            sums, fac + a.m, a.m, a.k, xsteps)
+                                            sums, fac + a.m, a.m, a.k, xsteps, look)
                 if (regs_iter <= 4) RUMUS_W4_REGS(4);
                 else if (regs_iter <= 8) RUMUS_W4_REGS(8);
                 else if (regs_iter <= 11) RUMUS_W4_REGS(11);
                 else RUMUS_W4_REGS(16);
 #undef RUMUS_W4_REGS
             } else if (perm_rows)
-                hipLaunchKernelGGL(w4_convert_x_rows_kernel, dim3(xtiles * 32 / perm_rows), dim3(256),
+                hipLaunchKernelGGL(w4_convert_x_rows_kernel, dim3(xtiles * 32 / perm_rows + look.blocks), dim3(256),
                                    (size_t)perm_rows * k4 * sizeof(float), s, a.x, a.perm, base, base + plane_bytes, sums,
-                                   a.m, a.k, xsteps, perm_rows, k4, fac + a.m);
+                                   a.m, a.k, xsteps, perm_rows, k4, fac + a.m, look);
             else if (vec) hipLaunchKernelGGL(w4_convert_x_kernel<true>, grid, dim3(256), 0, s, a.x, a.perm, base,
                                              base + plane_bytes, sums, a.m, a.k, xsteps, a.rinv);
             else hipLaunchKernelGGL(w4_convert_x_kernel<false>, grid, dim3(256), 0, s, a.x, a.perm, base,
@@ -979,14 +1013,6 @@ static int launch_tile(const W4Args& a_in, hipStream_t s) {
             a.xl = base + plane_bytes;
             a.xs = sums;
             a.xsteps = xsteps;
-        } else if (prepare) {
-            float* xp = static_cast<float*>(ws);
-            hipLaunchKernelGGL(w4_prepare_x_kernel, dim3(ceil_div(k4, 256), a.m), dim3(256), 0, s, a.x, a.perm, xp,
-                               a.k, k4);
-            if (int rc = check_launch("w4_prepare_x_kernel")) return rc;
-            a.x = xp;
-            a.perm = nullptr;
-            a.k = k4;                                     // the added columns are zero
         }
         if (splits > 1) out = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + x_bytes);
     }

@@ -22,7 +22,11 @@ def ops():
                                                (300, 512, 512, 64, True), (136, 520, 516, 32, False),
                                                (600, 1024, 2048, 128, True), (600, 1024, 2048, 128, False),
                                                (600, 1028, 2048, 128, False), (1024, 256, 11008, 128, False),
-                                               (600, 8192, 2048, 128, False), (600, 14336, 2048, 128, False)])
+                                               (600, 8192, 2048, 128, False), (600, 14336, 2048, 128, False),
+                                               # the launch of the rows' factors gathers or copies them: one round of 8192 columns, its edges,
+                                               # two and three; with and without the look at the zero-points
+                                               (10, 8192, 260, 32, True), (33, 8224, 132, 32, True), (140, 16416, 68, 32, True),
+                                               (40, 526, 260, 32, False), (130, 8190, 132, 32, False), (20, 64, 132, 32, True)])
 def test_rows_of_any_magnitude(ops, m, k, n, g, act_order):
     """Batches beyond 128 rows split x into two f16 planes: every row is first scaled by a power of two into
     f16's range, so rows of 1e-12, rows of 1e9 and a row with one element of 2e5 (beyond f16's 65504) come
