@@ -81,9 +81,10 @@ int rumus_hip_sync(rumus_hip_stream_t stream);
  *       them, converted once per call instead of once per 128 rows.  Same bits
  *       without;
  *       to reserve for it: 3 * (padded_k + 64) * (n + 512) / 4 on top;
- *   qmatmul_int4_t, m >= 8: 64 * m * k (partial sums, only below 512 tiles of
- *       64 x 128; 32 * m * k do from 65 rows on where there is no room for more,
- *       at some speed and with sums in another order) + 10 * num_groups * n +
+ *   qmatmul_int4_t, m >= 8: 64 * m * k (partial sums; 32 * m * k do from 65 rows
+ *       on, and none at 512 tiles of 64 x 128 or more, of 64 x 64 or 64 x 32 for such
+ *       groups, where there is no room for more, at some speed and with sums in
+ *       another order) + 10 * num_groups * n +
  *       4 * (m + num_groups) + 2048;
  *   i8_gemm: rumus_hip_i8_gemm_workspace_size(m, k, n) exactly; at most
  *       min(32 * m * n, 16 MiB) (with k % 64 != 0 only where there is room, as

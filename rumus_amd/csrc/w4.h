@@ -115,6 +115,8 @@ int w4_launch_gemm_f6(const W4Args& a, hipStream_t s, const W4BlockArgs& block =
 // 16-byte aligned buffers.
 bool w4_gemm_t_supported(uint32_t m, uint32_t k, uint32_t n, uint32_t group_size, const void* gy, const void* packed,
                          const void* scales, const void* zp, const void* out);
+// what it takes (an estimate of the whole call in us; 0 where it is the faster one by far)
+double w4_gemm_t_us(uint32_t m, uint32_t k, uint32_t n, uint32_t padded_k, uint32_t group_size);
 int w4_launch_gemm_t(const float* gy, const uint32_t* packed, const float* scales, const float* zp, float* out,
                      uint32_t m, uint32_t k, uint32_t n, uint32_t padded_k, uint32_t group_size, uint32_t num_groups,
                      hipStream_t s);

@@ -776,15 +776,55 @@ bool w4_gemm_t_supported(uint32_t m, uint32_t k, uint32_t n, uint32_t group_size
 // take twice as long: the vector unit and the matrix cores are busy all the time with one), so what counts is the most that any
 // gets; every share's partial result is written and read once, by one more launch.  Over 35 shapes (16 to 2048 rows) the choice is
 // within 3 % of the best of 1 .. 16: 4096 x 11008 at 512 rows 1 share 113.5 us, 4 shares 118.8; at 100 rows 91.5 and 37.5.
-static uint32_t w4t_wide_shares(uint32_t tiles, uint32_t m, uint32_t k, uint32_t n) {
-    uint32_t best = 1;
-    double least = 1e30;
+struct W4tShares { uint32_t shares; double us; };
+static W4tShares w4t_wide_shares(uint32_t tiles, uint32_t m, uint32_t k, uint32_t n) {
+    W4tShares best{1, 1e30};
     for (uint32_t shares = 1; shares <= (uint32_t)kTMaxSplits && n / 16 >= 8 * shares; shares++) {
-        const double us = ceil_div(tiles * shares, 256) * ceil_div(n / 16, 4 * shares) * 0.48 + (shares > 1 ? 3.0 + (shares + 1.0) * m * k * 4 / 4.5e6 : 0.0);
-        if (us < least) { least = us; best = shares; }
+        const double us = 8.7 + (double)ceil_div(tiles * shares, 256) * ceil_div(n / 16, 4 * shares) * 0.48 + (shares > 1 ? 3.0 + (shares + 1.0) * m * k * 4 / 4.5e6 : 0.0);
+        if (us < best.us) best = W4tShares{shares, us};
     }
     return best;
 }
+
+// Shares of n of the narrow kernel.  Four workgroups share a compute unit; a step of 32 columns then takes them `step` us, `beside` more for each
+// neighbour, and a round of them `start` us besides; partial results are added by one more launch (`add`, and 0.3 a share).  Fitted to 241 calls with
+// groups of 32, 64 and 128 (13 to 1024 rows, k and n 512 to 11008, 1 to 16 shares each; 3 to 5 % rms near the best): the choice is 1 % slower than
+// the best of a shape on average, 10 % at worst.  Shares of at least sixteen steps, as before, left weights of few columns on a few workgroups: groups of 32 1.25, of 64 1.13 times
+// as fast now, us: 50 x 1728 x 688 (k, n) groups of 32 37.1 -> 17.1, of 64 26.7 -> 15.4; 126 x 1024 x 1024 31.6 -> 19.1, 23.9 -> 17.0; 200 x 4096 x 4096 179.8 ->
+// 100.8 (groups of 32); 24 x 6912 x 688 22.3 -> 15.5 (64), 18.3 -> 13.6 (128).
+static W4tShares w4t_narrow_shares(uint32_t tiles, int kw, uint32_t m, uint32_t k, uint32_t n) {
+    struct Cost { double step, beside, start, add; };
+    const Cost c = kw == 1 ? Cost{1.26, 0.07, 2.8, 1.9} : kw == 4 ? (m <= 32 ? Cost{0.50, 0.19, 0.8, 1.8} : Cost{0.62, 0.25, 1.6, 2.0})
+                                                        : (m <= 32 ? Cost{0.65, 0.13, 2.0, 1.9} : Cost{0.84, 0.12, 1.5, 2.7});
+    const uint32_t nsteps = ceil_div(n, 32);
+    W4tShares best{1, 1e30};
+    for (uint32_t want = 1; want <= min((uint32_t)kTMaxSplits, nsteps); want++) {
+        const uint32_t steps = ceil_div(nsteps, want), shares = ceil_div(nsteps, steps);
+        const uint64_t on_one = ((uint64_t)tiles * shares + 255) / 256, last = on_one % 4;
+        double us = 6.0 + (double)(on_one / 4) * (steps * (c.step + 3 * c.beside) + c.start) + (last ? steps * (c.step + (last - 1) * c.beside) + c.start : 0.0);
+        if (shares > 1) us += c.add + 0.3 * shares + (shares + 1.0) * m * k * 4 / 4.5e6;
+        if (us < best.us) best = W4tShares{shares, us};
+    }
+    return best;
+}
+
+// Up to 32 rows half of the wide kernel's rows would be empty (11008 x 4096 at 16 rows 24.1 us on the narrow one, 24.6 there).
+static bool w4t_takes_wide(uint32_t m, uint32_t n, uint32_t group_size) { return group_size % 128 == 0 && n % 16 == 0 && m > 32; }
+
+static int w4t_waves(uint32_t group_size) { return group_size % 128 == 0 ? 4 : (int)group_size / 32; }
+
+static W4tShares w4t_shares(uint32_t m, uint32_t k, uint32_t n, uint32_t padded_k, uint32_t group_size) {
+    const int kw = w4t_waves(group_size);
+    const uint64_t tiles = (uint64_t)(padded_k / (32 * kw)) * ceil_div(m, 64);
+    if (tiles >= 1u << 20) return W4tShares{1, 0.0};
+    if (w4t_takes_wide(m, n, group_size)) {
+        if (tiles >= 512) return W4tShares{1, 0.0};
+        return w4t_wide_shares((uint32_t)tiles, m, k, n);
+    }
+    return w4t_narrow_shares((uint32_t)tiles, kw, m, k, n);
+}
+
+double w4_gemm_t_us(uint32_t m, uint32_t k, uint32_t n, uint32_t padded_k, uint32_t group_size) { return w4t_shares(m, k, n, padded_k, group_size).us; }
 
 template <int NS, int KW, bool HALF = false>
 static int launch_w4t(uint32_t ktiles, uint32_t mtiles, uint32_t shares, hipStream_t s, const float* gy,
@@ -813,26 +853,18 @@ static int launch_w4t(uint32_t ktiles, uint32_t mtiles, uint32_t shares, hipStre
 int w4_launch_gemm_t(const float* gy, const uint32_t* packed, const float* scales, const float* zp, float* out,
                      uint32_t m, uint32_t k, uint32_t n, uint32_t padded_k, uint32_t group_size, uint32_t num_groups,
                      hipStream_t s) {
-    const int kw = group_size % 128 == 0 ? 4 : group_size / 32;   // waves per workgroup: 32-column slices of one group
+    const int kw = w4t_waves(group_size);                    // waves per workgroup: 32-column slices of one group
     const uint32_t ktiles = padded_k / (32 * kw), mtiles = ceil_div(m, 64), nsteps = ceil_div(n, 32);
     RUMUS_REQUIRE(mtiles <= 65535, "qmatmul_int4_t: m %u is beyond the grid limit", m);
-    // fewer tiles than two per compute unit: n is shared out too, in shares of at least 16 steps
-    uint32_t shares = 1, steps_per = nsteps, wide_shares = 1;
+    const bool wide = w4t_takes_wide(m, n, group_size);
+    // n is shared out too where that is the faster
+    uint32_t shares = w4t_shares(m, k, n, padded_k, group_size).shares;
+    // Without room for the partial results of those shares: no more than the workspace has always had room for, which is what a capture
+    // may have been prepared with (tiles for less than two workgroups per compute unit, shares of at least 16 steps, 16 of one row tile, 8 of more).
+    uint32_t fewest = 1;
     const uint64_t tiles = (uint64_t)ktiles * mtiles;
-    // Up to 32 rows half of the wide kernel's rows would be empty (11008 x 4096 at 16 rows 24.1 us above, 24.6 there).
-    const bool wide = kw == 4 && n % 16 == 0 && m > 32;
-    if (wide && tiles < 512) wide_shares = w4t_wide_shares((uint32_t)tiles, m, k, n);
-    if (tiles < 512) {
-        shares = (uint32_t)(1024 / tiles);
-        // one row tile: up to 16 shares (46 us instead of 60 for up to 64 rows); beyond, the partial results
-        // of more than 8 shares cost more than the shares gain (128 rows: 84 us against 72)
-        const uint32_t cap = mtiles == 1 ? kTMaxSplits : kTMaxSplits / 2;
-        if (shares > cap) shares = cap;
-        if (shares > nsteps / 16) shares = nsteps / 16;
-        if (shares < 1) shares = 1;
-        steps_per = ceil_div(nsteps, shares);
-        shares = ceil_div(nsteps, steps_per);
-    }
+    if (tiles < 512) fewest = max(1u, min(min((uint32_t)(1024 / tiles), nsteps / 16), (uint32_t)(mtiles == 1 ? kTMaxSplits : kTMaxSplits / 2)));
+    fewest = min(fewest, shares);
     auto up = [](size_t v) { return (v + 255) & ~size_t(255); };
     const size_t gn = (size_t)num_groups * n;
     const size_t rowf_bytes = up((size_t)m * sizeof(float)), sgrp_bytes = up((size_t)num_groups * sizeof(float));
@@ -840,15 +872,13 @@ int w4_launch_gemm_t(const float* gy, const uint32_t* packed, const float* scale
     auto bytes = [&](uint32_t parts) {
         return rowf_bytes + sgrp_bytes + 2 * sp_bytes + zo_bytes + (parts > 1 ? (size_t)parts * m * k * sizeof(float) : 0);
     };
-    // The wide kernel's shares may be more than the narrow one's: it takes them where there is room for their partial results
-    // (100 rows, 11008 -> 512: 16 shares, 8), and no more than those where not, so that a capture runs in what it ran in.
-    const uint32_t fewest = wide ? min(shares, wide_shares) : shares;
-    if (wide) shares = wide_shares;
     void* ws = nullptr;
     size_t got = 0;
     WorkspaceLease lease;                                    // until the last kernel of this call is queued
     if (int rc = workspace_get_upto(s, bytes(fewest), bytes(shares), &got, &ws, lease)) return rc;
     if (got < bytes(shares)) shares = fewest;
+    const uint32_t steps_per = ceil_div(nsteps, shares);
+    if (!wide) shares = ceil_div(nsteps, steps_per);
     uint8_t* b = static_cast<uint8_t*>(ws);
     float* rowf = reinterpret_cast<float*>(b);
     float* sgrp = reinterpret_cast<float*>(b + rowf_bytes);

@@ -5,6 +5,8 @@
 //
 // Packed layout (rumus-vision/src/quant.rs:98-100): word (k/8)*N + col holds
 // rows 8*(k/8)..+7 of column col; scales / zero_points are f32 [groups, N].
+#include <algorithm>
+
 #include <mutex>
 
 #include "w4.h"
@@ -667,7 +669,12 @@ int rumus_hip_qmatmul_int4_t(const float* a, const uint32_t* packed, const float
     // 30 / 31 / 40 / 53 / 65 / 97 against 49-51, g64 against 59-61, g32 against 105-110; 11008 x 4096 32 / 39 / 46 / 65 /
     // 83 / 120 against 37-42, 56-60, 139-143; 4096 x 4096 17 / 15 / 20 / 26 / 33 / 46 against 31-34, 38-41, 45-50)
     const uint32_t mfma_from = group_size % 128 == 0 ? 13 : group_size == 64 ? 21 : 49;
-    if (m >= mfma_from && w4_gemm_t_supported(m, k, n, group_size, a, packed, scales, zero_points, out))
+    // ... and small weights beyond: a pass of the vector kernel takes 0.46 ns per k, from 1024 columns on with the columns (13 to 128 rows, k and n
+    // 512 to 11008, within 10 % from 5 us on), the matrix cores two or three launches.  From HBM, us there and here: groups of 128, 16 x 1024 x 1024 (k, n) 16.1
+    // and 4.7, 32 x 512 x 8192 20.9 and 10.2, 48 x 1024 x 1024 13.8 and 8.7, 24 x 2048 x 2048 17.3 and 10.8; of 64, 32 x 1728 x 688 14.2 and 9.7.
+    const double vector_us = 3.0 + (double)ceil_div(m, 4) * k * std::max(0.46e-3, 0.3e-3 + 1.5e-7 * n);
+    if (m >= mfma_from && w4_gemm_t_supported(m, k, n, group_size, a, packed, scales, zero_points, out) &&
+        vector_us > 0.95 * w4_gemm_t_us(m, k, n, padded_k, group_size))
         return w4_launch_gemm_t(a, packed, scales, zero_points, out, m, k, n, padded_k, group_size, num_groups, s);
     const uint32_t word_rows = padded_k / 8;
     const uintptr_t bits = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(packed) |

@@ -12,7 +12,9 @@ pytestmark = pytest.mark.gpu
 # n: one step of 32 (whole and ragged), two, three, four; 36 steps in two shares, 67 in four, the last share the shorter
 # one; 128 rows and more at few columns: several shares of many row tiles.  m: half a tile of 64, one over it, a whole one, one more.
 @pytest.mark.parametrize("n", [4, 32, 36, 64, 92, 96, 128, 1148, 2116])
-@pytest.mark.parametrize("m,k,g", [(32, 256, 128), (33, 128, 128), (64, 192, 64), (129, 256, 128), (49, 96, 32), (25, 128, 64)])
+@pytest.mark.parametrize("m,k,g", [(32, 256, 128), (33, 128, 128), (64, 192, 64), (129, 256, 128), (49, 96, 32), (25, 128, 64),
+                                   # weights too large for the vector kernel: one step a share, several, shares that end in a short one
+                                   (32, 4096, 128), (33, 3072, 128), (64, 1536, 64), (129, 1024, 128), (49, 2048, 32), (25, 4096, 64), (300, 512, 32)])
 def test_grad_x_steps(m, k, n, g):
     from rumus_amd import ops
     say(f"qmatmul_int4_t steps m={m} k={k} n={n} g={g}")

@@ -166,7 +166,7 @@ def test_q8_with_a_ragged_k_needs_no_partial_sums():
 
 
 # 100 rows: eight shares of n fit, sixteen would be faster; 40 rows with a short n: four fit
-@pytest.mark.parametrize("m,k,n,shares", [(100, 512, 11008, 8), (40, 512, 2048, 4)])
+@pytest.mark.parametrize("m,k,n,shares", [(100, 512, 11008, 8), (40, 512, 2048, 4), (100, 2048, 1028, 2), (32, 4096, 1028, 2)])
 def test_grad_x_with_room_for_fewer_shares(m, k, n, shares):
     import torch
     from rumus_amd import ops
