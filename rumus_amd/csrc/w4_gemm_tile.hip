@@ -933,37 +933,48 @@ static uint32_t convert_perm_rows(uint32_t kpad) {
     return fit >= 8 ? 8 : fit >= 4 ? 4 : fit >= 2 ? 2 : fit;
 }
 
+// A shape of workgroup, as launch_tile's template arguments, and how many of them share K.
+struct TilePlan {
+    uint32_t rt, waves;       // 32 rt rows, 64 waves columns
+    uint32_t splits, sps;     // shares of K, stages of each
+    bool pre() const { return rt >= 2; }
+    uint32_t tiles(const W4Args& a) const { return ceil_div(a.m, 32 * rt) * ceil_div(a.n, 64 * waves); }
+};
+// What a plan takes of the workspace: [flags, rows' factors][activations in the form the kernel reads][partial tiles]
+struct TileBytes { size_t fac, plane, sums, x, part; size_t all() const { return fac + x + part; } };
+static bool tile_copies_x(const W4Args& a) { return a.perm || a.k % 4 != 0 || (reinterpret_cast<uintptr_t>(a.x) & 15) != 0; }
+static TileBytes tile_bytes(const W4Args& a, const TilePlan& plan) {
+    auto up = [](size_t v) { return (v + 255) & ~size_t(255); };
+    const size_t blocks = (size_t)ceil_div(a.m, 32 * plan.rt) * plan.rt * ceil_div(a.padded_k, kStageK) * 8;    // whole workgroup tiles, whole stages
+    TileBytes b{kZpFlagWords * sizeof(uint32_t) + up((size_t)2 * a.m * sizeof(float)), blocks * 1024, blocks * 128, 0, 0};
+    if (plan.pre()) b.x = 2 * b.plane + b.sums;
+    else if (tile_copies_x(a)) b.x = up((size_t)a.m * ((a.k + 3) & ~3u) * sizeof(float));
+    if (plan.splits > 1) b.part = (size_t)plan.splits * a.m * a.n * sizeof(float);
+    return b;
+}
+
+// `ws`: tile_bytes(a_in, plan).all() of it.
 template <int RT, int WM, int TN, int WAVES, int DEPTH, int FOLD>
-static int launch_tile(const W4Args& a_in, hipStream_t s) {
+static int launch_tile(const W4Args& a_in, const TilePlan& plan, void* ws, hipStream_t s) {
     W4Args a = a_in;
     const uint32_t tn = ceil_div(a.n, (WAVES / WM) * 32 * TN), tm = ceil_div(a.m, 32 * RT * WM);
-    const uint32_t nstages = ceil_div(a.padded_k, kStageK);
-    uint32_t sps = nstages;
-    const uint32_t splits = pick_splits(tn * tm, nstages, &sps);
+    const uint32_t nstages = ceil_div(a.padded_k, kStageK), sps = plan.sps, splits = plan.splits;
     // 64-row tiles of eight waves: activations converted once, up front (10 % at m = 512).  The
     // four-wave shape has no registers to spare for the staged chunks and converts in place.
     constexpr bool PRE = RT * WM >= 2 && (WAVES == 8 || (WAVES == 4 && TN == 2));
     constexpr uint32_t BM = 32 * RT * WM;
-    // workspace: [activations in the form the kernel reads][partial tiles]
-    const bool prepare = !PRE && (a.perm || a.k % 4 != 0 || (reinterpret_cast<uintptr_t>(a.x) & 15) != 0);
+    const bool prepare = !PRE && tile_copies_x(a);
     const uint32_t k4 = (a.k + 3) & ~3u;
     const uint32_t xtiles = tm * (BM / 32), xsteps = nstages * 8;   // whole workgroup tiles, whole stages
     RUMUS_REQUIRE(!(prepare || PRE) || max(a.m, xtiles) <= 65535,
                   "qmatmul_int4: m %u is beyond the grid limit of the activation copy", a.m);
-    const size_t plane_bytes = (size_t)xtiles * xsteps * 1024, sums_bytes = (size_t)xtiles * xsteps * 128;
-    const size_t x_bytes = PRE ? 2 * plane_bytes + sums_bytes
-                               : prepare ? (((size_t)a.m * k4 * sizeof(float) + 255) & ~size_t(255)) : 0;
-    const size_t part_bytes = splits > 1 ? (size_t)splits * a.m * a.n * sizeof(float) : 0;
-    const size_t flag_bytes = kZpFlagWords * sizeof(uint32_t);
-    const size_t fac_bytes = flag_bytes + (((size_t)2 * a.m * sizeof(float) + 255) & ~size_t(255));   // flags, rinv[m], rfac[m]
+    const TileBytes bytes = tile_bytes(a, plan);
+    const size_t plane_bytes = bytes.plane;
     float* out = a.y;
-    WorkspaceLease lease;                                    // until the last kernel of this call is queued
     {
-        void* ws = nullptr;
-        if (int rc = workspace_get(s, fac_bytes + x_bytes + part_bytes, &ws, lease)) return rc;
         uint32_t* zflags = static_cast<uint32_t*>(ws);
-        float* fac = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + flag_bytes);
-        ws = static_cast<uint8_t*>(ws) + fac_bytes;
+        float* fac = reinterpret_cast<float*>(zflags + kZpFlagWords);
+        ws = static_cast<uint8_t*>(ws) + bytes.fac;
         // (fewer rows have the updates: what the look may save them is less than it costs)
         const bool look_first = !a.zp4 && a.m >= 128;
         const W4Look look{reinterpret_cast<const float4*>(a.zp), (uint32_t)((uint64_t)a.num_groups * a.n / 4), look_first ? kZpFlagWords : 0, zflags};
@@ -1014,7 +1025,7 @@ static int launch_tile(const W4Args& a_in, hipStream_t s) {
             a.xs = sums;
             a.xsteps = xsteps;
         }
-        if (splits > 1) out = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + x_bytes);
+        if (splits > 1) out = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + bytes.x);
     }
     if (a.zp4)
         hipLaunchKernelGGL((w4_gemm_tile_kernel<RT, WM, TN, WAVES, DEPTH, FOLD, true, PRE>), dim3(tn, tm, splits),
@@ -1034,39 +1045,94 @@ static int launch_tile(const W4Args& a_in, hipStream_t s) {
 }
 
 template <int RT, int WM, int TN, int WAVES, int DEPTH>
-static int launch_fold(const W4Args& a, hipStream_t s) {
+static int launch_fold(const W4Args& a, const TilePlan& plan, void* ws, hipStream_t s) {
     switch (a.group_size) {                              // MFMA steps of 16 per zero-point settlement
-        case 32: return launch_tile<RT, WM, TN, WAVES, DEPTH, 2>(a, s);
-        case 64: return launch_tile<RT, WM, TN, WAVES, DEPTH, 4>(a, s);
-        default: return launch_tile<RT, WM, TN, WAVES, DEPTH, 8>(a, s);  // a multiple of 128: once per stage
+        case 32: return launch_tile<RT, WM, TN, WAVES, DEPTH, 2>(a, plan, ws, s);
+        case 64: return launch_tile<RT, WM, TN, WAVES, DEPTH, 4>(a, plan, ws, s);
+        default: return launch_tile<RT, WM, TN, WAVES, DEPTH, 8>(a, plan, ws, s);  // a multiple of 128: once per stage
     }
+}
+
+// The workgroups' shape by how many tiles the problem makes (n = 4096 and n = 11008, m = 16 .. 8192), for outputs of 192 tiles of 64 x 512 and more, and
+// where the workspace has no room for the estimate's choice below:
+//   up to 72 tiles of 32 rows: 32 rows x 64 columns per wave; beyond: 64 rows x 64 columns per wave, so that a converted weight fragment serves
+//       two row tiles, on activations converted once.
+// (Four waves of 64 x 128 each, two workgroups per CU, halve the LDS fragment reads but have
+// no registers left for pre-converted activations: 3-20 % slower from m = 1024 to 4096.)
+// The 64-row workgroups run one per CU, in rounds of 256 that last the same full or not (4096 x 11008, 1024 rows:
+// 352 workgroups take as long as 512).  When the last round would be poorly filled, the same tile with four
+// waves over 256 columns runs two per CU and a CU's last one alone at 3/4 of the time, while a pair costs 5 %
+// more than one eight-wave workgroup (1024 rows: 255 -> 220 us, 768: 251 -> 210, but 2048: 405 -> 425).  Same
+// order of the sums over K, same bits.
+static TilePlan plan_by_tiles(const W4Args& a) {
+    const uint64_t col_tiles = ceil_div(a.n, kTileCols), row_tiles = ceil_div(a.m, 64);
+    TilePlan plan{2, 8, 1, 1};
+    if (ceil_div(a.m, 32) * col_tiles <= 72) {
+        plan.rt = 1;
+    } else {
+        const uint64_t full_rounds = ceil_div(row_tiles * col_tiles, 256);
+        const uint64_t halves = ceil_div(row_tiles * ceil_div(a.n, kTileCols / 2), 256);       // on the busiest CU
+        if (row_tiles * col_tiles >= 192 && (halves / 2) * 105 + (halves % 2) * 75 < full_rounds * 97) plan.waves = 4;
+    }
+    plan.splits = pick_splits(plan.tiles(a), ceil_div(a.padded_k, kStageK), &plan.sps);
+    return plan;
+}
+
+// Fewer than 192 tiles of 64 x 512: the cheapest of four shapes and of the shares of K that make up to 512 workgroups.  `side` of them run side by side on a
+// compute unit; a stage of 128 k takes one `step` us (more with smaller groups: their sums are settled more often, and with the updates
+// for zero-points that may be fractions), `beside` of that more for each neighbour, a round `start` us besides; partial tiles are written, and added by one more
+// launch (`add`).  `pre`: the activations' conversion, per MB of x.  Fitted to 109 layers (9 to 1900 rows, K and N 512 to 11008), each with every shape and up to
+// 128, 256 and 512 workgroups (7 to 8 % rms): the choice is 0.7 % slower than the best of a layer on average, 9 % at worst; the rule above 6 %
+// and 64 %.  us there and here: 769 x 640 -> 2560 28.2, 17.2; 1533 x 768 -> 1856 31.4, 21.9; 535 x 512 -> 4864, groups of 32, 32.0, 21.6; 10 x 8192 ->
+// 2944, groups of 32, 28.9, 24.9.  An f32 sum runs over no more of K than by the rule above, or over 1024: beyond, its roundings would show, in a row
+// that one element dominates above all.
+static TilePlan plan_by_estimate(const W4Args& a, const TilePlan& known) {
+    struct Shape { uint32_t rt, waves, side; double base, step, beside, start, add, pre, small, rest; };
+    static const Shape shapes[] = {{1, 8, 1, 7.1, 1.67, 0.0, 3.8, 0.6, 0.45, 0.86, 0.19},
+                                   {2, 8, 1, 10.9, 2.48, 0.0, 2.3, 1.7, 0.83, 0.92, 0.26},
+                                   {2, 4, 3, 6.7, 1.85, 0.69, 5.9, 2.2, 0.72, 0.85, 0.17},
+                                   {1, 4, 2, 7.6, 1.53, 0.52, 2.2, 1.6, 0.44, 0.67, 0.01}};
+    auto cost = [&](const Shape& c, const TilePlan& plan) {
+        const double settle = c.small * (a.group_size == 32 ? 1.0 : a.group_size == 64 ? 0.4 : 0.0) + c.rest * (a.zp4 ? 0.0 : a.m < 128 ? 1.0 : 0.5);
+        const double stages = plan.sps * c.step * (1.0 + settle);
+        const uint32_t on_one = ceil_div(plan.tiles(a) * plan.splits, 256), last = on_one % c.side;
+        double us = c.base + c.pre * 4e-6 * a.m * a.k + on_one / c.side * (stages * (1.0 + (c.side - 1) * c.beside) + c.start);
+        if (last) us += stages * (1.0 + (last - 1) * c.beside) + c.start;
+        return plan.splits > 1 ? us + c.add + (plan.splits + 1.0) * a.m * a.n * 4 / 4.5e6 : us;
+    };
+    const uint32_t nstages = ceil_div(a.padded_k, kStageK);
+    TilePlan best = known;
+    double least = 1e30;
+    for (const Shape& c : shapes)
+        if (c.rt == known.rt && c.waves == known.waves) least = 0.96 * cost(c, known);           // a gain within the fit's error is none
+    for (const Shape& c : shapes) {
+        TilePlan plan{c.rt, c.waves, 1, nstages};
+        const uint32_t most = min(min((uint32_t)kMaxSplits, nstages), max(1u, 512 / plan.tiles(a)));
+        for (uint32_t want = 1; want <= most; want++) {
+            plan.sps = ceil_div(nstages, want);
+            plan.splits = ceil_div(nstages, plan.sps);           // no empty split
+            if (plan.sps > max(known.sps, 8u)) continue;
+            const double us = cost(c, plan);
+            if (us < least) { least = us; best = plan; }
+        }
+    }
+    return best;
 }
 
 int w4_launch_gemm(const W4Args& a, hipStream_t s) {
     RUMUS_REQUIRE((uint64_t)a.m * a.n < (1ull << 32), "qmatmul_int4: m * n must fit 32 bits");
     RUMUS_REQUIRE(a.m <= 65535 * 32, "qmatmul_int4: m %u is beyond the grid limit", a.m);
-    // Two shapes of workgroup, eight waves side by side over 512 columns, chosen by how many
-    // tiles the problem makes (measured on n = 4096 and n = 11008, m = 16 .. 8192):
-    //   up to 72 tiles of 32 rows: 32 rows x 64 columns per wave; the small tile keeps more
-    //       workgroups in flight when there are fewer tiles than CUs, and converts its few
-    //       activations itself;
-    //   beyond: 64 rows x 64 columns per wave, so that a converted weight fragment serves two row
-    //       tiles, on activations converted once by w4_convert_x_kernel.
-    // (Four waves of 64 x 128 each, two workgroups per CU, halve the LDS fragment reads but have
-    // no registers left for pre-converted activations: 3-20 % slower from m = 1024 to 4096.)
-    const uint64_t col_tiles = ceil_div(a.n, kTileCols);
-    if (ceil_div(a.m, 32) * col_tiles <= 72) return launch_fold<1, 1, 2, 8, 1>(a, s);
-    // The 64-row workgroups run one per CU, in rounds of 256 that last the same full or not (4096 x 11008, 1024 rows:
-    // 352 workgroups take as long as 512).  When the last round would be poorly filled, the same tile with four
-    // waves over 256 columns runs two per CU and a CU's last one alone at 3/4 of the time, while a pair costs 5 %
-    // more than one eight-wave workgroup (1024 rows: 255 -> 220 us, 768: 251 -> 210, but 2048: 405 -> 425).  Same
-    // order of the sums over K, same bits.
-    const uint64_t row_tiles = ceil_div(a.m, 64);
-    const uint64_t full_rounds = ceil_div(row_tiles * col_tiles, 256);
-    const uint64_t halves = ceil_div(row_tiles * ceil_div(a.n, kTileCols / 2), 256);       // on the busiest CU
-    if (row_tiles * col_tiles >= 192 && (halves / 2) * 105 + (halves % 2) * 75 < full_rounds * 97)
-        return launch_fold<2, 1, 2, 4, 1>(a, s);
-    return launch_fold<2, 1, 2, 8, 1>(a, s);
+    const TilePlan known = plan_by_tiles(a);
+    TilePlan plan = known;
+    if ((uint64_t)ceil_div(a.m, 64) * ceil_div(a.n, kTileCols) < 192) plan = plan_by_estimate(a, known);
+    const size_t want = tile_bytes(a, plan).all(), least = min(want, tile_bytes(a, known).all());
+    void* ws = nullptr;
+    size_t got = 0;
+    WorkspaceLease lease;                                    // until the last kernel of this call is queued
+    if (int rc = workspace_get_upto(s, least, want, &got, &ws, lease)) return rc;
+    if (got < want) plan = known;
+    if (plan.rt == 1) return plan.waves == 8 ? launch_fold<1, 1, 2, 8, 1>(a, plan, ws, s) : launch_fold<1, 1, 2, 4, 1>(a, plan, ws, s);
+    return plan.waves == 8 ? launch_fold<2, 1, 2, 8, 1>(a, plan, ws, s) : launch_fold<2, 1, 2, 4, 1>(a, plan, ws, s);
 }
 
 }  // namespace rumus

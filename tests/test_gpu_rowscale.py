@@ -26,7 +26,10 @@ def ops():
                                                # the launch of the rows' factors gathers or copies them: one round of 8192 columns, its edges,
                                                # two and three; with and without the look at the zero-points
                                                (10, 8192, 260, 32, True), (33, 8224, 132, 32, True), (140, 16416, 68, 32, True),
-                                               (40, 526, 260, 32, False), (130, 8190, 132, 32, False), (20, 64, 132, 32, True)])
+                                               (40, 526, 260, 32, False), (130, 8190, 132, 32, False), (20, 64, 132, 32, True),
+                                               # the four shapes of workgroup, K shared and not, a last tile of few columns
+                                               (769, 640, 2560, 128, False), (535, 512, 4868, 32, False), (10, 8192, 2948, 32, False), (883, 896, 1524, 128, False),
+                                               (1541, 768, 2304, 32, True), (232, 4480, 1124, 32, False), (967, 736, 4548, 128, False)])
 def test_rows_of_any_magnitude(ops, m, k, n, g, act_order):
     """Batches beyond 128 rows split x into two f16 planes: every row is first scaled by a power of two into
     f16's range, so rows of 1e-12, rows of 1e9 and a row with one element of 2e5 (beyond f16's 65504) come
