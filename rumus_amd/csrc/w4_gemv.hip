@@ -405,23 +405,36 @@ static int validate(const W4Args& a, const char* who) {
 // Rows of x up to which the decode kernels beat the two launches of the integer kernel (g128, from HBM, us, decode kernel / integer kernel):
 // 4 rows 4096 x 12288 12.2 / 14.4, 4096 x 22016 18.4 / 23.4, 11008 x 4096 11.1 / 17.8; 8 rows 4096 x 4096 7.6 / 9.2, 11008 x 4096 17.7 / 17.8, 4096 x
 // 12288 17.6 / 14.4: eight up to four million packed words, four beyond.  Act-order rows wait in LDS beside their digits, 128 KB in all, and
-// a call whose rows do not fit takes them in parts, a launch each (8 x 4096 x 4096 17.1 / 10.9): as many as fit at once.
+// a call whose rows do not fit takes them in parts, a launch each (8 x 4096 x 4096 17.1 / 10.9): as many as fit at once.  Every workgroup gathers
+// all rows: with more than 512 of them the integer kernel's gather, once a call, wins from two rows on (4096 x 11008 4 rows 21.7 / 15.9, 2 rows
+// 17.3 / 15.8; 2048 x 11008 8 rows 18.3 / 14.1, 4 rows 9.7), with more than 256 and a long K from three (8192 x 8192 3 rows 24.3 / 20.2, 2 rows 20.3; 8192 x
+// 4096 3 rows 15.2 / 17.3).
+static uint32_t w4_rows_that_gather(uint32_t padded_k, uint32_t n) {
+    if (n > 8192) return padded_k <= 1024 ? 8 : padded_k <= 2048 ? 4 : 1;
+    if (padded_k <= 4096) return padded_k <= 2048 ? 8 : 4;
+    return n > 4096 ? 2 : padded_k <= 6144 ? 4 : padded_k <= 8192 ? 3 : 2;
+}
 uint32_t w4_decode_max_rows(uint32_t padded_k, uint32_t n, bool perm) {
     const double mw = (double)(padded_k / 8) * n * 1e-6;
-    if (perm && padded_k > 2048) return padded_k <= 4096 ? 4 : 2;
-    return mw <= 4.0 ? 8 : 4;
+    const uint32_t plain = mw <= 4.0 ? 8 : 4;
+    return perm ? min(plain, w4_rows_that_gather(padded_k, n)) : plain;
+}
+static bool w4_few_rows(const W4Args& a) {
+    if (a.m <= w4_decode_max_rows(a.padded_k, a.n, a.perm) || !w4_gemm_supported(a)) return true;
+    // not the integer kernel's: the f16 tiles take longer (4096 x 11008, groups of 32: 3 rows 25.3, 4 rows 27.2 / 24.5)
+    return a.perm && a.group_size % 64 != 0 && a.m <= 3 && a.padded_k <= 4096;
 }
 
 bool w4_routes_to_i8(const W4Args& a) {
     if (a.m == 0 || a.n == 0 || a.k == 0) return false;
-    const bool few_rows = a.m <= w4_decode_max_rows(a.padded_k, a.n, a.perm) || !w4_gemm_supported(a);
+    const bool few_rows = w4_few_rows(a);
     return !(few_rows && (w4_gemv_dot8_supported(a) || w4_gemv_supported(a))) && !w4_gemm_f6_chosen(a) && w4_gemm_i8_supported(a);
 }
 
 static int dispatch(const W4Args& a, hipStream_t s) {
     if (a.m == 0 || a.n == 0) return RUMUS_HIP_OK;
     RUMUS_REQUIRE(a.k > 0, "qmatmul_int4: k must be > 0");
-    const bool few_rows = a.m <= w4_decode_max_rows(a.padded_k, a.n, a.perm) || !w4_gemm_supported(a);
+    const bool few_rows = w4_few_rows(a);
     if (few_rows && w4_gemv_dot8_supported(a)) return w4_launch_gemv_dot8(a, s);
     if (few_rows && w4_gemv_supported(a)) return w4_launch_gemv(a, s);
     if (w4_gemm_f6_chosen(a)) return w4_launch_gemm_f6(a, s);

@@ -494,14 +494,19 @@ static int w4m_launch(const W4mArgs& a, hipStream_t s) {
     if (a.group_size % 64 == 0) return w4m_queue<&w4_gemv_mfma_kernel<MB, Q, 2, IN, S, U>>(grid, block, lds, a, s);
     return w4m_queue<&w4_gemv_mfma_kernel<MB, Q, 4, IN, S, U>>(grid, block, lds, a, s);
 }
-// Units of 128 k where 256 would leave waves without one; two in flight where the eight waves have more than that.
+// Of one launch's LDS: digits of the units in flight, and an act-order call's rows.
+static size_t w4m_gather_lds(uint32_t m, uint32_t k, uint32_t flight) {
+    return (size_t)kW4mWaves * flight * (m > 4 ? 2 : 1) * 4096 + (size_t)m * k * sizeof(float);
+}
+// Units of 128 k where 256 would leave waves without one; two in flight where the eight waves have more than that and the rows of
+// an act-order call leave room for both.
 template <int MB, int Q, W4mIn IN>
 static int w4m_sweep(const W4mArgs& a, hipStream_t s) {
     const uint32_t units = ceil_div(a.padded_k, 256);
     if (2 * units <= kW4mWaves) return w4m_launch<MB, Q, IN, 2, 1>(a, s);
     constexpr bool kTwo = MB * (IN == kW4mGlu ? 2 : 1) <= 2;       // (LDS)
     if constexpr (kTwo) {
-        if (units > kW4mWaves) return w4m_launch<MB, Q, IN, 4, 2>(a, s);
+        if (units > kW4mWaves && (IN != kW4mPerm || w4m_gather_lds(a.m, a.k, 2) <= kW4mLds)) return w4m_launch<MB, Q, IN, 4, 2>(a, s);
     }
     return w4m_launch<MB, Q, IN, 4, 1>(a, s);
 }
@@ -534,9 +539,7 @@ int w4_launch_gemv_mfma(const W4Args& a, const float* norm_w, float eps, const f
     // act-order rows are gathered from LDS; where all of them do not fit beside the digits, fewer at a time
     uint32_t part = a.m;
     if (a.perm && rows && (reinterpret_cast<uintptr_t>(a.perm) & 15) == 0) {
-        auto fits = [&](uint32_t m) {
-            return (size_t)kW4mWaves * (a.padded_k > 256 * kW4mWaves ? 2 : 1) * (m > 4 ? 2 : 1) * 4096 + (size_t)m * a.k * sizeof(float) <= kW4mLds;
-        };
+        auto fits = [&](uint32_t m) { return w4m_gather_lds(m, a.k, 1) <= kW4mLds; };
         if (!fits(part)) part = fits(4) ? 4 : fits(2) ? 2 : fits(1) ? 1 : 0;
     } else if (a.perm) {
         part = 0;
