@@ -67,7 +67,8 @@ def test_few_rows_against_float64(ops, m, k, n, g, tiled):
         np.testing.assert_array_equal(host(ops.qmatmul_int4_f16(dev(xh), *d, k, g)), f32.astype(np.float16))
 
 
-@pytest.mark.parametrize("m,k", [(2, 256), (8, 2048), (4, 4096), (8, 4096), (3, 8192), (5, 12288), (2, 16384), (2, 32768)])
+@pytest.mark.parametrize("m,k", [(2, 256), (8, 2048), (4, 4096), (8, 4096), (3, 8192), (5, 12288), (2, 16384), (2, 32768),
+                                 (4, 6144), (4, 6272), (3, 8320), (2, 12288), (2, 12416)])
 def test_act_order_rows_in_parts(ops, m, k):
     n, g = 48, 128
     say(f"few rows act-order m={m} k={k}")
