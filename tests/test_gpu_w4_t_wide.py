@@ -11,7 +11,9 @@ pytestmark = pytest.mark.gpu
 # n: one step of 16 (three of a workgroup's waves have none), two, five, six; 8 and 9 steps a wave in one share, shares of a few steps;
 # m: one row past the smallest batch, a tile of 64, one over it, several; k: part of a tile of 128, groups of 128 and 256
 @pytest.mark.parametrize("n", [16, 32, 80, 96, 512, 560, 2064])
-@pytest.mark.parametrize("m,k,g", [(33, 256, 128), (64, 128, 128), (65, 388, 128), (200, 512, 256), (129, 1500, 128)])
+@pytest.mark.parametrize("m,k,g", [(33, 256, 128), (64, 128, 128), (65, 388, 128), (200, 512, 256), (129, 1500, 128),
+                                   # the first three, with weights that the vector kernel does not take
+                                   (33, 3072, 128), (64, 2048, 128), (65, 1924, 128)])
 def test_grad_x_wide(m, k, n, g):
     from rumus_amd import ops
     say(f"qmatmul_int4_t wide m={m} k={k} n={n} g={g}")
