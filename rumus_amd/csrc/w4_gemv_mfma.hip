@@ -99,14 +99,19 @@ __global__ __launch_bounds__(kW4mThreads) void w4_gemv_mfma_kernel(W4mArgs a) {
     const uint32_t word_rows = a.padded_k / 8, num_groups = a.padded_k / a.group_size;
     const uint32_t units = (a.padded_k + 64 * S - 1) / (64 * S);
     const uint32_t tile = xcd_contiguous(blockIdx.x, (a.n + 16 * Q - 1) / (16 * Q));
-    // All arrays are read as buffers: an offset per lane that stays, one per wave (scalar), zeros beyond the end.  (gfx9 descriptor: no
-    // swizzle, raw 32-bit data.)  Per lane: where its column starts (a column past n: that of the last).
-    const auto array = [](const void* p, uint64_t bytes) __attribute__((always_inline)) {
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)(uint32_t)bytes, 0x00027000);
+    // All arrays are read as buffers: an offset per lane that stays, and zeros where it lies beyond the end.  (gfx9 descriptor: no
+    // swizzle, raw 32-bit data.)  A scalar offset is no part of that check, so what a step of K adds is taken off the buffer
+    // itself; of one past the end nothing is left.  Per lane: where its column starts (a column past n: that of the last).
+    const auto array = [](const void* p, uint32_t bytes) __attribute__((always_inline)) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);
+    };
+    const auto beyond = [&](const void* p, uint32_t bytes, uint32_t from) __attribute__((always_inline)) {
+        from = min(from, bytes);
+        return array(static_cast<const uint8_t*>(p) + from, bytes - from);
     };
     const uint32_t row_bytes = a.n * 4, word_row = a.tiled ? 64 : row_bytes, zp_row = a.zp4 ? word_row / 8 : word_row;
-    const auto b_packed = array(a.packed, (uint64_t)word_rows * row_bytes), b_scales = array(a.scales, (uint64_t)num_groups * row_bytes);
-    const auto b_zps = array(a.zps, (uint64_t)num_groups * (a.zp4 ? row_bytes / 8 : row_bytes));
+    const uint32_t packed_bytes = word_rows * row_bytes;
+    const auto b_scales = array(a.scales, num_groups * row_bytes), b_zps = array(a.zps, num_groups * (a.zp4 ? row_bytes / 8 : row_bytes));
     uint32_t words_at[Q], meta_at[Q], zp_at[Q];
 #pragma unroll
     for (int q = 0; q < Q; q++) {
@@ -127,9 +132,7 @@ __global__ __launch_bounds__(kW4mThreads) void w4_gemv_mfma_kernel(W4mArgs a) {
     const uint32_t even_at = quad * 16 + (d >> 1) * 8 + (d & 1) * 2, k_of = kb * 16 + (d >> 1) * 8 + (d & 1);   // k of a step: k_of + 0, 2, 4, 6
     const uint32_t k_in = kb * 16 + 4 * d;                         // what a lane reads of a step: k_in + 0, 1, 2, 3
     constexpr uint32_t kBytes = IN == kW4mHalf ? 2 : 4;
-    const auto b_x = array(a.x, (uint64_t)a.m * (kSrc * a.k) * kBytes);
-    const auto b_perm = array(kGather ? a.perm : nullptr, kGather ? (uint64_t)a.k * 4 : 0);
-    const auto b_norm = array(IN == kW4mNorm ? a.norm_w : nullptr, IN == kW4mNorm ? (uint64_t)a.k * 4 : 0);
+    const uint32_t x_bytes = a.m * (kSrc * a.k) * kBytes;
     const uint32_t x_at[2] = {(row_of[0] * (kSrc * a.k) + k_in) * kBytes, (row_of[1] * (kSrc * a.k) + k_in) * kBytes};
     float* const staged = reinterpret_cast<float*>(w4m_lds + kW4mWaves * U * MB * kSrc * kPart);
 
@@ -233,12 +236,15 @@ __global__ __launch_bounds__(kW4mThreads) void w4_gemv_mfma_kernel(W4mArgs a) {
     };
     auto load_weights = [&](uint32_t c, uint32_t (&w)[S][2][Q], float (&sc)[kFolds][Q], uint32_t (&z)[kFolds][Q]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int s = 0; s < S; s++)
+        for (int s = 0; s < S; s++) {
+            const uint32_t step = c * S + s;               // (word rows come in fours: a lane's second is there if its first is)
+            const auto b_packed = beyond(a.packed, packed_bytes, step * 64 < a.padded_k ? step * 8 * word_row : packed_bytes);
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
                 for (int q = 0; q < Q; q++)
-                    w[s][i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(b_packed, (int)words_at[q], (int)(((c * S + s) * 8 + i) * word_row), 0);
+                    w[s][i][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(b_packed, (int)words_at[q], (int)(i * word_row), 0);
+        }
 #pragma unroll
         for (int p = 0; p < kFolds; p++) {
             const uint32_t k32 = c * (2 * S) + p * (4 / G);
@@ -262,27 +268,29 @@ __global__ __launch_bounds__(kW4mThreads) void w4_gemv_mfma_kernel(W4mArgs a) {
         for (int u = 0; u < U; u++)
 #pragma unroll
             for (int s = 0; s < S; s++) {
-                const uint32_t step = ((c0 + u) * S + s) * 64;
+                const uint32_t step = ((c0 + u) * S + s) * 64, in_row = min(step, a.k);   // (a row's end: the next one's start, or the end)
+                const auto b_x = beyond(a.x, x_bytes, step < a.k ? step * kBytes : x_bytes);
 #pragma unroll
                 for (int b = 0; b < MB; b++) {
                     v4i& v = raw[u][s][b][0];
                     if constexpr (kGather) {
-                        if (b == 0) v = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(b_perm, (int)(k_in * 4), (int)(step * 4), 0));
+                        if (b == 0) v = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(beyond(a.perm, a.k * 4, in_row * 4), (int)(k_in * 4), 0, 0));
                     } else if constexpr (IN == kW4mHalf) {
-                        const v4h f = __builtin_bit_cast(v4h, __builtin_amdgcn_raw_buffer_load_b64(b_x, (int)x_at[b], (int)(step * 2), 0));
+                        const v4h f = __builtin_bit_cast(v4h, __builtin_amdgcn_raw_buffer_load_b64(b_x, (int)x_at[b], 0, 0));
                         v = v4i{__float_as_int((float)f[0]), __float_as_int((float)f[1]), __float_as_int((float)f[2]), __float_as_int((float)f[3])};
                     } else if constexpr (IN == kW4mAny) {
                         const uint32_t k0 = step + k_in;
                         v = v4i{__float_as_int(element(row_of[b], k0)), __float_as_int(element(row_of[b], k0 + 1)),
                                 __float_as_int(element(row_of[b], k0 + 2)), __float_as_int(element(row_of[b], k0 + 3))};
                     } else {                                       // (k % 4 == 0)
-                        v = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(b_x, (int)x_at[b], (int)(step * 4), 0));
+                        v = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(b_x, (int)x_at[b], 0, 0));
                         if constexpr (IN == kW4mGlu)
-                            raw[u][s][b][1] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(b_x, (int)x_at[b], (int)((step + a.k) * 4), 0));
+                            raw[u][s][b][1] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
+                                beyond(a.x, x_bytes, step < a.k ? (step + a.k) * 4 : x_bytes), (int)x_at[b], 0, 0));
                     }
                 }
                 if constexpr (IN == kW4mNorm)
-                    nw[u][s] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(b_norm, (int)(k_in * 4), (int)(step * 4), 0));
+                    nw[u][s] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(beyond(a.norm_w, a.k * 4, in_row * 4), (int)(k_in * 4), 0, 0));
             }
         if (base == 0) {
             __builtin_amdgcn_sched_barrier(0);

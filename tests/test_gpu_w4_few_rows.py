@@ -117,3 +117,54 @@ def test_not_finite_and_tiny(ops):
     got = host(ops.qmatmul_int4(dev(x), dev(packed), dev(scales), dev(zp), k, g))
     assert not np.isfinite(got[1:3]).any()
     check(got[[0, 3]], x[[0, 3]], w)
+
+
+# K of which the last sweep leaves units without elements, and a unit that ends inside a step of 64: every array the last thing in its
+# memory but for NaNs, which none of those may read
+@pytest.mark.parametrize("m,k,n,g", [(4, 4224, 12288, 128), (8, 2304, 8192, 128), (3, 1056, 48, 32), (6, 4192, 64, 32)])
+@pytest.mark.parametrize("form", ["plain", "tiled", "zp4", "act", "half", "norm", "glu"])
+def test_units_past_the_end(ops, m, k, n, g, form):
+    import torch
+    say(f"few rows, units past the end m={m} k={k} n={n} g={g} {form}")
+    gen = torch.Generator(device="cuda").manual_seed(m + k + n)
+
+    def last(t):
+        room = torch.full((t.numel() + 4096,), float("nan") if t.is_floating_point() else 0x7FC00000, dtype=t.dtype, device="cuda")
+        room[:t.numel()] = t.reshape(-1)
+        return room[:t.numel()].view(t.shape)
+
+    packed = torch.randint(-2 ** 31, 2 ** 31 - 1, (k // 8, n), generator=gen, device="cuda", dtype=torch.int32)
+    scales = 0.01 + 0.01 * torch.rand((k // g, n), generator=gen, device="cuda")
+    zp = torch.randint(0, 16, (k // g, n), generator=gen, device="cuda").float()
+    x = torch.randn((m, k), generator=gen, device="cuda")
+    perm = torch.randperm(k, generator=gen, device="cuda")
+    q = torch.stack([(packed >> (4 * i)) & 15 for i in range(8)], 1).reshape(k, n).double()
+    w = (q - zp.double().repeat_interleave(g, 0)) * scales.double().repeat_interleave(g, 0)
+    d = [last(t) for t in (packed, scales, zp)]
+    tiled = [last(t) for t in ops.w4_decode_layout(*d, g)]
+    if form == "plain":
+        got = ops.qmatmul_int4(last(x), *d, k, g)
+    elif form == "tiled":
+        got = ops.qmatmul_int4_decode(last(x), *tiled, k, g)
+    elif form == "zp4":
+        z4 = zp.to(torch.int64).view(k // g, n // 8, 8)
+        z4 = sum(z4[..., i] << (4 * i) for i in range(8))
+        got = ops.qmatmul_int4_zp4(last(x), d[0], d[1], last(torch.where(z4 >= 2 ** 31, z4 - 2 ** 32, z4).to(torch.int32)), k, g)
+    elif form == "act":
+        got = ops.qmatmul_int4_decode(last(x), *tiled, k, g, perm=last(perm.to(torch.int32)))
+        x = x[:, perm]
+    elif form == "half":
+        x = x.half()
+        got = ops.qmatmul_int4_f16(last(x), *d, k, g).float()
+    elif form == "norm":
+        scale = 1.0 + 0.1 * torch.randn(k, generator=gen, device="cuda")
+        got = ops.qmatmul_int4_decode_block(last(x), *tiled, k, g, norm_weight=last(scale), eps=1e-6)
+        x = x.double() * scale.double() / (x.double().square().mean(1, keepdim=True) + 1e-6).sqrt()
+    else:
+        up = torch.randn((m, k), generator=gen, device="cuda")
+        got = ops.qmatmul_int4_decode_block(last(torch.cat([x, up], 1)), *tiled, k, g, swiglu=True)
+        x = x.double() * torch.sigmoid(x.double()) * up.double()
+    want = x.double() @ w
+    # activations within 2^-20 of their unit's largest, f32 around them; one rounding to f16
+    bound = (2.0 ** -11 if form == "half" else 2.0 ** -18) * (x.double().abs() @ w.abs() + x.double().abs().amax(1, keepdim=True) * w.abs().sum(0))
+    assert float(((got.double() - want).abs() / bound).max()) <= 1.0
