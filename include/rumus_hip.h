@@ -264,7 +264,7 @@ int rumus_hip_f16_to_f32(const uint16_t* in, float* out, uint64_t numel,
  * 128 rows (up to 1024 where the integer matrix-core kernel is the faster one:
  * group_size % 64 == 0 and enough columns to fill the chip) x is held in fixed
  * point below the largest magnitude of a part of the row (20 bits per 32 k for
- * one row, or two of a long K; 21 bits per 128 or 256 k up to decode_max_rows
+ * one row, or two of a long K; 22 bits per 128 or 256 k up to decode_max_rows
  * rows, 22 bits per eighth of K beyond):
  * |error| <= max|x| * 2^-19 * sum|w| over that part.  Where elements
  * tower over their part by 2^8 or more the small ones keep their bits (in the

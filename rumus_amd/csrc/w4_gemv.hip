@@ -419,8 +419,19 @@ uint32_t w4_decode_max_rows(uint32_t padded_k, uint32_t n, bool perm) {
     const uint32_t plain = mw <= 4.0 ? 8 : 4;
     return perm ? min(plain, w4_rows_that_gather(padded_k, n)) : plain;
 }
+// Row-major arrays of wide weights are read in pieces of 128 bytes of every word row, with groups of 64 twice as many of the scales; rows a multiple of 8 KB
+// long fall on the same memory channels besides.  There the integer kernel, which reads a row's pieces side by side, is ahead from three rows on, beyond 19
+// million words from two (us, decode kernel / integer kernel: groups of 64, 3 x 4096 x 10240 15.2 / 13.6, but 4096 x 9216 13.4 / 13.4; 4 x 4096 x 28672
+// 29.8 / 25.4, 2 x 8192 x 28672 46.8 / 39.1; groups of 128, 2 x 8192 x 28672 42.3 / 38.6, but 8192 x 22016 31.1 / 34.9).
+static uint32_t w4_max_rows(const W4Args& a) {
+    const uint32_t rows = w4_decode_max_rows(a.padded_k, a.n, a.perm);
+    if (a.tiled || a.perm || a.group_size % 64 != 0 || a.padded_k <= 2048) return rows;
+    const bool large = (uint64_t)(a.padded_k / 8) * a.n > 19000000;
+    if (a.group_size % 128 == 0) return large && a.n > 24576 ? 1 : rows;
+    return a.n >= 12288 || (a.n > 8192 && a.n % 2048 == 0) ? (large ? 1 : 2) : rows;
+}
 static bool w4_few_rows(const W4Args& a) {
-    if (a.m <= w4_decode_max_rows(a.padded_k, a.n, a.perm) || !w4_gemm_supported(a)) return true;
+    if (a.m <= w4_max_rows(a) || !w4_gemm_supported(a)) return true;
     // not the integer kernel's: the f16 tiles take longer (4096 x 11008, groups of 32: 3 rows 25.3, 4 rows 27.2 / 24.5)
     return a.perm && a.group_size % 64 != 0 && a.m <= 3 && a.padded_k <= 4096;
 }
@@ -519,7 +530,7 @@ int rumus_hip_qmatmul_int4_f16(const uint16_t* x, const uint32_t* packed, const 
         a.y16 = reinterpret_cast<_Float16*>(y);
         a.x = nullptr;
         a.y = nullptr;
-        if (m <= w4_decode_max_rows(padded_k, n, false) && w4_gemv_half_takes(a)) return w4_launch_gemv_half(a, as_stream(stream));
+        if (m <= w4_max_rows(a) && w4_gemv_half_takes(a)) return w4_launch_gemv_half(a, as_stream(stream));
         if (w4_routes_to_i8(a)) return w4_launch_gemm_i8(a, as_stream(stream));
     }
     return w4_f16_staged(x, packed, scales, zero_points, bias, g_idx, y, m, k, n, padded_k, group_size, num_groups, stream);

@@ -496,8 +496,9 @@ static int launch_m(const W4Args& a, hipStream_t s) {
 }
 
 // Two rows of a plain weight with a long K stay here: the conversion of four rows, half of it for rows that are not there, is longer than two planes.
-// 2 x 2048 x 2048 4.5 us here, 3.7 on the matrix cores; 2 x 6528 x 512 6.8 and 7.2, 2 x 4096 x 12288 10.9 and 12.2.
-static bool w4_two_rows_long(const W4Args& a) { return a.m == 2 && a.padded_k > 2048 && !a.perm; }
+// 2 x 2048 x 2048 4.5 us here, 3.7 on the matrix cores; 2 x 6528 x 512 6.8 and 7.2, 2 x 4096 x 12288 10.9 and 12.2.  Beyond 19 million words the weight
+// is read for longer than either takes, and the matrix cores keep two bits more of the rows.
+static bool w4_two_rows_long(const W4Args& a) { return a.m == 2 && a.padded_k > 2048 && !a.perm && (uint64_t)(a.padded_k / 8) * a.n <= 19000000; }
 // f16 rows and result, row-major arrays with f32 zero-points: a call that came here in f32, k % 8 == 0 and 16-byte aligned rows
 template <int M>
 static int launch_half_m(const W4Args& a, hipStream_t s) {

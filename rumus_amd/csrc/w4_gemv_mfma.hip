@@ -2,7 +2,7 @@
 //
 //   y[m,n] = sum_c 2^-e[m,c] sum_{g in c} scale[g,n] * ( sum_{k in g} X[m,k] q[k,n]  -  zp[g,n] * sum_{k in g} X[m,k] )
 //
-// over units c of 128 or 256 consecutive k, with X = rint(x 2^e), e from the unit's largest magnitude, whose X is 2^20 to 2^21.
+// over units c of 128 or 256 consecutive k, with X = rint(x 2^e), e from the unit's largest magnitude, whose X is 2^21 to 2^22 (all but: w4m_digits).
 // X = d0 + 2^8 d1 + 2^16 d2 in signed bytes, and the sixteen rows of v_mfma_i32_16x16x64_i8 are three digits of four rows of x and, fourth, ones.
 // In its accumulator layout a lane then holds all digits' sums of one output, so folding a group takes eight vector instructions per
 // output and no exchange, and four rows cost the matrix cores what one does.
@@ -179,8 +179,9 @@ __global__ __launch_bounds__(kW4mThreads) void w4_gemv_mfma_kernel(W4mArgs a) {
         top = max(r[0], r[1]);
         const auto h = __builtin_amdgcn_permlane32_swap(top, top, false, false);
         top = max(h[0], h[1]);
-        // 2^(20 - E) for a largest magnitude in [2^E, 2^(E+1)); at most 2^126, its reciprocal is a normal number then
-        const uint32_t bits = min((274u << 23) - (top & 0x7f800000u), 253u << 23);
+        // 2^(21 - E) for a largest magnitude in [2^E, 2^(E+1)), half of that from 2^(E+1) (1 - 2^-6) on: |X| stays below 2^22 - 2^16, and byte 2
+        // of what w4m_digits adds up below 128.  At most 2^126, its reciprocal is a normal number then.
+        const uint32_t bits = min((275u << 23) - ((top + (1u << 18)) & 0x7f800000u), 253u << 23);
         f = __uint_as_float(bits);
         back = top >= 0x7f800000u ? __uint_as_float(0x7fc00000u) : __uint_as_float((254u << 23) - bits);
         return top;

@@ -168,3 +168,30 @@ def test_units_past_the_end(ops, m, k, n, g, form):
     # activations within 2^-20 of their unit's largest, f32 around them; one rounding to f16
     bound = (2.0 ** -11 if form == "half" else 2.0 ** -18) * (x.double().abs() @ w.abs() + x.double().abs().amax(1, keepdim=True) * w.abs().sum(0))
     assert float(((got.double() - want).abs() / bound).max()) <= 1.0
+
+
+# Activations of 22 bits, odd multiples of 2^-21 below 1.96, of which a column adds up four: 24 bits, nothing is rounded.  With activations cut
+# to 21 bits every one of them would be off by 2^-22.
+@pytest.mark.parametrize("m,k,n,g,form", [
+    (2, 512, 32, 128, "plain"), (2, 2048, 48, 64, "tiled"), (3, 4224, 36, 128, "plain"), (4, 1024, 20, 32, "plain"), (8, 4096, 4096, 128, "tiled"),
+    (5, 2304, 8224, 128, "plain"), (4, 4096, 11008, 128, "plain"), (3, 1001, 16, 256, "plain"), (6, 2048, 64, 128, "act"), (4, 4096, 48, 64, "act"),
+    # two rows of a weight that is read for longer than the rows are converted
+    (2, 16384, 9616, 128, "plain")])
+def test_bits_of_the_activations(ops, m, k, n, g, form):
+    say(f"few rows, 22 bits m={m} k={k} n={n} g={g} {form}")
+    rng = np.random.default_rng(m + k + n)
+    words = -(-k // g) * g // 8
+    at = np.stack([rng.choice(k, 4, replace=False) for _ in range(n)], 1)        # a column's four weights of one
+    packed = np.zeros((words, n), np.uint32)
+    np.bitwise_or.at(packed, (at // 8, np.arange(n)), np.uint32(1) << (4 * (at % 8)).astype(np.uint32))
+    scales, zp = np.ones((words * 8 // g, n), np.float32), np.zeros((words * 8 // g, n), np.float32)
+    d = [dev(a) for a in (packed, scales, zp)]
+    x = ((4.0 * rng.integers(-2 ** 18, 2 ** 18, (m, k)) + 1.0) * 2.0 ** -21).astype(np.float32)
+    large = x[:, ::64].shape
+    x[:, ::64] = (4.0 * rng.integers(2 ** 19, int(1.96 * 2 ** 19), large) + 1.0) * 2.0 ** -21 * rng.choice([-1.0, 1.0], large)
+    perm = rng.permutation(k) if form == "act" else np.arange(k)
+    if form == "plain":
+        got = host(ops.qmatmul_int4(dev(x), *d, k, g))
+    else:
+        got = host(ops.qmatmul_int4_decode(dev(x), *ops.w4_decode_layout(*d, g), k, g, perm=dev(perm.astype(np.int32)) if form == "act" else None))
+    np.testing.assert_array_equal(got, x[:, perm].astype(np.float64)[:, at].sum(axis=1))
