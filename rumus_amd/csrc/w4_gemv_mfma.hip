@@ -78,6 +78,10 @@ __device__ __forceinline__ uint32_t w4m_largest(const float (&v)[4]) {
 __device__ __forceinline__ float w4m_sum(const v4i& c) {      // of the digits' sums: exact but for two roundings
     return fmaf((float)(c[2] - 64 * c[3]), 65536.0f, (float)((c[1] << 8) + c[0]));
 }
+// the same where zero-points of up to 1023 have been taken off: 128 products of a digit then make up to 2^24, and not 256 times that in 32 bits
+__device__ __forceinline__ float w4m_wide_sum(const v4i& c) {
+    return fmaf((float)(c[2] - 64 * c[3]), 65536.0f, fmaf((float)c[1], 256.0f, (float)c[0]));
+}
 
 // MB: blocks of four rows.  Q: column tiles of 16.  S: steps of 64 k per unit.  G: groups per 128 k that a fold tells apart, 1, 2 or 4 (a group
 // of 32: the halves of a step are multiplied with the other half's digits zeroed).  U: units in flight.  The last unit may reach beyond K.
@@ -231,7 +235,7 @@ __global__ __launch_bounds__(kW4mThreads) void w4_gemv_mfma_kernel(W4mArgs a) {
 #pragma unroll
                     for (int i = 0; i < 4; i++) sq[i] -= (int)whole * sx[i];
                 }
-                to[q] = fmaf(fmaf(-rest, sum, w4m_sum(sq)) * sc[p][q], back, to[q]);
+                to[q] = fmaf(fmaf(-rest, sum, EXACT.value ? w4m_wide_sum(sq) : w4m_sum(sq)) * sc[p][q], back, to[q]);
             }
         }
     };

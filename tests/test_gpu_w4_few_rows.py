@@ -195,3 +195,23 @@ def test_bits_of_the_activations(ops, m, k, n, g, form):
     else:
         got = host(ops.qmatmul_int4_decode(dev(x), *ops.w4_decode_layout(*d, g), k, g, perm=dev(perm.astype(np.int32)) if form == "act" else None))
     np.testing.assert_array_equal(got, x[:, perm].astype(np.float64)[:, at].sum(axis=1))
+
+
+@pytest.mark.parametrize("m,k,g", [(8, 256, 128), (4, 1024, 64), (8, 2304, 128), (7, 512, 32)])
+@pytest.mark.parametrize("large", [240.0, 700.0, 1000.0])
+def test_elements_far_apart_and_zero_points_far_away(ops, m, k, g, large):
+    """Rows of one value and a few tiny ones, zero-points of several hundred: the digits' sums times the zero-points."""
+    say(f"few rows far apart m={m} k={k} g={g}, zero-points up to {large}")
+    n = 32
+    rng = np.random.default_rng(m + k)
+    packed, scales, zp, _ = weights(rng, k, n, g)
+    zp = (large * rng.uniform(0.9, 1.0, zp.shape) * rng.choice([-1.0, 1.0], zp.shape)).astype(np.float32)
+    q = oracle.w4_unpack(packed, packed.shape[0] * 8).astype(np.float64)[:k]
+    rows = np.arange(k) // g
+    w = (q - zp[rows].astype(np.float64)) * scales[rows].astype(np.float64)
+    x = np.repeat(np.linspace(1.0, 1.95, m * 16).astype(np.float32).reshape(16, m, 1), k, axis=2)
+    x[:, :, np.arange(k) % 64 < 8] *= np.float32(2.0 ** -12)     # all elements of some lanes: every unit is multiplied in parts then
+    d = [dev(a) for a in (packed, scales, zp)]
+    for rows_of in x:
+        got = host(ops.qmatmul_int4(dev(rows_of), *d, k, g))
+        check(got, rows_of, w)
