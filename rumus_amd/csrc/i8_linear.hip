@@ -91,7 +91,8 @@ __global__ __launch_bounds__(512) void i8_linear_kernel(const float* __restrict_
         for (int i = 0; i < NV; i++) {
             const uint32_t kk = k0 + i * 256 + lane * 4;
             const float4 v = make_float4(__int_as_float(raw[r][i][0]), __int_as_float(raw[r][i][1]), __int_as_float(raw[r][i][2]), __int_as_float(raw[r][i][3]));
-            if (kk < steps * 64) *reinterpret_cast<uint32_t*>(xs + row * pitch + kk) = pack_i8x4(v, inv);
+            // (zeros from K on as such: in a row of 1e-37 `inv` is an infinity, and its product with zero no number)
+            if (kk < steps * 64) *reinterpret_cast<uint32_t*>(xs + row * pitch + kk) = kk < K ? pack_i8x4(v, inv) : 0u;
         }
     }
     __syncthreads();

@@ -49,6 +49,18 @@ def test_i8_linear_rows_that_are_not_finite(ops):
     assert torch.equal(torch.nan_to_num(ops.i8_linear(x, wq, sw), nan=7.0), torch.nan_to_num(want, nan=7.0))
 
 
+# 127 / 1e-37 is an infinity: what stands between the end of a row and that of its last step of 64 has to be zero all the same
+@pytest.mark.parametrize("m,k,n", [(1, 80, 40), (1, 8208, 20), (2, 1040, 33), (3, 4112, 17), (5, 1040, 40), (8, 2064, 33), (12, 16, 5), (16, 1040, 18)])
+def test_i8_linear_rows_of_tiny_values(ops, m, k, n):
+    say(f"i8_linear m={m} k={k} n={n}, rows of 1e-37")
+    x, wq, sw, bias = operands(m, k, n)
+    x[::2] = 1e-37
+    xq, sx = ops.i8_quantize_rows(x)
+    for b in (None, bias):
+        want, _ = ops.i8_gemm(xq, wq, sx, sw, b)
+        assert torch.equal(ops.i8_linear(x, wq, sw, b), want)
+
+
 def test_i8_linear_from_rows_of_any_alignment(ops):
     say("i8_linear, x at an odd float")
     x, wq, sw, bias = operands(3, 528, 200)
