@@ -779,7 +779,7 @@ bool w4_gemm_t_supported(uint32_t m, uint32_t k, uint32_t n, uint32_t group_size
 struct W4tShares { uint32_t shares; double us; };
 static W4tShares w4t_wide_shares(uint32_t tiles, uint32_t m, uint32_t k, uint32_t n) {
     W4tShares best{1, 1e30};
-    for (uint32_t shares = 1; shares <= (uint32_t)kTMaxSplits && n / 16 >= 8 * shares; shares++) {
+    for (uint32_t shares = 1; shares == 1 || (shares <= (uint32_t)kTMaxSplits && n / 16 >= 8 * shares); shares++) {
         const double us = 8.7 + (double)ceil_div(tiles * shares, 256) * ceil_div(n / 16, 4 * shares) * 0.48 + (shares > 1 ? 3.0 + (shares + 1.0) * m * k * 4 / 4.5e6 : 0.0);
         if (us < best.us) best = W4tShares{shares, us};
     }

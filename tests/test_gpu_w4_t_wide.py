@@ -8,6 +8,25 @@ from gpu_util import dev, host, say
 pytestmark = pytest.mark.gpu
 
 
+def takes_the_matrix_cores(m, k, n, g):
+    """Whether the call wants workspace, which the vector kernel does not: asked for on a stream that has none and is being captured."""
+    import torch
+    from rumus_amd import ops
+    words = torch.zeros((k // 8, n), dtype=torch.int32, device="cuda")
+    meta = torch.ones((-(-k // g), n), dtype=torch.float32, device="cuda")
+    gy, out = torch.zeros((m, n), device="cuda"), torch.empty((m, k), device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        out.zero_()
+        try:
+            ops.qmatmul_int4_t(gy, words, meta, meta, k, g, out=out)
+        except ops.RumusError as e:
+            assert "workspace of" in str(e)
+            return True
+    return False
+
+
 # n: one step of 16 (three of a workgroup's waves have none), two, five, six; 8 and 9 steps a wave in one share, shares of a few steps;
 # m: one row past the smallest batch, a tile of 64, one over it, several; k: part of a tile of 128, groups of 128 and 256
 @pytest.mark.parametrize("n", [16, 32, 80, 96, 512, 560, 2064])
@@ -39,3 +58,15 @@ def test_grad_x_wide(m, k, n, g):
     assert err.max() < 2e-5
     assert not got[2].any()
     assert not np.isfinite(got[4]).any() and not np.isfinite(got[m - 1]).any()
+
+
+# few columns: the last three weights of the test above at each of its n, and one of 512 tiles and more
+@pytest.mark.parametrize("m,k,n", [(m, k, n) for n in (16, 32, 80, 96, 512, 560, 2064) for m, k in ((33, 3072), (64, 2048), (65, 1920))] +
+                         [(512, 4096, 112), (256, 11008, 112), (384, 11008, 112)])
+def test_few_columns_take_the_matrix_cores(m, k, n):
+    say(f"qmatmul_int4_t route m={m} k={k} n={n}")
+    assert takes_the_matrix_cores(m, k, n, 128)
+
+
+def test_few_columns_of_many_tiles():
+    test_grad_x_wide(384, 11008, 112, 128)
