@@ -82,6 +82,8 @@ bool w4_gemv_half_takes(const W4Args& a);
 int w4_launch_gemv_half(const W4Args& a, hipStream_t s);
 int w4_launch_gemv_mfma(const W4Args& a, const float* norm_w, float eps, const float* resid, hipStream_t s);
 
+// the array of rumus_hip_qmatmul_int4_perm_static
+constexpr size_t kStaticScratchBytes = size_t(32) << 20;
 // f16 MFMA kernel for larger m (needs group_size 32, 64 or a multiple of 128,
 // n % 4 == 0, 16-byte aligned buffers, no g_idx).
 bool w4_gemm_supported(const W4Args& a);

@@ -47,6 +47,7 @@
 // Few output tiles (small m): K is split over gridDim.z workgroups, each
 // writes its partial tile to the workspace, and a second kernel adds the
 // partials in a fixed order (deterministic, no atomics) and the bias.
+#include <algorithm>
 #include <type_traits>
 
 #include "w4.h"
@@ -1086,7 +1087,10 @@ static TilePlan plan_by_tiles(const W4Args& a) {
 // and 64 %.  us there and here: 769 x 640 -> 2560 28.2, 17.2; 1533 x 768 -> 1856 31.4, 21.9; 535 x 512 -> 4864, groups of 32, 32.0, 21.6; 10 x 8192 ->
 // 2944, groups of 32, 28.9, 24.9.  An f32 sum runs over no more of K than by the rule above, or over 1024: beyond, its roundings would show, in a row
 // that one element dominates above all.
+// Nor does it want more of the workspace than that rule, or than the array of the entry point that allocates nothing: that one runs the
+// same plan as the others, with the same order of the sums.
 static TilePlan plan_by_estimate(const W4Args& a, const TilePlan& known) {
+    const size_t room = std::max(kStaticScratchBytes, tile_bytes(a, known).all());
     struct Shape { uint32_t rt, waves, side; double base, step, beside, start, add, pre, small, rest; };
     static const Shape shapes[] = {{1, 8, 1, 7.1, 1.67, 0.0, 3.8, 0.6, 0.45, 0.86, 0.19},
                                    {2, 8, 1, 10.9, 2.48, 0.0, 2.3, 1.7, 0.83, 0.92, 0.26},
@@ -1111,7 +1115,7 @@ static TilePlan plan_by_estimate(const W4Args& a, const TilePlan& known) {
         for (uint32_t want = 1; want <= most; want++) {
             plan.sps = ceil_div(nstages, want);
             plan.splits = ceil_div(nstages, plan.sps);           // no empty split
-            if (plan.sps > max(known.sps, 8u)) continue;
+            if (plan.sps > max(known.sps, 8u) || tile_bytes(a, plan).all() > room) continue;
             const double us = cost(c, plan);
             if (us < least) { least = us; best = plan; }
         }

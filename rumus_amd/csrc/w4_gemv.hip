@@ -477,7 +477,6 @@ static int dispatch(const W4Args& a, hipStream_t s) {
 // the stream's workspace.  Every GPU the library runs on holds its own copy, at its own address, until
 // the process ends.  In host code the array's name is only a handle for hipGetSymbolAddress: the
 // address the kernels get is the one looked up below, once per device.
-constexpr size_t kStaticScratchBytes = size_t(32) << 20;
 static __device__ __align__(256) uint8_t scratch[kStaticScratchBytes];
 
 constexpr int kMaxDevices = 64;

@@ -85,3 +85,27 @@ def test_static_scratch_refuses_what_does_not_fit(ops):
     # the refusal left nothing behind: the next call that fits runs
     y = ops.qmatmul_int4_perm_static(x[:16].contiguous(), padded_words, meta, meta, k, g)
     assert float(host(y).max()) == 0.0
+
+
+# Plans whose partial tiles are more than the array: fewer workgroups share K then, in both entry points.  The last two need more than the
+# array by any plan: refused.
+@pytest.mark.parametrize("m,k,n,g,fits", [(368, 4096, 11008, 32, True), (952, 4096, 5120, 32, True), (560, 8192, 2048, 32, True), (345, 4096, 11008, 32, None),
+                                          (1100, 8192, 2048, 32, None), (3000, 4096, 2048, 32, False)])
+def test_static_scratch_plans_that_fit(ops, m, k, n, g, fits):
+    import torch
+    from rumus_amd._lib import RumusError
+    say(f"qmatmul_int4_perm_static m={m} k={k} n={n} g={g}")
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    packed = torch.randint(-2 ** 31, 2 ** 31 - 1, (k // 8, n), generator=gen, device="cuda", dtype=torch.int32)
+    scales = torch.rand((k // g, n), generator=gen, device="cuda") + 0.5
+    zp = 15.0 * torch.rand((k // g, n), generator=gen, device="cuda")
+    x = torch.randn((m, k), generator=gen, device="cuda")
+    perm = torch.randperm(k, generator=gen, device="cuda").to(torch.int32)
+    for order in (None, perm):
+        try:
+            got = ops.qmatmul_int4_perm_static(x, packed, scales, zp, k, g, perm=order)
+        except RumusError as e:
+            assert "bytes of scratch memory" in str(e) and not fits
+            continue
+        assert fits is not False
+        assert torch.equal(got, ops.qmatmul_int4_perm(x, packed, scales, zp, k, g, perm=order))
