@@ -403,31 +403,37 @@ static int validate(const W4Args& a, const char* who) {
 }
 
 // Rows of x up to which the decode kernels beat the two launches of the integer kernel (g128, from HBM, us, decode kernel / integer kernel):
-// 4 rows 4096 x 12288 12.2 / 14.4, 4096 x 22016 18.4 / 23.4, 11008 x 4096 11.1 / 17.8; 8 rows 4096 x 4096 7.6 / 9.2, 11008 x 4096 17.7 / 17.8, 4096 x
-// 12288 17.6 / 14.4: eight up to four million packed words, four beyond.  Act-order rows wait in LDS beside their digits, 128 KB in all, and
+// 4 rows 4096 x 12288 12.0 / 14.4, 4096 x 22016 17.6 / 23.1, 11008 x 4096 10.6 / 17.5; 8 rows 4096 x 4096 6.7 / 8.2, 5120 x 5120 12.2 / 15.8, 11008 x 4096
+// 17.7 / 17.8, 4096 x 12288 14.5 / 14.4: eight up to four million packed words, four beyond, and four of a long K whose workgroups come in more than one
+// round (3200 x 9600 14.8 / 12.8, groups of 64 16.7 / 12.8; 7168 x 4416 16.1 / 15.9).  Act-order rows wait in LDS beside their digits, 128 KB in all, and
 // a call whose rows do not fit takes them in parts, a launch each (8 x 4096 x 4096 17.1 / 10.9): as many as fit at once.  Every workgroup gathers
 // all rows: with more than 512 of them the integer kernel's gather, once a call, wins from two rows on (4096 x 11008 4 rows 21.7 / 15.9, 2 rows
-// 17.3 / 15.8; 2048 x 11008 8 rows 18.3 / 14.1, 4 rows 9.7), with more than 256 and a long K from three (8192 x 8192 3 rows 24.3 / 20.2, 2 rows 20.3; 8192 x
-// 4096 3 rows 15.2 / 17.3).
+// 17.3 / 15.8; 2048 x 11008 8 rows 18.3 / 14.1, 4 rows 9.7; 2048 x 8192, 512 of them, 8 rows 12.9 / 11.5), with more than 256 and a long K from three (8192 x
+// 8192 3 rows 24.3 / 20.2, 2 rows 20.3; 8192 x 4096 3 rows 15.2 / 17.3).
 static uint32_t w4_rows_that_gather(uint32_t padded_k, uint32_t n) {
     if (n > 8192) return padded_k <= 1024 ? 8 : padded_k <= 2048 ? 4 : 1;
-    if (padded_k <= 4096) return padded_k <= 2048 ? 8 : 4;
+    if (padded_k <= 4096) return padded_k > 2048 ? 4 : padded_k > 1024 && n > 7680 ? 7 : 8;
     return n > 4096 ? 2 : padded_k <= 6144 ? 4 : padded_k <= 8192 ? 3 : 2;
 }
 uint32_t w4_decode_max_rows(uint32_t padded_k, uint32_t n, bool perm) {
     const double mw = (double)(padded_k / 8) * n * 1e-6;
-    const uint32_t plain = mw <= 4.0 ? 8 : 4;
+    const uint32_t plain = mw > 4.0 || (n > 8192 && padded_k > 2048) || (n > 4096 && padded_k > 6144) ? 4 : 8;
     return perm ? min(plain, w4_rows_that_gather(padded_k, n)) : plain;
 }
+
 // Row-major arrays of wide weights are read in pieces of 128 bytes of every word row, with groups of 64 twice as many of the scales; rows a multiple of 8 KB
 // long fall on the same memory channels besides.  There the integer kernel, which reads a row's pieces side by side, is ahead from three rows on, beyond 19
 // million words from two (us, decode kernel / integer kernel: groups of 64, 3 x 4096 x 10240 15.2 / 13.6, but 4096 x 9216 13.4 / 13.4; 4 x 4096 x 28672
-// 29.8 / 25.4, 2 x 8192 x 28672 46.8 / 39.1; groups of 128, 2 x 8192 x 28672 42.3 / 38.6, but 8192 x 22016 31.1 / 34.9).
+// 29.8 / 25.4, 2 x 8192 x 28672 46.8 / 39.1; groups of 128, 2 x 8192 x 28672 42.3 / 38.6, but 8192 x 22016 31.1 / 34.9; 3 x 8192 x 10240, a second round of
+// workgroups mostly empty, 22.2 / 19.7).
 static uint32_t w4_max_rows(const W4Args& a) {
     const uint32_t rows = w4_decode_max_rows(a.padded_k, a.n, a.perm);
     if (a.tiled || a.perm || a.group_size % 64 != 0 || a.padded_k <= 2048) return rows;
     const bool large = (uint64_t)(a.padded_k / 8) * a.n > 19000000;
-    if (a.group_size % 128 == 0) return large && a.n > 24576 ? 1 : rows;
+    if (a.group_size % 128 == 0) {
+        if (large && a.n > 24576) return 1;
+        return a.padded_k > 6144 && a.n > 8192 && a.n < 12288 && a.n % 2048 == 0 ? 2 : rows;
+    }
     return a.n >= 12288 || (a.n > 8192 && a.n % 2048 == 0) ? (large ? 1 : 2) : rows;
 }
 static bool w4_few_rows(const W4Args& a) {

@@ -12,7 +12,7 @@
 // From HBM, us, there -> here: 4 x 1024 x 1024 6.8 -> 2.9, 4 x 4096 x 4096 7.8 -> 5.4, 4 x 1152 x 8064 12.0 -> 4.5, 8 x 2048 x 2048 11.9 -> 4.9, groups of 32 the same
 // shape 11.4 -> 4.1 (1024); act-order 4 x 4096 x 4096 17.4 -> 8.9, 8 x 512 x 11008 82 -> 6.4; f16 rows 4 x 4096 x 4096 11.9 (with two launches that convert) -> 5.9.
 // What bounds it: vector issue of the conversion (half of the launch at 4 x 4096 x 4096), then latency.  Error against float64 with some channels 20
-// times as large 3.3e-6 -> 2.0e-6, N(0,1) 2.0e-6 -> 0.6e-6.
+// times as large 3.3e-6 -> 1.1e-6, N(0,1) 2.0e-6 -> 0.3e-6.
 //
 // A workgroup owns 16 Q columns over the whole of K (no partial sums in memory); its eight waves take units in turn, all loads of U units
 // in flight, activations first.  Every activation is loaded and converted once per workgroup; the byte transposition that the digits need
@@ -263,7 +263,7 @@ __global__ __launch_bounds__(kW4mThreads) void w4_gemv_mfma_kernel(W4mArgs a) {
     };
 
     for (uint32_t base = 0; base < units; base += kW4mWaves * U) {
-        const uint32_t c0 = base + wave * U;
+        const uint32_t c0 = base + wave;                           // and every eighth after it: the same units whatever U
         // ---- loads of U units: activations first (their digits are made while the weights are on their way)
         v4i raw[U][S][MB][kSrc], nw[IN == kW4mNorm ? U : 1][S];
         uint32_t word[U][S][2][Q], zp[U][kFolds][Q];
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(kW4mThreads) void w4_gemv_mfma_kernel(W4mArgs a) {
         for (int u = 0; u < U; u++)
 #pragma unroll
             for (int s = 0; s < S; s++) {
-                const uint32_t step = ((c0 + u) * S + s) * 64, in_row = min(step, a.k);   // (a row's end: the next one's start, or the end)
+                const uint32_t step = ((c0 + kW4mWaves * u) * S + s) * 64, in_row = min(step, a.k);   // (a row's end: the next one's start, or the end)
                 const auto b_x = beyond(a.x, x_bytes, step < a.k ? step * kBytes : x_bytes);
 #pragma unroll
                 for (int b = 0; b < MB; b++) {
@@ -303,7 +303,7 @@ __global__ __launch_bounds__(kW4mThreads) void w4_gemv_mfma_kernel(W4mArgs a) {
             __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
-        for (int u = 0; u < U; u++) load_weights(c0 + u, word[u], scale[u], zp[u]);
+        for (int u = 0; u < U; u++) load_weights(c0 + kW4mWaves * u, word[u], scale[u], zp[u]);
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
@@ -315,7 +315,7 @@ __global__ __launch_bounds__(kW4mThreads) void w4_gemv_mfma_kernel(W4mArgs a) {
                         if (kGather && b) continue;
                         v4i v = raw[u][s][b][i];
                         if constexpr (IN == kW4mNorm) {
-                            const bool in = ((c0 + u) * S + s) * 64 + k_in < a.k;
+                            const bool in = ((c0 + kW4mWaves * u) * S + s) * 64 + k_in < a.k;
 #pragma unroll
                             for (int j = 0; j < 4; j++) {
                                 const float f = __int_as_float(v[j]);
@@ -329,7 +329,7 @@ __global__ __launch_bounds__(kW4mThreads) void w4_gemv_mfma_kernel(W4mArgs a) {
                     }
 
         // ---- digits, in the place of the activations
-        const uint32_t live = c0 < units ? min((uint32_t)U, units - c0) : 0;
+        const uint32_t live = c0 < units ? min((uint32_t)U, (units - c0 + kW4mWaves - 1) / kW4mWaves) : 0;
         if (lane < U * MB * 4) back_of[wave][0][lane] = 0.0f;      // (a unit that is not there adds nothing)
         uint32_t deep = 0;                                         // bit per (unit, block) with towering elements
 #pragma unroll 1
@@ -355,11 +355,11 @@ __global__ __launch_bounds__(kW4mThreads) void w4_gemv_mfma_kernel(W4mArgs a) {
                     for (int j = 0; j < 4; j++) t[s][j] = w4m_silu(t[s][j], __int_as_float(up[j]));
                 }
             }
-            if ((c0 + u + 1) * (64 * S) > a.k) {
+            if ((c0 + kW4mWaves * u + 1) * (64 * S) > a.k) {
 #pragma unroll
                 for (int s = 0; s < S; s++)
 #pragma unroll
-                    for (int j = 0; j < 4; j++) t[s][j] = ((c0 + u) * S + s) * 64 + k_of + 2 * j < a.k ? t[s][j] : 0.0f;
+                    for (int j = 0; j < 4; j++) t[s][j] = ((c0 + kW4mWaves * u) * S + s) * 64 + k_of + 2 * j < a.k ? t[s][j] : 0.0f;
             }
 #pragma unroll
             for (int s = 0; s < S; s++) top = max(top, w4m_largest(t[s]));
@@ -396,7 +396,7 @@ __global__ __launch_bounds__(kW4mThreads) void w4_gemv_mfma_kernel(W4mArgs a) {
 #pragma unroll 1
             for (uint32_t i = 0; i < live * MB; i++) {
                 if (!((deep >> i) & 1)) continue;
-                const uint32_t c = c0 + i / MB, b = i % MB, row = b ? row_of[1] : row_of[0];
+                const uint32_t c = c0 + kW4mWaves * (i / MB), b = i % MB, row = b ? row_of[1] : row_of[0];
                 uint32_t w[S][2][Q], z[kFolds][Q];
                 float sc[kFolds][Q];
                 load_weights(c, w, sc, z);
@@ -484,10 +484,6 @@ __global__ __launch_bounds__(kW4mThreads) void w4_gemv_mfma_kernel(W4mArgs a) {
     }
 }
 
-bool w4_gemv_mfma_supported(const W4Args& a) {
-    return a.m >= 2 && a.m <= 8 && !a.g_idx && a.group_size % 32 == 0 && a.k > 0;
-}
-
 template <auto KERNEL>
 static int w4m_queue(dim3 grid, dim3 block, size_t lds, const W4mArgs& a, hipStream_t s) {
     static std::atomic<bool> allowed{false};
@@ -505,29 +501,38 @@ static int w4m_launch(const W4mArgs& a, hipStream_t s) {
     const size_t lds = (size_t)kW4mWaves * U * MB * (IN == kW4mGlu ? 2 : 1) * S * 1024 + (IN == kW4mPerm ? (size_t)a.m * a.k * sizeof(float) : 0);
     if (a.group_size % 128 == 0) return w4m_queue<&w4_gemv_mfma_kernel<MB, Q, 1, IN, S, U>>(grid, block, lds, a, s);
     if (a.group_size % 64 == 0) return w4m_queue<&w4_gemv_mfma_kernel<MB, Q, 2, IN, S, U>>(grid, block, lds, a, s);
-    return w4m_queue<&w4_gemv_mfma_kernel<MB, Q, 4, IN, S, U>>(grid, block, lds, a, s);
+    if constexpr (U == 1) return w4m_queue<&w4_gemv_mfma_kernel<MB, Q, 4, IN, S, U>>(grid, block, lds, a, s);
+    return set_error(RUMUS_HIP_EINVAL, "w4 gemv: groups of 32 take one unit at a time");
 }
 // Of one launch's LDS: digits of the units in flight, and an act-order call's rows.
 static size_t w4m_gather_lds(uint32_t m, uint32_t k, uint32_t flight) {
     return (size_t)kW4mWaves * flight * (m > 4 ? 2 : 1) * 4096 + (size_t)m * k * sizeof(float);
 }
-// Units of 128 k where 256 would leave waves without one; two in flight where the eight waves have more than that and the rows of
-// an act-order call leave room for both.
+// Two units in flight for up to four rows where the eight waves have more than that and the rows of an act-order call leave room for both.  Not for
+// eight rows, whose digits of two units are 128 KB, one workgroup a compute unit, nor for groups of 32, whose folds take the registers (us with two
+// and one: 8 x 4096 x 5632 12.7 and 10.1, 8 x 5120 x 5120 18.1 and 12.2, 8 x 4096 x 22016 24.7 and 21.6; groups of 32, 3 x 4096 x 12288 16.2 and 14.1, 5 x
+// 4096 x 12288 through RMSNorm 28.7 and 22.3).
+// Units of 128 k where 256 would leave waves without one, and for groups of 32 where there are more workgroups than compute units: half the registers
+// let two share one (3 x 4096 x 12288 14.1 -> 12.0, 5 x 4096 x 5632 15.8 -> 13.9, 8 x 5120 x 5120 20.5 -> 16.6; but 3 x 4096 x 8192, 256 of them, 8.3 -> 9.1).
+// The rows of an act-order call hold the LDS of a compute unit anyway.  None of it depends on the number of rows but the units in flight, which
+// leave a wave its units in their order: a row's bits are the same in calls of three to eight.
 template <int MB, int Q, W4mIn IN>
 static int w4m_sweep(const W4mArgs& a, hipStream_t s) {
-    const uint32_t units = ceil_div(a.padded_k, 256);
-    if (2 * units <= kW4mWaves) return w4m_launch<MB, Q, IN, 2, 1>(a, s);
-    constexpr bool kTwo = MB * (IN == kW4mGlu ? 2 : 1) <= 2;       // (LDS)
-    if constexpr (kTwo) {
-        if (units > kW4mWaves && (IN != kW4mPerm || w4m_gather_lds(a.m, a.k, 2) <= kW4mLds)) return w4m_launch<MB, Q, IN, 4, 2>(a, s);
+    const uint32_t units = ceil_div(a.padded_k, 256), columns = a.n >= 8192 ? 32 : 16;     // of a workgroup (w4m_pick)
+    const bool shared = IN != kW4mPerm && a.group_size % 64 != 0 && ceil_div(a.n, columns) > 256;
+    if (2 * units <= kW4mWaves || shared) return w4m_launch<MB, Q, IN, 2, 1>(a, s);
+    if constexpr (MB == 1) {
+        if (a.group_size % 64 == 0 && units > kW4mWaves && (IN != kW4mPerm || w4m_gather_lds(a.m, a.k, 2) <= kW4mLds)) return w4m_launch<MB, Q, IN, 4, 2>(a, s);
     }
     return w4m_launch<MB, Q, IN, 4, 1>(a, s);
 }
+// (f16 rows come with row-major arrays: pieces of 128 bytes only where the rows of all columns begin on the same memory channels, us with 16 and 32
+// columns 4 x 4096 x 8192 9.0 and 7.8, 4 x 8192 x 8192 14.4 and 12.3, but 4 x 4096 x 11008 11.1 and 12.1)
 template <W4mIn IN>
 static int w4m_pick(const W4mArgs& a, hipStream_t s) {
-    constexpr bool kWide = IN == kW4mVec || IN == kW4mNorm || IN == kW4mGlu;
+    constexpr bool kWide = IN == kW4mVec || IN == kW4mHalf || IN == kW4mNorm || IN == kW4mGlu;
     if constexpr (kWide) {
-        if (a.n >= 8192) return a.m <= 4 ? w4m_sweep<1, 2, IN>(a, s) : w4m_sweep<2, 2, IN>(a, s);
+        if (a.n >= 8192 && (IN != kW4mHalf || a.n % 2048 == 0)) return a.m <= 4 ? w4m_sweep<1, 2, IN>(a, s) : w4m_sweep<2, 2, IN>(a, s);
     }
     return a.m <= 4 ? w4m_sweep<1, 1, IN>(a, s) : w4m_sweep<2, 1, IN>(a, s);
 }

@@ -39,7 +39,9 @@ def check(got, x, w, largest=None):
 
 SHAPES = [(2, 32, 16, 32), (3, 96, 20, 32), (8, 160, 48, 32), (2, 1000, 52, 64), (5, 1088, 64, 64), (4, 128, 4, 128), (7, 1152, 36, 128),
           (2, 2048, 80, 128), (6, 2176, 16, 128), (3, 4096, 64, 256), (8, 4224, 32, 128), (4, 8320, 32, 64), (4, 512, 8192, 128),
-          (8, 300, 8224, 32), (3, 1001, 16, 8 * 32)]
+          (8, 300, 8224, 32), (3, 1001, 16, 8 * 32),
+          # groups of 32 on more workgroups than compute units; eight rows on two of them; wide row-major weights of groups of 64
+          (5, 1088, 4112, 32), (3, 2176, 4128, 32), (7, 2176, 4128, 128), (3, 2176, 12288, 64)]
 
 
 @pytest.mark.parametrize("m,k,n,g", SHAPES)
