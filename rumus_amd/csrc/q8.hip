@@ -434,11 +434,23 @@ static int launch_q8_rows(const T* a, const uint32_t* b, T* c, uint32_t k, uint3
                     : launch_q8_rows_form<M, 4, false>(a, b, c, k, n, bs, stride, bpc, kpad, s);
 }
 
+// Rows of one launch of a call of m, as many as fit the LDS but for calls of more than four (blocks of 16 or 48, unaligned rows; us): with several blocks a
+// column four at a time from eight rows on, whose instance spills (8 x 4096 x 4096, blocks of 16, 29.6, and 34.7 in one launch; 16 x 3072 x 4096, unaligned,
+// 59.7 and 73.7), and with one block on more columns than 256 workgroups have as many as 80 KB hold, evenly, for two workgroups a compute unit (6 x
+// 4096 x 11008 42.5 and 45.4, 8 x 4608 x 11008 60.2 and 75.5; on 4096 columns 8 rows of 4096 in one launch 34.9, in two 39.0).
+static uint32_t q8_rows_at_once(uint32_t m, uint32_t n, uint32_t kpad, uint32_t bpc) {
+    const uint32_t most = min(8u, kQ8RowsFloats / kpad);
+    if (m <= 4) return most;
+    if (bpc > 1) return m >= 8 && kpad <= 4096 ? 4 : most;
+    const uint32_t two = kQ8RowsFloats * 5 / 8 / kpad;
+    return n > 8192 && two < 8 ? ceil_div(m, ceil_div(m, max(two, 1u))) : most;
+}
+
 // Rows that do not go to the matrix cores (block_size % 16 == 0, kpad <= 16384), in groups whose x fits the LDS.
 template <typename T>
 static int q8_rows(const T* a, const uint32_t* b, T* c, uint32_t m, uint32_t k, uint32_t n, uint32_t bs, uint32_t stride, uint32_t bpc,
                    hipStream_t s) {
-    const uint32_t kpad = (k + 15) & ~15u, group = min(8u, kQ8RowsFloats / kpad);
+    const uint32_t kpad = (k + 15) & ~15u, group = q8_rows_at_once(m, n, kpad, bpc);
     for (uint32_t r0 = 0; r0 < m; r0 += group) {
         const T* ar = a + (uint64_t)r0 * k;
         T* cr = c + (uint64_t)r0 * n;

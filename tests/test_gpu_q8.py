@@ -139,6 +139,23 @@ def test_matmul_q8_vs_oracle(ops, m, k, n, bs):
     np.testing.assert_array_equal(deq.reshape(-1), oracle.q8_dequantize(words, k * n, bs))
 
 
+# rows that the matrix cores do not take: blocks of 16 and 48, or x one float off; one launch, as many rows as fit, four at a time, evenly
+@pytest.mark.parametrize("m,k,n,bs", [(5, 2064, 40, 16), (8, 4096, 24, 16), (8, 4112, 17, 16), (7, 4080, 20, 48), (9, 1040, 20, 16), (16, 3072, 33, 128),
+                                      (15, 4608, 12, 128), (6, 4096, 8208, 4096), (8, 4608, 8200, 4608), (13, 2560, 8201, 2560), (5, 8192, 9, 8192),
+                                      (5, 16384, 5, 16384), (6, 16384, 8193, 16384)])
+def test_matmul_q8_more_rows_without_the_matrix_cores(ops, m, k, n, bs):
+    import torch
+    from rumus_amd import nn
+    say(f"matmul_q8 m={m} k={k} n={n} bs={bs}, x one float off")
+    gen = torch.Generator(device="cuda").manual_seed(m + k + n)
+    wq = nn.quantize(0.02 * torch.randn((k, n), generator=gen, device="cuda"), bs)
+    x = torch.randn(m * k + 1, generator=gen, device="cuda")[1:].view(m, k)
+    got, w = nn.matmul(x, wq).double(), nn.dequantize_kn(wq).double()
+    # a lane adds up every sixty-fourth run of 16, then the lanes: roundings of 2^-24 of what has been added up
+    bound = (k / 64 + 32) * 2.0 ** -24 * (x.double().abs() @ w.abs())
+    assert float(((got - x.double() @ w).abs() / bound).max()) <= 1.0
+
+
 def test_matmul_q8_row_split_inside_on_a_fresh_stream(ops):
     # 520 rows become 2080 rows of digit planes; the int8 GEMM inside splits them into 2048 rows of wide
     # blocks and 32 rows that share K over workgroups, whose partial sums must fit behind this call's own
