@@ -43,7 +43,6 @@ int i8_launch_gemv(const int8_t* xq, const int8_t* wq, const float* sx, const fl
 
 // 5 to 32 rows, K % 256 == 0: MFMA tiles fed straight from global memory (i8_gemv.hip).
 // 5..64 rows with the activations resident in registers, where i8_resident_takes says so
-uint32_t i8_resident_grid(uint32_t n);
 bool i8_resident_takes(uint32_t m, uint32_t k, uint32_t n);
 int i8_launch_resident(const int8_t* xq, const int8_t* wq, const float* sx, const float* sw, const float* bias, int32_t* acc,
                        float* y, uint32_t m, uint32_t k, uint32_t n, hipStream_t s);

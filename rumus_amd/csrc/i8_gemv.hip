@@ -305,7 +305,7 @@ __global__ __launch_bounds__(512) void i8_resident_kernel(
 }
 
 // the fewest workgroups, one per compute unit at most, that keep the longest walk over column tiles as short
-uint32_t i8_resident_grid(uint32_t n) {
+static uint32_t resident_grid(uint32_t n) {
     const uint32_t tiles = ceil_div(n, 16);
     return ceil_div(tiles, ceil_div(tiles, 256));
 }
@@ -321,7 +321,7 @@ bool i8_resident_takes(uint32_t m, uint32_t k, uint32_t n) {
 int i8_launch_resident(const int8_t* xq, const int8_t* wq, const float* sx, const float* sw, const float* bias, int32_t* acc,
                        float* y, uint32_t m, uint32_t k, uint32_t n, hipStream_t s) {
     const uint32_t ch = ceil_div(ceil_div(k / 64, 8), 8), rt = ceil_div(m, 16);
-    const dim3 grid(i8_resident_grid(n)), block(512);
+    const dim3 grid(resident_grid(n)), block(512);
 #define RUMUS_RESIDENT(RT, CH) \
     hipLaunchKernelGGL((i8_resident_kernel<RT, CH>), grid, block, 0, s, xq, wq, sx, sw, bias, acc, y, m, k, n)
     if (ch == 1) {

@@ -86,13 +86,16 @@ __global__ __launch_bounds__(512) void i8_linear_kernel(const float* __restrict_
         const uint32_t row = row0 + 8 * r;
         if (row >= M) continue;
         const float inv = top[r] == 0.0f ? 0.0f : __fdiv_rn(127.0f, top[r]);
-        if (lane == 0) scale_of[row] = top[r] == 0.0f ? 1.0f : __fdiv_rn(top[r], 127.0f);
+        if (lane == 0) {
+            scale_of[row] = top[r] == 0.0f ? 1.0f : __fdiv_rn(top[r], 127.0f);
+            // zeros as such: in a row of 1e-37 `inv` is an infinity, and its product with a zero no number
+            for (uint32_t kk = K; kk < steps * 64; kk += 16) *reinterpret_cast<v4i*>(xs + row * pitch + kk) = v4i{0, 0, 0, 0};
+        }
 #pragma unroll
         for (int i = 0; i < NV; i++) {
             const uint32_t kk = k0 + i * 256 + lane * 4;
             const float4 v = make_float4(__int_as_float(raw[r][i][0]), __int_as_float(raw[r][i][1]), __int_as_float(raw[r][i][2]), __int_as_float(raw[r][i][3]));
-            // (zeros from K on as such: in a row of 1e-37 `inv` is an infinity, and its product with zero no number)
-            if (kk < steps * 64) *reinterpret_cast<uint32_t*>(xs + row * pitch + kk) = kk < K ? pack_i8x4(v, inv) : 0u;
+            if (kk < K) *reinterpret_cast<uint32_t*>(xs + row * pitch + kk) = pack_i8x4(v, inv);
         }
     }
     __syncthreads();

@@ -69,7 +69,7 @@ __global__ __launch_bounds__(256) void i8_quantize_rows_kernel(const float* __re
 
 // One launch, w read once (n % 4 == 0, k % 4 == 0 up to 12288, 16-byte aligned w, 4-byte aligned wq).  A workgroup owns 4 QUADS columns over
 // all of K: thread = four adjacent columns of four consecutive rows, 4096 / QUADS rows a sweep.  All sweeps stay in registers between
-// the maximum and the digits, all their loads in flight at once.  A thread's four rows are four bytes of a column of wq: a wave
+// the maximum and the digits (of six, four words a thread go through scratch memory), all their loads in flight at once.  A thread's four rows are four bytes of a column of wq: a wave
 // stores 64 (QUADS = 4) contiguous bytes of 16 columns, no trip through LDS.
 // What bounds it: HBM in segments of 64 bytes of w (the other half of a line belongs to the neighbour, on the same L2), and one
 // workgroup a compute unit from 3072 rows on, which loads and then stores; a small matrix the launch.

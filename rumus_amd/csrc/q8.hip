@@ -454,16 +454,17 @@ static int q8_rows(const T* a, const uint32_t* b, T* c, uint32_t m, uint32_t k, 
     for (uint32_t r0 = 0; r0 < m; r0 += group) {
         const T* ar = a + (uint64_t)r0 * k;
         T* cr = c + (uint64_t)r0 * n;
-        int rc;
+        constexpr bool kMore = sizeof(T) == sizeof(float);     // (f16 rows: up to four, q8_few_rows_take)
+        int rc = RUMUS_HIP_EINVAL;
         switch (min(group, m - r0)) {
             case 1: rc = launch_q8_rows<1>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
             case 2: rc = launch_q8_rows<2>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
             case 3: rc = launch_q8_rows<3>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
             case 4: rc = launch_q8_rows<4>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
-            case 5: rc = launch_q8_rows<5>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
-            case 6: rc = launch_q8_rows<6>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
-            case 7: rc = launch_q8_rows<7>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
-            default: rc = launch_q8_rows<8>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
+            case 5: if constexpr (kMore) rc = launch_q8_rows<5>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
+            case 6: if constexpr (kMore) rc = launch_q8_rows<6>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
+            case 7: if constexpr (kMore) rc = launch_q8_rows<7>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
+            default: if constexpr (kMore) rc = launch_q8_rows<8>(ar, b, cr, k, n, bs, stride, bpc, kpad, s); break;
         }
         if (rc) return rc;
     }

@@ -450,7 +450,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void q8_gemm_blocks_f16_kernel(
 // instead of two, and a step issues 40 vector instructions and 10 LDS reads per 16 MFMAs.  One wave per SIMD, so every
 // latency has to be hidden inside it: a step is one pair of 32 k, and while its 16 MFMAs run the wave reads the next
 // step's fragments into a second set of registers (the loop is unrolled over the two sets) and converts its bytes; NS
-// steps are on their way to LDS meanwhile.  Products and sums in the order of the kernel above: the same bits.
+// steps are on their way to LDS meanwhile.  Products and sums in the order of the kernel above, the same bits, for
+// blocks of up to 1024; this one folds once a block, that one of longer blocks at least every 1024 k.
 // What bounds it is the address side of the loads: a wave's load that touches 64 cache lines (headers, 4 bytes each) costs
 // the compute unit eight times one that reads 1 KB in a row.  Hence steps of 64 k (64 bytes of a column at a time), headers
 // only with the last step of a block, and activations laid out by q8_split_rows_f16_kernel<true> as a step wants them.
