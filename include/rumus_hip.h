@@ -72,7 +72,9 @@ int rumus_hip_sync(rumus_hip_stream_t stream);
  *   qmatmul_int4 / _perm / _zp4 / _block, m > 5: 5 * (m + 64) * (padded_k + 128) (activations
  *       in matrix-core order and a scale factor per row) + 64 * m * n (partial
  *       sums, only while the output has fewer than 192 tiles of 64 x 512) + 1280
- *       (the last kilobyte: flags of the look at the zero-point table).  Large
+ *       (the last kilobyte: flags of the look at the zero-point table; batches of
+ *       fewer tiles than that whose faster plan finds no room, in a capture or a
+ *       reserved size, run another one, with sums in another order).  Large
  *       batches take up to 3/4 of a byte per weight more, at most 256 MiB, where
  *       the workspace has room for it or can grow (not while capturing, and not
  *       beyond a size reserved here; what it had before stays allocated until
@@ -265,7 +267,8 @@ int rumus_hip_f16_to_f32(const uint16_t* in, float* out, uint64_t numel,
  * group_size % 64 == 0 and enough columns to fill the chip) x is held in fixed
  * point below the largest magnitude of a part of the row (20 bits per 32 k for
  * one row, or two of a long K; 22 bits per 128 or 256 k up to decode_max_rows
- * rows, 22 bits per eighth of K beyond):
+ * rows, 22 bits per eighth of K beyond; so a row's bits depend on how many rows
+ * the call has):
  * |error| <= max|x| * 2^-19 * sum|w| over that part.  Where elements
  * tower over their part by 2^8 or more the small ones keep their bits (in the
  * few-row kernels all of that part, in f32 or in further digits; beyond, up to 16
@@ -325,7 +328,7 @@ int rumus_hip_f16_staging_reserve(rumus_hip_stream_t stream, uint64_t bytes);
  * workgroups of the f16 tile kernel (few output tiles) need room for their
  * partial sums.  With k = 4096, n = 11008 and groups of 128 every call up to
  * about 1900 rows runs; with groups of 32 (which the integer kernel does not
- * take) calls of 318 to 383 rows are refused.
+ * take) calls of 318 to 320 rows are refused.
  * All calls on one GPU share the one array, whatever their stream: calls that
  * overlap in time on one GPU race (calls on one stream do not overlap).
  * Nothing in the array has to start at zero: every byte a kernel reads from
@@ -386,7 +389,8 @@ int rumus_hip_w4_decode_layout(const uint32_t* packed, const float* scales,
                                float* zero_points_t, rumus_hip_stream_t stream);
 
 /* EXTENSION: QLinear::forward for m <= 8 on the decode layout; same arithmetic
- * and results as rumus_hip_qmatmul_int4_perm (bit for bit).  perm may be NULL.
+ * and results as rumus_hip_qmatmul_int4_perm, bit for bit where that call runs
+ * the decode kernels too (see decode_max_rows below).  perm may be NULL.
  * EINVAL unless m <= 8, n % 16 == 0, group_size % 32 == 0. */
 int rumus_hip_qmatmul_int4_decode(const float* x, const uint32_t* packed_t,
                                   const float* scales_t, const float* zero_points_t,
@@ -398,7 +402,13 @@ int rumus_hip_qmatmul_int4_decode(const float* x, const uint32_t* packed_t,
 /* Rows of x up to which the decode entry points are the faster way to run a
  * [padded_k, n] weight (between 1 and 8, from measurements; beyond it
  * rumus_hip_qmatmul_int4 takes the matrix cores).  The dispatch inside
- * rumus_hip_qmatmul_int4 uses the same number.  No counterpart in the reference. */
+ * rumus_hip_qmatmul_int4 uses the same number, but two rows, or one of weights of
+ * more than 150 million elements, for row-major arrays that are slow to read a few
+ * columns at a time: K above 2048, group_size % 64 == 0 and some n above 8192
+ * (groups of 64: from 12288 on and multiples of 2048; of 128: beyond 24576 on
+ * such large weights, and 10240 with K above 6144); and up to three rows of
+ * act-order weights of groups that are no multiple of 64.  No counterpart in the
+ * reference. */
 uint32_t rumus_hip_qmatmul_int4_decode_max_rows(uint32_t padded_k, uint32_t n);
 /* the same for act-order weights (a `perm`): as many rows as the kernel gathers in one launch */
 uint32_t rumus_hip_qmatmul_int4_decode_max_rows_perm(uint32_t padded_k, uint32_t n);
@@ -407,8 +417,8 @@ uint32_t rumus_hip_qmatmul_int4_decode_max_rows_perm(uint32_t padded_k, uint32_t
  * rumus_hip_w4_quantize_pack_awq): packed_t and scales_t as in
  * rumus_hip_w4_decode_layout; qzeros_t[(c*num_groups + g)*2 + h] =
  * qzeros[g*(n/8) + 2*c + h], the two zero-point words of tile c's 16 columns.
- * Same bits as rumus_hip_qmatmul_int4_zp4 on the row-major arrays while m is
- * within rumus_hip_qmatmul_int4_decode_max_rows, except for one row with
+ * Same bits as rumus_hip_qmatmul_int4_zp4 on the row-major arrays where that call
+ * runs the decode kernels (rumus_hip_qmatmul_int4_decode_max_rows), except for one row with
  * group_size % 64 == 0: that case fixes the point of x per 64 rows instead of
  * 32 here (same tolerance, other bits).
  * EINVAL as for the f32 zero-point forms.  No counterpart in the reference. */

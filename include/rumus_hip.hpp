@@ -191,7 +191,7 @@ struct QLinear {
     }
 
     // y[m, out] = x[m, in] . dequant(W) + bias; x and y are device pointers.
-    // Few rows take the decode kernel on the tile-major copy (same result bit for bit).
+    // Few rows take the decode kernel on the tile-major copy.
     void forward(const float* x, uint32_t m, float* y, hipStream_t stream = nullptr) const {
         const int32_t* perm = weight.perm.size() ? weight.perm.data() : nullptr;
         if (weight.has_decode_layout() && m <= (perm ? rumus_hip_qmatmul_int4_decode_max_rows_perm(weight.padded_k, weight.n)

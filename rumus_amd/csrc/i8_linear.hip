@@ -4,7 +4,7 @@
 //
 // The same bits as rumus_hip_i8_quantize_rows and rumus_hip_i8_gemm on its result; every workgroup quantizes all of the rows for itself.
 // What bounds it: the weights' stream where they are large (8 x 4096 x 11008 3.5 TB/s), else the launch and two trips to memory.  Two
-// launches, the quantizer's 2.6 us first -> one, from HBM, called from Python: 1 x 1024 x 1024 8.8 -> 5.1 us, 2 x 4096 x 4096 9.3 -> 6.7, 4 x 768 x 10800
+// launches, the quantizer's 2.6 us first -> one, called from Python on 500 MB of weights in turn: 1 x 1024 x 1024 8.8 -> 5.1 us, 2 x 4096 x 4096 9.3 -> 6.7, 4 x 768 x 10800
 // 11.1 -> 5.2, 4 x 4096 x 11008 13.6 -> 12.2, 8 x 1152 x 7200 9.4 -> 5.3, 8 x 4096 x 11008 15.2 -> 13.2, 16 x 2048 x 11008 11.8 -> 9.8.
 #include "i8_gemm.h"
 

@@ -1,8 +1,9 @@
 """INT4 forward for 2 to 8 rows on the int8 matrix cores (``w4_gemv_mfma.hip``): units of 128 and 256 k and their tails, groups of 32, 64 and
 128, column tiles, act-order rows in one launch and in parts, f16 rows, elements far apart in a unit, NaN and infinity.
 
-The bound, against float64: an activation is rounded to 2^-21 of the power of two above its unit's largest magnitude, so an output is off by at
-most max|x| 2^-20 sum|w|; the f32 sums around it lose less than 2^-20 of the summed magnitudes (up to K/128 + 8 additions of 2^-24 each)."""
+The bound, against float64: an activation is rounded to 2^-22 of its unit's largest magnitude (2^-21 where that lies within 1.6 % below a power of
+two), so an output is off by at most max|x| 2^-21 sum|w|, half of what ``check`` allows; the f32 sums around it lose less than 2^-20 of the
+summed magnitudes (up to K/128 + 8 additions of 2^-24 each)."""
 import numpy as np
 import pytest
 

@@ -184,3 +184,21 @@ def test_grad_x_with_room_for_fewer_shares(m, k, n, shares):
     for got in _captured_in(room, lambda: ops.qmatmul_int4_t(gy, packed, scales, zp, k, 128, out=out), out):
         # test_gpu_w4_t_wide.py's bound of an ordinary sum, far above both share counts' rounding
         assert float(((got.double() - want).abs() / size).max()) < 2e-6
+
+
+# the plan of 256 columns a workgroup wants more shares of K than that of 512, for which there is room; stages of 128 k of each of these
+@pytest.mark.parametrize("m,k,n,shares,stages", [(257, 4096, 768, 11, 3), (540, 2048, 768, 6, 3)])
+def test_f16_tiles_with_room_for_fewer_shares(m, k, n, shares, stages):
+    import torch
+    from rumus_amd import ops
+    say(f"qmatmul_int4 {m} x {k} -> {n}, groups of 32, captured with room for {shares} shares of K")
+    packed, scales, zp = _weight(k, n, 32, 5)
+    x, out = _rows(m, k, 6), torch.empty((m, n), device="cuda")
+    room = 1024 + -(-8 * m // 256) * 256 + shares * m * n * 4      # flags, the rows' factors, partial tiles
+    q = torch.stack([(packed.view(torch.int32) >> (4 * i)) & 15 for i in range(8)], 1).reshape(k, n).double()
+    each = lambda t: t.double().repeat_interleave(32, 0)
+    w = (q - each(zp)) * each(scales)
+    want, size = x.double() @ w, x.double().abs() @ w.abs()
+    for got in _captured_in(room, lambda: ops.qmatmul_int4(x, packed, scales, zp, k, 32, out=out), out):
+        # f32 additions: eight steps a stage, two products each, a settlement every two, then the shares; zero-points up to half a step off
+        assert float(((got.double() - want).abs() / size).max()) < (20 * stages + shares + 16) * 2.0 ** -24
