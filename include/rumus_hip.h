@@ -69,7 +69,8 @@ int rumus_hip_sync(rumus_hip_stream_t stream);
  * inside the call that needs it.  A caller that must not allocate later
  * (graph capture, serving loop) reserves the largest size up front.  Upper
  * bounds per call, in bytes:
- *   qmatmul_int4 / _perm / _zp4 / _block, m > 5: 5 * (m + 64) * (padded_k + 128) (activations
+ *   qmatmul_int4 / _perm / _zp4 / _block, m > 1 (up to eight rows of some weights
+ *       run without, in other bits, where there is none): 5 * (m + 64) * (padded_k + 128) (activations
  *       in matrix-core order and a scale factor per row) + 64 * m * n (partial
  *       sums, only while the output has fewer than 192 tiles of 64 x 512) + 1280
  *       (the last kilobyte: flags of the look at the zero-point table; batches of

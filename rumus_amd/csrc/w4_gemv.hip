@@ -410,9 +410,10 @@ static int validate(const W4Args& a, const char* who) {
 // all rows: with more than 512 of them the integer kernel's gather, once a call, wins from two rows on (4096 x 11008 4 rows 21.7 / 15.9, 2 rows
 // 17.3 / 15.8; 2048 x 11008 8 rows 18.3 / 14.1, 4 rows 9.7; 2048 x 8192, 512 of them, 8 rows 12.9 / 11.5), with more than 256 and a long K from three (8192 x
 // 8192 3 rows 24.3 / 20.2, 2 rows 20.3; 8192 x 4096 3 rows 15.2 / 17.3).
-static uint32_t w4_rows_that_gather(uint32_t padded_k, uint32_t n) {
+// `fit`: how many fit, not how many of these the integer kernel is behind on.
+static uint32_t w4_rows_that_gather(uint32_t padded_k, uint32_t n, bool fit = false) {
     if (n > 8192) return padded_k <= 1024 ? 8 : padded_k <= 2048 ? 4 : 1;
-    if (padded_k <= 4096) return padded_k > 2048 ? 4 : padded_k > 1024 && n > 7680 ? 7 : 8;
+    if (padded_k <= 4096) return padded_k > 2048 ? 4 : padded_k > 1024 && n > 7680 && !fit ? 7 : 8;
     return n > 4096 ? 2 : padded_k <= 6144 ? 4 : padded_k <= 8192 ? 3 : 2;
 }
 uint32_t w4_decode_max_rows(uint32_t padded_k, uint32_t n, bool perm) {
@@ -442,6 +443,13 @@ static bool w4_few_rows(const W4Args& a) {
     return a.perm && a.group_size % 64 != 0 && a.m <= 3 && a.padded_k <= 4096;
 }
 
+// Where a call that another kernel is faster on finds no workspace (a capture on a stream that has none), the decode kernels, which need none, run it:
+// up to eight rows of four million packed words, four beyond.
+static bool w4_runs_without_workspace(const W4Args& a) {
+    const uint32_t rows = (uint64_t)(a.padded_k / 8) * a.n <= 4000000 ? 8 : 4;
+    return a.m <= (a.perm ? min(rows, w4_rows_that_gather(a.padded_k, a.n, true)) : rows) && w4_gemv_dot8_supported(a);
+}
+
 bool w4_routes_to_i8(const W4Args& a) {
     if (a.m == 0 || a.n == 0 || a.k == 0) return false;
     const bool few_rows = w4_few_rows(a);
@@ -455,8 +463,10 @@ static int dispatch(const W4Args& a, hipStream_t s) {
     if (few_rows && w4_gemv_dot8_supported(a)) return w4_launch_gemv_dot8(a, s);
     if (few_rows && w4_gemv_supported(a)) return w4_launch_gemv(a, s);
     if (w4_gemm_f6_chosen(a)) return w4_launch_gemm_f6(a, s);
-    if (w4_gemm_i8_supported(a)) return w4_launch_gemm_i8(a, s);
-    if (w4_gemm_supported(a)) return w4_launch_gemm(a, s);
+    if (const bool i8 = w4_gemm_i8_supported(a); i8 || w4_gemm_supported(a)) {
+        const int rc = i8 ? w4_launch_gemm_i8(a, s) : w4_launch_gemm(a, s);          // (EINVAL: nothing has been queued)
+        return rc == RUMUS_HIP_EINVAL && w4_runs_without_workspace(a) ? w4_launch_gemv_dot8(a, s) : rc;
+    }
     // Batches the matrix-core kernel does not take (group sizes that are no multiple of 32): the
     // decode kernel, a few rows at a time, is far ahead of the reference-order kernel
     // (16 x 4096 x 11008, group 8: 1.2 ms there).
@@ -536,7 +546,10 @@ int rumus_hip_qmatmul_int4_f16(const uint16_t* x, const uint32_t* packed, const 
         a.x = nullptr;
         a.y = nullptr;
         if (m <= w4_max_rows(a) && w4_gemv_half_takes(a)) return w4_launch_gemv_half(a, as_stream(stream));
-        if (w4_routes_to_i8(a)) return w4_launch_gemm_i8(a, as_stream(stream));
+        if (w4_routes_to_i8(a)) {
+            const int rc = w4_launch_gemm_i8(a, as_stream(stream));
+            return rc == RUMUS_HIP_EINVAL && w4_runs_without_workspace(a) && w4_gemv_half_takes(a) ? w4_launch_gemv_half(a, as_stream(stream)) : rc;
+        }
     }
     return w4_f16_staged(x, packed, scales, zero_points, bias, g_idx, y, m, k, n, padded_k, group_size, num_groups, stream);
 }

@@ -202,3 +202,27 @@ def test_f16_tiles_with_room_for_fewer_shares(m, k, n, shares, stages):
     for got in _captured_in(room, lambda: ops.qmatmul_int4(x, packed, scales, zp, k, 32, out=out), out):
         # f32 additions: eight steps a stage, two products each, a settlement every two, then the shares; zero-points up to half a step off
         assert float(((got.double() - want).abs() / size).max()) < (20 * stages + shares + 16) * 2.0 ** -24
+
+
+# few rows on which the integer kernel is the faster one, and needs workspace: eight of two rounds of workgroups, wide row-major arrays, act-order
+@pytest.mark.parametrize("m,k,n,group,form", [(6, 3200, 9600, 64, "plain"), (8, 7168, 4416, 128, "plain"), (3, 4096, 12288, 64, "plain"),
+                                              (4, 4096, 12288, 64, "half"), (8, 2048, 8192, 128, "act"), (5, 2560, 8704, 32, "plain")])
+def test_few_rows_without_workspace(m, k, n, group, form):
+    import torch
+    from rumus_amd import ops
+    say(f"qmatmul_int4 {m} x {k} -> {n}, groups of {group}, {form}, captured without workspace")
+    packed, scales, zp = _weight(k, n, group, 5)
+    x = _rows(m, k, 6).to(torch.float16 if form == "half" else torch.float32)
+    out = torch.empty((m, n), dtype=x.dtype, device="cuda")
+    perm = torch.randperm(k, generator=torch.Generator(device="cuda").manual_seed(7), device="cuda").to(torch.int32)
+    call = {"plain": lambda: ops.qmatmul_int4(x, packed, scales, zp, k, group, out=out),
+            "half": lambda: ops.qmatmul_int4_f16(x, packed, scales, zp, k, group, out=out),
+            "act": lambda: ops.qmatmul_int4_perm(x, packed, scales, zp, k, group, perm=perm, out=out)}[form]
+    q = torch.stack([(packed.view(torch.int32) >> (4 * i)) & 15 for i in range(8)], 1).reshape(k, n).double()
+    each = lambda t: t.double().repeat_interleave(group, 0)
+    w, rows = (q - each(zp)) * each(scales), (x[:, perm.long()] if form == "act" else x).double()
+    want, size = rows @ w, rows.abs() @ w.abs() + rows.abs().amax(1, keepdim=True) * w.abs().sum(0)
+    free_workspaces()
+    for got in _captured_in(0, call, out):
+        # test_gpu_w4_few_rows.py's bound; one rounding to f16
+        assert float(((got.double() - want).abs() / size).max()) < (2.0 ** -11 if form == "half" else 2.0 ** -20)
